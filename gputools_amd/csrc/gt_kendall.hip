@@ -11,32 +11,16 @@
 // It runs one 256-thread block per pair of variables, each re-comparing the
 // raw values of both variables n^2/2 times.
 //
-// Here the comparisons are made once per variable.  A planes pass encodes
-// each sample pair (i, j), i < j, of a variable as three bits: P (x_j > x_i),
-// N (x_j < x_i) and E (x_j == x_i); a NaN on either side clears all three.
-// A wave compares x_i with 64 consecutive x_j at once (the loads of up to 32
-// such steps issued together) and __ballot turns the comparisons into bit
-// words, which v_writelane collects across lanes for coalesced 256-byte
-// stores.  In a variable without NaN every sample pair is exactly one of P,
-// N and E, so only P and E are compared and N = ~(P | E) within the row.
-// The sample pairs of row i take
-// ceil((n - 1 - i) / 32) words (the tail bits are zero), so
-//   concordant(x, y) = sum over words of popc(Px & Py) + popc(Nx & Ny)
-//                      + popc(Ex & Ey)
-// exactly, 6 VALU operations per 32 sample pairs per pair of variables (AND
-// and v_bcnt_u32_b32, which adds the count to an accumulator), or 4 where the
-// E words of the staged chunk are all zero (ties are rare bits in continuous
-// data; a side without any tied variable does not even load them).  In a
-// tile without NaN, a chunk without E bits has exactly one of the P and N
-// bits of every sample pair set, so
-//   concordant(x, y) = sum over words of popc(~(Px ^ Py)) - (bits past row ends),
-// 2 operations per 32 sample pairs (the bits past row ends depend on the
-// layout alone: a small pass tabulates them per chunk).  The count
-// kernel tiles 128 x 128 pairs of variables over 256 lanes (8 x 8 each),
-// stages word chunks of both sides through LDS and splits the word range over
-// workgroups, adding its counts with 64-bit atomics.  A last pass applies the
-// reference's FP32 / FP64 formula to the exact count.
-//
+// Here the comparisons are made once per variable, and the counting is a
+// contraction on the matrix cores.  A planes pass writes each sample pair of a
+// variable as bits: P (x_j > x_i) always, N (x_j < x_i) and E (x_j == x_i)
+// only where a tie or a non-finite value makes them more than ~P and 0.
+// Where every sample pair of two variables is exactly one of P and N, the
+// number of agreeing pairs is (bits + sum s s') / 2 with s = +1 or -1: the
+// count pass expands the bits to FP4 values (E2M1: the sign is the bit, the
+// magnitude 1) in registers and sums the products with
+// v_mfma_f32_32x32x64_f8f6f4, exactly, as FP32 sums of integers below 2^24.
+// Elsewhere it sums the 0/1 products of the three planes, also in FP4.
 // The reference accumulates the count in FP32 (kendall.cu:14, 23, 28-38):
 // below 2^24 concordant pairs (always when n <= 5793) that sum is exact and
 // the results are identical; above it the reference's sum can round, and this
@@ -44,458 +28,493 @@
 #include "gt_common.h"
 #include "gt_internal.h"
 
-#include <type_traits>
-
 namespace gt {
 namespace {
 
-// Words of the rows with m = 1 .. M sample pairs: sum_{t=1}^{M} ceil(t / 32).
-__host__ __device__ __forceinline__ int64_t words_upto(int64_t m)
+// ---------------------------------------------------------------------------
+// Layout of the sample pairs
+// ---------------------------------------------------------------------------
+// Sample pairs (i, j) are cut into tiles of 64 rows i by 32 columns j: tile
+// (rb, jw) holds i = 64 rb + r and j = 32 jw + u, for every rb and every jw
+// from 2 rb on (j > i).  A tile is 64 words per variable, word r = row r, bit
+// u = column u.  The bits of the tile that are no sample pair (j <= i, or past
+// the end) have P = E = 0 and N = 1 for every variable, so they count as
+// agreeing everywhere and the finish pass subtracts their number.
+//
+// Variables are taken in blocks of 32 and words in groups of 8, the operand of
+// four matrix products: group g of block vb is 1 KB, 16 bytes for each of 64
+// lanes, lane 32 h + v holding words 8 q + 4 h .. + 3 of variable 32 vb + v.
+// The count pass moves groups as they are from memory to LDS to registers.
+constexpr int KVB = 32;      // variables per block
+constexpr int KGW = 8;       // words per group
+constexpr int KTG = 8;       // groups per tile of sample pairs (64 words)
+constexpr int KGWORDS = KVB * KGW;   // words of one group (256, 1 KB)
+
+// Tiles before row block rb (jwn = ceil(n / 32) column words).
+__host__ __device__ __forceinline__ int64_t tiles_before(int64_t rb, int64_t jwn)
 {
-    const int64_t q = m / 32, r = m % 32;
-    return 16 * q * (q + 1) + r * (q + 1);
+    return rb * jwn - rb * (rb - 1);
 }
 
-// v_writelane_b32 through the compiler's own intrinsic (this clang has no
-// builtin for it), so that the compiler sees the instruction and places the
-// wait states between the compare that writes the ballot's SGPRs and the
-// lane write that reads them.
-extern "C" __device__ int gt_amdgcn_writelane(int value, int lane, int old)
-    __asm("llvm.amdgcn.writelane.i32");
+__host__ __device__ __forceinline__ int64_t column_words(int64_t n) { return (n + 31) / 32; }
 
-// One plane's two words of one step (a 64-bit ballot) into lanes L and
-// L + 1 of the plane words: v_writelane_b32 with the lane select as an
-// inline constant.
-template <int L>
-__device__ __forceinline__ void put_plane(uint32_t &w, unsigned long long bits)
+__host__ __device__ __forceinline__ int64_t pair_tiles(int64_t n)
 {
-    w = (uint32_t)gt_amdgcn_writelane((int)(uint32_t)bits, L, (int)w);
-    w = (uint32_t)gt_amdgcn_writelane((int)(uint32_t)(bits >> 32), L + 1, (int)w);
-}
-
-// The three planes' words of one step.
-template <int L>
-__device__ __forceinline__ void put_step(uint32_t &wp, uint32_t &wn, uint32_t &we,
-                                         unsigned long long gt, unsigned long long lt,
-                                         unsigned long long eq)
-{
-    put_plane<L>(wp, gt);
-    put_plane<L>(wn, lt);
-    put_plane<L>(we, eq);
-}
-
-// f(std::integral_constant<int, U>) for U = 0 .. N - 1, in order.
-template <int U, int N, typename F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (U < N) {
-        f(std::integral_constant<int, U>{});
-        static_for<U + 1, N>(f);
-    }
+    return tiles_before((n - 1 + 63) / 64, column_words(n));
 }
 
 // ---------------------------------------------------------------------------
-// Planes pass: one workgroup per (variable, row split), one wave per sample i.
+// Planes pass
 // ---------------------------------------------------------------------------
-// Plane p (0 = P, 1 = N, 2 = E) of variable v, word w at
-// planes[(p * nvar + v) * wpad + w]; row i starts at word
-// words_upto(n - 1) - words_upto(n - 1 - i).  Words past the last row are
-// zero (written by this pass in P and N; the E planes are cleared before it,
-// since E words are written only where a step has a tie).  flags[v] (cleared before) gets bit 0 when
-// any sample pair of v is tied (its E plane has a set bit) and bit 1 when v
-// holds a NaN (a block-wide vote over all n values).
-template <bool LX>
-__global__ __launch_bounds__(256) void kendall_planes_kernel(const float *__restrict__ x,
-                                                             int64_t nvar, int64_t n, int64_t ldx,
-                                                             uint32_t *__restrict__ planes,
-                                                             int64_t wpad,
-                                                             uint32_t *__restrict__ ties,
-                                                             int rsplit)
+struct PlanesArgs {
+    const float *x;
+    int64_t nvar, n, ldx;
+    uint32_t *planes;    // plane p (0 = P, 1 = N, 2 = E), block vb, group g at
+                         // ((p * nvb + vb) * ngroups + g) * KGWORDS
+    uint8_t *flags;      // flags[g * fstride + vb]: the group's N and E words are stored
+    int64_t nvb, fstride, ngroups;
+    int64_t tile_begin, ntiles;   // this segment's tiles of sample pairs
+    int64_t runs;
+};
+
+constexpr int KRUN = 4;      // tiles per workgroup
+
+// x read through the scalar cache: uniform addresses, not written by the kernel
+typedef const __attribute__((address_space(4))) float uniform_float_t;
+
+// One workgroup per (variable block, run of tiles); a wave takes 8 variables,
+// a lane one row i.  The bit of (i, j) is the sign of x_i - x_j, shifted into
+// the lane's word by v_alignbit_b32: a subtract and a shift per 64 sample
+// pairs, plus half a v_min3_u32 that notices a zero difference.  x_i has its
+// zero made +0, so that equal values always give the difference +0.  x_j is
+// uniform and comes through scalar loads.  This took 1024 variables x 2048
+// samples from 0.52 ms (a ballot per 64 pairs, moved between lanes) to
+// 0.23 ms.  Bound: VALU issue (1.2e8 wave instructions, 108 per word of 64
+// lanes: 80 in the column loop, the rest masks, tests and the LDS transpose).
+// A word with a zero difference or a non-finite value is redone with the
+// three comparisons; if it holds a tie (or a NaN may be about), its group is
+// flagged and the N and E words of the whole group are stored.
+__global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
 {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t wtot = words_upto(n - 1);
-    const float qnan = __builtin_nanf("");
-    const int64_t pstride = nvar * wpad;
-    // workgroup (variable v, split rs); its waves take rows
-    // i = 4 rs + wave + 4 rsplit k, a mix of long and short rows
-    const int64_t v = blockIdx.x / rsplit;
-    const int rs = (int)(blockIdx.x % rsplit);
-    const float *xv = x + v * ldx;
-    uint32_t *const pv = planes + v * wpad;
-    // Does the variable hold a NaN?  Without one, every sample pair in a row
-    // is exactly one of P, N and E, so the N word is ~(P | E) within the row
-    // and needs no compare of its own; the E words need lane writes only in
-    // steps with a tie.  That takes a step from 3 compares and 6 lane writes
-    // to 2 and 2.
-    // LX: the variable's n values are staged in LDS (the same pass), followed
-    // by 2048 NaNs, and the rows read them from there instead of through the
-    // vector memory path.  A group reads all 32 steps, up to x_j with
-    // j = n - 1 + 63 + 31 * 64, so the NaN tail stands in for the bounds and
-    // step tests (a NaN compares false).
-    extern __shared__ float xs[];
-    bool nan_here = false;
-    for (int64_t t = threadIdx.x; t < n; t += blockDim.x) {
-        const float val = xv[t];
-        nan_here = nan_here || val != val;
-        if (LX) xs[t] = val;
+    // a tile's P words, padded so that the 16 four-word pieces of a wave's
+    // store fall in different banks
+    constexpr int HS = 132, QS = 264;
+    __shared__ __attribute__((aligned(16))) uint32_t buf[2][KTG * QS];
+    __shared__ unsigned special[3];   // per tile: groups whose N and E words are needed
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t n = args.n, jwn = column_words(n);
+    const int64_t vb = blockIdx.x / args.runs, run = blockIdx.x % args.runs;
+    const int64_t tb = run * KRUN;
+    const int nt = (int)(args.ntiles - tb < KRUN ? args.ntiles - tb : KRUN);
+    const int64_t t0 = args.tile_begin + tb;
+    // row block of tile t0: the last rb with tiles_before(rb) <= t0
+    int64_t rb;
+    {
+        const double b = (double)(jwn + 1);
+        rb = (int64_t)((b - sqrt(fmax(b * b - 4.0 * (double)t0, 0.0))) * 0.5);
+        while (rb > 0 && tiles_before(rb, jwn) > t0) --rb;
+        while (tiles_before(rb + 1, jwn) <= t0) ++rb;
     }
-    if (LX)
-        for (int t = threadIdx.x; t < 2048; t += blockDim.x) xs[n + t] = qnan;
-    const bool has_nan = __syncthreads_or(nan_here) != 0;   // (and the LDS copy is complete)
-    // P and N are written in full, up to wpad: split 0 zeroes the words after
-    // the last row (fewer than KKW); the E planes are cleared before this pass
-    if (rs == 0 && threadIdx.x < wpad - wtot) {
-        pv[wtot + threadIdx.x] = 0u;
-        pv[pstride + wtot + threadIdx.x] = 0u;
-    }
-    bool tied = false;
-    for (int64_t i = 4 * rs + wave; i < n - 1; i += 4 * (int64_t)rsplit) {
-        const int64_t m = n - 1 - i;
-        const float xi = LX ? xs[i] : xv[i];
-        const float *xr = xv + i + 1;                    // x_j, j = i + 1 + q
-        uint32_t *const row = pv + (wtot - words_upto(m));
-        const int64_t wr = (m + 31) / 32;
-        const int64_t steps = (m + 63) / 64;
-        // groups of 32 steps: lanes 2u and 2u + 1 collect the words of step
-        // u (a compile-time lane, so each word is one v_writelane), and the
-        // group's 64 words per plane go out in one store per plane
-        for (int64_t g0 = 0; g0 < steps; g0 += 32) {
-            int nst = (int)((steps - g0) < 32 ? (steps - g0) : 32);
-            // a 32-bit scalar: the step tests below stay scalar compares
-            // (the compiler otherwise tests the 64-bit value on the VALU)
-            asm("" : "+s"(nst));
-            float xj[32];
-            // every xj[u] a register of its own (compile-time u): a loop with
-            // a run-time exit would index xj dynamically and wait on each load
-            if (LX) {
-                // n <= 8192: 32-bit offsets; step u is an immediate offset
-                const float *xl = xs + (int)(i + 1 + g0 * 64) + lane;
-                static_for<0, 32>([&](auto uc) {
-                    constexpr int u = decltype(uc)::value;
-                    xj[u] = xl[u * 64];
-                });
-            } else {
-                static_for<0, 32>([&](auto uc) {
-                    constexpr int u = decltype(uc)::value;
-                    if (u < nst) {
-                        const int64_t q = (g0 + u) * 64 + lane;
-                        xj[u] = q < m ? xr[q] : qnan;
-                    }
-                });
-            }
-            uint32_t wp = 0, wn = 0, we = 0;
-            bool group_tied = false;
-            const int64_t w = 2 * g0 + lane;
-            if (has_nan) {
-                static_for<0, 32>([&](auto uc) {
-                    constexpr int u = decltype(uc)::value;
-                    if (u < nst) {
-                        const unsigned long long gt = __builtin_amdgcn_ballot_w64(xj[u] > xi);
-                        const unsigned long long lt = __builtin_amdgcn_ballot_w64(xj[u] < xi);
-                        const unsigned long long eq = __builtin_amdgcn_ballot_w64(xj[u] == xi);
-                        put_step<2 * u>(wp, wn, we, gt, lt, eq);
-                        group_tied = group_tied || eq != 0ull;
-                    }
-                });
-            } else {
-                static_for<0, 32>([&](auto uc) {
-                    constexpr int u = decltype(uc)::value;
-                    if (u < nst) {
-                        const unsigned long long gt = __builtin_amdgcn_ballot_w64(xj[u] > xi);
-                        const unsigned long long eq = __builtin_amdgcn_ballot_w64(xj[u] == xi);
-                        put_plane<2 * u>(wp, gt);
-                        if (eq != 0ull) {
-                            put_plane<2 * u>(we, eq);
-                            group_tied = true;
-                        }
-                    }
-                });
-                // the sample pairs of word w are q = 32 w .. 32 w + 31 < m
-                const int64_t rem = m - 32 * w;
-                const uint32_t valid = rem >= 32 ? 0xffffffffu : rem > 0 ? (1u << rem) - 1u : 0u;
-                wn = ~(wp | we) & valid;
-            }
-            // lanes at or past `used` hold no word of this group; w < wr
-            // drops the odd last word of the row (it belongs to the next row)
-            const int used = 2 * nst;
-            if (lane < used && w < wr) {
-                row[w] = wp;
-                row[pstride + w] = wn;
-                // E words that are zero stay as cleared
-                if (group_tied) row[2 * pstride + w] = we;
-            }
-            tied = tied || group_tied;
+    int64_t jw = 2 * rb + (t0 - tiles_before(rb, jwn));
+    const int64_t v0 = vb * KVB + wave * 8;
+    const float *const x = args.x;
+    const int64_t pstride = args.nvb * args.ngroups * KGWORDS;
+    uint32_t *const pv = args.planes + vb * args.ngroups * KGWORDS;
+    const int slot = (lane >> 3) * QS + ((lane >> 2) & 1) * HS + (lane & 3);
+
+    float xi[8];
+    auto load_rows = [&]() {
+        int64_t i = rb * 64 + lane;
+        if (i > n - 1) i = n - 1;
+#pragma unroll
+        for (int vv = 0; vv < 8; ++vv) {
+            const int64_t v = v0 + vv < args.nvar ? v0 + vv : args.nvar - 1;
+            xi[vv] = x[v * args.ldx + i] + 0.0f;
         }
-    }
-    const uint32_t bits = (tied ? 1u : 0u) | (has_nan ? 2u : 0u);
-    if (lane == 0 && bits) atomicOr(ties + v, bits);
-}
-
-// ---------------------------------------------------------------------------
-// Count pass: popcount tiles.
-// ---------------------------------------------------------------------------
-constexpr int KBM = 128;                 // variables per tile side
-constexpr int KKW = 8;                   // words per LDS chunk (256 sample pairs)
-constexpr int KTHREADS = 256;            // 16 x 16 lanes, 8 x 8 pairs each
-constexpr int KUNITS = 2 * 3 * KBM * 2 / KTHREADS;  // 16-byte staging units per lane
-
-// Bits past row ends per chunk of KKW words, from the layout alone: the last
-// word of row i (m = n - 1 - i sample pairs) holds m % 32 of them when that is
-// not 0, and the words after the last row (up to wpad) are past the end
-// entirely.  pe (cleared before) gets one count per chunk.
-__global__ __launch_bounds__(256) void kendall_pastend_kernel(int64_t n, int64_t wpad,
-                                                              uint32_t *__restrict__ pe)
-{
-    const int64_t wtot = words_upto(n - 1);
-    const int64_t rows = n - 1, tail = wpad - wtot;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < rows + tail;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        if (t < rows) {
-            const int64_t m = n - 1 - t;
-            if (m % 32 != 0) {
-                const int64_t last = wtot - words_upto(m) + (m + 31) / 32 - 1;
-                atomicAdd(pe + last / KKW, 32u - (uint32_t)(m % 32));
+    };
+    // the three comparisons of 32 columns, column u in bit u; the columns from
+    // cols on repeat the last one
+    auto exact = [&](float a, uniform_float_t *xj, int cols, uint32_t &gt, uint32_t &lt, uint32_t &eq) {
+        gt = lt = eq = 0u;
+#pragma unroll 8
+        for (int u = 31; u >= 0; --u) {
+            const float b = xj[u < cols ? u : cols - 1];
+            gt = (gt << 1) | (b > a ? 1u : 0u);
+            lt = (lt << 1) | (b < a ? 1u : 0u);
+            eq = (eq << 1) | (b == a ? 1u : 0u);
+        }
+    };
+    load_rows();
+    if (tid == 0) special[0] = 0u;
+    __syncthreads();
+    for (int k = 0; k < nt; ++k) {
+        if (tid == 0) special[(k + 1) % 3] = 0u;   // last read two tiles ago
+        const int64_t j0 = jw * 32;
+        const int cols = n - j0 < 32 ? (int)(n - j0) : 32;
+        // bits of the columns i < j < n
+        const int lo = (int)(rb * 64 - j0) + lane + 1;   // -n .. 64
+        uint32_t valid = cols >= 32 ? 0xffffffffu : (1u << cols) - 1u;
+        if (lo > 0) valid &= lo >= 32 ? 0u : 0xffffffffu << lo;
+        unsigned sp = 0;
+        uint32_t *const pb = buf[k & 1] + slot + wave * 8 * 4;
+#pragma unroll
+        for (int vv = 0; vv < 8; ++vv) {
+            const int64_t v = v0 + vv < args.nvar ? v0 + vv : args.nvar - 1;
+            const float *xv = x + v * args.ldx + j0;
+            uniform_float_t *xj = (uniform_float_t *)xv;
+            const float xl = xv[(lane & 31) < cols ? lane & 31 : cols - 1];
+            uint32_t w = 0u, m = 0xffffffffu;
+            if (cols == 32) {
+#pragma unroll
+                for (int u = 31; u >= 0; --u) {
+                    const uint32_t d = __float_as_uint(xi[vv] - xj[u]);
+                    w = __builtin_amdgcn_alignbit(w, d, 31);
+                    m = d < m ? d : m;
+                }
+            } else {
+                m = 0u;
             }
-        } else {
-            atomicAdd(pe + (wtot + (t - rows)) / KKW, 32u);
+            const bool odd = !(fabsf(xi[vv]) < INFINITY) || !(fabsf(xl) < INFINITY);
+            const unsigned long long oddw = __builtin_amdgcn_ballot_w64(odd);
+            if (__builtin_amdgcn_ballot_w64(m == 0u) | oddw) {
+                uint32_t lt, eq;
+                exact(xi[vv], xj, cols, w, lt, eq);
+                const unsigned long long tied = __builtin_amdgcn_ballot_w64((eq & valid) != 0u);
+                if (oddw) {
+                    sp = 0xffu;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < KTG; ++q)
+                        if ((tied >> (8 * q)) & 0xffull) sp |= 1u << q;
+                }
+            }
+            pb[vv * 4] = w & valid;
+        }
+        if (sp != 0u && lane == 0) atomicOr(&special[k % 3], sp);
+        __syncthreads();
+        const int64_t g = (tb + k) * KTG;
+        uint32_t *const pt = pv + g * KGWORDS;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int unit = tid + 256 * h, q = unit >> 6, l = unit & 63;
+            *reinterpret_cast<uint4 *>(pt + unit * 4) =
+                *reinterpret_cast<const uint4 *>(buf[k & 1] + q * QS + (l >> 5) * HS + (l & 31) * 4);
+        }
+        const unsigned mask = special[k % 3];
+        if (tid < KTG) args.flags[(g + tid) * args.fstride + vb] = (uint8_t)((mask >> tid) & 1u);
+        if (mask != 0u) {
+            const int q = lane >> 3;
+            uint32_t *const po = pt + q * KGWORDS + ((lane >> 2) & 1) * 128 + (lane & 3);
+            for (int vv = 0; vv < 8; ++vv) {
+                const int64_t v = v0 + vv < args.nvar ? v0 + vv : args.nvar - 1;
+                uint32_t gt, lt, eq;
+                exact(xi[vv], (uniform_float_t *)(x + v * args.ldx + j0), cols, gt, lt, eq);
+                if ((mask >> q) & 1u) {
+                    po[pstride + (wave * 8 + vv) * 4] = (lt & valid) | ~valid;
+                    po[2 * pstride + (wave * 8 + vv) * 4] = eq & valid;
+                }
+            }
+        }
+        if (++jw == jwn && k + 1 < nt) {
+            ++rb;
+            jw = 2 * rb;
+            load_rows();
         }
     }
 }
+
+// ---------------------------------------------------------------------------
+// Count pass
+// ---------------------------------------------------------------------------
+constexpr int KBX = 256, KBY = 128;      // variables per tile side
+constexpr int KTX = KBX / KVB, KTY = KBY / KVB;   // blocks per tile side
+constexpr int KTHREADS = 256;            // 4 waves, 2 (x) x 2 (y), 128 x 64 pairs each
+constexpr int KSTAGE = (KTX + KTY) * KGWORDS * 4;   // bytes of one group of both sides (12 KB)
+constexpr int KNSTAGE = 4;
+// FP32 sums of +-2 per bit stay exact below 2^24: 32768 groups of 256 bits
+constexpr int64_t KMAXGROUPS = 32000;
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+typedef float kf32x16_t __attribute__((ext_vector_type(16)));
 
 struct KendallArgs {
-    const uint32_t *pa, *pb;   // planes of A (na variables) and B (nb variables)
-    int64_t na, nb, wpad;
+    const uint32_t *pa, *pb;   // planes of A and B (PlanesArgs)
+    const uint8_t *fa, *fb;
+    int64_t nvb_a, nvb_b, fs_a, fs_b, ngroups;
+    int64_t na, nb;
     unsigned long long *count; // na x nb (row stride ldc), pair (x, y) at x * ldc + y
     int64_t ldc;
-    int64_t tiles_a, tiles_b, ntiles;
-    int64_t split_w;           // words per workgroup (multiple of KKW)
-    const uint32_t *pe;        // per chunk of KKW words: bits past row ends
-    const uint32_t *ties_a, *ties_b;   // per variable: bit 0 a tie (E bit set), bit 1 a NaN
+    int64_t tiles_b, ntiles;
+    int64_t split_g;           // groups per workgroup
     int64_t id_offset, ids_this;
 };
 
-// Accumulate one staged chunk into the 8 x 8 counts of this lane: per plane
-// and pair one AND and one v_bcnt_u32_b32 (popcount plus accumulator); the
-// empty asm keeps the compiler from regrouping the sums into an extra v_add3.
-template <int NP>
-__device__ __forceinline__ void count_chunk(const uint32_t (&lds)[2][3][KKW][KBM], int tx, int ty,
-                                            uint32_t (&cnt)[8][8])
+// 32 bits -> 32 FP4 values: nibble t of dword s is bit 4 t + s of w, placed at
+// mask's bit of the nibble, over the other bits of one.  Signs: mask 8, one 2
+// (+1 where the bit is clear, -1 where it is set).  0 / 1: w rotated right by
+// 2, mask 2; 0 / 2: w rotated right by 1, mask 4; one 0.
+__device__ __forceinline__ i32x8_t expand(uint32_t w, uint32_t mask, uint32_t one)
 {
-#pragma unroll 2
-    for (int kw = 0; kw < KKW; ++kw) {
-        uint32_t xa[NP][8], yb[NP][8];
+    i32x8_t r = {};
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const uint4 a0 = *reinterpret_cast<const uint4 *>(&lds[0][p][kw][ty * 4]);
-            const uint4 a1 = *reinterpret_cast<const uint4 *>(&lds[0][p][kw][64 + ty * 4]);
-            const uint4 b0 = *reinterpret_cast<const uint4 *>(&lds[1][p][kw][tx * 4]);
-            const uint4 b1 = *reinterpret_cast<const uint4 *>(&lds[1][p][kw][64 + tx * 4]);
-            xa[p][0] = a0.x; xa[p][1] = a0.y; xa[p][2] = a0.z; xa[p][3] = a0.w;
-            xa[p][4] = a1.x; xa[p][5] = a1.y; xa[p][6] = a1.z; xa[p][7] = a1.w;
-            yb[p][0] = b0.x; yb[p][1] = b0.y; yb[p][2] = b0.z; yb[p][3] = b0.w;
-            yb[p][4] = b1.x; yb[p][5] = b1.y; yb[p][6] = b1.z; yb[p][7] = b1.w;
-        }
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                uint32_t s = cnt[r][c];
-#pragma unroll
-                for (int p = 0; p < NP; ++p) {
-                    s += __builtin_popcount(xa[p][r] & yb[p][c]);
-                    asm("" : "+v"(s));
-                }
-                cnt[r][c] = s;
-            }
-    }
+    for (int s = 0; s < 4; ++s)
+        r[s] = (int)(((s < 3 ? __builtin_rotateleft32(w, 3 - s) : w) & mask) | one);
+    return r;
 }
 
-// Chunks without E bits in tiles without NaN: every sample pair has exactly
-// one of its P and N bits, so the pair is concordant where the P bits agree:
-// one XNOR and one v_bcnt_u32_b32 per word and pair.  The bits past the end
-// of a row agree too (all zero); the caller subtracts them per chunk.
-__device__ __forceinline__ void count_chunk_xnor(const uint32_t (&lds)[2][3][KKW][KBM], int tx,
-                                                 int ty, uint32_t (&cnt)[8][8])
+// Four blocks of side A and two of side B, 16 bytes a lane, loaded and waited
+// for here: as ordinary loads in the loop they would make the compiler wait
+// for every load in flight, the ring's among them, in groups that do not take
+// this path (634 against 612 us for the whole pass).
+__device__ __forceinline__ void load_six(const uint32_t *a, const int64_t (&sa)[4], const uint32_t *b,
+                                         const int64_t (&sb)[2], u32x4_t (&w)[6])
 {
-    // fully unrolled: a rolled loop here is a loop of its own, and the
-    // compiler then copies the 64 counts into and out of its registers on
-    // every chunk
-#pragma unroll
-    for (int kw = 0; kw < KKW; ++kw) {
-        const uint4 a0 = *reinterpret_cast<const uint4 *>(&lds[0][0][kw][ty * 4]);
-        const uint4 a1 = *reinterpret_cast<const uint4 *>(&lds[0][0][kw][64 + ty * 4]);
-        const uint4 b0 = *reinterpret_cast<const uint4 *>(&lds[1][0][kw][tx * 4]);
-        const uint4 b1 = *reinterpret_cast<const uint4 *>(&lds[1][0][kw][64 + tx * 4]);
-        const uint32_t xa[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-        const uint32_t yb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                uint32_t s = cnt[r][c];
-                s += __builtin_popcount(~(xa[r] ^ yb[c]));
-                asm("" : "+v"(s));
-                cnt[r][c] = s;
-            }
-    }
+    const uint32_t *a0 = a + sa[0], *a1 = a + sa[1], *a2 = a + sa[2], *a3 = a + sa[3];
+    const uint32_t *b0 = b + sb[0], *b1 = b + sb[1];
+    asm volatile("global_load_dwordx4 %0, %6, off\n\t"
+                 "global_load_dwordx4 %1, %7, off\n\t"
+                 "global_load_dwordx4 %2, %8, off\n\t"
+                 "global_load_dwordx4 %3, %9, off\n\t"
+                 "global_load_dwordx4 %4, %10, off\n\t"
+                 "global_load_dwordx4 %5, %11, off\n\t"
+                 "s_waitcnt vmcnt(0)"
+                 : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5])
+                 : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b0), "v"(b1)
+                 : "memory");
 }
 
-// SYM: pa == pb; tiles with J <= I only (the finish pass reads the other half
-// from the transposed position).
+__device__ __forceinline__ kf32x16_t mfma_fp4(i32x8_t a, i32x8_t b, kf32x16_t c)
+{
+    // format 4 = E2M1 on both sides, block scales 2^0
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 4, 4, 0, 127, 0, 127);
+}
+
+// A 256 x 128 tile of pairs of variables over a range of groups.  Both sides'
+// groups stream from memory through a four-stage LDS ring (direct loads); a
+// wave expands its 4 + 2 blocks in registers, 7 VALU instructions per operand
+// of two (A) or four (B) products, which leaves the matrix cores the longer
+// side (256 against 168 cycles per 64 sample pairs and wave).  The popcount
+// form this replaces spent 2 VALU operations per 32 sample pairs and pair.
+// 1024 variables x 2048 samples, self case: 3.18 -> 0.61 ms, 4.6 PFLOP/s.
+// Bound: the matrix cores at the clock they hold on such data; a register-only
+// loop of the same products and expansions takes 0.51 - 0.61 ms (constant
+// operands would run at 7.5 PFLOP/s, 0.38 ms).  256 x 256 tiles of 8 waves, one
+// workgroup per CU, took 0.72 ms.
+// SYM: pa == pb; tiles with J <= I only, and only x >= y is stored.
 template <bool SYM>
-__global__ __launch_bounds__(KTHREADS) void kendall_count_kernel(KendallArgs args)
+__global__ __launch_bounds__(KTHREADS, 2) void kendall_count_kernel(KendallArgs args)
 {
-    __shared__ uint32_t lds[2][3][KKW][KBM];   // [side][plane][word][variable]
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;    // y = tx*4 + {0..3, 64..67}, x likewise with ty
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[KNSTAGE * KSTAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wx = wave >> 1, wy = wave & 1;
     const int64_t id = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
     const int64_t split = id / args.ntiles, t = id % args.ntiles;
     int64_t I, J;
     if (SYM) {
-        int ti, tj;
-        tri_tile(t, ti, tj);
-        I = ti;
-        J = tj;
+        // tile row I has 2 (I + 1) tiles
+        I = (int64_t)((sqrt(4.0 * (double)t + 1.0) - 1.0) * 0.5);
+        while ((I + 1) * (I + 2) <= t) ++I;
+        while (I * (I + 1) > t) --I;
+        J = t - I * (I + 1);
     } else {
         I = t / args.tiles_b;
         J = t % args.tiles_b;
     }
-    const int64_t x0 = I * KBM, y0 = J * KBM;
-    const int64_t w_begin = split * args.split_w;
-    int64_t w_end = w_begin + args.split_w;
-    if (w_end > args.wpad) w_end = args.wpad;
-    if (w_begin >= w_end) return;
+    const int64_t x0 = I * KBX, y0 = J * KBY;
+    const int64_t g0 = split * args.split_g;
+    int64_t g1 = g0 + args.split_g;
+    if (g1 > args.ngroups) g1 = args.ngroups;
+    if (g0 >= g1) return;
+    const int ng = (int)(g1 - g0);
+    // a wave with no pair x >= y only helps to load
+    const bool idle = SYM && y0 + wy * 64 > x0 + wx * 128 + 127;
 
-    // Flags of the tile's variables (A in lanes 0..127, B in 128..255).  The
-    // E planes only matter when a variable on each side has a tie; for
-    // tie-free tiles (continuous data) they are all zero and are skipped:
-    // two planes, 4 instead of 6 operations per word.  A tile with no tie and
-    // no NaN at all takes the XOR form below.
-    uint32_t f = 0;
-    if (tid < KBM) {
-        const int64_t v = x0 + tid;
-        f = v < args.na ? args.ties_a[v] : 0u;
-    } else {
-        const int64_t v = y0 + (tid - KBM);
-        f = v < args.nb ? args.ties_b[v] : 0u;
-    }
-    const bool tie_x = __syncthreads_or(tid < KBM && (f & 1u)) != 0;
-    const bool tie_y = __syncthreads_or(tid >= KBM && (f & 1u)) != 0;
-    const bool use_e = tie_x && tie_y;
-    // any NaN in the tile: the XNOR form below is not used
-    const bool nan_tile = __syncthreads_or((f & 2u) != 0u) != 0;
-
-    // staging unit u = tid + 256 q: half u & 1 (words 4 half .. +3 of the
-    // chunk), variable (u >> 1) & 127, side/plane u >> 8 (side = sp / 3)
-    const uint32_t *src[KUNITS];
-    bool ok[KUNITS], inr[KUNITS];
+    // wave w loads blocks 3 w .. 3 w + 2 of the 8 + 4; blocks past a side's last
+    // one repeat it (they only feed pairs that are not stored)
+    typedef __attribute__((address_space(3))) void lds_void_t;
+    typedef const __attribute__((address_space(1))) void gbl_void_t;
+    const uint32_t *src[3];
 #pragma unroll
-    for (int q = 0; q < KUNITS; ++q) {
-        const int u = tid + KTHREADS * q;
-        const int sp = u >> 8, v = (u >> 1) & (KBM - 1), half = u & 1;
-        const int side = sp / 3, plane = sp % 3;
-        const int64_t nside = side ? args.nb : args.na;
-        const int64_t gv = (side ? y0 : x0) + v;
-        // E words are loaded for a side with a tied variable: E & E needs
-        // both sides, the XNOR form's check needs either.  N words are loaded
-        // ahead only in a tile with a NaN; other chunks that need them load
-        // them when their E bits show up.
-        inr[q] = gv < nside;
-        ok[q] = inr[q] && (plane == 0 || (plane == 1 && nan_tile) ||
-                           (plane == 2 && (side ? tie_y : tie_x)));
-        src[q] = (side ? args.pb : args.pa) + ((int64_t)plane * nside + (inr[q] ? gv : 0)) * args.wpad +
-                 half * 4;
+    for (int q = 0; q < 3; ++q) {
+        const int blk = wave * 3 + q;
+        const bool sb = blk >= KTX;
+        const int64_t nvb = sb ? args.nvb_b : args.nvb_a;
+        int64_t v = sb ? J * KTY + blk - KTX : I * KTX + blk;
+        if (v >= nvb) v = nvb - 1;
+        src[q] = (sb ? args.pb : args.pa) + (v * args.ngroups + g0) * KGWORDS + lane * 4;
     }
-    uint4 stage[KUNITS];
-    auto gload = [&](int64_t w) {
+    auto issue = [&](int c) {
+        unsigned char *const st = smem + (c % KNSTAGE) * KSTAGE + wave * 3 * (KGWORDS * 4);
 #pragma unroll
-        for (int q = 0; q < KUNITS; ++q)
-            stage[q] = ok[q] ? *reinterpret_cast<const uint4 *>(src[q] + w) : make_uint4(0, 0, 0, 0);
+        for (int q = 0; q < 3; ++q)
+            __builtin_amdgcn_global_load_lds((gbl_void_t *)(src[q] + (int64_t)c * KGWORDS),
+                                             (lds_void_t *)(st + q * KGWORDS * 4), 16, 0, 0);
+    };
+    // which of the next 64 groups hold N and E words for a block of this wave
+    const int64_t la = args.nvb_a - (I * KTX + wx * 4), lb = args.nvb_b - (J * KTY + wy * 2);
+    const uint32_t ma = la >= 4 ? 0xffffffffu : la > 0 ? (1u << (8 * (int)la)) - 1u : 0u;
+    const uint32_t mb = lb >= 2 ? 0xffffu : lb > 0 ? 0xffu : 0u;
+    const uint8_t *const fa = args.fa + I * KTX + wx * 4, *const fb = args.fb + J * KTY + wy * 2;
+    auto flags_of = [&](int c, uint32_t &ua, uint32_t &ub) {
+        ua = *reinterpret_cast<const uint32_t *>(fa + (g0 + c) * args.fs_a) & ma;
+        ub = *reinterpret_cast<const uint16_t *>(fb + (g0 + c) * args.fs_b) & mb;
     };
 
-    uint32_t cnt[8][8];
+    // this wave's blocks in the N and E planes of group g0 (blocks past the end
+    // repeat the last one)
+    int64_t step_a[4], step_b[2];
 #pragma unroll
-    for (int r = 0; r < 8; ++r)
+    for (int a = 0; a < 4; ++a)
+        step_a[a] = (a < la ? a : la > 0 ? la - 1 : args.nvb_a - 1 - (I * KTX + wx * 4)) *
+                    args.ngroups * KGWORDS;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) cnt[r][c] = 0;
+    for (int b = 0; b < 2; ++b)
+        step_b[b] = (b < lb ? b : lb > 0 ? lb - 1 : args.nvb_b - 1 - (J * KTY + wy * 2)) *
+                    args.ngroups * KGWORDS;
+    const int64_t pstride_a = args.nvb_a * args.ngroups * KGWORDS;
+    const int64_t pstride_b = args.nvb_b * args.ngroups * KGWORDS;
+    const uint32_t *const pside_a =
+        args.pa + ((I * KTX + wx * 4) * args.ngroups + g0) * KGWORDS + lane * 4;
+    const uint32_t *const pside_b =
+        args.pb + ((J * KTY + wy * 2) * args.ngroups + g0) * KGWORDS + lane * 4;
 
-    uint32_t past_end = 0;   // XNOR chunks: bits past row ends, counted for every pair
-    gload(w_begin);
-    for (int64_t w = w_begin; w < w_end; w += KKW) {
-        __syncthreads();
+    kf32x16_t acc[4][2];
 #pragma unroll
-        for (int q = 0; q < KUNITS; ++q) {
-            const int u = tid + KTHREADS * q;
-            const int sp = u >> 8, v = (u >> 1) & (KBM - 1), half = u & 1;
-            uint32_t *d = &lds[sp / 3][sp % 3][half * 4][v];
-            d[0 * KBM] = stage[q].x;
-            d[1 * KBM] = stage[q].y;
-            d[2 * KBM] = stage[q].z;
-            d[3 * KBM] = stage[q].w;
-        }
-        // units 2 and 5 of every lane are the E words of the two sides: a
-        // chunk where none is set (ties are rare bits) counts two planes
-        const uint4 e0 = stage[2], e1 = stage[5];
-        const bool e_here = (e0.x | e0.y | e0.z | e0.w | e1.x | e1.y | e1.z | e1.w) != 0u;
-        const bool any_e = __syncthreads_or(e_here) != 0;
-        if (any_e && !nan_tile) {
-            // this chunk counts P and N: load its N words (units 1 and 4)
-            uint4 sn[2];
+    for (int a = 0; a < 4; ++a)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int q = 1 + 3 * h;
-                sn[h] = inr[q] ? *reinterpret_cast<const uint4 *>(src[q] + w) : make_uint4(0, 0, 0, 0);
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
+
+    int nfast = 0;
+    unsigned long long slow = 0;
+#pragma unroll
+    for (int c = 0; c < KNSTAGE - 1; ++c)
+        if (c < ng) issue(c);
+    for (int c = 0; c < ng; ++c) {
+        if ((c & 63) == 0) {
+            bool f = false;
+            if (c + lane < ng) {
+                uint32_t ua, ub;
+                flags_of(c + lane, ua, ub);
+                f = (ua | ub) != 0u;
             }
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int u = tid + KTHREADS * (1 + 3 * h);
-                const int sp = u >> 8, v = (u >> 1) & (KBM - 1), half = u & 1;
-                uint32_t *d = &lds[sp / 3][sp % 3][half * 4][v];
-                d[0 * KBM] = sn[h].x;
-                d[1 * KBM] = sn[h].y;
-                d[2 * KBM] = sn[h].z;
-                d[3 * KBM] = sn[h].w;
-            }
-            __syncthreads();
+            slow = __builtin_amdgcn_ballot_w64(f);
         }
-        if (w + KKW < w_end) gload(w + KKW);
-        if (!any_e && !nan_tile) {
-            // the chunk's bits past row ends (the same for every variable)
-            past_end += args.pe[w / KKW];
-            count_chunk_xnor(lds, tx, ty, cnt);
-        } else if (any_e && use_e) {
-            count_chunk<3>(lds, tx, ty, cnt);
+        // group c landed when at most the two later groups' loads are
+        // outstanding (vector memory loads complete in order)
+        if (c + 2 < ng)
+            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        else if (c + 1 < ng)
+            asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // every wave's part of group c is in LDS, and every wave is done with
+        // group c - 1, whose stage the next issue overwrites
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (c + KNSTAGE - 1 < ng) issue(c + KNSTAGE - 1);
+        if (idle) continue;
+        const unsigned char *const st = smem + (c % KNSTAGE) * KSTAGE + lane * 16;
+        const bool flagged = ((slow >> (c & 63)) & 1ull) != 0ull;
+        uint32_t ua = 0, ub = 0, mask_a = 0x88888888u, mask_b = 0x88888888u, one = 0x22222222u;
+        if (flagged) {
+            // P P' + N N' + E E', twice: 0/1 on one side, 0/2 on the other
+            flags_of(c, ua, ub);
+            ua = __builtin_amdgcn_readfirstlane(ua);
+            ub = __builtin_amdgcn_readfirstlane(ub);
+            mask_a = 0x22222222u;
+            mask_b = 0x44444444u;
+            one = 0u;
         } else {
-            count_chunk<2>(lds, tx, ty, cnt);
+            ++nfast;
+        }
+        // one in a VGPR: v_and_or_b32 takes the mask as its only scalar
+        asm("" : "+v"(one));
+#pragma unroll 1
+        for (int p = 0; p < (flagged ? 3 : 1); ++p) {
+            u32x4_t pa[4], pb[2];
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                pa[a] = *reinterpret_cast<const u32x4_t *>(st + (wx * 4 + a) * (KGWORDS * 4));
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                pb[b] = *reinterpret_cast<const u32x4_t *>(st + (KTX + wy * 2 + b) * (KGWORDS * 4));
+            if (flagged) {
+                // the stored N or E words; a block whose group is not flagged
+                // has N = ~P and E = 0
+                if (p > 0) {
+                    u32x4_t w[6];
+                    load_six(pside_a + p * pstride_a + (int64_t)c * KGWORDS, step_a,
+                             pside_b + p * pstride_b + (int64_t)c * KGWORDS, step_b, w);
+#pragma unroll
+                    for (int a = 0; a < 4; ++a)
+                        pa[a] = ((ua >> (8 * a)) & 0xffu) ? w[a] : p == 1 ? ~pa[a] : (u32x4_t)0u;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        pb[b] = ((ub >> (8 * b)) & 0xffu) ? w[4 + b] : p == 1 ? ~pb[b] : (u32x4_t)0u;
+                }
+#pragma unroll
+                for (int a = 0; a < 4; ++a) pa[a] = (pa[a] >> 2) | (pa[a] << 30);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) pb[b] = (pb[b] >> 1) | (pb[b] << 31);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                i32x8_t vb[2];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) vb[b] = expand(pb[b][k], mask_b, one);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const i32x8_t va = expand(pa[a][k], mask_a, one);
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) acc[a][b] = mfma_fp4(va, vb[b], acc[a][b]);
+                }
+                // keeps the expansions of later steps, and their registers,
+                // behind this step's products
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
+    if (idle) return;
 
+    // acc = 2 agreeing - bits over the +-1 groups, 2 agreeing over the others.
+    // 32 x 32 accumulator layout: element r of lane l is x row 8 (r / 4) +
+    // 4 (l / 32) + r % 4 and y column l % 32.
+    const int bits = nfast * (KGW * 32);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const int64_t x = x0 + (r < 4 ? ty * 4 + r : 64 + ty * 4 + (r - 4));
-        if (x >= args.na) continue;
+    for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const int64_t y = y0 + (c < 4 ? tx * 4 + c : 64 + tx * 4 + (c - 4));
-            if (y >= args.nb) continue;
-            atomicAdd(args.count + x * args.ldc + y, (unsigned long long)(cnt[r][c] - past_end));
+        for (int r = 0; r < 16; ++r) {
+            const int64_t x = x0 + wx * 128 + a * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const int64_t y = y0 + wy * 64 + b * 32 + (lane & 31);
+                if (x < args.na && y < args.nb && (!SYM || x >= y))
+                    atomicAdd(args.count + x * args.ldc + y,
+                              (unsigned long long)(((int)acc[a][b][r] + bits) >> 1));
+            }
         }
-    }
 }
 
 // tau from the exact count, with the reference's arithmetic (kendall.cu:40-45);
-// count == nullptr: no sample pairs (n < 2), the count is 0.
+// count == nullptr: no sample pairs (n < 2), the count is 0.  nopair: bits of
+// the tiles that are no sample pair, which the count pass counted.
 __global__ void kendall_finish_kernel(const unsigned long long *__restrict__ count, int64_t ldc,
                                       int64_t na, int64_t nb, int64_t n, int sym,
-                                      double *__restrict__ tau, int64_t ldt)
+                                      unsigned long long nopair, double *__restrict__ tau,
+                                      int64_t ldt)
 {
     const int64_t total = na * nb;
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
         const int64_t x = e % na, y = e / na;
-        const bool lower = !sym || (x / KBM >= y / KBM);
-        const unsigned long long c = count ? (lower ? count[x * ldc + y] : count[y * ldc + x]) : 0ull;
+        const bool lower = !sym || x >= y;
+        const unsigned long long c =
+            count ? (lower ? count[x * ldc + y] : count[y * ldc + x]) - nopair : 0ull;
         const float concordant = (float)c;
         float denom = (float)n;
         denom = (denom * (denom - 1.0f)) / 2.0f;
@@ -515,10 +534,63 @@ unsigned grid_for(int64_t total, int threads)
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
-int64_t padded_words(int64_t n)
+// Workspace: planes and flags of one segment of the tiles of sample pairs,
+// then the counts.  A segment takes as many tiles as keep the planes within
+// three bits per sample pair and variable (blocks of 32 variables hold more
+// than that when there are few variables), and at least 64 MiB; the segments
+// run one after the other.
+struct KendallPlan {
+    int64_t tiles, seg;                  // tiles of sample pairs in all, per segment
+    int64_t nvb_a, nvb_b, fs_a, fs_b;
+    size_t off_pb, off_fa, off_fb, off_count, bytes;
+};
+
+KendallPlan kendall_plan(int64_t na, int64_t nb, bool same, int64_t n)
 {
-    const int64_t w = n > 1 ? words_upto(n - 1) : 0;
-    return (w + KKW - 1) / KKW * KKW;
+    KendallPlan k;
+    k.tiles = pair_tiles(n);
+    k.nvb_a = (na + KVB - 1) / KVB;
+    k.nvb_b = same ? 0 : (nb + KVB - 1) / KVB;
+    k.fs_a = (k.nvb_a + KTX - 1) / KTX * KTX;
+    k.fs_b = (k.nvb_b + KTX - 1) / KTX * KTX;
+    const double tile_bytes = 3.0 * KTG * KGWORDS * 4 * (double)(k.nvb_a + k.nvb_b);
+    double cap = 3.0 / 8.0 * ((double)n * (double)(n - 1) / 2.0) * (double)(same ? na : na + nb);
+    if (cap < 67108864.0) cap = 67108864.0;
+    // a whole problem that is over by the tiles' rounding stays one segment
+    const double want = cap * 1.07 / tile_bytes;
+    k.seg = want < 1.0 ? 1 : want < (double)k.tiles ? (int64_t)want : k.tiles;
+    size_t p = 3 * (size_t)k.nvb_a * (size_t)k.seg * KTG * KGWORDS * 4;
+    k.off_pb = p;
+    p += 3 * (size_t)k.nvb_b * (size_t)k.seg * KTG * KGWORDS * 4;
+    k.off_fa = p;
+    p += align256((size_t)k.seg * KTG * (size_t)k.fs_a);
+    k.off_fb = p;
+    p += align256((size_t)k.seg * KTG * (size_t)k.fs_b);
+    k.off_count = p;
+    k.bytes = p + align256((size_t)na * (size_t)nb * 8);
+    return k;
+}
+
+hipError_t launch_planes(const float *x, int64_t nvar, int64_t n, int64_t ldx, uint32_t *planes,
+                         uint8_t *flags, int64_t nvb, int64_t fstride, int64_t seg, int64_t begin,
+                         int64_t tiles, hipStream_t stream)
+{
+    PlanesArgs args;
+    args.x = x;
+    args.nvar = nvar;
+    args.n = n;
+    args.ldx = ldx;
+    args.planes = planes;
+    args.flags = flags;
+    args.nvb = nvb;
+    args.fstride = fstride;
+    args.ngroups = seg * KTG;
+    args.tile_begin = begin;
+    args.ntiles = tiles;
+    args.runs = (tiles + KRUN - 1) / KRUN;
+    hipLaunchKernelGGL(kendall_planes_kernel, dim3((unsigned)(nvb * args.runs)), dim3(256), 0,
+                       stream, args);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -526,12 +598,7 @@ int64_t padded_words(int64_t n)
 size_t kendall_workspace_bytes(int64_t na, int64_t nb, bool same, int64_t n)
 {
     if (na <= 0 || nb <= 0 || n < 2) return 0;
-    const size_t wpad = (size_t)padded_words(n);
-    const size_t planes = align256(3 * (size_t)na * wpad * 4) +
-                          (same ? 0 : align256(3 * (size_t)nb * wpad * 4));
-    const size_t ties = align256((size_t)na * 4) + (same ? 0 : align256((size_t)nb * 4));
-    const size_t pe = align256(wpad / KKW * 4);
-    return planes + ties + pe + align256((size_t)na * (size_t)nb * 8);
+    return kendall_plan(na, nb, same, n).bytes;
 }
 
 hipError_t launch_kendall(const float *a, int64_t na, int64_t lda, const float *b, int64_t nb,
@@ -540,113 +607,86 @@ hipError_t launch_kendall(const float *a, int64_t na, int64_t lda, const float *
 {
     if (na <= 0 || nb <= 0) return hipSuccess;
     hipError_t e;
-    const int64_t wpad = padded_words(n);
-    char *ws = static_cast<char *>(workspace);
-    uint32_t *pa = nullptr, *pb = nullptr, *ta = nullptr, *tb = nullptr, *pe = nullptr;
     unsigned long long *count = nullptr;
+    unsigned long long nopair = 0;
     if (n >= 2) {
-        pa = reinterpret_cast<uint32_t *>(ws);
-        ws += align256(3 * (size_t)na * (size_t)wpad * 4);
-        pb = pa;
-        if (!same) {
-            pb = reinterpret_cast<uint32_t *>(ws);
-            ws += align256(3 * (size_t)nb * (size_t)wpad * 4);
-        }
-        ta = reinterpret_cast<uint32_t *>(ws);
-        ws += align256((size_t)na * 4);
-        tb = ta;
-        if (!same) {
-            tb = reinterpret_cast<uint32_t *>(ws);
-            ws += align256((size_t)nb * 4);
-        }
-        pe = reinterpret_cast<uint32_t *>(ws);
-        ws += align256((size_t)(wpad / KKW) * 4);
-        count = reinterpret_cast<unsigned long long *>(ws);
-        // zero the E planes (written only where a step has a tie), tie flags,
-        // past-end counts and counts with fill kernels, not memset nodes, so
-        // that a captured graph replays correctly; the planes pass writes P
-        // and N in full
-        e = launch_fill(reinterpret_cast<float *>(pa + 2 * (size_t)na * (size_t)wpad),
-                        na * wpad, 0.0f, stream);
+        const KendallPlan k = kendall_plan(na, nb, same, n);
+        char *ws = static_cast<char *>(workspace);
+        uint32_t *pa = reinterpret_cast<uint32_t *>(ws);
+        uint32_t *pb = same ? pa : reinterpret_cast<uint32_t *>(ws + k.off_pb);
+        uint8_t *fa = reinterpret_cast<uint8_t *>(ws + k.off_fa);
+        uint8_t *fb = same ? fa : reinterpret_cast<uint8_t *>(ws + k.off_fb);
+        count = reinterpret_cast<unsigned long long *>(ws + k.off_count);
+        nopair = (unsigned long long)k.tiles * KTG * KGW * 32 - (unsigned long long)n * (n - 1) / 2;
+        // the counts are added to: cleared by a fill kernel, not a memset
+        // node, so that a captured graph replays correctly
+        e = launch_fill(reinterpret_cast<float *>(count), na * nb * 2, 0.0f, stream);
         if (e != hipSuccess) return e;
-        if (!same) {
-            e = launch_fill(reinterpret_cast<float *>(pb + 2 * (size_t)nb * (size_t)wpad),
-                            nb * wpad, 0.0f, stream);
-            if (e != hipSuccess) return e;
-        }
-        const size_t zero_floats =
-            (size_t)(reinterpret_cast<char *>(count + (size_t)na * (size_t)nb) -
-                     reinterpret_cast<char *>(ta)) / 4;
-        e = launch_fill(reinterpret_cast<float *>(ta), (int64_t)zero_floats, 0.0f, stream);
-        if (e != hipSuccess) return e;
-        {
-            // row splits per variable: about 16 rows per wave, within the
-            // grid limit (every row is still covered: waves stride over rows)
-            int64_t rs64 = (n + 63) / 64;
-            const int64_t nv = na > nb ? na : nb;
-            if (nv * rs64 > 0x7fffffff) rs64 = 0x7fffffff / nv;
-            const int rsplit = (int)(rs64 > 0 ? rs64 : 1);
-            // up to 8192 samples (32 KB + an 8 KB tail) the rows read the variable from LDS
-            const bool lx = n <= 8192;
-            const unsigned lds = lx ? (unsigned)((n + 2048) * 4) : 0u;
-            auto planes_fn = lx ? kendall_planes_kernel<true> : kendall_planes_kernel<false>;
-            hipLaunchKernelGGL(planes_fn, dim3((unsigned)(na * rsplit)), dim3(256), lds, stream,
-                               a, na, n, lda, pa, wpad, ta, rsplit);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-            if (!same) {
-                hipLaunchKernelGGL(planes_fn, dim3((unsigned)(nb * rsplit)), dim3(256), lds,
-                                   stream, b, nb, n, ldb, pb, wpad, tb, rsplit);
-                if ((e = hipGetLastError()) != hipSuccess) return e;
-            }
-        }
-        {
-            const int64_t items = (n - 1) + (wpad - words_upto(n - 1));
-            hipLaunchKernelGGL(kendall_pastend_kernel, dim3(grid_for(items, 256)), dim3(256), 0,
-                               stream, n, wpad, pe);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
         KendallArgs args;
-        args.pe = pe;
         args.pa = pa;
         args.pb = pb;
+        args.fa = fa;
+        args.fb = fb;
+        args.nvb_a = k.nvb_a;
+        args.nvb_b = same ? k.nvb_a : k.nvb_b;
+        args.fs_a = k.fs_a;
+        args.fs_b = same ? k.fs_a : k.fs_b;
         args.na = na;
         args.nb = nb;
-        args.wpad = wpad;
         args.count = count;
         args.ldc = nb;
-        args.ties_a = ta;
-        args.ties_b = tb;
-        args.tiles_a = (na + KBM - 1) / KBM;
-        args.tiles_b = (nb + KBM - 1) / KBM;
-        args.ntiles = same ? args.tiles_a * (args.tiles_a + 1) / 2 : args.tiles_a * args.tiles_b;
-        // split the words so that about 2048 workgroups run (8 per CU)
-        int64_t splits = (2048 + args.ntiles - 1) / args.ntiles;
-        const int64_t chunks = wpad / KKW;
-        if (splits > chunks) splits = chunks;
-        if (splits < 1) splits = 1;
-        args.split_w = (chunks + splits - 1) / splits * KKW;
-        // a workgroup's counts are 32-bit: fewer than 2^32 sample pairs
-        // (32 per word) per word range
-        const int64_t max_split_w = ((int64_t(1) << 27) - KKW) / KKW * KKW;
-        if (args.split_w > max_split_w) args.split_w = max_split_w;
-        splits = (wpad + args.split_w - 1) / args.split_w;
-        const int64_t ids = args.ntiles * splits;
-        const int64_t max_ids = int64_t(1) << 23;
-        for (int64_t off = 0; off < ids; off += max_ids) {
-            args.id_offset = off;
-            args.ids_this = (ids - off) < max_ids ? (ids - off) : max_ids;
-            if (same)
-                hipLaunchKernelGGL(kendall_count_kernel<true>, dim3((unsigned)args.ids_this),
-                                   dim3(KTHREADS), 0, stream, args);
-            else
-                hipLaunchKernelGGL(kendall_count_kernel<false>, dim3((unsigned)args.ids_this),
-                                   dim3(KTHREADS), 0, stream, args);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
+        const int64_t ta = (na + KBX - 1) / KBX;
+        args.tiles_b = (nb + KBY - 1) / KBY;
+        args.ntiles = same ? ta * (ta + 1) : ta * args.tiles_b;
+        for (int64_t begin = 0; begin < k.tiles; begin += k.seg) {
+            const int64_t tiles = k.tiles - begin < k.seg ? k.tiles - begin : k.seg;
+            e = launch_planes(a, na, n, lda, pa, fa, k.nvb_a, k.fs_a, tiles, begin, tiles, stream);
+            if (e != hipSuccess) return e;
+            if (!same) {
+                e = launch_planes(b, nb, n, ldb, pb, fb, k.nvb_b, k.fs_b, tiles, begin, tiles,
+                                  stream);
+                if (e != hipSuccess) return e;
+            }
+            args.ngroups = tiles * KTG;
+            // Ranges of groups: two workgroups run on a CU at a time (out of
+            // step, so that one's barrier and LDS waits lie under the other's
+            // products), so the number of workgroups is kept just under a
+            // multiple of 512 (the multiple, up to 4, that leaves the fewest
+            // idle), with at least 16 groups each to fill and drain the ring.
+            int64_t splits = 1;
+            double best = 0.0;
+            for (int r = 1; r <= 4; ++r) {
+                const int64_t s = 512 * r / args.ntiles;
+                if (s < 1) continue;
+                const double used = (double)(s * args.ntiles) / (512.0 * r) - 0.02 * r;
+                if (used > best) {
+                    best = used;
+                    splits = s;
+                }
+            }
+            if (splits > args.ngroups / 16) splits = args.ngroups / 16;
+            if (splits < 1) splits = 1;
+            args.split_g = (args.ngroups + splits - 1) / splits;
+            if (args.split_g > KMAXGROUPS) args.split_g = KMAXGROUPS;
+            splits = (args.ngroups + args.split_g - 1) / args.split_g;
+            const int64_t ids = args.ntiles * splits;
+            const int64_t max_ids = int64_t(1) << 22;
+            for (int64_t off = 0; off < ids; off += max_ids) {
+                args.id_offset = off;
+                args.ids_this = (ids - off) < max_ids ? (ids - off) : max_ids;
+                if (same)
+                    hipLaunchKernelGGL(kendall_count_kernel<true>, dim3((unsigned)args.ids_this),
+                                       dim3(KTHREADS), 0, stream, args);
+                else
+                    hipLaunchKernelGGL(kendall_count_kernel<false>, dim3((unsigned)args.ids_this),
+                                       dim3(KTHREADS), 0, stream, args);
+                if ((e = hipGetLastError()) != hipSuccess) return e;
+            }
         }
     }
     // n < 2 leaves count null: no sample pair, tau = 0 / 0
     hipLaunchKernelGGL(kendall_finish_kernel, dim3(grid_for(na * nb, 256)), dim3(256), 0, stream,
-                       count, nb, na, nb, n, same ? 1 : 0, tau, ldt);
+                       count, nb, na, nb, n, same ? 1 : 0, nopair, tau, ldt);
     return hipGetLastError();
 }
 

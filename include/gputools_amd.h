@@ -2,7 +2,7 @@
  * gputools_amd.h -- C-ABI of the MI355X (gfx950) pairwise-distance library,
  * of the hierarchical-clustering stage built on its output, and of gpuCor's
  * all-pairs correlations (Pearson: the same contraction on standardised
- * variables; Kendall: popcounts over sample-pair bit planes).
+ * variables; Kendall: FP4 matrix products of sample-pair signs).
  *
  * Two groups of entry points:
  *

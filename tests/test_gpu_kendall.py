@@ -195,3 +195,47 @@ def test_kendall_invariant_under_monotone_maps():
     t2 = gt.kendall(-da, db).cpu().numpy()
     np.testing.assert_array_equal(t1, t0)
     np.testing.assert_array_equal(t2, -t0)
+
+
+@pytest.mark.parametrize("n,na,nb", [(64, 32, 33), (65, 128, 129), (66, 256, 127), (97, 257, 0),
+                                     (130, 96, 385), (161, 513, 0)])
+def test_kendall_matrix_tile_edges(n, na, nb):
+    """Sizes at the edges of the sample-pair tiles (64 x 32), the variable
+    blocks (32) and the count tiles (256 x 128), each with: variables without
+    a tie, one late tie, signed zeros (equal), infinities (equal to
+    themselves) and NaN.  The count is exact: bit for bit."""
+    rng = np.random.default_rng(n + na + nb)
+    sets = []
+    for nv in (na, nb):
+        x = rng.standard_normal((max(nv, 1), n)).astype(np.float32)
+        x[0, n - 2] = x[0, n - 1]
+        x[nv // 3, : n // 2 : 3] = 0.0
+        x[nv // 3, 1 : n // 2 : 3] = -0.0
+        x[nv // 2, ::7] = np.inf
+        x[nv // 2, 3::7] = -np.inf
+        x[(2 * nv) // 3, n // 2] = np.nan
+        sets.append(x)
+    a, b = sets
+    print("case kendall tile edges n=%d na=%d nb=%d" % (n, na, nb), flush=True)
+    got = gt.kendall(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda() if nb else None)
+    torch.cuda.synchronize()
+    want, _ = orc.kendall(a, b if nb else a, nthreads=8)
+    assert_same(got.cpu().numpy(), want)
+
+
+def test_kendall_segments():
+    """Few variables and many samples: the planes are made and counted one
+    segment of the sample pairs at a time (12000 samples, 64 MiB a segment)."""
+    rng = np.random.default_rng(81)
+    n = 12000
+    a = rng.standard_normal((3, n)).astype(np.float32)
+    b = rng.standard_normal((2, n)).astype(np.float32)
+    a[1] = rng.integers(0, 9, n)
+    b[0] = a[0] + rng.standard_normal(n).astype(np.float32)
+    b[1, n - 1] = np.nan
+    print("case kendall segments", flush=True)
+    for bb in (b, None):
+        got = gt.kendall(torch.from_numpy(a).cuda(), None if bb is None else torch.from_numpy(bb).cuda())
+        torch.cuda.synchronize()
+        want, _ = orc.kendall(a, a if bb is None else bb, nthreads=8)
+        assert_same(got.cpu().numpy(), want)
