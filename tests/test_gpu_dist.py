@@ -461,3 +461,41 @@ def test_mixture_65536x512_fp32_sampled():
     want = orc.dist_pairs(x, ii, jj, "euclidean")
     err = np.max(np.abs(vals - want) / want)
     assert err <= RTOL, err
+
+
+@pytest.mark.parametrize("method,k", [("euclidean", 37), ("maximum", 16), ("manhattan", 81),
+                                      ("minkowski", 130), ("canberra", 37)])
+def test_tile_sides_agree(method, k):
+    """The tile side follows the number of points: 32 up to about 2100, then
+    64, and 128 where its rounds fill the chip (3968 points).  The order of a
+    pair's sums does not depend on it, so the distances among the first 2049
+    points are the same bits from all three (canberra picks its form per tile:
+    within its tolerance, and 9000 points reach its 64 tile); ragged edges of
+    each against the oracle; the pitched layouts against the packed one."""
+    p = 3.0 if method == "minkowski" else 2.0
+    big = 9100 if method == "canberra" else 3968
+    x = wl.method_input(method, big, k, seed=31)
+    print("case tile sides %s k=%d" % (method, k), flush=True)
+    m = 2049
+    small = run(x[:m], method, p)
+    assert_parity(small, orc.dist(x[:m], method, p), method)
+    j, i = np.triu_indices(m, 1)
+    for n in (2305, big):
+        full = run(x[:n], method, p, layout="full")
+        got = full[:m, :m]
+        np.testing.assert_array_equal(got, got.T)
+        if method == "canberra":
+            assert_parity(got[i, j], orc.dist(x[:m], method, p), method)
+        else:
+            np.testing.assert_array_equal(got[i, j], small)
+        packed = run(x[:n], method, p)
+        jj, ii = np.triu_indices(n, 1)
+        np.testing.assert_array_equal(packed, full[ii, jj])
+        cross = gt.dist_cross(dev(x[:n]), dev(x[:1037]), method, p)
+        torch.cuda.synchronize()
+        cross = cross.cpu().numpy()
+        if method == "canberra":
+            np.testing.assert_allclose(cross[:, 1037:], full[:1037, 1037:], rtol=1e-5)
+        else:
+            off = ~np.eye(1037, n, dtype=bool)
+            np.testing.assert_array_equal(cross[off], full[:1037][off])
