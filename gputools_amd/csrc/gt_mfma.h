@@ -7,6 +7,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace gt {
 
@@ -15,6 +16,17 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 enum { SPLIT_BF16 = 0, SPLIT_FP16 = 1 };
+
+// Operand blocks: split terms lie in memory as the matrix product takes them.
+// A block is 32 rows x 16 features of one term, 1 KB: lane 32 h + r of a wave
+// holds features 8 h .. 8 h + 7 of row r, 16 bytes.  The NT terms of a block
+// are consecutive, then the blocks of the same rows along the features:
+// block (rb, ch), term t at ((rb * nch + ch) * NT + t) * OPERAND_VALUES.
+constexpr int OPERAND_K = 16;
+constexpr int OPERAND_VALUES = 512;
+constexpr int OPERAND_BYTES = OPERAND_VALUES * 2;
+
+__host__ __device__ __forceinline__ int64_t operand_rows(int64_t n) { return (n + 31) / 32 * 32; }
 
 template <int SPLIT>
 struct Split;
