@@ -27,7 +27,7 @@
 // held from module load until the process ends.  Its name is a host-side
 // stand-in; host code uses only the device address that hipGetSymbolAddress
 // returns for the current device (scratch_address below).
-static __device__ __align__(256) unsigned char scratch[GT_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[GT_NOALLOC_SCRATCH_BYTES + gt::GRAM_ROW_SLACK];
 
 namespace {
 
@@ -513,9 +513,12 @@ int pmcc_host(int use, int precision, const float *a_host, int64_t na, const flo
     const size_t bbytes = (size_t)nb * (size_t)dim * sizeof(float);
     if ((s = da.alloc(abytes, "hipMalloc(variables a)")) != GT_OK) return s;
     if (!same && (s = db.alloc(bbytes, "hipMalloc(variables b)")) != GT_OK) return s;
-    if ((s = dout.alloc(3 * round_up(out * sizeof(float), 256), "hipMalloc(correlations)")) != GT_OK)
+    // the pairwise workspace shares the outputs' allocation
+    const size_t out_bytes = 3 * round_up(out * sizeof(float), 256);
+    const bool joint = use == GT_USE_PAIRWISE;
+    if ((s = dout.alloc(out_bytes + (joint ? ws_bytes : 0), "hipMalloc(correlations)")) != GT_OK)
         return s;
-    if ((s = dws.alloc(ws_bytes, "hipMalloc(workspace)")) != GT_OK) return s;
+    if (!joint && (s = dws.alloc(ws_bytes, "hipMalloc(workspace)")) != GT_OK) return s;
     if (abytes) GT_HIP(hipMemcpy(da.ptr, a_host, abytes, hipMemcpyHostToDevice));
     if (!same && bbytes) GT_HIP(hipMemcpy(db.ptr, b_host, bbytes, hipMemcpyHostToDevice));
     char *o = static_cast<char *>(dout.ptr);
@@ -524,7 +527,7 @@ int pmcc_host(int use, int precision, const float *a_host, int64_t na, const flo
           *dt = reinterpret_cast<float *>(o + 2 * part);
     const float *dbp = same ? static_cast<const float *>(da.ptr) : static_cast<const float *>(db.ptr);
     GT_HIP(gt::launch_pmcc(use, precision, static_cast<const float *>(da.ptr), na, dim, dbp, nb, dim,
-                           same, dim, dp, dc, dt, nb, dws.ptr, nullptr));
+                           same, dim, dp, dc, dt, nb, joint ? o + out_bytes : dws.ptr, nullptr));
     GT_HIP(hipMemcpy(pairs, dp, out * sizeof(float), hipMemcpyDeviceToHost));
     GT_HIP(hipMemcpy(corr, dc, out * sizeof(float), hipMemcpyDeviceToHost));
     GT_HIP(hipMemcpy(ts, dt, out * sizeof(float), hipMemcpyDeviceToHost));
@@ -653,7 +656,11 @@ int gt_dist_noalloc(const float *x, int64_t n, int64_t k, int64_t ldx, int metho
     if (s != GT_OK) return s;
     size_t need = 0;
     workspace_bytes(n, k, method, precision, &need);
-    if (need > GT_NOALLOC_SCRATCH_BYTES)
+    // the split forms round their rows up to 32: the limit is on the rows
+    // themselves, and the scratch has room for the rounding
+    const size_t rounding =
+        need > 0 && precision != GT_PREC_FP32 ? gt::gram_rounding_bytes(n, k, precision) : 0;
+    if (need - rounding > GT_NOALLOC_SCRATCH_BYTES)
         return fail(GT_ERR_WORKSPACE,
                     "gt_dist_noalloc: this call needs %zu bytes of workspace, above the %zu of "
                     "its static scratch; call gt_dist_ws with a workspace instead",
@@ -858,9 +865,13 @@ int gt_pmcc(int use, int precision, const float *a, int64_t na, int64_t lda, con
     int s = check_pmcc_args(use, precision, a, na, lda, b, nb, ldb, dim, pairs, corr, ts, ldo);
     if (s != GT_OK) return s;
     const size_t need = gt::pmcc_workspace_bytes(use, precision, na, nb, same, dim);
-    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
-        return fail(GT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need,
-                    workspace_bytes);
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
+        // pairwise.complete.obs runs without a workspace too (on the VALU)
+        if (use != GT_USE_PAIRWISE)
+            return fail(GT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need,
+                        workspace_bytes);
+        workspace = nullptr;
+    }
     GT_HIP(gt::launch_pmcc(use, precision, a, na, lda, b, nb, ldb, same, dim, pairs, corr, ts, ldo,
                            workspace, static_cast<hipStream_t>(stream)));
     return GT_OK;

@@ -809,11 +809,23 @@ int64_t colstats_blocks(int64_t n) { return (n + CS_ROWS - 1) / CS_ROWS; }
 // 32), then norms, scales and
 // inverse scales (n floats each), the column centres (k floats) and the
 // partial column statistics (3 x ceil(n / 256) x k floats).
+static size_t terms_bytes(int64_t rows, int64_t k, int precision)
+{
+    return align256((size_t)split_terms(precision) * (size_t)rows * (size_t)padded_k(k) *
+                    sizeof(unsigned short));
+}
+
+// Bytes of gram_workspace_bytes that come from rounding the rows up to 32: at
+// most GRAM_ROW_SLACK at the feature counts that use them (GRAM_TAU_MAX below:
+// up to 8304 in BF16, 15456 in FP16).
+size_t gram_rounding_bytes(int64_t n, int64_t k, int precision)
+{
+    return terms_bytes(operand_rows(n), k, precision) - terms_bytes(n, k, precision);
+}
+
 size_t gram_workspace_bytes(int64_t n, int64_t k, int precision)
 {
-    const size_t terms = align256((size_t)split_terms(precision) * (size_t)operand_rows(n) *
-                                  (size_t)padded_k(k) * sizeof(unsigned short));
-    return terms + 3 * align256((size_t)n * sizeof(float)) + align256((size_t)k * sizeof(float)) +
+    return terms_bytes(operand_rows(n), k, precision) + 3 * align256((size_t)n * sizeof(float)) + align256((size_t)k * sizeof(float)) +
            3 * align256((size_t)colstats_blocks(n) * (size_t)k * sizeof(float));
 }
 

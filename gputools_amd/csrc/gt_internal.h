@@ -53,6 +53,8 @@ hipError_t launch_fill_full(float *out, int64_t n, int64_t ldd, float offdiag,
 // Split-precision MFMA Gram path (euclidean).  Workspace: split terms, row
 // norms and row scales (gram_workspace_bytes).
 size_t gram_workspace_bytes(int64_t n, int64_t k, int precision);
+size_t gram_rounding_bytes(int64_t n, int64_t k, int precision);
+constexpr size_t GRAM_ROW_SLACK = (size_t)2 << 20;
 hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int64_t k,
                        int64_t ldx, float *out, int64_t ldd, void *workspace,
                        hipStream_t stream);

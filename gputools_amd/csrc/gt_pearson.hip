@@ -18,8 +18,13 @@
 // dot-product term).
 //
 // use = "pairwise.complete.obs": a pair uses the samples where both values
-// are present, so means and deviations are per pair.  A VALU tile kernel keeps
-// the reference's two passes per pair: counts and sums give the pair's means,
+// are present, so means and deviations are per pair.  The six sums a pair needs
+// (count, two sums, three second moments of shifted values) are products of
+// values, squares and presence masks: the matrix cores form them from split
+// operands that a pre-pass lays out once (pmcc_moments_kernel).  Pairs whose
+// moments cancel, or whose data is not finite, and calls without a workspace
+// take a VALU tile kernel (pmcc_pairwise_kernel), which keeps the reference's
+// two passes per pair where it must: counts and sums give the pair's means,
 // then the centred second moments give the correlation
 //     sum d_x d_y / (sqrt(sum d_x^2) sqrt(sum d_y^2)).
 //
@@ -430,6 +435,10 @@ struct PairwiseArgs {
     int64_t tiles_b;
     int64_t tile_offset, tiles_this;
     bool vec;   // ldo and the output pointers allow 16-byte stores
+    // tiles that pmcc_moments_kernel left (one byte per tile, 1 = left): only
+    // those run, with two passes; null: every tile runs
+    const uint8_t *left;
+    const float *scale_a, *scale_b;   // with left: each variable's power of two
 };
 
 // A sample of a pair counts when both values are present (not NaN): counts
@@ -445,6 +454,7 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     const int tid = threadIdx.x;
     const int tx = tid & 15, ty = tid >> 4;   // y = 4 tx + j, x = 4 ty + i
     const int64_t t = args.tile_offset + xcd_remap(blockIdx.x, args.tiles_this);
+    if (args.left && args.left[t] == 0) return;
     int64_t I, J;
     if (SYM) {
         int ti, tj;
@@ -465,13 +475,15 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     const float *pa = args.a + (va_ok ? (x0 + sv) * args.lda : 0);
     const float *pb = args.b + (vb_ok ? (y0 + sv) * args.ldb : 0);
     const float qnan = __builtin_nanf("");
+    const float fa = args.left && va_ok ? args.scale_a[x0 + sv] : 1.0f;
+    const float fb = args.left && vb_ok ? args.scale_b[y0 + sv] : 1.0f;
     float ra[8], rb[8];
     auto gload = [&](int64_t kb) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const int64_t kk = kb + sk + q;
-            ra[q] = (va_ok && kk < dim) ? pa[kk] : qnan;
-            rb[q] = (vb_ok && kk < dim) ? pb[kk] : qnan;
+            ra[q] = (va_ok && kk < dim) ? pa[kk] * fa : qnan;
+            rb[q] = (vb_ok && kk < dim) ? pb[kk] * fb : qnan;
         }
     };
     auto stage = [&]() {
@@ -493,7 +505,7 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     // Where that subtraction cancels (Caa <= Saa / 16: a subset mean far from
     // c, a constant subset, fewer than two samples) or a sum is not finite
     // (Inf in the data), the tile runs the two passes below instead.
-    {
+    if (!args.left) {
         __shared__ float lds1[3][2][WBK][WLD];   // a', a'^2, presence; [side]
         gload(0);
         float csum[2] = {0.0f, 0.0f}, ccnt[2] = {0.0f, 0.0f};
@@ -787,6 +799,285 @@ finish:
 }
 
 // ---------------------------------------------------------------------------
+// Matrix-core form of use = "pairwise.complete.obs"
+// ---------------------------------------------------------------------------
+// Per variable and sample seven BF16 values, in operand blocks (gt_mfma.h, NT =
+// 7): the shifted and scaled value a' in three terms, its FP32 square q in three
+// terms (both splits are exact), the presence mask m.  Missing samples, samples
+// past dim and rows past the last variable are zero in all seven.  The shift c
+// is the mean of the present values among the first 32 samples; the scale is
+// the power of two that brings max |v - c| to [1, 2), so that the terms stay
+// clear of the denormal range (the correlation does not depend on it; the
+// two passes over the tiles that are left use it as well).
+constexpr int QT = 7;
+enum { Q_VALUE = 0, Q_SQUARE = 3, Q_MASK = 6 };
+constexpr int QTHREADS = 1024;
+
+// `split` workgroups per block of 32 variables: each finds the shift and the
+// scale from all samples and writes its share of the chunks (few variables
+// would otherwise leave CUs idle).  Lane 32 h + r of a wave reads samples 8 h
+// .. + 7 of 16 of variable r.  Also clears `left`.
+__global__ __launch_bounds__(QTHREADS) void pmcc_moments_prep_kernel(const float *__restrict__ x, int64_t n,
+                                                                     int64_t dim, int64_t ldx, int64_t nch,
+                                                                     int split,
+                                                                     unsigned short *__restrict__ terms,
+                                                                     float *__restrict__ scales,
+                                                                     uint8_t *__restrict__ left, int64_t nleft)
+{
+    __shared__ float row_shift[32], row_scale[32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
+    for (int64_t t = (int64_t)blockIdx.x * QTHREADS + threadIdx.x; t < nleft;
+         t += (int64_t)gridDim.x * QTHREADS)
+        left[t] = 0;
+    const int64_t rb = blockIdx.x / split, part = blockIdx.x % split;
+    // shift and scale, a wave per variable
+    for (int q = wave; q < 32; q += QTHREADS / 64) {
+        const int64_t row = rb * 32 + q;
+        float shift = 0.0f, m = 0.0f;
+        if (row < n) {
+            const float *xr = x + row * ldx;
+            const float first = lane < 32 && lane < dim ? xr[lane] : __builtin_nanf("");
+            const bool present = fabsf(first) < INFINITY;
+            const float s = wave_sum(present ? first : 0.0f), c = wave_sum(present ? 1.0f : 0.0f);
+            shift = c > 0.0f ? s / c : 0.0f;
+#pragma unroll 4
+            for (int64_t k = lane; k < dim; k += 64) {
+                const float d = fabsf(xr[k] - shift);
+                if (d < INFINITY) m = fmaxf(m, d);
+            }
+            m = wave_max(m);
+        }
+        if (lane == 0) {
+            int e = m > 0.0f ? ilogbf(m) : 0;
+            e = e < -120 ? -120 : (e > 120 ? 120 : e);
+            row_shift[q] = shift;
+            row_scale[q] = ldexpf(1.0f, -e);
+            if (part == 0 && row < n) scales[row] = row_scale[q];
+        }
+    }
+    __syncthreads();
+    const int64_t row = rb * 32 + r;
+    const bool in = row < n;
+    const float *xr = x + (in ? row : 0) * ldx;
+    const float shift = row_shift[r], scale = row_scale[r];
+    float v[8];
+    auto load = [&](int64_t ch) {
+        const int64_t k0 = ch * OPERAND_K + h * 8;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = (in && k0 + k < dim) ? xr[k0 + k] : __builtin_nanf("");
+    };
+    for (int64_t ch = part * (QTHREADS / 64) + wave; ch < nch; ch += (int64_t)split * (QTHREADS / 64)) {
+        load(ch);
+        unsigned short t[8][QT];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const bool present = v[k] == v[k];
+            const float d = present ? (v[k] - shift) * scale : 0.0f;
+            Split<SPLIT_BF16>::split(d, t[k] + Q_VALUE);
+            Split<SPLIT_BF16>::split(d * d, t[k] + Q_SQUARE);
+            t[k][Q_MASK] = present ? 0x3f80 : 0;   // BF16 1.0
+        }
+        unsigned short *const out = terms + (rb * nch + ch) * QT * OPERAND_VALUES + lane * 8;
+#pragma unroll
+        for (int q = 0; q < QT; ++q) {
+            uint4 w;
+            w.x = t[0][q] | ((unsigned)t[1][q] << 16);
+            w.y = t[2][q] | ((unsigned)t[3][q] << 16);
+            w.z = t[4][q] | ((unsigned)t[5][q] << 16);
+            w.w = t[6][q] | ((unsigned)t[7][q] << 16);
+            *reinterpret_cast<uint4 *>(out + q * OPERAND_VALUES) = w;
+        }
+    }
+}
+
+constexpr double MOMENTS_MAX_BYTES = 1073741824.0;
+
+constexpr int QBM = WBM;                 // variables per tile side
+constexpr int QWAVES = 4;                // 2 (x) x 2 (y), 32 x 32 pairs each
+constexpr int QSTAGE = 2 * QBM / 32 * QT * OPERAND_BYTES;   // one chunk of 16 samples (28 KB)
+constexpr int QNSTAGE = 2;
+constexpr int QTRL = 33;                 // row of a wave's transposed 32 x 32 block
+
+struct MomentsArgs {
+    const unsigned short *ta, *tb;   // operand blocks of pmcc_moments_prep_kernel
+    int64_t na, nb;
+    int nch, fold;                   // chunks, chunks per partial second moment
+    float *corr, *ts, *pairs;
+    int64_t ldo;
+    uint8_t *left;                   // per WBM x WBM tile: a pair here is left to two passes
+    int64_t tiles_b;                 // tiles along y (rectangular schedule)
+    int64_t id_offset, ids_this;
+};
+
+// A 128 x 64 tile of pairs; the operand blocks stream through a three-stage
+// LDS ring (direct loads; wave w < 7 moves term w of the six blocks).  A wave
+// holds 32 x 32 pairs: n = m m', Sa = a m', Sb = m b', Saa = q m', Sbb = m q'
+// and Sab = a b' take 1, 3, 3, 3, 3 and 6 products of 16 samples, all with
+// FP32 accumulation.  The second moments are two-level sums: `fold` chunks in
+// the accumulator, then added to a total, which keeps their error at that of
+// the VALU form's two levels.  With two levels and six sums a 32 x 32 block
+// takes 144 registers, which is what sets the tile.
+// Two workgroups share a CU, so one's waits lie under the other's products.
+// Bound: the matrix cores (19 products, 0.9 PFLOP/s of a measured 1.1 for a
+// large BF16 product).  4001 variables x 777 samples, self case: 1.14 ms on
+// the VALU (6 fused products per pair and sample), 0.28 ms here; 128 x 64
+// tiles of 8 waves, one workgroup per CU, took 0.34 ms (five rounds of tiles,
+// the last nearly empty).
+// SYM: a == b; tiles on and below the diagonal, each pair stored twice.
+template <bool SYM>
+__global__ __launch_bounds__(QWAVES * 64, 2) void pmcc_moments_kernel(MomentsArgs args)
+{
+    typedef Split<SPLIT_BF16> S;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[QNSTAGE * QSTAGE];
+    static_assert(QWAVES * 32 * QTRL * 4 <= (int)sizeof(smem), "transpose regions");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wx = wave >> 1, wy = wave & 1;
+    const int64_t t = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
+    int64_t I, J;
+    if (SYM) {
+        int ti, tj;
+        tri_tile(t, ti, tj);
+        I = ti;
+        J = tj;
+    } else {
+        I = t / args.tiles_b;
+        J = t % args.tiles_b;
+    }
+    const int64_t x0 = I * QBM + wx * 32, y0 = J * QBM + wy * 32;   // this wave's pairs
+    const int64_t na = args.na, nb = args.nb;
+    const int nch = args.nch;
+
+    typedef __attribute__((address_space(3))) void lds_void_t;
+    typedef const __attribute__((address_space(1))) void gbl_void_t;
+    // wave w moves block w: side x in waves 0 and 1, side y in 2 and 3
+    const unsigned short *src;
+    {
+        const bool sb = wave >= 2;
+        const int64_t last = operand_rows(sb ? nb : na) / 32 - 1;
+        int64_t rb = (sb ? J : I) * (QBM / 32) + (wave & 1);
+        if (rb > last) rb = last;   // only feeds pairs that are not stored
+        src = (sb ? args.tb : args.ta) + rb * nch * QT * OPERAND_VALUES + lane * 8;
+    }
+    auto issue = [&](int c) {
+        unsigned char *const st = smem + (c % QNSTAGE) * QSTAGE + wave * QT * OPERAND_BYTES;
+#pragma unroll
+        for (int q = 0; q < QT; ++q)
+            __builtin_amdgcn_global_load_lds((gbl_void_t *)(src + ((int64_t)c * QT + q) * OPERAND_VALUES),
+                                             (lds_void_t *)(st + q * OPERAND_BYTES), 16, 0, 0);
+    };
+    // blocks above the diagonal or past the end only help to load
+    const bool idle = x0 >= na || y0 >= nb || (SYM && y0 > x0);
+
+    f32x16_t cn, sa, sb, paa, pbb, pab, saa, sbb, sab;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        cn[r] = sa[r] = sb[r] = paa[r] = pbb[r] = pab[r] = saa[r] = sbb[r] = sab[r] = 0.0f;
+
+#pragma unroll
+    for (int c = 0; c < QNSTAGE - 1; ++c)
+        if (c < nch) issue(c);
+    int folded = 0;
+    for (int c = 0; c < nch; ++c) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // every wave's part of chunk c is in LDS, and every wave is done with
+        // chunk c - 1, whose stage the next issue overwrites
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (c + QNSTAGE - 1 < nch) issue(c + QNSTAGE - 1);
+        if (idle) continue;
+        const unsigned char *const st = smem + (c % QNSTAGE) * QSTAGE + lane * 16;
+        bf16x8_t av[QT], bv[QT];
+#pragma unroll
+        for (int q = 0; q < QT; ++q) {
+            av[q] = *reinterpret_cast<const bf16x8_t *>(st + (wx * QT + q) * OPERAND_BYTES);
+            bv[q] = *reinterpret_cast<const bf16x8_t *>(st + ((QBM / 32 + wy) * QT + q) * OPERAND_BYTES);
+        }
+        cn = S::mfma(av[Q_MASK], bv[Q_MASK], cn);
+#pragma unroll
+        for (int q = 2; q >= 0; --q) {
+            sa = S::mfma(av[Q_VALUE + q], bv[Q_MASK], sa);
+            sb = S::mfma(av[Q_MASK], bv[Q_VALUE + q], sb);
+            paa = S::mfma(av[Q_SQUARE + q], bv[Q_MASK], paa);
+            pbb = S::mfma(av[Q_MASK], bv[Q_SQUARE + q], pbb);
+            // the products of three terms down to 2^-16: 1 1, 0 2, 2 0, 0 1, 1 0, 0 0
+            if (q == 2) {
+                pab = S::mfma(av[Q_VALUE + 1], bv[Q_VALUE + 1], pab);
+                pab = S::mfma(av[Q_VALUE], bv[Q_VALUE + 2], pab);
+            } else if (q == 1) {
+                pab = S::mfma(av[Q_VALUE + 2], bv[Q_VALUE], pab);
+                pab = S::mfma(av[Q_VALUE], bv[Q_VALUE + 1], pab);
+            } else {
+                pab = S::mfma(av[Q_VALUE + 1], bv[Q_VALUE], pab);
+                pab = S::mfma(av[Q_VALUE], bv[Q_VALUE], pab);
+            }
+        }
+        if (++folded == args.fold || c + 1 == nch) {
+            folded = 0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                saa[r] += paa[r];
+                sbb[r] += pbb[r];
+                sab[r] += pab[r];
+                paa[r] = pbb[r] = pab[r] = 0.0f;
+            }
+        }
+    }
+    // the stages become the transpose regions
+    __syncthreads();
+    if (idle) return;
+
+    // 32 x 32 accumulator layout: element r of lane l is x row 8 (r / 4) +
+    // 4 (l / 32) + r % 4 and y column l % 32
+    const bool diag = SYM && x0 == y0;
+    const int64_t y = y0 + (lane & 31);
+    bool ill = false;
+    float rv[16], tv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int64_t x = x0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        const float n = cn[r];
+        // Sa Sb / n with the product first, so (x, y) and (y, x) round alike
+        const float qa = saa[r] - sa[r] * sa[r] / n;
+        const float qb = sbb[r] - sb[r] * sb[r] / n;
+        const float qab = sab[r] - sa[r] * sb[r] / n;
+        const bool inside = x < na && y < nb && (!diag || x >= y);
+        ill = ill || (inside && !(qa > saa[r] * 0.0625f && qb > sbb[r] * 0.0625f));
+        rv[r] = qab / (sqrtf(qa) * sqrtf(qb));
+        tv[r] = t_score<true>(n, rv[r]);
+        if (inside) {
+            const int64_t o = x * args.ldo + y;
+            args.corr[o] = rv[r];
+            args.ts[o] = tv[r];
+            args.pairs[o] = n;
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(ill) != 0 && lane == 0) args.left[t] = 1;
+    if (!SYM) return;
+    // the mirrored block, transposed through this wave's own LDS region, as
+    // rows of 32 consecutive x
+    float *const tr = reinterpret_cast<float *>(smem) + wave * 32 * QTRL;
+    auto mirror = [&](const float (&v)[16], float *out) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            tr[(lane & 31) * QTRL + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] = v[r];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int it = 0; it < 16; ++it) {
+            const int ly = 2 * it + (lane >> 5), lx = lane & 31;
+            if (y0 + ly < nb && x0 + lx < na && (!diag || lx > ly))
+                out[(y0 + ly) * args.ldo + x0 + lx] = tr[ly * QTRL + lx];
+        }
+    };
+    float nv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nv[r] = cn[r];
+    mirror(rv, args.corr);
+    mirror(tv, args.ts);
+    mirror(nv, args.pairs);
+}
+
+// ---------------------------------------------------------------------------
 // Elementwise kernels
 // ---------------------------------------------------------------------------
 
@@ -927,12 +1218,74 @@ hipError_t launch_tile_split(bool same, bool vec, PmccTileArgs &args, int64_t id
     return launch_tile<SPLIT, false, false>(args, ids, stream);
 }
 
+// Workspace of the matrix-core form of use = "pairwise.complete.obs": the
+// operand blocks of a, then (unless same) of b, the scales, the tile flags.  bytes is
+// 0 where the VALU form is taken: few samples, where three launches cost
+// more than the sums (500 x 300 variables, times in us, VALU and here: 28 and
+// 37 at 48 samples, 44 and 30 at 100), unless the pairs are many (3000
+// variables x 20 samples: 70 and 50), and above a gigabyte of operands.
+struct MomentsPlan {
+    int64_t nch, tiles64;
+    size_t off_b, off_scale, off_left, bytes;
+};
+
+MomentsPlan moments_plan(int64_t na, int64_t nb, bool same, int64_t dim)
+{
+    MomentsPlan m;
+    m.nch = (dim + OPERAND_K - 1) / OPERAND_K;
+    const int64_t ta = (na + WBM - 1) / WBM, tb = (nb + WBM - 1) / WBM;
+    m.tiles64 = same ? ta * (ta + 1) / 2 : ta * tb;
+    const double row = 2.0 * QT * OPERAND_K * (double)m.nch;
+    const double all = row * ((double)operand_rows(na) + (same ? 0.0 : (double)operand_rows(nb)));
+    if (!(dim >= 80 || (dim >= 16 && m.tiles64 >= 1000)) || all > MOMENTS_MAX_BYTES) {
+        m.bytes = 0;
+        return m;
+    }
+    m.off_b = (size_t)operand_rows(na) * (size_t)m.nch * OPERAND_K * QT * sizeof(unsigned short);
+    m.off_scale = m.off_b + (same ? 0 : (size_t)operand_rows(nb) * (size_t)m.nch * OPERAND_K * QT *
+                                            sizeof(unsigned short));
+    m.off_left = m.off_scale + align256(((size_t)na + (same ? 0 : (size_t)nb)) * sizeof(float));
+    m.bytes = m.off_left + align256((size_t)m.tiles64);
+    return m;
+}
+
+hipError_t launch_moments_prep(const float *x, int64_t n, int64_t dim, int64_t ldx, int64_t nch,
+                               unsigned short *terms, float *scales, uint8_t *left, int64_t nleft,
+                               hipStream_t stream)
+{
+    const int64_t blocks = operand_rows(n) / 32;
+    int64_t split = (512 + blocks - 1) / blocks;
+    const int64_t rounds = (nch + QTHREADS / 64 - 1) / (QTHREADS / 64);   // chunks per wave
+    if (split > rounds) split = rounds;
+    hipLaunchKernelGGL(pmcc_moments_prep_kernel, dim3((unsigned)(blocks * split)), dim3(QTHREADS), 0, stream,
+                       x, n, dim, ldx, nch, (int)split, terms, scales, left, nleft);
+    return hipGetLastError();
+}
+
+template <bool SYM>
+hipError_t launch_moments(const MomentsPlan &m, MomentsArgs &args, hipStream_t stream)
+{
+    args.tiles_b = (args.nb + QBM - 1) / QBM;
+    const int64_t ids = m.tiles64;
+    const int64_t max_ids = int64_t(1) << 22;
+    for (int64_t off = 0; off < ids; off += max_ids) {
+        args.id_offset = off;
+        args.ids_this = (ids - off) < max_ids ? (ids - off) : max_ids;
+        hipLaunchKernelGGL(pmcc_moments_kernel<SYM>, dim3((unsigned)args.ids_this), dim3(QWAVES * 64), 0,
+                           stream, args);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 }  // namespace
 
 size_t pmcc_workspace_bytes(int use, int precision, int64_t na, int64_t nb, bool same,
                             int64_t dim)
 {
-    if (use != 0 || dim <= 0 || na <= 0 || nb <= 0) return 0;
+    if (dim <= 0 || na <= 0 || nb <= 0) return 0;
+    if (use == 1) return moments_plan(na, nb, same, dim).bytes;
     return side_bytes(precision, na, dim) + (same ? 0 : side_bytes(precision, nb, dim));
 }
 
@@ -964,6 +1317,41 @@ hipError_t launch_pmcc(int use, int precision, const float *a, int64_t na, int64
                                        reinterpret_cast<uintptr_t>(pairs)) & 15u) == 0;
         const int64_t ta = (na + WBM - 1) / WBM, tb = (nb + WBM - 1) / WBM;
         args.tiles_b = tb;
+        args.left = nullptr;
+        args.scale_a = args.scale_b = nullptr;
+        const MomentsPlan m = moments_plan(na, nb, same, dim);
+        if (m.bytes > 0 && workspace != nullptr) {
+            char *ws = static_cast<char *>(workspace);
+            MomentsArgs ma;
+            unsigned short *terms_a = reinterpret_cast<unsigned short *>(ws);
+            unsigned short *terms_b = same ? terms_a : reinterpret_cast<unsigned short *>(ws + m.off_b);
+            float *scale_a = reinterpret_cast<float *>(ws + m.off_scale);
+            float *scale_b = same ? scale_a : scale_a + na;
+            ma.left = reinterpret_cast<uint8_t *>(ws + m.off_left);
+            hipError_t e = launch_moments_prep(a, na, dim, lda, m.nch, terms_a, scale_a, ma.left,
+                                               m.tiles64, stream);
+            if (e == hipSuccess && !same)
+                e = launch_moments_prep(b, nb, dim, ldb, m.nch, terms_b, scale_b, ma.left, 0, stream);
+            if (e != hipSuccess) return e;
+            ma.ta = terms_a;
+            ma.tb = terms_b;
+            ma.na = na;
+            ma.nb = nb;
+            ma.nch = (int)m.nch;
+            // about sqrt(chunks) chunks per partial sum, so that both levels
+            // add about as many
+            ma.fold = 1;
+            while ((int64_t)(ma.fold + 1) * (ma.fold + 1) <= m.nch) ++ma.fold;
+            ma.corr = corr;
+            ma.ts = ts;
+            ma.pairs = pairs;
+            ma.ldo = ldo;
+            e = same ? launch_moments<true>(m, ma, stream) : launch_moments<false>(m, ma, stream);
+            if (e != hipSuccess) return e;
+            args.left = ma.left;   // the tiles left to two passes
+            args.scale_a = scale_a;
+            args.scale_b = scale_b;
+        }
         const int64_t total = same ? ta * (ta + 1) / 2 : ta * tb;
         const int64_t max_tiles = int64_t(1) << 23;
         for (int64_t off = 0; off < total; off += max_tiles) {

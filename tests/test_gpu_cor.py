@@ -280,3 +280,68 @@ def test_gputtest_matches_gpusignif():
     dt = gt.ttest(torch.from_numpy(n.astype(np.float32)).cuda(),
                   torch.from_numpy(r.astype(np.float32)).cuda())
     assert_bits_equal(dt.cpu().numpy(), want)
+
+
+def _pmcc_capi(a, b, workspace):
+    """gt_pmcc, pairwise.complete.obs, with the workspace it asks for or none."""
+    import ctypes
+    L = gt.lib()
+    same = b is None
+    bb = a if same else b
+    na, dim = a.shape
+    nb = bb.shape[0]
+    outs = [torch.full((na, nb), 7.0, device="cuda") for _ in range(3)]
+    need = ctypes.c_size_t()
+    assert L.gt_pmcc_workspace_size(1, 0, na, nb, dim, int(same), ctypes.byref(need)) == 0
+    ws = torch.full((max(need.value, 1),), 0xFF, dtype=torch.uint8, device="cuda")
+    s = L.gt_pmcc(1, 0, a.data_ptr(), na, a.stride(0), None if same else b.data_ptr(), nb,
+                  bb.stride(0), dim, outs[0].data_ptr(), outs[1].data_ptr(), outs[2].data_ptr(), nb,
+                  ws.data_ptr() if workspace else None, need.value if workspace else 0, None)
+    assert s == 0
+    torch.cuda.synchronize()
+    return need.value, [o.cpu().numpy() for o in outs]
+
+
+@pytest.mark.parametrize("dim,na,nb,scale", [(80, 31, 33, 1.0), (81, 64, 65, 1e-20), (95, 32, 0, 1e18),
+                                             (96, 65, 1, 1.0), (97, 129, 0, 1e-30), (128, 1, 0, 1.0),
+                                             (400, 96, 161, 1e-4), (777, 130, 0, 1.0)])
+def test_pairwise_matrix_form_edges(dim, na, nb, scale):
+    """The matrix-core form at the edges of its blocks (32 variables, 16
+    samples, 64 x 64 tiles), on unaligned strided rows, at extreme scales (the
+    pre-pass scales each variable by a power of two), with an Inf, a constant
+    variable and an empty one (their tiles are left to the two passes), from
+    a workspace full of garbage; and the same call without a workspace, which
+    runs on the VALU.  Both within 1e-5 of the oracle, counts exact."""
+    rng = np.random.default_rng(dim + na)
+
+    def make(n):
+        base = np.full((n, dim + 5), np.nan, np.float32)
+        v = _data(rng, dim, n, shift=3.0).T * np.float32(scale)
+        v[rng.random(v.shape) < 0.15] = np.nan
+        base[:, 3:3 + dim] = v
+        return base
+
+    xa = make(na)
+    if na > 96:
+        xa[1, 7] = np.inf
+        xa[2, 3:] = 2.0 * scale
+        xa[70, 3:] = np.nan
+    xb = make(nb) if nb else None
+    a = torch.from_numpy(xa).cuda()[:, 3:3 + dim]
+    b = None if xb is None else torch.from_numpy(xb).cuda()[:, 3:3 + dim]
+    print("case pairwise matrix form dim=%d na=%d nb=%d scale=%g" % (dim, na, nb, scale), flush=True)
+    av = np.ascontiguousarray(xa[:, 3:3 + dim])
+    bv = av if xb is None else np.ascontiguousarray(xb[:, 3:3 + dim])
+    # the oracle's sums in FP64 do not over- or underflow
+    pairs, corr = orc.pmcc(av, bv, "pairwise.complete.obs")
+    for workspace in (True, False):
+        need, (p, c, t) = _pmcc_capi(a, b, workspace)
+        assert need > 0
+        np.testing.assert_array_equal(p, pairs)
+        if not workspace and not 1e-15 < scale < 1e15:
+            continue   # the VALU form squares unscaled values
+        inf_rows = np.isinf(av).any(1)[:, None] | np.isinf(bv).any(1)[None, :]
+        ok = np.isfinite(corr) & ~inf_rows
+        assert np.max(np.abs(c[ok] - corr[ok]), initial=0.0) <= 1e-5
+        if xb is None:
+            np.testing.assert_array_equal(c, c.T)
