@@ -21,11 +21,17 @@
 // per row block, which write partial dX into a workspace; a second kernel
 // adds the JS partials in a fixed order.  No atomics: deterministic.
 //
-// The same kernel computes the metric-MDS stress S = sum_{i<j} (d_ij - delta_ij)^2
+// Euclidean gradients of up to 128 features run on the matrix cores instead
+// (gradient_kernel below): the distances in the split-precision Gram form of
+// gt_gram.hip, with near pairs recomputed from differences, and the
+// accumulation sum_j w_ij x_j as a product of split operands.
+//
+// The same sweep computes the metric-MDS stress S = sum_{i<j} (d_ij - delta_ij)^2
 // of an embedding Y and its gradient (G_ij = 2 (d_ij - delta_ij)); S is summed
 // in FP64 from per-workgroup partials (the only FP64 on the device).
 #include "gt_common.h"
 #include "gt_internal.h"
+#include "gt_mfma.h"
 
 namespace gt {
 namespace {
@@ -50,6 +56,9 @@ struct BwArgs {
     float *dxp;            // JS > 1: JS partial dX slices, n x k each
     double *partials;      // MODE_MDS: one per (row block, j split) workgroup
     float p, pm1;          // p and p - 1
+    // row blocks that gradient_kernel left (1 = left): only those run; null:
+    // every block runs
+    const uint8_t *left;
 };
 
 template <int OP>
@@ -79,6 +88,7 @@ __global__ __launch_bounds__(BTH) void backward_kernel(BwArgs args)
     const int tid = threadIdx.x;
     const int64_t n = args.n, k = args.k, ldx = args.ldx;
     const int64_t i0 = (int64_t)blockIdx.x * BI;
+    if (MODE == MODE_GRAD && args.left && args.left[blockIdx.x] == 0) return;
     const int64_t f0 = (int64_t)blockIdx.y * KB;
     const int64_t fcount = (k - f0) < KB ? (k - f0) : KB;
 
@@ -321,6 +331,394 @@ __global__ __launch_bounds__(BTH) void backward_kernel(BwArgs args)
     }
 }
 
+// ---------------------------------------------------------------------------
+// Euclidean gradient on the matrix cores
+// ---------------------------------------------------------------------------
+// dX_i = x_i sum_j w_ij - sum_j w_ij x_j with w_ij = G_ij / d_ij, on the centred
+// rows (both terms move alike).  A wave owns 32 rows i and visits blocks of 32
+// rows j.  The Gram block is computed with j along the accumulator's rows and i
+// along its columns, so element r of lane l is pair (i = l % 32, j = 8 (r / 4) +
+// 4 (l / 32) + r % 4): as it stands, registers 8 s .. 8 s + 7 of the weights are
+// the A operand of the second product for sixteen j, whose B operand (x_j, one
+// feature per lane) a pre-pass lays out in the same order of j.  Weights never
+// leave the registers.
+constexpr int GW = 8;                  // waves per workgroup, 32 rows i each
+constexpr int GROWS = GW * 32;
+constexpr int GTL = 36;                // row of a wave's transposed block of G
+constexpr int GOWN = 512 + 1024;       // floats of a wave's region: G, or near pairs and distances
+static_assert(32 * GTL <= GOWN, "transpose region");
+constexpr float GRAD_W_MIN = 0x1p-100f;
+constexpr int GRAD_NEAR_MAX = 160;     // near pairs of a 32 x 32 block, on average
+
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));   // rows start anywhere
+
+// This lane's rank among the set bits of m.
+__device__ __forceinline__ int rank_in(unsigned long long m)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+// norms read through the scalar cache: uniform addresses, not written by the kernel
+typedef const __attribute__((address_space(4))) float uniform_float_t;
+
+struct GradArgs {
+    const float *x;                    // FP32 rows (exact pairs)
+    int64_t n, k, ldx;
+    const unsigned short *terms;       // operand blocks of the centred rows (gt_mfma.h)
+    const unsigned short *tterms;      // the same values, features along the rows
+    const float *norms;                // squared norms of the centred rows
+    const float *center;
+    const float *g;                    // packed dL/dD
+    float *dx;
+    int64_t lddx;
+    float *dxp;                        // gridDim.y > 1: partial dX slices
+    uint8_t *left;                     // per BI rows: 1 = left to backward_kernel
+    int64_t jblocks;                   // blocks of 32 rows j, per workgroup
+    float tau;
+};
+
+// B operands of the second product: block jb (32 rows j), feature block cb (32
+// features), step s (sixteen j: 16 s + 8 p + 4 h + e, p < 2, e < 4), term t at
+// (((jb * ncb + cb) * 2 + s) * 3 + t) * OPERAND_VALUES, lane 32 h + c.  Also
+// clears `left`.
+__global__ __launch_bounds__(256) void gradient_terms_kernel(const float *__restrict__ x, int64_t n,
+                                                             int64_t k, int64_t ldx, int64_t ncb,
+                                                             const float *__restrict__ center,
+                                                             unsigned short *__restrict__ tterms,
+                                                             uint8_t *__restrict__ left)
+{
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int64_t nleft = (n + BI - 1) / BI;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < nleft; t += (int64_t)gridDim.x * 256)
+        left[t] = 0;
+    const int64_t blocks = operand_rows(n) / 32 * ncb * 2;
+    for (int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); blk < blocks;
+         blk += (int64_t)gridDim.x * 4) {
+        const int64_t s = blk & 1, cb = (blk >> 1) % ncb, jb = (blk >> 1) / ncb;
+        const int64_t c = cb * 32 + (lane & 31);
+        unsigned short t[8][3];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int64_t j = jb * 32 + s * 16 + (e >> 2) * 8 + h * 4 + (e & 3);
+            const float v = (j < n && c < k) ? x[j * ldx + c] - center[c] : 0.0f;
+            Split<SPLIT_BF16>::split(v, t[e]);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            uint4 w;
+            w.x = t[0][q] | ((unsigned)t[1][q] << 16);
+            w.y = t[2][q] | ((unsigned)t[3][q] << 16);
+            w.z = t[4][q] | ((unsigned)t[5][q] << 16);
+            w.w = t[6][q] | ((unsigned)t[7][q] << 16);
+            *reinterpret_cast<uint4 *>(tterms + (blk * 3 + q) * OPERAND_VALUES + lane * 8) = w;
+        }
+    }
+}
+
+// NC: chunks of 16 features (2, 4, 6 or 8).  A workgroup owns 256 rows i (blockIdx.x)
+// and a range of row blocks j (blockIdx.y); each block's two operand forms
+// stream through a two-stage LDS ring, G through registers.
+// Bound: the matrix cores and the VALU about alike (per 32 x 32 block and wave
+// 96 products, 3072 cycles, and about 500 VALU instructions, 2000 cycles, the
+// weights and their split).  Two waves a SIMD, from registers that hold the
+// wave's rows of the Gram product and its share of dX.  16384 x 128: 5.2 ms for
+// the sweep (two distances and an fma per feature and ordered pair on the
+// VALU), 1.1 ms here; the relative error of dX against FP64 8.2e-7 -> 4.0e-7.
+// A pair with d^2 < tau (||x_i||^2 + ||x_j||^2), or a d^2 that is not a normal
+// number, is recomputed from FP32 differences.  Rows with a weight that is not
+// finite or too small for three BF16 terms, or with many near pairs, are left to
+// backward_kernel (8000 x 128 in 32, 8 and 4 clusters: 0.52, 0.90 and 1.35 ms
+// with every near pair taken here, 1.28 ms for the sweep).
+template <int NC>
+__global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
+{
+    typedef Split<SPLIT_BF16> S;
+    constexpr int NCB = NC / 2;                       // blocks of 32 features
+    constexpr int HALF = NC * 3 * OPERAND_BYTES;      // one block j in one form
+    // [two stages of both operand forms][a region per wave].  One array: with
+    // two, the compiler waits for the direct loads in flight before every LDS
+    // read.
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * 2 * HALF + GW * GOWN * 4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float *const own = reinterpret_cast<float *>(smem + 2 * 2 * HALF) + wave * GOWN;
+    const int h = lane >> 5, col = lane & 31;
+    const int64_t n = args.n, k = args.k;
+    const int64_t i0 = (int64_t)blockIdx.x * GROWS + wave * 32;
+    const int64_t nblk = operand_rows(n) / 32;
+    const int64_t jb0 = (int64_t)blockIdx.y * args.jblocks;
+    const int64_t jb1 = jb0 + args.jblocks < nblk ? jb0 + args.jblocks : nblk;
+    bool idle = i0 >= n;                              // only helps to load
+    const int64_t i = i0 + col;
+    const int64_t ic = i < n ? i : n - 1;
+
+    typedef __attribute__((address_space(3))) void lds_void_t;
+    typedef const __attribute__((address_space(1))) void gbl_void_t;
+    auto issue = [&](int64_t jb) {
+        unsigned char *const st = smem + (jb & 1) * 2 * HALF;
+        const unsigned short *const a = args.terms + jb * NC * 3 * OPERAND_VALUES + lane * 8;
+        const unsigned short *const b = args.tterms + jb * NC * 3 * OPERAND_VALUES + lane * 8;
+        for (int u = wave; u < NC * 3; u += GW) {
+            __builtin_amdgcn_global_load_lds((gbl_void_t *)(a + u * OPERAND_VALUES),
+                                             (lds_void_t *)(st + u * OPERAND_BYTES), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gbl_void_t *)(b + u * OPERAND_VALUES),
+                                             (lds_void_t *)(st + HALF + u * OPERAND_BYTES), 16, 0, 0);
+        }
+    };
+    // G of block j0: below the diagonal (i > j) the packed index runs along i,
+    // the lanes; above it along j, so the lanes take j and the block is
+    // transposed through LDS when it is used
+    float gq[16] = {};
+    auto gfetch = [&](int64_t jb) {
+        const int64_t j0 = jb * 32;
+        if (j0 < i0) {
+            const float *const base = args.g + packed_base(n, j0) + ic;
+            const unsigned cw = (unsigned)(n - 1 - j0);
+            // row j0 + d + 4 h starts d cw - d (d + 1) / 2 + h (4 cw - 4 d - 10) on
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const unsigned d = 8 * (r >> 2) + (r & 3);
+                gq[r] = base[d * cw - d * (d + 1) / 2 + (h ? 4 * cw - 4 * d - 10 : 0u)];
+            }
+        } else if (j0 > i0) {
+            const int64_t j = j0 + col < n ? j0 + col : n - 1;
+            const float *const base = args.g + packed_base(n, i0) + j;
+            unsigned cw = (unsigned)(n - 1 - i0);
+            // the sixteen offsets do not change with jb: computed here each
+            // time, or they would be kept in registers that are not there
+            asm volatile("" : "+s"(cw));
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const unsigned d = 2 * r;
+                gq[r] = base[d * cw - d * (d + 1) / 2 + (h ? cw - d - 1 : 0u)];
+            }
+        } else {
+            int h4 = 4 * h;
+            asm volatile("" : "+v"(h4));
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t j = j0 + 8 * (r >> 2) + (r & 3) + h4;
+                const int64_t hi = i > j ? i : j, lo = i > j ? j : i;
+                gq[r] = (hi < n && lo != hi) ? args.g[packed_base(n, lo) + hi] : 0.0f;
+            }
+        }
+    };
+
+    bf16x8_t xi[NC][3];
+    f32x16_t dacc[NCB];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            xi[c][t] = *reinterpret_cast<const bf16x8_t *>(
+                args.terms + (((idle ? nblk - 1 : i0 / 32) * NC + c) * 3 + t) * OPERAND_VALUES + lane * 8);
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dacc[cb][r] = 0.0f;
+    const float ni = args.norms[ic];
+    float rowsum = 0.0f;
+    bool bad = false;
+    int seen = 0, seen_near = 0;                      // blocks, near pairs in them
+
+    if (jb0 < jb1) {
+        issue(jb0);
+        if (!idle) gfetch(jb0);
+    }
+    for (int64_t jb = jb0; jb < jb1; ++jb) {
+        const int64_t j0 = jb * 32;
+        // this block's operands (and G) have landed, in every wave, and every
+        // wave is done with the stage that the next issue overwrites
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // (a use of G here, or the compiler would wait for the next block's
+        // loads at its first use below)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(gq[r]));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (jb + 1 < jb1) issue(jb + 1);
+        if (idle) continue;
+        const unsigned char *const st = smem + (jb & 1) * 2 * HALF + lane * 16;
+        // ---- Gram block, smaller products first ------------------------------
+        f32x16_t w;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) w[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            bf16x8_t a[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                a[t] = *reinterpret_cast<const bf16x8_t *>(st + (c * 3 + t) * OPERAND_BYTES);
+            w = S::mfma(a[1], xi[c][1], w);
+            w = S::mfma(a[2], xi[c][0], w);
+            w = S::mfma(a[0], xi[c][2], w);
+            w = S::mfma(a[1], xi[c][0], w);
+            w = S::mfma(a[0], xi[c][1], w);
+            w = S::mfma(a[0], xi[c][0], w);
+            // keeps the later chunks' operands out of the registers
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // ---- weights -----------------------------------------------------------
+        if (j0 > i0) {
+            // G back with lanes along i (a wave's own region; LDS is in order)
+            float *const tr = own;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tr[(2 * r + h) * GTL + col] = gq[r];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 v = *reinterpret_cast<const float4 *>(tr + col * GTL + 8 * q + 4 * h);
+                gq[4 * q] = v.x;
+                gq[4 * q + 1] = v.y;
+                gq[4 * q + 2] = v.z;
+                gq[4 * q + 3] = v.w;
+            }
+        }
+        const bool edge = j0 == i0 || j0 + 32 > n || i0 + 32 > n;
+        unsigned flags = 0;
+        float part = 0.0f;
+        // (past the last row these read what follows the norms: no pair uses it)
+        uniform_float_t *const nj = (uniform_float_t *)(args.norms + j0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int lj = 8 * (r >> 2) + 4 * h + (r & 3);
+            const int64_t j = j0 + lj;
+            const float ss = ni + (h ? nj[8 * (r >> 2) + 4 + (r & 3)] : nj[8 * (r >> 2) + (r & 3)]);
+            const float d2 = fmaf(-2.0f, w[r], ss);
+            bool ok = d2 >= fmaf(args.tau, ss, GRAM_SQRT_MIN) && d2 < 0x1p127f;
+            // 1 / sqrt(d^2): the hardware estimate and one Newton step
+            float y = __builtin_amdgcn_rsqf(d2);
+            y = fmaf(0.5f * y, fmaf(-d2 * y, y, 1.0f), y);
+            float v = gq[r] * y;
+            if (edge) {
+                const bool pair = i < n && j < n && i != j;
+                ok = ok || !pair;
+                v = pair ? v : 0.0f;
+            }
+            w[r] = ok ? v : 0.0f;
+            flags |= ok ? 0u : 1u << r;
+        }
+        if (__builtin_amdgcn_ballot_w64(flags != 0u)) {
+            // Near pairs from differences: their list goes to LDS (the wave's
+            // own region), four lanes take a pair, sixteen pairs at a time,
+            // and the distances come back through LDS.
+            unsigned short *const list = reinterpret_cast<unsigned short *>(own);
+            float *const res = own + 512;
+            int near = 0;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const bool f = (flags >> r) & 1u;
+                const unsigned long long m = __builtin_amdgcn_ballot_w64(f);
+                if (f) list[near + rank_in(m)] = (unsigned short)(lane | (r << 6));
+                near += __popcll(m);
+            }
+            __builtin_amdgcn_wave_barrier();
+            seen_near += near;
+            if (seen >= 1 && seen_near > (seen + 1) * GRAD_NEAR_MAX) {
+                // points in a few clusters: differences throughout are cheaper
+                bad = idle = true;
+                continue;
+            }
+#pragma unroll 1
+            for (int e0 = 0; e0 < near; e0 += 16) {
+                const int e = e0 + (lane >> 2);
+                const int ent = list[e < near ? e : near - 1];
+                const int src = ent & 63, q = ent >> 6;
+                const float *const pi = args.x + (i0 + (src & 31)) * args.ldx;
+                const float *const pj = args.x + (j0 + 8 * (q >> 2) + 4 * (src >> 5) + (q & 3)) * args.ldx;
+                float s = 0.0f;
+#pragma unroll 2
+                for (int f = (lane & 3) * 4; f < (int)k; f += 16) {
+                    if (f + 4 <= (int)k) {
+                        const f32x4u_t d = *reinterpret_cast<const f32x4u_t *>(pi + f) -
+                                           *reinterpret_cast<const f32x4u_t *>(pj + f);
+                        s = fmaf(d[0], d[0], s);
+                        s = fmaf(d[1], d[1], s);
+                        s = fmaf(d[2], d[2], s);
+                        s = fmaf(d[3], d[3], s);
+                    } else {
+                        for (int u = f; u < (int)k; ++u) {
+                            const float d = pi[u] - pj[u];
+                            s = fmaf(d, d, s);
+                        }
+                    }
+                }
+                s += __shfl_xor(s, 1, 64);
+                s += __shfl_xor(s, 2, 64);
+                if ((lane & 3) == 0 && e < near) res[e] = sqrtf(s);
+            }
+            __builtin_amdgcn_wave_barrier();
+            near = 0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const bool f = (flags >> r) & 1u;
+                const unsigned long long m = __builtin_amdgcn_ballot_w64(f);
+                if (f) {
+                    const float dist = res[near + rank_in(m)];
+                    w[r] = dist > 0.0f ? gq[r] / dist : 0.0f;
+                }
+                near += __popcll(m);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        ++seen;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float a = fabsf(w[r]);
+            bad = bad || !(a < INFINITY) || (a < GRAD_W_MIN && a != 0.0f);
+            part += w[r];
+        }
+        rowsum += part;
+        if (jb + 1 < jb1) gfetch(jb + 1);
+        // ---- dX += W x_J ---------------------------------------------------------
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            bf16x8_t a[3];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                unsigned short t[3];
+                S::split(w[8 * s + e], t);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) a[q][e] = __builtin_bit_cast(__bf16, t[q]);
+            }
+#pragma unroll
+            for (int cb = 0; cb < NCB; ++cb) {
+                bf16x8_t b[3];
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    b[t] = *reinterpret_cast<const bf16x8_t *>(st + HALF + ((cb * 2 + s) * 3 + t) * OPERAND_BYTES);
+                dacc[cb] = S::mfma(a[1], b[1], dacc[cb]);
+                dacc[cb] = S::mfma(a[2], b[0], dacc[cb]);
+                dacc[cb] = S::mfma(a[0], b[2], dacc[cb]);
+                dacc[cb] = S::mfma(a[1], b[0], dacc[cb]);
+                dacc[cb] = S::mfma(a[0], b[1], dacc[cb]);
+                dacc[cb] = S::mfma(a[0], b[0], dacc[cb]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) args.left[i0 / BI] = 1;
+    if (idle) return;
+
+    rowsum += __shfl_xor(rowsum, 32, 64);
+    const bool slices = gridDim.y > 1;
+    float *const out = slices ? args.dxp + (int64_t)blockIdx.y * n * k : args.dx;
+    const int64_t ldo = slices ? k : args.lddx;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int li = 8 * (r >> 2) + 4 * h + (r & 3);
+        const float rs = __shfl(rowsum, li, 64);
+        const int64_t row = i0 + li;
+        if (row >= n) continue;
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            const int64_t c = cb * 32 + col;
+            if (c < k) out[row * ldo + c] = fmaf(args.x[row * args.ldx + c] - args.center[c], rs, -dacc[cb][r]);
+        }
+    }
+}
+
 // Sum of the per-workgroup FP64 partials, fixed order (deterministic).
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const double *partials, int64_t count,
                                                               double *out)
@@ -337,18 +735,69 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const double *part
     if (threadIdx.x == 0) *out = s_[0];
 }
 
-// dx = sum over the JS partial slices, in slice order.
+// dx = sum over the JS partial slices, in slice order (left_count slices for
+// the rows of the BI-row blocks marked in left).
 __global__ __launch_bounds__(256) void sum_partial_dx_kernel(const float *__restrict__ dxp, int64_t n,
                                                              int64_t k, int js_count,
+                                                             const uint8_t *__restrict__ left, int left_count,
                                                              float *__restrict__ dx, int64_t lddx)
 {
     const int64_t total = n * k;
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
         float s = dxp[e];
-        for (int q = 1; q < js_count; ++q) s += dxp[(int64_t)q * total + e];
+        const int count = left && left[e / k / BI] ? left_count : js_count;
+        for (int q = 1; q < count; ++q) s += dxp[(int64_t)q * total + e];
         dx[(e / k) * lddx + e % k] = s;
     }
+}
+
+// Workspace of gradient_kernel: the Gram pre-passes' (gt_gram.hip), the second
+// operand form, the flags and the partial slices.
+struct GradPlan {
+    int64_t kp, ncb, slices, jblocks;
+    int sweep_slices;      // of the rows that are left
+    size_t off_tterms, off_left, off_slices, bytes;
+};
+
+int j_splits(int64_t n, int64_t k);
+
+size_t align256(size_t v) { return (v + 255) / 256 * 256; }
+
+// Whether the matrix-core gradient takes the call.  Its operands of a block of
+// rows fit the registers up to 128 features; below 16 most pairs are near by
+// its rule (5 features, 4000 points: 206 us, and 115 for the sweep); with few
+// points the pre-passes cost more than they save (times in us, sweep and here:
+// 1000 x 96 50 and 55, 2000 x 96 88 and 70; 2000 x 32 41 and 58, 4000 x 32 122
+// and 77).  A sweep that needs no workspace can be captured; it stays.
+bool gradient_applies(int op, int64_t n, int64_t k)
+{
+    return op == OP_EUCLID && k <= 128 && ((k > 32 && n >= 1500) || (k >= 16 && n >= 3000)) &&
+           j_splits(n, k) > 1;
+}
+
+GradPlan gradient_plan(int64_t n, int64_t k)
+{
+    GradPlan g;
+    g.kp = (k + 31) / 32 * 32;
+    g.ncb = g.kp / 32;
+    const int64_t rows = (n + GROWS - 1) / GROWS, nblk = operand_rows(n) / 32;
+    // about 1024 workgroups in all, at most 16 slices, at least two blocks each
+    int64_t js = (1024 + rows - 1) / rows;
+    if (js > 16) js = 16;
+    if (js > (nblk + 1) / 2) js = (nblk + 1) / 2;
+    g.jblocks = (nblk + js - 1) / js;
+    g.slices = (nblk + g.jblocks - 1) / g.jblocks;
+    g.sweep_slices = j_splits(n, k) < g.slices ? j_splits(n, k) : (int)g.slices;
+    size_t p = align256(gram_workspace_bytes(n, k, 1));
+    g.off_tterms = p;
+    p += (size_t)operand_rows(n) * (size_t)g.kp * 3 * sizeof(unsigned short);
+    g.off_left = p;
+    p += align256((size_t)nblk);
+    g.off_slices = p;
+    if (g.slices > 1) p += (size_t)g.slices * (size_t)n * (size_t)k * sizeof(float);
+    g.bytes = p;
+    return g;
 }
 
 int feature_block(int64_t k) { return k <= 4 ? 4 : (k <= 32 ? 32 : KBMAX); }
@@ -362,6 +811,16 @@ int j_splits(int64_t n, int64_t k)
     if (js > 16) js = 16;
     if (js > gx) js = gx;
     return (int)(js < 1 ? 1 : js);
+}
+
+hipError_t launch_sum(const float *dxp, int64_t n, int64_t k, int slices, const uint8_t *left, int left_slices,
+                      float *dx, int64_t lddx, hipStream_t stream)
+{
+    int64_t blocks = (n * k + 255) / 256;
+    if (blocks > 65536) blocks = 65536;
+    hipLaunchKernelGGL(sum_partial_dx_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, dxp, n, k, slices,
+                       left, left_slices, dx, lddx);
+    return hipGetLastError();
 }
 
 template <int MODE, int KB>
@@ -378,29 +837,83 @@ hipError_t launch_kb(int op, BwArgs &args, int js, hipStream_t stream)
 }
 
 template <int MODE>
+hipError_t launch_sweep(int op, BwArgs &args, int js, hipStream_t stream)
+{
+    if (args.k <= 4) return launch_kb<MODE, 4>(op, args, js, stream);
+    if (args.k <= 32) return launch_kb<MODE, 32>(op, args, js, stream);
+    return launch_kb<MODE, KBMAX>(op, args, js, stream);
+}
+
+template <int MODE>
 hipError_t launch_mode(int op, BwArgs &args, hipStream_t stream)
 {
     const int js = j_splits(args.n, args.k);
-    hipError_t e;
-    if (args.k <= 4)
-        e = launch_kb<MODE, 4>(op, args, js, stream);
-    else if (args.k <= 32)
-        e = launch_kb<MODE, 32>(op, args, js, stream);
-    else
-        e = launch_kb<MODE, KBMAX>(op, args, js, stream);
+    const hipError_t e = launch_sweep<MODE>(op, args, js, stream);
     if (e != hipSuccess || js == 1 || args.dx == nullptr) return e;
-    int64_t blocks = (args.n * args.k + 255) / 256;
+    return launch_sum(args.dxp, args.n, args.k, js, nullptr, 0, args.dx, args.lddx, stream);
+}
+
+// The matrix-core gradient: pre-passes, products, the sweep over the rows that
+// were left, sum of the slices.
+hipError_t launch_gradient(BwArgs &args, void *workspace, hipStream_t stream)
+{
+    const GradPlan g = gradient_plan(args.n, args.k);
+    char *ws = static_cast<char *>(workspace);
+    GramPrep prep;
+    hipError_t e = gram_prepare(1, args.x, args.n, args.k, args.ldx, workspace, prep, stream);
+    if (e != hipSuccess) return e;
+    GradArgs ga;
+    ga.x = args.x;
+    ga.n = args.n;
+    ga.k = args.k;
+    ga.ldx = args.ldx;
+    ga.terms = prep.terms;
+    ga.tterms = reinterpret_cast<unsigned short *>(ws + g.off_tterms);
+    ga.norms = prep.norms;
+    ga.center = prep.center;
+    ga.g = args.g;
+    ga.dx = args.dx;
+    ga.lddx = args.lddx;
+    ga.dxp = reinterpret_cast<float *>(ws + g.off_slices);
+    ga.left = reinterpret_cast<uint8_t *>(ws + g.off_left);
+    ga.jblocks = g.jblocks;
+    // pairs this near lose more in the Gram form than differences do
+    ga.tau = fmaxf(gram_tau(1, args.k), 0.25f);
+    int64_t blocks = (operand_rows(args.n) / 32 * g.ncb * 2 + 3) / 4;
     if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(sum_partial_dx_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, args.dxp,
-                       args.n, args.k, js, args.dx, args.lddx);
-    return hipGetLastError();
+    hipLaunchKernelGGL(gradient_terms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, args.x, args.n,
+                       args.k, args.ldx, g.ncb, prep.center, const_cast<unsigned short *>(ga.tterms), ga.left);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const dim3 grid((unsigned)((args.n + GROWS - 1) / GROWS), (unsigned)g.slices);
+    switch (g.ncb) {
+    case 1: hipLaunchKernelGGL(gradient_kernel<2>, grid, dim3(GW * 64), 0, stream, ga); break;
+    case 2: hipLaunchKernelGGL(gradient_kernel<4>, grid, dim3(GW * 64), 0, stream, ga); break;
+    case 3: hipLaunchKernelGGL(gradient_kernel<6>, grid, dim3(GW * 64), 0, stream, ga); break;
+    default: hipLaunchKernelGGL(gradient_kernel<8>, grid, dim3(GW * 64), 0, stream, ga); break;
+    }
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    // the rows that were left, over their slices
+    args.left = ga.left;
+    args.dxp = ga.dxp;
+    e = launch_sweep<MODE_GRAD>(BW_EUCLID, args, g.sweep_slices, stream);
+    if (e != hipSuccess || g.slices == 1) return e;
+    // (sweep_slices > 1 here: gradient_applies)
+    return launch_sum(ga.dxp, args.n, args.k, (int)g.slices, ga.left, g.sweep_slices, args.dx, args.lddx,
+                      stream);
 }
 
 }  // namespace
 
 int64_t mds_partials_count(int64_t n, int64_t q) { return (n + BI - 1) / BI * j_splits(n, q); }
 
-size_t backward_workspace_bytes(int64_t n, int64_t k)
+size_t backward_workspace_bytes(int op, int64_t n, int64_t k)
+{
+    if (n < 2 || k < 1) return 0;
+    if (gradient_applies(op, n, k)) return gradient_plan(n, k).bytes;
+    return sweep_workspace_bytes(n, k);
+}
+
+size_t sweep_workspace_bytes(int64_t n, int64_t k)
 {
     if (n < 2 || k < 1) return 0;
     const int js = j_splits(n, k);
@@ -424,6 +937,8 @@ hipError_t launch_backward(int op, const float *x, int64_t n, int64_t k, int64_t
     args.partials = nullptr;
     args.p = p;
     args.pm1 = p - 1.0f;
+    args.left = nullptr;
+    if (gradient_applies(op, n, k)) return launch_gradient(args, workspace, stream);
     const int bop = (op == OP_EUCLID) ? BW_EUCLID : (op == OP_MINK3) ? BW_MINK3 : BW_MINKP;
     return launch_mode<MODE_GRAD>(bop, args, stream);
 }
@@ -444,6 +959,7 @@ hipError_t launch_mds(const float *y, int64_t n, int64_t q, int64_t ldy, const f
     args.partials = partials;
     args.p = 2.0f;
     args.pm1 = 1.0f;
+    args.left = nullptr;
     hipError_t e = launch_mode<MODE_MDS>(BW_EUCLID, args, stream);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, stream, partials,

@@ -47,7 +47,6 @@ constexpr int FCAP = 1024;      // flagged pairs per fix-up pass
 // Gram-form values are finished with the hardware square root (v_sqrt_f32)
 // plus one residual correction (sqrt_rn), which rounds correctly for normal
 // inputs; d^2 below 2^-100 goes to the exact pass instead.
-constexpr float GRAM_SQRT_MIN = 0x1p-100f;
 constexpr int TERM_BYTES = GBM / 32 * OPERAND_BYTES;   // one split term of one side, one chunk (8 KB)
 constexpr int FIX_BYTES = 2 * GBM * FLD * 4;   // fix-up staging, both sides
 constexpr int LIST_BYTES = FCAP * 4;
@@ -771,28 +770,33 @@ hipError_t launch_tiles(GramArgs &args, int64_t ids, hipStream_t stream)
 }
 
 template <int SPLIT>
-hipError_t launch_split(int layout, bool vec4, GramArgs &args, const float *center,
-                        const float *scales, int64_t ids, hipStream_t stream)
+hipError_t launch_layout(int layout, bool vec4, GramArgs &args, int64_t ids, hipStream_t stream)
 {
-    {
-        int64_t blocks = (operand_rows(args.n) / 32 * (args.kp / OPERAND_K) + 3) / 4;
-        if (blocks > 65536) blocks = 65536;
-        if (vec4)
-            hipLaunchKernelGGL((split_kernel<SPLIT, true>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                               args.x, args.n, args.k, args.ldx, args.kp, center, scales,
-                               const_cast<unsigned short *>(args.terms));
-        else
-            hipLaunchKernelGGL((split_kernel<SPLIT, false>), dim3((unsigned)blocks), dim3(256), 0,
-                               stream, args.x, args.n, args.k, args.ldx, args.kp, center, scales,
-                               const_cast<unsigned short *>(args.terms));
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
     if (layout == OUT_PACKED)
         return vec4 ? launch_tiles<SPLIT, OUT_PACKED, true>(args, ids, stream)
                     : launch_tiles<SPLIT, OUT_PACKED, false>(args, ids, stream);
     return vec4 ? launch_tiles<SPLIT, OUT_FULL, true>(args, ids, stream)
                 : launch_tiles<SPLIT, OUT_FULL, false>(args, ids, stream);
+}
+
+template <int SPLIT>
+hipError_t launch_split(bool vec4, const float *x, int64_t n, int64_t k, int64_t ldx, const GramPrep &prep,
+                        hipStream_t stream)
+{
+    int64_t blocks = (operand_rows(n) / 32 * (prep.kp / OPERAND_K) + 3) / 4;
+    if (blocks > 65536) blocks = 65536;
+    if (vec4)
+        hipLaunchKernelGGL((split_kernel<SPLIT, true>), dim3((unsigned)blocks), dim3(256), 0, stream, x, n, k,
+                           ldx, prep.kp, prep.center, prep.scales, prep.terms);
+    else
+        hipLaunchKernelGGL((split_kernel<SPLIT, false>), dim3((unsigned)blocks), dim3(256), 0, stream, x, n,
+                           k, ldx, prep.kp, prep.center, prep.scales, prep.terms);
+    return hipGetLastError();
+}
+
+bool rows_vec4(const float *x, int64_t k, int64_t ldx)
+{
+    return (k % 4 == 0) && (ldx % 4 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15u) == 0);
 }
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -856,29 +860,23 @@ float gram_tau(int precision, int64_t k)
     return (float)(tau > 0.125 ? tau : 0.125);
 }
 
-// Above this tau nearly every pair would be recomputed: the request is
-// computed by the FP32 difference kernel instead.
-constexpr float GRAM_TAU_MAX = 0.9f;
-
-hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int64_t k,
-                       int64_t ldx, float *out, int64_t ldd, void *workspace, hipStream_t stream)
+// The pre-passes: column centres, row norms (FP16: row scales) and the split
+// terms, all in the workspace (gram_workspace_bytes).
+hipError_t gram_prepare(int precision, const float *x, int64_t n, int64_t k, int64_t ldx, void *workspace,
+                        GramPrep &prep, hipStream_t stream)
 {
-    if (n < 2 && layout == OUT_PACKED) return hipSuccess;
-    const float tau = gram_tau(precision, k);
-    if (tau > GRAM_TAU_MAX)
-        return launch_plain(OP_EUCLID, layout, x, n, ldx, x, n, ldx, k, 2.0f, out, ldd, stream);
-    const int64_t kp = padded_k(k);
+    prep.kp = padded_k(k);
     char *ws = static_cast<char *>(workspace);
-    unsigned short *terms = reinterpret_cast<unsigned short *>(ws);
-    ws += align256((size_t)split_terms(precision) * (size_t)operand_rows(n) * (size_t)kp *
+    prep.terms = reinterpret_cast<unsigned short *>(ws);
+    ws += align256((size_t)split_terms(precision) * (size_t)operand_rows(n) * (size_t)prep.kp *
                    sizeof(unsigned short));
-    float *norms = reinterpret_cast<float *>(ws);
+    prep.norms = reinterpret_cast<float *>(ws);
     ws += align256((size_t)n * sizeof(float));
-    float *scales = reinterpret_cast<float *>(ws);
+    prep.scales = reinterpret_cast<float *>(ws);
     ws += align256((size_t)n * sizeof(float));
-    float *iscales = reinterpret_cast<float *>(ws);
+    prep.iscales = reinterpret_cast<float *>(ws);
     ws += align256((size_t)n * sizeof(float));
-    float *center = reinterpret_cast<float *>(ws);
+    prep.center = reinterpret_cast<float *>(ws);
     ws += align256((size_t)k * sizeof(float));
     const int64_t csb = colstats_blocks(n);
     const size_t pbytes = align256((size_t)csb * (size_t)k * sizeof(float));
@@ -894,7 +892,7 @@ hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int
         if (e != hipSuccess) return e;
         const int64_t fb = (k + CS_COLS - 1) / CS_COLS;
         hipLaunchKernelGGL(colstats_finish_kernel, dim3((unsigned)(fb < 65536 ? fb : 65536)), dim3(256),
-                           0, stream, psum, pmin, pmax, csb, n, k, center);
+                           0, stream, psum, pmin, pmax, csb, n, k, prep.center);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -902,29 +900,49 @@ hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int
         int64_t blocks = (n + 3) / 4;
         if (blocks > 65536) blocks = 65536;
         hipLaunchKernelGGL(row_prep_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, k,
-                           ldx, center, norms, fp16 ? scales : nullptr, fp16 ? iscales : nullptr);
+                           ldx, prep.center, prep.norms, fp16 ? prep.scales : nullptr,
+                           fp16 ? prep.iscales : nullptr);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
+    const bool vec4 = rows_vec4(x, k, ldx);
+    return fp16 ? launch_split<SPLIT_FP16>(vec4, x, n, k, ldx, prep, stream)
+                : launch_split<SPLIT_BF16>(vec4, x, n, k, ldx, prep, stream);
+}
+
+// Above this tau nearly every pair would be recomputed: the request is
+// computed by the FP32 difference kernel instead.
+constexpr float GRAM_TAU_MAX = 0.9f;
+
+hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int64_t k,
+                       int64_t ldx, float *out, int64_t ldd, void *workspace, hipStream_t stream)
+{
+    if (n < 2 && layout == OUT_PACKED) return hipSuccess;
+    const float tau = gram_tau(precision, k);
+    if (tau > GRAM_TAU_MAX)
+        return launch_plain(OP_EUCLID, layout, x, n, ldx, x, n, ldx, k, 2.0f, out, ldd, stream);
+    GramPrep prep;
+    hipError_t e = gram_prepare(precision, x, n, k, ldx, workspace, prep, stream);
+    if (e != hipSuccess) return e;
+    const bool fp16 = (precision == 2);
     GramArgs args;
     args.x = x;
     args.n = n;
     args.k = k;
     args.ldx = ldx;
-    args.terms = terms;
-    args.kp = kp;
-    args.norms = norms;
-    args.iscale = iscales;
+    args.terms = prep.terms;
+    args.kp = prep.kp;
+    args.norms = prep.norms;
+    args.iscale = prep.iscales;
     args.out = out;
     args.ldd = ldd;
     args.T = (n + GBM - 1) / GBM;
     args.tau = tau;
     const int64_t S = (args.T + GSUPER - 1) / GSUPER;
     const int64_t ids = S * (S + 1) / 2 * GSUPER * GSUPER;
-    const bool vec4 = (k % 4 == 0) && (ldx % 4 == 0) &&
-                      ((reinterpret_cast<uintptr_t>(x) & 15u) == 0);
-    return fp16 ? launch_split<SPLIT_FP16>(layout, vec4, args, center, scales, ids, stream)
-                : launch_split<SPLIT_BF16>(layout, vec4, args, center, scales, ids, stream);
+    const bool vec4 = rows_vec4(x, k, ldx);
+    return fp16 ? launch_layout<SPLIT_FP16>(layout, vec4, args, ids, stream)
+                : launch_layout<SPLIT_BF16>(layout, vec4, args, ids, stream);
 }
 
 }  // namespace gt

@@ -55,14 +55,28 @@ hipError_t launch_fill_full(float *out, int64_t n, int64_t ldd, float offdiag,
 size_t gram_workspace_bytes(int64_t n, int64_t k, int precision);
 size_t gram_rounding_bytes(int64_t n, int64_t k, int precision);
 constexpr size_t GRAM_ROW_SLACK = (size_t)2 << 20;
+// Its pre-passes, and what they leave in the workspace.
+struct GramPrep {
+    int64_t kp;              // k padded
+    unsigned short *terms;   // split terms, in operand blocks (gt_mfma.h)
+    float *norms;            // squared norms of the centred rows
+    float *scales, *iscales; // FP16: power-of-two row scales and their inverses
+    float *center;           // column centres
+};
+hipError_t gram_prepare(int precision, const float *x, int64_t n, int64_t k, int64_t ldx, void *workspace,
+                        GramPrep &prep, hipStream_t stream);
+float gram_tau(int precision, int64_t k);
+constexpr float GRAM_SQRT_MIN = 0x1p-100f;   // smaller squared distances go to the exact pass
 hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int64_t k,
                        int64_t ldx, float *out, int64_t ldd, void *workspace,
                        hipStream_t stream);
 
 // Backward (dL/dX) and fused MDS stress.  op: OP_EUCLID, OP_MINK3 or OP_MINKP.
-// workspace: backward_workspace_bytes(n, k) (partial dX slices when the j
-// blocks are split over workgroups; 0 otherwise).
-size_t backward_workspace_bytes(int64_t n, int64_t k);
+// workspace: backward_workspace_bytes(op, n, k) (partial dX slices when the j
+// blocks are split over workgroups, and the matrix-core form's operands; 0
+// otherwise); the MDS sweep takes sweep_workspace_bytes.
+size_t backward_workspace_bytes(int op, int64_t n, int64_t k);
+size_t sweep_workspace_bytes(int64_t n, int64_t k);
 hipError_t launch_backward(int op, const float *x, int64_t n, int64_t k, int64_t ldx,
                            float p, const float *g_packed, float *dx, int64_t lddx,
                            float *workspace, hipStream_t stream);

@@ -125,3 +125,72 @@ def test_backward_rejects_other_methods():
         gt.dist_backward(x, g, "manhattan")
     with pytest.raises(gt.GputoolsError, match="INVALID"):
         gt.dist_backward(x, g, "minkowski", 0.5)
+
+
+@pytest.mark.parametrize("n,k,data", [(1500, 33, "normal"), (1537, 64, "offset"), (1793, 97, "mixture"),
+                                      (2049, 128, "normal"), (3000, 16, "uniform"), (3009, 31, "clusters"),
+                                      (1600, 128, "clusters"), (1700, 50, "duplicates"),
+                                      (1700, 96, "upstream")])
+def test_matrix_core_gradient(n, k, data):
+    """The matrix-core form (euclidean, up to 128 features) at the edges of its
+    blocks, on strided rows that start anywhere, where the Gram form needs its
+    near pairs recomputed (mixture, duplicates: subgradient 0), where most
+    pairs are near (two clusters: rows left to the sweep), and with upstream
+    gradients that three BF16 terms cannot hold (1e-36: rows left).  Centred
+    data far from the origin: the reference is the oracle on the FP32 values;
+    its gradient cancels, so the bound is relative to the terms there."""
+    rng = np.random.default_rng(n + k)
+    base = rng.standard_normal((n, k + 3)).astype(np.float32)
+    x = base[:, 1:k + 1]
+    if data == "uniform":
+        x[:] = rng.random((n, k))
+    elif data == "offset":
+        x += np.float32(100.0)
+    elif data == "mixture":
+        x[:] = x * np.float32(1e-3) + rng.standard_normal((64, k)).astype(np.float32)[np.arange(n) % 64]
+    elif data == "clusters":
+        x[:] = x * np.float32(1e-2) + rng.standard_normal((2, k)).astype(np.float32)[rng.integers(0, 2, n)]
+    elif data == "duplicates":
+        x[n // 2:n // 2 + 90] = x[:90]
+        x[33] = x[32]
+    g = rng.standard_normal(n * (n - 1) // 2).astype(np.float32)
+    if data == "upstream":
+        g[::1001] = 1e-36
+        g[5::977] = 0.0
+    print("case matrix-core gradient n=%d k=%d %s" % (n, k, data), flush=True)
+    xd = dev(base)[:, 1:k + 1]
+    got = gt.dist_backward(xd, dev(g), "euclidean").cpu().numpy()
+    again = gt.dist_backward(xd, dev(g), "euclidean").cpu().numpy()
+    np.testing.assert_array_equal(got, again)          # deterministic
+    want = orc.dist_backward(np.ascontiguousarray(x), g.astype(np.float64), "euclidean")
+    # near pairs have large weights whose sum cancels against w x_j: FP32 sums
+    # of terms |w| |x| 1e-2 or 1e-3 apart carry that factor (the sweep's error
+    # there is 1e-5 to 8e-5)
+    close = {"mixture": 2e-4, "clusters": 5e-5}.get(data, 1e-5)
+    assert_grad_close(got, want, frob=close, elem=max(1e-4, 2 * close))
+
+
+def test_matrix_core_gradient_non_finite_upstream():
+    """An infinite and a NaN entry of dL/dD reach the rows of their pairs and no
+    other: the other rows equal those without the entries."""
+    n, k = 1600, 40
+    rng = np.random.default_rng(7)
+    x = dev(rng.standard_normal((n, k)))
+    g = rng.standard_normal(n * (n - 1) // 2).astype(np.float32)
+
+    def at(i, j):   # i > j
+        return j * n - j * (j + 1) // 2 + i - j - 1
+
+    clean = g.copy()
+    clean[at(700, 3)] = clean[at(1300, 900)] = 0.0
+    g[at(700, 3)] = np.inf
+    g[at(1300, 900)] = np.nan
+    print("case matrix-core gradient non-finite", flush=True)
+    got = gt.dist_backward(x, dev(g)).cpu().numpy()
+    want = gt.dist_backward(x, dev(clean)).cpu().numpy()
+    hit = np.zeros(n, bool)
+    hit[[700, 3, 1300, 900]] = True
+    assert not np.isfinite(got[hit]).all(1).any()
+    assert np.isfinite(got[~hit]).all()
+    rel = np.linalg.norm(got[~hit].astype(np.float64) - want[~hit]) / np.linalg.norm(want[~hit])
+    assert rel <= 1e-5
