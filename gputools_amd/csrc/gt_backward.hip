@@ -719,6 +719,240 @@ __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
     }
 }
 
+// ---------------------------------------------------------------------------
+// MDS of few features
+// ---------------------------------------------------------------------------
+// Up to 8 features a pair is a handful of instructions and four bytes of
+// delta, so each pair is visited once and serves both of its rows.  A workgroup
+// owns 256 rows i and 4 jw columns j < i, a wave jw of the columns; a lane holds
+// four rows i (lanes along i, as the packed columns run) and walks the columns,
+// whose rows are uniform (scalar loads).  The sums of row i stay in its lane;
+// those of row j are added over the lane's four rows, then over the wave by
+// data-parallel adds.  Each term is w (y_i - y_j): sums of w and of w y_j apart
+// cancel where points are close.  Both sides go to partial slices, which
+// mds_finish_kernel adds in a fixed order: deterministic, no atomics.
+// Bound: VALU issue (about 45 instructions per pair with 2 features, two of them
+// FP64; delta alone would take 0.11 ms).  16384 x 2: 0.67 ms for the sweep, which
+// visits each pair from both rows and pads 2 features to 4, 0.18 ms here; the
+// relative error of dY against FP64 9.0e-7 -> 1.9e-7.
+constexpr int MI = 256;                            // rows of a workgroup
+constexpr int MR = MI / 64;                        // rows per lane
+constexpr int MSUM = 8;                            // threads per row in mds_finish_kernel
+
+struct MdsArgs {
+    const float *y;
+    int64_t n, q, ldy;
+    const float *delta;
+    int jw;                    // columns per wave: 16, 32 or 64
+    float *ipart, *jpart;      // [slice][feature][row]: rows i by column block, rows j by row block
+    double *partials;          // stress, one per workgroup
+};
+
+// Sum over the wave, in lane 63.
+__device__ __forceinline__ float wave_total(float v)
+{
+#define GT_DPP_ADD(ctrl, rows) \
+    v += __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), ctrl, rows, 0xf, false))
+    GT_DPP_ADD(0x111, 0xf);   // row_shr:1
+    GT_DPP_ADD(0x112, 0xf);   // row_shr:2
+    GT_DPP_ADD(0x114, 0xf);   // row_shr:4
+    GT_DPP_ADD(0x118, 0xf);   // row_shr:8
+    GT_DPP_ADD(0x142, 0xa);   // row_bcast:15
+    GT_DPP_ADD(0x143, 0xc);   // row_bcast:31
+#undef GT_DPP_ADD
+    return v;
+}
+
+extern "C" __device__ int gt_mds_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
+// One column j against the lane's rows.  EDGE: rows at or before j, or past
+// the end, do not count.
+template <int Q, bool GRAD, bool EDGE>
+__device__ __forceinline__ void mds_column(const float (&xi)[MR][Q], const float (&xj)[Q], const float (&dl)[MR],
+                                           int64_t i0, int64_t j, int64_t n, int lane, double &stress,
+                                           float (&wi)[MR][Q], float (&wj)[Q])
+{
+#pragma unroll
+    for (int c = 0; c < Q; ++c) wj[c] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+        float t[Q], d2 = 0.0f;
+#pragma unroll
+        for (int c = 0; c < Q; ++c) {
+            t[c] = xi[r][c] - xj[c];
+            d2 = fmaf(t[c], t[c], d2);
+        }
+        // d = sqrt(d2) and inv = 1 / d: the hardware estimate of the inverse
+        // root, one correction of the root
+        float inv = __builtin_amdgcn_rsqf(d2);
+        float d = d2 * inv;
+        d = fmaf(0.5f * inv, fmaf(-d, d, d2), d);
+        bool apart = true;
+        if (!(d2 >= 0x1p-100f && d2 <= 0x1p120f)) {   // 0, tiny, huge, not a number
+            d = sqrtf(d2);
+            inv = 1.0f / d;
+            apart = d > 0.0f;
+        }
+        float res = apart ? d - dl[r] : -dl[r];
+        if (EDGE) {
+            const int64_t i = i0 + r * 64 + lane;
+            const bool pair = i > j && i < n;
+            res = pair ? res : 0.0f;
+            apart = apart && pair;
+        }
+        stress = fma((double)res, (double)res, stress);
+        if (GRAD) {
+            const float w = apart ? 2.0f * res * inv : 0.0f;
+#pragma unroll
+            for (int c = 0; c < Q; ++c) {
+                wi[r][c] = fmaf(w, t[c], wi[r][c]);
+                wj[c] = fmaf(-w, t[c], wj[c]);
+            }
+        }
+    }
+}
+
+template <int Q, bool GRAD>
+__global__ __launch_bounds__(256) void mds_small_kernel(MdsArgs args)
+{
+    __shared__ float red[3][MI][Q];
+    __shared__ double red_s[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t n = args.n;
+    // row block ci has f (ci + 1) column blocks, f = 256 / (4 jw)
+    const int64_t t = blockIdx.x;
+    const int f = 64 / args.jw;
+    int ci, cm;
+    tri_tile(t / f, ci, cm);
+    const int64_t cj = (int64_t)cm * f + t % f;
+    const int64_t i0 = (int64_t)ci * MI;
+    const int64_t j0 = (cj * 4 + wave) * args.jw;
+    int64_t j1 = j0 + args.jw < n ? j0 + args.jw : n;
+
+    float xi[MR][Q], wi[MR][Q];
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+        const int64_t i = i0 + r * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < Q; ++c) xi[r][c] = (i < n && c < args.q) ? args.y[i * args.ldy + c] : 0.0f;
+#pragma unroll
+        for (int c = 0; c < Q; ++c) wi[r][c] = 0.0f;
+    }
+    double stress = 0.0;
+    const bool edge = j1 > i0 || i0 + MI > n;
+    auto load = [&](int64_t j, float (&xj)[Q], float (&dl)[MR]) {
+        uniform_float_t *const yj = (uniform_float_t *)(args.y + j * args.ldy);
+#pragma unroll
+        for (int c = 0; c < Q; ++c) xj[c] = c < args.q ? yj[c] : 0.0f;
+        const float *const col = args.delta + packed_base(n, j) + i0;
+#pragma unroll
+        for (int r = 0; r < MR; ++r) {
+            const int li = r * 64 + lane;
+            dl[r] = (!edge || (i0 + li > j && i0 + li < n)) ? col[li] : 0.0f;
+        }
+    };
+    if (j0 < j1) {
+        const int64_t jc = j0;
+        const int count = (int)(j1 - j0);
+        float out[Q];   // lane l: the sums of row jc + l
+#pragma unroll
+        for (int c = 0; c < Q; ++c) out[c] = 0.0f;
+        for (int l = 0; l < count; l += 4) {
+            float xj[4][Q], dl[4][MR];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                load(l + u < count ? jc + l + u : jc + count - 1, xj[u], dl[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (l + u >= count) break;
+                float wj[Q];
+                if (edge)
+                    mds_column<Q, GRAD, true>(xi, xj[u], dl[u], i0, jc + l + u, n, lane, stress, wi, wj);
+                else
+                    mds_column<Q, GRAD, false>(xi, xj[u], dl[u], i0, jc + l + u, n, lane, stress, wi, wj);
+                if (GRAD) {
+#pragma unroll
+                    for (int c = 0; c < Q; ++c) {
+                        const int total = __builtin_amdgcn_readlane((int)__float_as_uint(wave_total(wj[c])), 63);
+                        out[c] = __uint_as_float((unsigned)gt_mds_writelane(total, l + u, (int)__float_as_uint(out[c])));
+                    }
+                }
+            }
+        }
+        if (GRAD && lane < count) {
+#pragma unroll
+            for (int c = 0; c < Q; ++c)
+                if (c < args.q) args.jpart[(ci * args.q + c) * n + jc + lane] = out[c];
+        }
+    }
+    // the four waves' sums of the rows i, in order
+    if (GRAD) {
+        if (wave > 0)
+#pragma unroll
+            for (int r = 0; r < MR; ++r)
+#pragma unroll
+                for (int c = 0; c < Q; ++c) red[wave - 1][r * 64 + lane][c] = wi[r][c];
+        __syncthreads();
+        if (wave == 0)
+#pragma unroll
+            for (int r = 0; r < MR; ++r) {
+                const int64_t i = i0 + r * 64 + lane;
+#pragma unroll
+                for (int c = 0; c < Q; ++c) {
+                    float v = wi[r][c];
+                    for (int w = 0; w < 3; ++w) v += red[w][r * 64 + lane][c];
+                    if (i < n && c < args.q) args.ipart[(cj * args.q + c) * n + i] = v;
+                }
+            }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) stress += __shfl_xor(stress, d, 64);
+    if (lane == 0) red_s[wave] = stress;
+    __syncthreads();
+    if (tid == 0) args.partials[t] = ((red_s[0] + red_s[1]) + red_s[2]) + red_s[3];
+}
+
+// dY_r from the slices of row r: its column blocks as a
+// row i, then the row blocks from its own on as a row j.  MSUM threads a row;
+// the last workgroup adds the stress partials.
+__global__ __launch_bounds__(256) void mds_finish_kernel(MdsArgs args, float *__restrict__ dy, int64_t lddy,
+                                                         int64_t count, double *__restrict__ stress)
+{
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ double s_[256];
+        double s = 0.0;
+        for (int64_t e = threadIdx.x; e < count; e += 256) s += args.partials[e];
+        s_[threadIdx.x] = s;
+        __syncthreads();
+        for (int d = 128; d >= 1; d >>= 1) {
+            if ((int)threadIdx.x < d) s_[threadIdx.x] += s_[threadIdx.x + d];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *stress = s_[0];
+        return;
+    }
+    constexpr int ROWS = 256 / MSUM;
+    __shared__ float red[MSUM][ROWS];
+    const int lr = threadIdx.x % ROWS, part = threadIdx.x / ROWS;
+    const int64_t n = args.n, row = (int64_t)blockIdx.x * ROWS + lr, ci = row / MI;
+    const int64_t islices = 64 / args.jw * (ci + 1), slices = islices + (n + MI - 1) / MI - ci;
+    for (int64_t c = 0; c < args.q; ++c) {
+        float v = 0.0f;
+        if (row < n)
+#pragma unroll 4
+            for (int64_t e = part; e < slices; e += MSUM)
+                v += e < islices ? args.ipart[(e * args.q + c) * n + row]
+                                 : args.jpart[((ci + e - islices) * args.q + c) * n + row];
+        __syncthreads();
+        red[part][lr] = v;
+        __syncthreads();
+        float total = red[0][lr];
+#pragma unroll
+        for (int e = 1; e < MSUM; ++e) total += red[e][lr];
+        if (part == 0 && row < n) dy[row * lddy + c] = total;
+    }
+}
+
 // Sum of the per-workgroup FP64 partials, fixed order (deterministic).
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const double *partials, int64_t count,
                                                               double *out)
@@ -904,7 +1138,53 @@ hipError_t launch_gradient(BwArgs &args, void *workspace, hipStream_t stream)
 
 }  // namespace
 
-int64_t mds_partials_count(int64_t n, int64_t q) { return (n + BI - 1) / BI * j_splits(n, q); }
+namespace {
+
+// Columns per wave of mds_small_kernel: few for few points, where there would be
+// too few waves and each one's chain of loads would show (2000 x 2: 111 us with
+// 128 columns a wave, 31 with 16; 16384 x 2: 229 with 128, 182 with 64).
+int mds_jw(int64_t n) { return n <= 2500 ? 16 : n <= 6000 ? 32 : 64; }
+
+// Its workgroups: row block ci has 64 / jw (ci + 1) column blocks.
+int64_t mds_tiles(int64_t n)
+{
+    const int64_t ni = (n + MI - 1) / MI;
+    return 64 / mds_jw(n) * (ni * (ni + 1) / 2);
+}
+
+// Few features: each pair once (mds_small_kernel).  Times in us, sweep and here:
+// 16384 x 8 1738 and 502, 4000 x 6 125 and 70, 2000 x 6 42 and 41, 2000 x 8 42
+// and 50; with 16 features its sums no longer fit the registers (4000: 128 and
+// 329).
+bool mds_small_applies(int64_t n, int64_t q) { return n >= 2 && (q <= 6 || (q <= 8 && n >= 3000)); }
+
+// Slices of the rows as i (column blocks) and as j (row blocks).
+int64_t mds_islices(int64_t n) { return 64 / mds_jw(n) * ((n + MI - 1) / MI); }
+size_t mds_slices(int64_t n) { return (size_t)mds_islices(n) + (size_t)((n + MI - 1) / MI); }
+
+template <int Q>
+void launch_mds_small(const MdsArgs &args, bool grad, hipStream_t stream)
+{
+    const dim3 grid((unsigned)mds_tiles(args.n));
+    if (grad)
+        hipLaunchKernelGGL((mds_small_kernel<Q, true>), grid, dim3(256), 0, stream, args);
+    else
+        hipLaunchKernelGGL((mds_small_kernel<Q, false>), grid, dim3(256), 0, stream, args);
+}
+
+}  // namespace
+
+int64_t mds_partials_count(int64_t n, int64_t q)
+{
+    if (mds_small_applies(n, q)) return mds_tiles(n);
+    return (n + BI - 1) / BI * j_splits(n, q);
+}
+
+size_t mds_workspace_bytes(int64_t n, int64_t q)
+{
+    if (mds_small_applies(n, q)) return mds_slices(n) * (size_t)n * (size_t)q * sizeof(float);
+    return sweep_workspace_bytes(n, q);
+}
 
 size_t backward_workspace_bytes(int op, int64_t n, int64_t k)
 {
@@ -947,6 +1227,32 @@ hipError_t launch_mds(const float *y, int64_t n, int64_t q, int64_t ldy, const f
                       float *dy, int64_t lddy, double *stress, double *partials, float *workspace,
                       hipStream_t stream)
 {
+    if (mds_small_applies(n, q)) {
+        MdsArgs ma;
+        ma.y = y;
+        ma.n = n;
+        ma.q = q;
+        ma.ldy = ldy;
+        ma.delta = delta;
+        ma.ipart = workspace;
+        ma.jw = mds_jw(n);
+        ma.jpart = dy ? workspace + (size_t)mds_islices(n) * (size_t)n * (size_t)q : nullptr;
+        ma.partials = partials;
+        switch (q) {
+        case 1: launch_mds_small<1>(ma, dy != nullptr, stream); break;
+        case 2: launch_mds_small<2>(ma, dy != nullptr, stream); break;
+        case 3: launch_mds_small<3>(ma, dy != nullptr, stream); break;
+        case 4: launch_mds_small<4>(ma, dy != nullptr, stream); break;
+        case 5: case 6: launch_mds_small<6>(ma, dy != nullptr, stream); break;
+        default: launch_mds_small<8>(ma, dy != nullptr, stream); break;
+        }
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const unsigned rows = dy ? (unsigned)((n + 256 / MSUM - 1) / (256 / MSUM)) : 0u;
+        hipLaunchKernelGGL(mds_finish_kernel, dim3(rows + 1), dim3(256), 0, stream, ma, dy, lddy, mds_tiles(n),
+                           stress);
+        return hipGetLastError();
+    }
     BwArgs args;
     args.x = y;
     args.n = n;

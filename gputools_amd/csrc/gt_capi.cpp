@@ -1158,7 +1158,7 @@ int gt_mds_stress(const float *y, int64_t n, int64_t q, int64_t ldy, const float
     hipStream_t hs = static_cast<hipStream_t>(stream);
     const int64_t parts = n > 1 ? gt::mds_partials_count(n, q) : 1;
     const size_t pbytes = round_up((size_t)parts * sizeof(double), 256);
-    const size_t dbytes = (n > 1 && dy != nullptr) ? gt::sweep_workspace_bytes(n, q) : 0;
+    const size_t dbytes = (n > 1 && dy != nullptr) ? gt::mds_workspace_bytes(n, q) : 0;
     Scratch ws;
     int s = ws.acquire(pbytes + dbytes, hs);
     if (s != GT_OK) return s;

@@ -194,3 +194,32 @@ def test_matrix_core_gradient_non_finite_upstream():
     assert np.isfinite(got[~hit]).all()
     rel = np.linalg.norm(got[~hit].astype(np.float64) - want[~hit]) / np.linalg.norm(want[~hit])
     assert rel <= 1e-5
+
+
+@pytest.mark.parametrize("n,q", [(2, 1), (64, 2), (255, 3), (256, 4), (257, 5), (300, 6), (2500, 2), (2501, 3),
+                                 (3073, 8), (3100, 7), (6001, 1)])
+def test_mds_few_features(n, q):
+    """The form that visits each pair once (few features) at the edges of its
+    blocks (256 rows; 16, 32 or 64 columns a wave), on strided rows, with
+    coincident points (distance 0: no gradient, full residual), with and
+    without the gradient."""
+    rng = np.random.default_rng(n * 10 + q)
+    base = rng.standard_normal((n, q + 2)).astype(np.float32)
+    if n > 10:
+        base[n - 1] = base[0]
+        base[n // 2] = base[n // 2 - 1]
+    y = np.ascontiguousarray(base[:, 1:q + 1])
+    delta = (rng.random(n * (n - 1) // 2) * 3.0).astype(np.float32)
+    print("case mds few features n=%d q=%d" % (n, q), flush=True)
+    s_ref, dy_ref = orc.mds_stress(y, delta.astype(np.float64))
+    yd = dev(base)[:, 1:q + 1]
+    dd = dev(delta)
+    from gputools_amd.autograd import _mds
+    for grad in (True, False):
+        s, dy = _mds(yd, dd, grad)
+        assert abs(s.item() - s_ref) <= 1e-6 * s_ref
+        if grad:
+            assert_grad_close(dy.cpu().numpy(), dy_ref)
+            s2, dy2 = _mds(yd, dd, True)
+            assert s2.item() == s.item()                              # deterministic
+            np.testing.assert_array_equal(dy.cpu().numpy(), dy2.cpu().numpy())
