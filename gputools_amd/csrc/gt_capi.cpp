@@ -358,10 +358,10 @@ int hclust_method_from_name(const char *name)
     return GT_HC_SINGLE;
 }
 
-size_t hclust_ws_bytes(int64_t n)
-{
-    return 3 * round_up((size_t)(n > 0 ? n : 0) * 4, 256);
-}
+// Rows' state; with the meeting point of the several-workgroup form behind it
+// (without: one workgroup does the rounds).
+size_t hclust_ws_min(int64_t n) { return 3 * round_up((size_t)(n > 0 ? n : 0) * 4, 256); }
+size_t hclust_ws_bytes(int64_t n) { return hclust_ws_min(n) + gt::HC_GROUP_BYTES; }
 
 int check_hclust_args(int64_t n, int64_t ldd, int method)
 {
@@ -375,14 +375,14 @@ int check_hclust_args(int64_t n, int64_t ldd, int method)
 }
 
 int run_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float beta, int *sub,
-               int *sup, float *height, void *ws, hipStream_t stream,
+               int *sup, float *height, void *ws, size_t ws_bytes, hipStream_t stream,
                int state = gt::HC_STATE_AUTO)
 {
     char *w = static_cast<char *>(ws);
     const size_t part = round_up((size_t)n * 4, 256);
     GT_HIP(gt::launch_hclust(d, n, ldd, method, lambda, beta, reinterpret_cast<float *>(w),
                              reinterpret_cast<float *>(w + part), reinterpret_cast<int *>(w + 2 * part),
-                             sub, sup, height, state, stream));
+                             ws_bytes >= hclust_ws_bytes(n) ? w + 3 * part : nullptr, sub, sup, height, state, stream));
     return GT_OK;
 }
 
@@ -401,7 +401,8 @@ int hclust_device_to_host(float *d, int64_t n, int64_t ldd, int method, float la
     int *dsub = reinterpret_cast<int *>(o);
     int *dsup = reinterpret_cast<int *>(o + part);
     float *dh = reinterpret_cast<float *>(o + 2 * part);
-    if ((s = run_hclust(d, n, ldd, method, lambda, beta, dsub, dsup, dh, ws.ptr, nullptr)) != GT_OK)
+    if ((s = run_hclust(d, n, ldd, method, lambda, beta, dsub, dsup, dh, ws.ptr,
+                        hclust_ws_bytes(n), nullptr)) != GT_OK)
         return s;
     GT_HIP(hipMemcpy(sub_h, dsub, len * 4, hipMemcpyDeviceToHost));
     GT_HIP(hipMemcpy(sup_h, dsup, len * 4, hipMemcpyDeviceToHost));
@@ -787,10 +788,10 @@ int gt_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float 
     if (s != GT_OK) return s;
     if (n < 2) return GT_OK;
     if (!d || !sub || !sup || !height) return fail(GT_ERR_INVALID, "null pointer");
-    if (workspace == nullptr || workspace_bytes < hclust_ws_bytes(n))
+    if (workspace == nullptr || workspace_bytes < hclust_ws_min(n))
         return fail(GT_ERR_WORKSPACE, "clustering workspace of %zu bytes needed (got %zu)",
-                    hclust_ws_bytes(n), workspace_bytes);
-    return run_hclust(d, n, ldd, method, lambda, beta, sub, sup, height, workspace,
+                    hclust_ws_min(n), workspace_bytes);
+    return run_hclust(d, n, ldd, method, lambda, beta, sub, sup, height, workspace, workspace_bytes,
                       static_cast<hipStream_t>(stream));
 }
 
@@ -807,12 +808,12 @@ int gt_hclust_state(float *d, int64_t n, int64_t ldd, int method, float lambda, 
                     (long long)gt::HC_LDS_MAX_N, (long long)n);
     if (n < 2) return GT_OK;
     if (!d || !sub || !sup || !height) return fail(GT_ERR_INVALID, "null pointer");
-    if (workspace == nullptr || workspace_bytes < hclust_ws_bytes(n))
+    if (workspace == nullptr || workspace_bytes < hclust_ws_min(n))
         return fail(GT_ERR_WORKSPACE, "clustering workspace of %zu bytes needed (got %zu)",
-                    hclust_ws_bytes(n), workspace_bytes);
+                    hclust_ws_min(n), workspace_bytes);
     static_assert((int)GT_HC_STATE_LDS == (int)gt::HC_STATE_LDS &&
                   (int)GT_HC_STATE_GLOBAL == (int)gt::HC_STATE_GLOBAL, "state values");
-    return run_hclust(d, n, ldd, method, lambda, beta, sub, sup, height, workspace,
+    return run_hclust(d, n, ldd, method, lambda, beta, sub, sup, height, workspace, workspace_bytes,
                       static_cast<hipStream_t>(stream), state);
 }
 

@@ -13,8 +13,10 @@
 //   - hclust_init_kernel (many workgroups, one wave per row) puts +inf on the
 //     diagonal, sets every count to 1 and computes each row's minimum over
 //     columns 0..r-1 (value and column);
-//   - hclust_merge_kernel (one persistent workgroup of 1024 threads) runs all
-//     n - 1 rounds.  Per round: the argmin over the cached row minima, the
+//   - hclust_group_kernel (32 workgroups on one XCD, see there) runs the n - 1
+//     rounds from 8 to 32768 points;
+//   - hclust_merge_kernel (one persistent workgroup of 1024 threads) runs them
+//     elsewhere, and where the 32 found no room together.  Per round: the argmin over the cached row minima, the
 //     update of row and column sup (row and column sub become +inf), then the
 //     cached minima are repaired: row sup is rescanned; a row r > sup takes
 //     the new D[r][sup] if it beats its cached minimum, and is rescanned only
@@ -65,7 +67,21 @@ struct HclustArgs {
     int *sub, *sup;
     float *height;
     bool vec4;         // rows start 16 B aligned
+    struct HcGroup *group;   // hclust_group_kernel's meeting point; null without it
 };
+
+// Meeting point of the workgroups of hclust_group_kernel (cleared by the init
+// kernel).
+constexpr int GP = 32;               // workgroups, all on one XCD
+constexpr int GMAX_N = 32768;        // a tie key fits 15 bits
+constexpr unsigned G_ABORT = 0xffffu;
+struct HcGroup {
+    unsigned arrive[16];             // workgroups seen, per XCD
+    unsigned chosen;                 // 0 none yet, 1 + XCD, or G_ABORT
+    unsigned pad[47];
+    unsigned long long rec[2][GP][2];   // [round parity][workgroup]: what it found
+};
+static_assert(sizeof(HcGroup) + 255 <= HC_GROUP_BYTES, "workspace share, any alignment");
 
 // Order of equal values in the reference's 32-lane reductions: lane t keeps
 // the first of its indices t, t+32, ...; the tree then folds lanes t and
@@ -244,6 +260,9 @@ __global__ __launch_bounds__(256) void hclust_init_kernel(HclustArgs a)
 {
     const int lane = threadIdx.x & 63;
     const int64_t waves = (int64_t)gridDim.x * 4;
+    if (a.group && blockIdx.x == 0)
+        for (unsigned t = threadIdx.x; t < sizeof(HcGroup) / 4; t += 256)
+            reinterpret_cast<unsigned *>(a.group)[t] = 0u;
     for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < a.n; r += waves) {
         float *row = a.d + r * a.ldd;
         if (lane == 0) {
@@ -274,6 +293,9 @@ __global__ __launch_bounds__(HTHREADS) void hclust_merge_kernel(HclustArgs a)
     __shared__ int rescan[RESCAN_CAP];
     __shared__ float part_v[HWAVES];
     __shared__ int part_i[HWAVES];
+
+    // after hclust_group_kernel: only when its workgroups did not come together
+    if (a.group && a.group->chosen != G_ABORT) return;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = a.n;
@@ -593,11 +615,565 @@ __global__ __launch_bounds__(HTHREADS) void hclust_merge_kernel(HclustArgs a)
     }
 }
 
+// ---------------------------------------------------------------------------
+// The merge rounds on the 32 CUs of one XCD
+// ---------------------------------------------------------------------------
+// One workgroup's round is a chain of memory round trips with LDS work on all
+// rows' state between them, and one CU issues every scattered store.  Here GP
+// workgroups share the rounds.  Rows are owned in blocks of 32, round robin; a
+// workgroup keeps the cached minima of its rows in LDS, and every workgroup
+// keeps all sizes (each sees every merge).  Per round:
+//   - wave 0 sends out the workgroup's best row and its part of the minimum of
+//     the row rewritten last round as two tagged 64-bit words, reads all GP
+//     records and comes to the same pair as the others (the order on (value,
+//     tie key) is total, so the grouping does not matter), and lists its rows
+//     whose cached minimum is at column sub or sup;
+//   - one wave per 64 rows reads its columns of rows sup and sub, stores the
+//     new values to row and column sup and lets them beat the cached minima;
+//   - at the same time the other waves scan the listed rows' remaining live
+//     columns (a bit each), a row over up to 16 waves; the new value in column
+//     sup joins afterwards.
+// The workgroups must run on one XCD: they exchange data through its L2, where
+// stores complete and which loads that pass the L1 by read.  GLAUNCH are
+// launched, the first XCD that has GP of them is chosen and the others leave.
+// If none has GP within 50 ms (a busy device), nobody starts and
+// hclust_merge_kernel, launched behind, does the work; otherwise that leaves
+// at once.
+// Bound: the round's latency, most of it dependent instructions of single
+// waves.  Average linkage, n = 8192 (independent normal points): 4.2 us a
+// round, of which 0.2 gather, 0.5 exchange, 0.4 choice of the pair, 0.35 list,
+// 1.0 rewrite and 1.3 beside it where some workgroup scans a row (0.8 of the
+// rounds have one).  One workgroup took 21.6 us; whole runs 177 -> 34 ms, at
+// 1024 points 8.9 -> 3.2 ms, at 32768 4680 -> 299 ms.
+// From 8 points (51 us against 66; at 3 points 38 against 36, the larger launch)
+// to what 15-bit tie keys and the LDS hold (9.1 against 143 us a round there).
+constexpr int GROUP_MIN_N = 8;
+constexpr int GTHREADS = 1024, GWAVES = GTHREADS / 64;
+constexpr int GLAUNCH = 320;
+constexpr unsigned long long GJOIN_TICKS = 5000000ull;      // 50 ms of the 100 MHz clock
+
+// End of a round: also this wave's stores are complete.
+__device__ __forceinline__ void round_barrier()
+{
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Loads that pass the L1 by; stores and records complete in the L2 (a store
+// of agent scope would go on to memory).
+__device__ __forceinline__ float load_shared(const float *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long load_shared(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void store_shared(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Four 16 B loads past the L1 at byte offsets from a row, and their wait.
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+__device__ __forceinline__ void load_four(const float *row, int o0, int o1, int o2, int o3, f32x4 (&x)[4])
+{
+    asm volatile("s_nop 4\n\t"   // a lane read into the address is five wait states away
+                 "global_load_dwordx4 %0, %4, %8 sc1\n\t"
+                 "global_load_dwordx4 %1, %5, %8 sc1\n\t"
+                 "global_load_dwordx4 %2, %6, %8 sc1\n\t"
+                 "global_load_dwordx4 %3, %7, %8 sc1\n\t"
+                 "s_waitcnt vmcnt(0)"
+                 : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
+                 : "v"(o0), "v"(o1), "v"(o2), "v"(o3), "s"(row)
+                 : "memory");
+}
+
+// Rows and columns as their tie keys in 15 bits: (value, key) then has the
+// order of beats().  No candidate: (+inf, NO_KEY).
+constexpr unsigned NO_KEY = 0x7fffu + 1u;
+__device__ __forceinline__ unsigned key_of(int i)
+{
+    return ((__builtin_bitreverse32((unsigned)i) >> 27) << 10) | ((unsigned)i >> 5);
+}
+__device__ __forceinline__ int index_of(unsigned k)
+{
+    return (int)(((k & 1023u) << 5) | (__builtin_bitreverse32(k >> 10) >> 27));
+}
+
+// One step of a wave-wide reduction in registers: lanes without a source, or
+// in rows that the mask leaves out, keep their value.  A DPP read needs two
+// wait states after the write of its source.
+#define GT_DPP_STEP(op, x, ctrl) "s_nop 1\n\t" op " " x ", " x ", " x " " ctrl "\n\t"
+#define GT_DPP_STEPS(op, x)                                                                        \
+    GT_DPP_STEP(op, x, "row_shr:1 row_mask:0xf bank_mask:0xf")                                     \
+    GT_DPP_STEP(op, x, "row_shr:2 row_mask:0xf bank_mask:0xf")                                     \
+    GT_DPP_STEP(op, x, "row_shr:4 row_mask:0xf bank_mask:0xf")                                     \
+    GT_DPP_STEP(op, x, "row_shr:8 row_mask:0xf bank_mask:0xf")                                     \
+    GT_DPP_STEP(op, x, "row_bcast:15 row_mask:0xa bank_mask:0xf")                                  \
+    GT_DPP_STEP(op, x, "row_bcast:31 row_mask:0xc bank_mask:0xf")                                  \
+    "s_nop 1"
+
+__device__ __forceinline__ float lane_of(float v, int lane)
+{
+    return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
+}
+
+// The lane that wins among those with (v, k) at the wave's minimum m; -1
+// when m is +inf.
+__device__ __forceinline__ int winner(float v, unsigned k, float m)
+{
+    unsigned long long at = __builtin_amdgcn_ballot_w64(v == m);
+    if (!(m < INFINITY)) return -1;
+    if (at & (at - 1)) {
+        const unsigned own = v == m ? k : ~0u;
+        unsigned q = own;
+        asm volatile(GT_DPP_STEPS("v_min_u32_dpp", "%0") : "+v"(q));
+        at = __builtin_amdgcn_ballot_w64(own == (unsigned)__builtin_amdgcn_readlane((int)q, 63));
+    }
+    return __builtin_ctzll(at);
+}
+
+// Wave-wide minimum.  (fminf would bring each step's operands into canonical
+// form first.)  No candidate is a NaN.
+__device__ __forceinline__ float wave_min(float v)
+{
+    asm volatile(GT_DPP_STEPS("v_min_f32_dpp", "%0") : "+v"(v));
+    return lane_of(v, 63);
+}
+
+// two at once: each fills the other's wait states
+#define GT_DPP_STEP2(ctrl)                                                                         \
+    "s_nop 0\n\tv_min_f32_dpp %0, %0, %0 " ctrl "\n\tv_min_f32_dpp %1, %1, %1 " ctrl "\n\t"
+__device__ __forceinline__ void wave_min2(float v, float w, float &mv, float &mw)
+{
+    asm volatile("s_nop 0\n\t"
+                 GT_DPP_STEP2("row_shr:1 row_mask:0xf bank_mask:0xf")
+                 GT_DPP_STEP2("row_shr:2 row_mask:0xf bank_mask:0xf")
+                 GT_DPP_STEP2("row_shr:4 row_mask:0xf bank_mask:0xf")
+                 GT_DPP_STEP2("row_shr:8 row_mask:0xf bank_mask:0xf")
+                 GT_DPP_STEP2("row_bcast:15 row_mask:0xa bank_mask:0xf")
+                 GT_DPP_STEP2("row_bcast:31 row_mask:0xc bank_mask:0xf")
+                 "s_nop 1"
+                 : "+v"(v), "+v"(w));
+    mv = lane_of(v, 63);
+    mw = lane_of(w, 63);
+}
+
+// rows per workgroup, a multiple of 32
+__host__ __device__ __forceinline__ int group_rows(int n) { return ((n + 31) / 32 + GP - 1) / GP * 32; }
+
+template <int METHOD>
+__global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
+{
+    extern __shared__ float hs_dyn[];
+    __shared__ int s_g, s_nres, s_rw, s_cw;
+    __shared__ float s_val, s_np, s_nq;
+    // per wave: its rows' best (value, row and column), its part of row sup's
+    // minimum, its part of a rescan
+    __shared__ float best_v[GWAVES], sup_v[GWAVES], scan_v[GWAVES];
+    __shared__ unsigned best_k[GWAVES], best_c[GWAVES], sup_k[GWAVES], scan_k[GWAVES];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    HcGroup *const grp = a.group;
+    if (tid == 0) {
+        const unsigned xcc = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & 15u;   // HW_REG_XCC_ID
+        const unsigned t = atomicAdd(&grp->arrive[xcc], 1u);
+        if (t == GP - 1) atomicCAS(&grp->chosen, 0u, xcc + 1u);
+        const unsigned long long began = wall_clock64();
+        unsigned c = 0u;
+        while (c == 0u) {
+            const bool late = wall_clock64() - began > GJOIN_TICKS;
+            c = atomicCAS(&grp->chosen, 0u, late ? G_ABORT : 0u);
+            if (late) break;
+            __builtin_amdgcn_s_sleep(4);
+        }
+        s_g = (c == xcc + 1u && t < GP) ? (int)t : -1;
+    }
+    __syncthreads();
+    const int g = s_g;
+    if (g < 0) return;
+
+    const int n = a.n, rows = group_rows(n), words = (n + 31) / 32;
+    const int64_t ldd = a.ldd;
+    float *const minv = hs_dyn;                                   // own rows: cached minimum,
+    unsigned *const mink = reinterpret_cast<unsigned *>(minv + rows);   // its column's key,
+    float *const newv = minv + 2 * rows;                          // D[sup][row] as rewritten,
+    int *const list = reinterpret_cast<int *>(minv + 3 * rows);   // rows to rescan
+    float *const scanv = minv + 4 * rows;                         // and what each scan found
+    unsigned *const scank = reinterpret_cast<unsigned *>(minv + 5 * rows);
+    unsigned *const live = reinterpret_cast<unsigned *>(minv + 6 * rows);   // bit per cluster, sup's off
+    float *const cnt = reinterpret_cast<float *>(live + words);   // sizes of all clusters
+    auto row_of = [&](int l) { return ((l >> 5) * GP + g) * 32 + (l & 31); };
+    auto mine = [&](int r) { return ((r >> 5) & (GP - 1)) == g; };
+    auto local = [&](int r) { return (r >> 5) / GP * 32 + (r & 31); };
+    for (int c = tid; c < n; c += GTHREADS) cnt[c] = 1.0f;
+    for (int w = tid; w < words; w += GTHREADS)
+        live[w] = n - w * 32 >= 32 ? ~0u : (1u << (n - w * 32)) - 1;
+    for (int l = tid; l < rows; l += GTHREADS) {
+        const int r = row_of(l);
+        const int c = r < n ? a.minc[r] : NO_COL;
+        minv[l] = c >= 0 ? a.minv[r] : INFINITY;
+        mink[l] = c >= 0 ? key_of(c) : NO_KEY;
+    }
+    __syncthreads();
+
+    if (tid < GWAVES) best_v[tid] = sup_v[tid] = INFINITY;
+    __syncthreads();
+
+    const unsigned lane_key = (__builtin_bitreverse32((unsigned)lane) >> 27) << 10;
+    const bool updates = wave * 64 < rows;      // 64 rows each
+    const int first = rows <= 256 ? 8 : 0;      // waves that rescan
+    // the best of this wave's rows and its part of row sup, to LDS
+    auto publish = [&](float v, unsigned k, unsigned c, float pv, unsigned pk) {
+        float m, pm;
+        wave_min2(v, pv, m, pm);
+        const int w = winner(v, k, m), pw = winner(pv, pk, pm);
+        if (lane == 0) {
+            best_v[wave] = w < 0 ? INFINITY : lane_of(v, w & 63);
+            best_k[wave] = (unsigned)__builtin_amdgcn_readlane((int)k, w & 63);
+            best_c[wave] = (unsigned)__builtin_amdgcn_readlane((int)c, w & 63);
+            sup_v[wave] = pw < 0 ? INFINITY : lane_of(pv, pw & 63);
+            sup_k[wave] = (unsigned)__builtin_amdgcn_readlane((int)pk, pw & 63);
+        }
+    };
+    if (updates) {
+        const int l = wave * 64 + lane;
+        const bool in = l < rows;
+        publish(in ? minv[l] : INFINITY, key_of(row_of(l)), in ? mink[l] : NO_KEY, INFINITY, NO_KEY);
+    }
+    __syncthreads();
+
+    int last = -1;      // the row rewritten last round
+    float rv = INFINITY;                      // best of the rows rescanned last round
+    unsigned rk = NO_KEY, rc = NO_KEY;
+    for (int iter = 0; iter + 1 < n; ++iter) {
+        if (wave == 0) {
+            const unsigned tag = (unsigned)(iter >> 1) % 3u + 1u;
+            // ---- this workgroup's best row, and its part of row `last` ------
+            float bv = rv, pv = INFINITY;
+            unsigned bk = rk, bc = rc, pk = NO_KEY;
+            if (lane < GWAVES) {
+                pv = sup_v[lane];
+                pk = sup_k[lane];
+                const float v = best_v[lane];
+                const unsigned k = best_k[lane], c = best_c[lane];
+                const bool t = v < bv || (v == bv && k < bk && v < INFINITY);
+                bv = t ? v : bv;
+                bk = t ? k : bk;
+                bc = t ? c : bc;
+            }
+            if (last >= 0 && lane == 0) atomicOr(&live[last >> 5], 1u << (last & 31));
+            // (the last round's stores are complete, so the record may go out)
+            unsigned long long *const rec = grp->rec[iter & 1][0];
+            {
+                float mb, mp;
+                wave_min2(bv, pv, mb, mp);
+                const int wb = winner(bv, bk, mb), wp = winner(pv, pk, mp);
+                const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)bk, wb & 63) & 0x7fffu;
+                const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)bc, wb & 63) & 0x7fffu;
+                const unsigned q = (unsigned)__builtin_amdgcn_readlane((int)pk, wp & 63) & 0x7fffu;
+                const float v = wb < 0 ? INFINITY : lane_of(bv, wb & 63);
+                const float qv = wp < 0 ? INFINITY : lane_of(pv, wp & 63);
+                if (lane < 2) {
+                    const unsigned hi = __float_as_uint(lane == 0 ? v : qv);
+                    const unsigned lo = lane == 0 ? (k << 17 | c << 2 | tag) : (q << 2 | tag);
+                    store_shared(rec + g * 2 + lane, ((unsigned long long)hi << 32) | lo);
+                }
+            }
+            // ---- all records ---------------------------------------------------
+            unsigned long long w0 = 0, w1 = 0;
+            bool failed = false;
+            for (unsigned spin = 0;; ++spin) {
+                w0 = load_shared(rec + (lane & (GP - 1)) * 2);
+                w1 = load_shared(rec + (lane & (GP - 1)) * 2 + 1);
+                if (__builtin_amdgcn_ballot_w64((w0 & 3u) != tag || (w1 & 3u) != tag) == 0) break;
+                if (spin == 5000000u) {
+                    failed = true;   // a partner is gone: about a second
+                    break;
+                }
+            }
+            asm volatile("" ::: "memory");
+            if (failed) {
+                // never seen: what is left is marked as no merge
+                for (int i = iter + lane; g == 0 && i + 1 < n; i += 64) {
+                    a.height[i] = __builtin_nanf("");
+                    a.sub[i] = a.sup[i] = 0;
+                }
+                if (lane == 0) s_nres = -1;
+            } else {
+                const float v = lane < GP ? __uint_as_float((unsigned)(w0 >> 32)) : INFINITY;
+                const float lv = lane < GP ? __uint_as_float((unsigned)(w1 >> 32)) : INFINITY;
+                const unsigned k = (unsigned)w0 >> 17, kc = ((unsigned)w0 >> 2) & 0x7fffu;
+                const unsigned lk = ((unsigned)w1 >> 2) & 0x7fffu;
+                float mv, ml;
+                wave_min2(v, lv, mv, ml);
+                const int wr = winner(v, k, mv);
+                float val = INFINITY;
+                unsigned krw = NO_KEY, kcw = NO_KEY;
+                if (wr >= 0) {
+                    val = lane_of(v, wr);
+                    krw = (unsigned)__builtin_amdgcn_readlane((int)k, wr);
+                    kcw = (unsigned)__builtin_amdgcn_readlane((int)kc, wr);
+                }
+                if (last >= 0) {
+                    const int wl = winner(lv, lk, ml);
+                    float lval = INFINITY;
+                    unsigned lkey = NO_KEY;
+                    if (wl >= 0) {
+                        lval = lane_of(lv, wl);
+                        lkey = (unsigned)__builtin_amdgcn_readlane((int)lk, wl);
+                        const unsigned kl = key_of(last);
+                        if (lval < val || (lval == val && kl < krw)) {
+                            val = lval;
+                            krw = kl;
+                            kcw = lkey;
+                        }
+                    }
+                    if (mine(last) && lane == 0) {
+                        minv[local(last)] = lval;
+                        mink[local(last)] = lkey;
+                    }
+                }
+                int cw = -1, rw = -1;
+                if (krw != NO_KEY) {
+                    rw = index_of(krw);
+                    cw = index_of(kcw);
+                } else {
+                    // no finite distance left: the two lowest-index clusters
+                    for (int i = 0; i < words && rw < 0; ++i) {
+                        unsigned m = live[i];
+                        if (m && cw < 0) {
+                            cw = i * 32 + __builtin_ctz(m);
+                            m &= m - 1;
+                        }
+                        if (m && cw >= 0) rw = i * 32 + __builtin_ctz(m);
+                    }
+                    rw = __builtin_amdgcn_readfirstlane(rw);
+                    cw = __builtin_amdgcn_readfirstlane(cw);
+                    krw = key_of(rw);
+                    kcw = key_of(cw);
+                }
+                last = rw;
+                // the other waves are past the last round's reads
+                const float nq = cnt[rw], np = cnt[cw];
+                // rows whose cached minimum is at column sub or sup: their
+                // other columns are scanned while row and column sup are made
+                int nres = 0;
+                const int own = mine(rw) ? local(rw) : -1;
+                for (int l0 = 0; l0 < rows; l0 += 256) {
+                    const int l = l0 + lane * 4;
+                    uint4 mk = make_uint4(NO_KEY, NO_KEY, NO_KEY, NO_KEY);
+                    if (l < rows) mk = *reinterpret_cast<const uint4 *>(mink + l);   // (rows: of 32)
+                    auto hit = [&](unsigned k, int at) { return (k == kcw || k == krw) && at != own; };
+                    const bool h0 = hit(mk.x, l), h1 = hit(mk.y, l + 1), h2 = hit(mk.z, l + 2), h3 = hit(mk.w, l + 3);
+                    if (__builtin_amdgcn_ballot_w64(h0 || h1 || h2 || h3) == 0) continue;
+                    auto add = [&](bool h, int at) {
+                        const unsigned long long who = __builtin_amdgcn_ballot_w64(h);
+                        if (h)
+                            list[nres + (int)__builtin_amdgcn_mbcnt_hi(
+                                            (unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, 0u))] = at;
+                        nres += __popcll(who);
+                    };
+                    add(h0, l);
+                    add(h1, l + 1);
+                    add(h2, l + 2);
+                    add(h3, l + 3);
+                }
+                if (lane == 0) {
+                    s_val = val;
+                    s_cw = cw;
+                    s_rw = rw;
+                    s_np = np;
+                    s_nq = nq;
+                    s_nres = nres;
+                    cnt[rw] = nq + np;
+                    cnt[cw] = 0.0f;
+                    atomicAnd(&live[cw >> 5], ~(1u << (cw & 31)));
+                    atomicAnd(&live[rw >> 5], ~(1u << (rw & 31)));
+                    if (g == 0) {
+                        a.height[iter] = val;
+                        a.sub[iter] = cw;
+                        a.sup[iter] = rw;
+                    }
+                }
+            }
+        }
+        lds_barrier();
+        const int listed_row = list[min(lane, rows - 1)];
+        const int nres = __builtin_amdgcn_readfirstlane(s_nres);
+        if (nres < 0) return;
+        const int rw = __builtin_amdgcn_readfirstlane(s_rw);
+        const unsigned krw = key_of(rw);
+        if (updates) {
+            // ---- row and column sup at 64 of this workgroup's rows -------------
+            const int cw = __builtin_amdgcn_readfirstlane(s_cw);
+            const unsigned kcw = key_of(cw);
+            const float np = s_np, nq = s_nq, val = s_val;
+            const float *const dcw = a.d + (int64_t)cw * ldd;
+            float *const drw = a.d + (int64_t)rw * ldd;
+            const int l = wave * 64 + lane, c = row_of(l);
+            const bool in = l < rows && c < n;
+            float bot = 0.0f, top = 0.0f, nk = 0.0f, m = INFINITY;
+            unsigned mk = NO_KEY;
+            if (in) {
+                bot = load_shared(drw + c);
+                top = load_shared(dcw + c);
+                nk = cnt[c];
+                m = minv[l];
+                mk = mink[l];
+            }
+            const float nr = nq + np;
+            const bool alive = nk > 0.0f, other = alive && c != rw;
+            float f = lw_update<METHOD>(bot, top, nr, np, nq, nk, val, a.lambda, a.beta);
+            f = other ? f : INFINITY;
+            if (alive) {
+                store_shared(drw + c, f);
+                store_shared(a.d + (int64_t)c * ldd + rw, f);
+            }
+            const bool part = other && c < rw && f < INFINITY;
+            const unsigned kc = lane_key | ((unsigned)c >> 5);
+            // ---- the cached minimum of each row: the new value may beat it.  Row
+            // sup's is put together from all parts; listed rows follow below.
+            const bool drop = c == rw || c == cw;
+            const bool listed = (mk == kcw || mk == krw) && !drop;
+            if (other && c > rw && f < INFINITY && (f < m || (f == m && krw < mk))) {
+                m = f;
+                mk = krw;
+            }
+            m = drop ? INFINITY : m;
+            mk = drop ? NO_KEY : mk;
+            if (in) newv[l] = f;
+            if (in && !listed) {
+                minv[l] = m;
+                mink[l] = mk;
+            }
+            publish(listed ? INFINITY : m, kc, mk, part ? f : INFINITY, kc);
+        }
+        // ---- listed rows: the live columns but sup, a row over several waves ----
+        const int lgw = first ? 3 : 4;
+        const int lgs = nres <= 1 ? lgw : max(lgw - (32 - __builtin_clz(nres - 1)), 0), S = 1 << lgs;
+        for (int q = (wave - first) >> lgs; wave >= first && q < nres; q += 1 << (lgw - lgs)) {
+            const int l = q < 64 ? __builtin_amdgcn_readlane(listed_row, q & 63)
+                                 : __builtin_amdgcn_readfirstlane(list[q]);
+            const int r = row_of(l), sg = (wave - first) & (S - 1);
+            const float *const row = a.d + (int64_t)r * ldd;
+            const int r4 = r & ~3, per = ((((r + 255) >> 8) + S - 1) >> lgs) * 256;
+            const int c0 = min(r4, sg * per), c1 = min(r4, (sg + 1) * per);
+            float v = INFINITY;
+            unsigned k = NO_KEY;
+            // 1024 columns at a time, 4 x 4 per lane
+            for (int cb = c0; cb < c1; cb += 1024) {
+                const int cc = cb + lane * 4;
+                f32x4 x[4];
+                load_four(row, min(cc, c1 - 4) * 4, min(cc + 256, c1 - 4) * 4, min(cc + 512, c1 - 4) * 4,
+                          min(cc + 768, c1 - 4) * 4, x);
+                float best = INFINITY;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (cb + u * 256 >= c1) {
+                        x[u] = f32x4{INFINITY, INFINITY, INFINITY, INFINITY};
+                        continue;
+                    }
+                    const int cu = cc + u * 256;
+                    const unsigned w = cu < c1 ? live[cu >> 5] >> (cu & 31) : 0u;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        x[u][e] = (w >> e) & 1u ? x[u][e] : INFINITY;
+                        best = x[u][e] < best ? x[u][e] : best;   // (passes NaN over)
+                    }
+                }
+                const float m = wave_min(best);
+                if (m < INFINITY && m <= v) {
+                    // this lane's first in key order: columns 0, 2, 1, 3 of four
+                    int at = -1;
+#pragma unroll
+                    for (int o = 15; o >= 0; --o) {
+                        const int e = (o >> 3) | ((o >> 1) & 2), u = o & 3;
+                        at = x[u][e] == m ? o : at;
+                    }
+                    const unsigned bk =
+                        at < 0 ? NO_KEY : key_of(cc) + ((unsigned)(at >> 2) << 13) + ((unsigned)(at & 3) << 3);
+                    const int w = winner(at < 0 ? INFINITY : m, bk, m);
+                    const unsigned wk = (unsigned)__builtin_amdgcn_readlane((int)bk, w);
+                    if (m < v || wk < k) {
+                        v = m;
+                        k = wk;
+                        if (m == 0.0f) v = load_shared(row + index_of(wk));   // its sign
+                    }
+                }
+            }
+            if (sg == S - 1 && r4 < r) {
+                // the last one to three columns
+                const int c = min(r4 + lane, r - 1);
+                float x = load_shared(row + c);
+                x = (live[c >> 5] >> (c & 31)) & 1u && r4 + lane < r && x < INFINITY ? x : INFINITY;
+                const unsigned ck = key_of(c);
+                const float m = wave_min(x);
+                const int w = winner(x, ck, m);
+                if (w >= 0) {
+                    const unsigned wk = (unsigned)__builtin_amdgcn_readlane((int)ck, w);
+                    if (m < v || (m == v && wk < k)) {
+                        v = lane_of(x, w);
+                        k = wk;
+                    }
+                }
+            }
+            if (lane == 0) {
+                scanv[q * S + sg] = v;
+                scank[q * S + sg] = k;
+            }
+        }
+        round_barrier();
+        if (wave == 0) {
+            rv = INFINITY;
+            if (nres > 0) {
+                float sv = INFINITY;
+                unsigned sk = NO_KEY;
+                if (S > 1) {
+                    // (at most 8 rows, 16 parts)
+                    const float ov = lane < nres * S ? scanv[lane] : INFINITY;
+                    const unsigned ok = lane < nres * S ? scank[lane] : NO_KEY;
+                    for (int q = 0; q < nres; ++q) {
+                        const float v = (lane >> lgs) == q ? ov : INFINITY;
+                        const int w = winner(v, ok, wave_min(v));
+                        if (lane == q && w >= 0) {
+                            sv = lane_of(ov, w);
+                            sk = (unsigned)__builtin_amdgcn_readlane((int)ok, w);
+                        }
+                    }
+                }
+                for (int q = lane; q < nres; q += 64) {
+                    const int l = list[q], r = row_of(l);
+                    float m = S > 1 ? sv : scanv[q];
+                    unsigned mk = S > 1 ? sk : scank[q];
+                    const float f = newv[l];
+                    if (r > rw && f < INFINITY && (f < m || (f == m && krw < mk))) {
+                        m = f;
+                        mk = krw;
+                    }
+                    minv[l] = m;
+                    mink[l] = mk;
+                    const unsigned k = key_of(r);
+                    if (m < rv || (m == rv && m < INFINITY && k < rk)) {
+                        rv = m;
+                        rk = k;
+                        rc = mk;
+                    }
+                }
+            }
+        }
+    }
+}
+
+unsigned group_lds(int n) { return (unsigned)((n + 31) / 32 * 4 + 4 * n + 24 * group_rows(n)); }
+
 }  // namespace
 
 hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float beta,
-                         float *count, float *minv, int *minc, int *sub, int *sup, float *height,
-                         int state, hipStream_t stream)
+                         float *count, float *minv, int *minc, void *group, int *sub, int *sup,
+                         float *height, int state, hipStream_t stream)
 {
     if (n < 2) return hipSuccess;
     HclustArgs a;
@@ -614,6 +1190,9 @@ hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lam
     a.sup = sup;
     a.height = height;
     a.vec4 = (ldd % 4 == 0) && ((reinterpret_cast<uintptr_t>(d) & 15) == 0);
+    a.group = nullptr;
+    if (state == HC_STATE_AUTO && group && n >= GROUP_MIN_N && n <= GMAX_N)
+        a.group = reinterpret_cast<HcGroup *>((reinterpret_cast<uintptr_t>(group) + 255) & ~(uintptr_t)255);
     int64_t blocks = (n + 3) / 4;
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL(hclust_init_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a);
@@ -628,6 +1207,15 @@ hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lam
     switch (method) {
 #define GT_HC_CASE(m)                                                                          \
     case m:                                                                                    \
+        if (a.group) {                                                                         \
+            const unsigned gl = group_lds((int)n);                                             \
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(hclust_group_kernel<m>),    \
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)gl);      \
+            if (e != hipSuccess) return e;                                                     \
+            hipLaunchKernelGGL(hclust_group_kernel<m>, dim3(GLAUNCH), dim3(GTHREADS), gl,      \
+                               stream, a);                                                     \
+            if ((e = hipGetLastError()) != hipSuccess) return e;                               \
+        }                                                                                      \
         if (lds) {                                                                             \
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(hclust_merge_kernel<m, true>), \
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);     \

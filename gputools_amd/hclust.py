@@ -154,9 +154,10 @@ def hclust(d, method="complete", lam: float = 0.5, beta: float = 0.5, stream=Non
     tensor on the GPU, consumed: it is overwritten).  Returns device int32
     tensors ``sub``, ``sup`` and float32 ``height`` of length n - 1: at step s
     the clusters represented by sub[s] < sup[s] merge at height[s].
-    ``state`` places the kernel's per-row state: "auto" (LDS up to 9216
-    points, global memory above), "lds" or "global"; every placement gives
-    the same result."""
+    ``state`` places the kernel's per-row state: "auto" (shared among
+    workgroups from 8 to 32768 points; else one workgroup, in LDS up to 9216
+    points, in global memory above), "lds" or "global" (one workgroup); every
+    placement gives the same result."""
     import torch
     if not isinstance(d, torch.Tensor) or not d.is_cuda or d.dtype != torch.float32:
         raise TypeError("d must be a float32 torch tensor on the GPU")

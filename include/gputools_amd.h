@@ -259,7 +259,8 @@ int gt_free(void *device_ptr);
  * GT_HC_SINGLE. */
 int gt_hclust_method_from_name(const char *name);
 
-/* Bytes of device workspace gt_hclust needs for n points. */
+/* Bytes of device workspace for gt_hclust on n points.  Without the last 4096
+ * (the meeting point of its workgroups) one workgroup does the work. */
 int gt_hclust_workspace_size(int64_t n, size_t *bytes);
 
 /* Hierarchical clustering of the full, symmetric n x n FP32 device matrix d
@@ -273,10 +274,11 @@ int gt_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float 
               int *sup, float *height, void *workspace, size_t workspace_bytes, void *stream);
 
 /* Where the clustering kernel keeps its per-row state (counts, cached row
- * minima, the rewritten row): GT_HC_STATE_AUTO as gt_hclust does (LDS up to
- * GT_HC_LDS_MAX_N points, global memory above), or one placement forced (LDS
- * only up to GT_HC_LDS_MAX_N).  Both placements run the same merge rounds and
- * give the same merges and heights bit for bit. */
+ * minima, the rewritten row): GT_HC_STATE_AUTO as gt_hclust does (shared among
+ * workgroups from 8 to 32768 points; else one workgroup, in LDS up to
+ * GT_HC_LDS_MAX_N points, in global memory above), or one workgroup and its
+ * placement forced (LDS only up to GT_HC_LDS_MAX_N).  All run the same merge
+ * rounds and give the same merges and heights bit for bit. */
 enum gt_hc_state {
     GT_HC_STATE_AUTO = 0,
     GT_HC_STATE_LDS = 1,

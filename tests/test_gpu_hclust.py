@@ -215,3 +215,32 @@ def test_hclust_power_of_two_scaling(method, state):
     np.testing.assert_array_equal(sub1, sub0)
     np.testing.assert_array_equal(sup1, sup0)
     np.testing.assert_array_equal(h1, h0 * np.float32(8.0))
+
+
+@pytest.mark.parametrize("n", [7, 8, 31, 33, 1023, 1024, 1025, 2049, 8193])
+@pytest.mark.parametrize("data", ["normal", "ties", "holes"])
+def test_hclust_workgroup_edges(n, data):
+    """The form with several workgroups at the edges of its blocks of 32 rows,
+    of one, two and more than four updating waves per workgroup, and of its
+    smallest size, on a matrix whose row stride is odd, with equal distances,
+    and with infinities and NaN (two halves that never get a finite
+    distance): bit for bit what the one-workgroup form gives."""
+    rng = np.random.default_rng(4000 + n)
+    x = rng.integers(0, 4, size=(n, 3)) if data == "ties" else rng.standard_normal((n, 6))
+    d = full_matrix(x)
+    if data == "holes":
+        d[: n // 2, n // 2 :] = np.inf
+        d[n // 2 :, : n // 2] = np.inf
+        i = rng.integers(0, n // 2, size=(2, n))
+        d[i[0], i[1]] = np.nan
+        d[i[1], i[0]] = np.nan
+    ldd = n + 1 + n % 2
+    print("case hclust workgroups n=%d %s" % (n, data), flush=True)
+    for method in ("average", "single") if n > 2000 else ("average", "centroid", "ward"):
+        res = []
+        for state in ("auto", "global"):
+            buf = torch.zeros((n, ldd), dtype=torch.float32, device="cuda")
+            buf[:, :n] = torch.from_numpy(d).cuda()
+            res.append([t.cpu().numpy() for t in gt.hclust(buf[:, :n], method, state=state)])
+        for a, b in zip(*res):
+            np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
