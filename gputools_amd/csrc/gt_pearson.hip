@@ -69,73 +69,120 @@ __device__ __forceinline__ float wave_max(float v)
 }
 
 // ---------------------------------------------------------------------------
-// Pre-pass of use = "everything": one wave per variable.
+// Pre-pass of use = "everything"
 // ---------------------------------------------------------------------------
-enum { PREP_BF16 = SPLIT_BF16, PREP_FP16 = SPLIT_FP16, PREP_FP32 = 2 };
-
 // z = (v - mean) / sqrt(sum (v - mean)^2), the mean and the sum over all dim
 // samples (NaN in, NaN out; a constant variable gives 0 / 0 = NaN, as the
-// reference's zero standard deviation does).  PREP_FP32 writes z (n x dim);
-// the split forms write the terms of z in operand blocks (gt_mfma.h), samples
-// dim..kp-1 zero.  FP16 scales z by a
-// power of two that brings max |z| into [2^14, 2^15) and records the inverse.
-template <int PREP>
-__global__ __launch_bounds__(256) void pmcc_prep_kernel(const float *__restrict__ x, int64_t n,
-                                                        int64_t dim, int64_t ldx, int64_t kp,
-                                                        unsigned short *__restrict__ terms,
-                                                        float *__restrict__ iscale,
-                                                        float *__restrict__ z)
+// reference's zero standard deviation does), and max |v - mean| for the FP16
+// scale.  One wave per variable; the sums' order is the same in every form.
+struct RowStats {
+    float mean, root, mx;
+};
+__device__ __forceinline__ RowStats row_stats(const float *xr, int64_t dim)
+{
+    const int lane = threadIdx.x & 63;
+    RowStats st;
+    float s = 0.0f;
+#pragma unroll 8
+    for (int64_t c = lane; c < dim; c += 64) s += xr[c];
+    st.mean = wave_sum(s) / (float)dim;
+    float q = 0.0f, mx = 0.0f;
+#pragma unroll 8
+    for (int64_t c = lane; c < dim; c += 64) {
+        const float d = xr[c] - st.mean;
+        q = fmaf(d, d, q);
+        mx = fmaxf(mx, fabsf(d));
+    }
+    st.root = sqrtf(wave_sum(q));
+    st.mx = wave_max(mx);
+    return st;
+}
+
+// z (n x dim) for the FP32 form
+__global__ __launch_bounds__(256) void pmcc_zscore_kernel(const float *__restrict__ x, int64_t n,
+                                                          int64_t dim, int64_t ldx, float *__restrict__ z)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t rows = PREP == PREP_FP32 ? n : operand_rows(n);
-    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
-        // rows past n fill their block with the last row; they only feed
-        // pairs that are never stored
-        const float *xr = x + (row < n ? row : n - 1) * ldx;
-        float s = 0.0f;
-        for (int64_t c = lane; c < dim; c += 64) s += xr[c];
-        const float mean = wave_sum(s) / (float)dim;
-        float q = 0.0f, mx = 0.0f;
-        for (int64_t c = lane; c < dim; c += 64) {
-            const float d = xr[c] - mean;
-            q = fmaf(d, d, q);
-            mx = fmaxf(mx, fabsf(d));
-        }
-        const float root = sqrtf(wave_sum(q));
-        mx = wave_max(mx);
-        if constexpr (PREP == PREP_FP32) {
-            for (int64_t c = lane; c < dim; c += 64) z[row * dim + c] = (xr[c] - mean) / root;
-        } else {
+    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < n; row += (int64_t)gridDim.x * 4) {
+        const float *xr = x + row * ldx;
+        const RowStats st = row_stats(xr, dim);
+        for (int64_t c = lane; c < dim; c += 64) z[row * dim + c] = (xr[c] - st.mean) / st.root;
+    }
+}
+
+// The split forms: the terms of z in operand blocks (gt_mfma.h), samples
+// dim..kp-1 zero.  FP16 scales z by a power of two that brings max |z| into
+// [2^14, 2^15) and records the inverse.  `split` workgroups per block of 32
+// variables: each finds the statistics, a wave per variable, and writes its
+// share of the chunks, a wave per chunk, so that a store is a whole 1 KB
+// block (few variables would otherwise leave CUs idle).  Rows past n fill
+// their block with the last row; they only feed pairs that are never stored.
+// Bound: memory (a read, then one from the caches, and six bytes out per
+// value).  8192 x 1024, BF16: 25 us; a wave that wrote its own variable's
+// 16-byte pieces of the blocks took 51.
+constexpr int PTHREADS = 1024;
+template <int PREP>
+__global__ __launch_bounds__(PTHREADS) void pmcc_prep_kernel(const float *__restrict__ x, int64_t n,
+                                                             int64_t dim, int64_t ldx, int64_t kp, int split,
+                                                             bool vec,
+                                                             unsigned short *__restrict__ terms,
+                                                             float *__restrict__ iscale)
+{
+    constexpr int NT = Split<PREP>::NT;
+    __shared__ float row_mean[32], row_root[32], row_scale[32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
+    const int64_t part = blockIdx.x % split, blocks = operand_rows(n) / 32;
+    for (int64_t rb = blockIdx.x / split; rb < blocks; rb += gridDim.x / split) {
+        __syncthreads();   // the last block's statistics are read
+        for (int q = wave; q < 32; q += PTHREADS / 64) {
+            const int64_t row = rb * 32 + q;
+            const RowStats st = row_stats(x + (row < n ? row : n - 1) * ldx, dim);
             float sc = 1.0f;
-            if (PREP == PREP_FP16) {
-                const float m = mx / root;   // max |z|
+            if (PREP == SPLIT_FP16) {
+                const float m = st.mx / st.root;   // max |z|
                 int e = 0;
                 if (m > 0.0f && m < INFINITY) {
                     e = ilogbf(m);
                     e = e < -100 ? -100 : (e > 100 ? 100 : e);
                 }
                 sc = ldexpf(1.0f, 14 - e);
-                if (lane == 0 && row < n) iscale[row] = ldexpf(1.0f, e - 14);
+                if (lane == 0 && part == 0 && row < n) iscale[row] = ldexpf(1.0f, e - 14);
             }
-            constexpr int NT = Split<PREP>::NT;
-            for (int64_t c0 = (int64_t)lane * 8; c0 < kp; c0 += 512) {
-                unsigned short t[8][NT];
+            if (lane == 0) {
+                row_mean[q] = st.mean;
+                row_root[q] = st.root;
+                row_scale[q] = sc;
+            }
+        }
+        __syncthreads();
+        const int64_t row = rb * 32 + r, nch = kp / OPERAND_K;
+        const float *xr = x + (row < n ? row : n - 1) * ldx;
+        const float mean = row_mean[r], root = row_root[r], sc = row_scale[r];
+        for (int64_t ch = part * (PTHREADS / 64) + wave; ch < nch; ch += (int64_t)split * (PTHREADS / 64)) {
+            const int64_t c0 = ch * OPERAND_K + h * 8;
+            float v[8];
+            if (vec && c0 + 8 <= dim) {
+                const float4 a = *reinterpret_cast<const float4 *>(xr + c0);
+                const float4 b = *reinterpret_cast<const float4 *>(xr + c0 + 4);
+                v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+                v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+            } else {
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const float v = (c0 + c < dim) ? ((xr[c0 + c] - mean) / root) * sc : 0.0f;
-                    Split<PREP>::split(v, t[c]);
-                }
+                for (int c = 0; c < 8; ++c) v[c] = c0 + c < dim ? xr[c0 + c] : 0.0f;
+            }
+            unsigned short t[8][NT];
 #pragma unroll
-                for (int q2 = 0; q2 < NT; ++q2) {
-                    uint4 w;
-                    w.x = t[0][q2] | ((unsigned)t[1][q2] << 16);
-                    w.y = t[2][q2] | ((unsigned)t[3][q2] << 16);
-                    w.z = t[4][q2] | ((unsigned)t[5][q2] << 16);
-                    w.w = t[6][q2] | ((unsigned)t[7][q2] << 16);
-                    const int64_t blk = (row >> 5) * (kp / OPERAND_K) + c0 / OPERAND_K;
-                    *reinterpret_cast<uint4 *>(terms + (blk * NT + q2) * OPERAND_VALUES +
-                                               ((c0 >> 3) & 1) * 256 + (row & 31) * 8) = w;
-                }
+            for (int c = 0; c < 8; ++c)
+                Split<PREP>::split(c0 + c < dim ? ((v[c] - mean) / root) * sc : 0.0f, t[c]);
+            unsigned short *const out = terms + (rb * nch + ch) * NT * OPERAND_VALUES + lane * 8;
+#pragma unroll
+            for (int q = 0; q < NT; ++q) {
+                uint4 w;
+                w.x = t[0][q] | ((unsigned)t[1][q] << 16);
+                w.y = t[2][q] | ((unsigned)t[3][q] << 16);
+                w.z = t[4][q] | ((unsigned)t[5][q] << 16);
+                w.w = t[6][q] | ((unsigned)t[7][q] << 16);
+                *reinterpret_cast<uint4 *>(out + q * OPERAND_VALUES) = w;
             }
         }
     }
@@ -144,13 +191,14 @@ __global__ __launch_bounds__(256) void pmcc_prep_kernel(const float *__restrict_
 // ---------------------------------------------------------------------------
 // MFMA tile of use = "everything": corr(x, y) = z_x . z_y.
 // ---------------------------------------------------------------------------
-constexpr int MBM = 256;        // tile side (variables)
+constexpr int MBM = 256;        // variables along x of a tile
+constexpr int MBN = 128;        // along y: two workgroups share a square of 256
 constexpr int MBK = 16;         // samples per main-loop chunk (one MFMA k-step)
 constexpr int MKPAD = 32;       // split terms are zero-padded to a multiple of this
-constexpr int MTHREADS = 1024;  // 16 waves, 4 (x) x 4 (y), 64 x 64 pairs each
+constexpr int MTHREADS = 512;   // 8 waves, 4 (x) x 2 (y), 64 x 64 pairs each
 constexpr int MSUPER = 2;       // super-tile side in tiles (L2 locality)
-constexpr int MTERM = MBM / 32 * OPERAND_BYTES;   // one term of one side, one chunk (8 KB)
-constexpr int MNSTAGE = 3;
+constexpr int MBLOCKS = (MBM + MBN) / 32;   // operand blocks of one term, one chunk
+constexpr int MNSTAGE = 2;
 
 struct PmccTileArgs {
     const unsigned short *ta, *tb;   // split terms, in operand blocks (gt_mfma.h)
@@ -166,27 +214,35 @@ struct PmccTileArgs {
 
 // SYM: a == b; tiles with J <= I, values mirrored to (y, x).  VEC: ldo and the
 // output pointers allow 16-byte mirrored stores.
+// Two workgroups share a CU, so one's stores and waits lie under the other's
+// products, and the last round of tiles is shorter: one workgroup of 16 waves
+// on a 256 x 256 tile with a three-stage ring ran 8192 variables x 1024 samples
+// (BF16, self) in 572 us, two of 8 waves on 256 x 128 with two stages in 491.
+// Bound: the matrix cores (six products, 0.41 TFLOP: 361 us at the 1.14
+// PFLOP/s of a large BF16 product) and 0.8 GB of results (117 us) beneath.
+// Unaligned rows, 4001 x 201: 153 us with 4-byte mirrored stores, 111 as rows.
 template <int SPLIT, bool SYM, bool VEC>
-__global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
+__global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs args)
 {
     typedef typename Split<SPLIT>::vec vec;
     constexpr int NT = Split<SPLIT>::NT;
-    constexpr int STAGE = 2 * NT * MTERM;
+    constexpr int STAGE = MBLOCKS * NT * OPERAND_BYTES;
     // after the main loop the stages hold each wave's transpose region for
     // the mirrored stores: 64 rows of MTRL floats
     constexpr int MTRL = 36;
     constexpr int TRBYTES = (MTHREADS / 64) * 64 * MTRL * 4;
     constexpr int SBYTES = MNSTAGE * STAGE > TRBYTES ? MNSTAGE * STAGE : TRBYTES;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[SBYTES + 2 * MBM * 4];
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[SBYTES + (MBM + MBN) * 4];
     float *iA = reinterpret_cast<float *>(smem + SBYTES);
     float *iB = iA + MBM;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave >> 2, wc = wave & 3;   // x rows wr*64.., y rows wc*64..
+    const int wr = wave >> 1, wc = wave & 1;   // x rows wr*64.., y rows wc*64..
 
     // Super-tiled schedule: super-tile st covers MSUPER x MSUPER tiles; tiles
     // past the edge (or above the diagonal when SYM) exit at once.
-    const int64_t id = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
+    const int64_t gid = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
+    const int64_t id = gid / 2;
     const int64_t st = id / (MSUPER * MSUPER);
     const int w = (int)(id % (MSUPER * MSUPER));
     int64_t SI, SJ;
@@ -202,14 +258,15 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
     const int64_t I = SI * MSUPER + w / MSUPER;
     const int64_t J = SJ * MSUPER + w % MSUPER;
     if (I >= args.tiles_a || J >= args.tiles_b || (SYM && J > I)) return;
-    const int64_t x0 = I * MBM, y0 = J * MBM;
+    const int64_t x0 = I * MBM, y0 = J * MBM + (gid & 1) * MBN;
     const int64_t na = args.na, nb = args.nb, kp = args.kp;
+    if (y0 >= nb) return;
 
     if (SPLIT == SPLIT_FP16) {
         if (tid < MBM) {
             const int64_t r = x0 + tid;
             iA[tid] = r < na ? args.isa[r] : 1.0f;
-        } else if (tid < 2 * MBM) {
+        } else if (tid < MBM + MBN) {
             const int64_t r = y0 + (tid - MBM);
             iB[tid - MBM] = r < nb ? args.isb[r] : 1.0f;
         }
@@ -226,21 +283,25 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
     // self, BF16, 643 -> 613 us.)
     typedef __attribute__((address_space(3))) void lds_void_t;
     typedef const __attribute__((address_space(1))) void gbl_void_t;
-    const unsigned short *gsrc;
-    {
-        const int lside = wave >> 3;
+    constexpr int PIECES = MBLOCKS * NT, PMAX = (PIECES + 7) / 8;
+    const unsigned short *gsrc[PMAX];
+#pragma unroll
+    for (int q = 0; q < PMAX; ++q) {
+        const int p = min(wave + 8 * q, PIECES - 1), blk = p / NT;
+        const int lside = blk >= MBM / 32;
         const int64_t last = operand_rows(lside ? nb : na) / 32 - 1;
-        const int64_t rb = (lside ? y0 : x0) / 32 + (wave & 7);
-        gsrc = (lside ? args.tb : args.ta) +
-               (rb < last ? rb : last) * (kp / OPERAND_K) * NT * OPERAND_VALUES + lane * 8;
+        const int64_t rb = lside ? y0 / 32 + blk - MBM / 32 : x0 / 32 + blk;
+        gsrc[q] = (lside ? args.tb : args.ta) +
+                  ((rb < last ? rb : last) * (kp / OPERAND_K) * NT + p % NT) * OPERAND_VALUES + lane * 8;
     }
     auto issue = [&](int chunk) {
         const int g = chunk % MNSTAGE;
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-            __builtin_amdgcn_global_load_lds(
-                (gbl_void_t *)(gsrc + ((int64_t)chunk * NT + t) * OPERAND_VALUES),
-                (lds_void_t *)(smem + g * STAGE + (wave * NT + t) * OPERAND_BYTES), 16, 0, 0);
+        for (int q = 0; q < PMAX; ++q)
+            if (wave + 8 * q < PIECES)
+                __builtin_amdgcn_global_load_lds(
+                    (gbl_void_t *)(gsrc[q] + (int64_t)chunk * NT * OPERAND_VALUES),
+                    (lds_void_t *)(smem + g * STAGE + (wave + 8 * q) * OPERAND_BYTES), 16, 0, 0);
     };
     const int roff = lane * 16;
 
@@ -257,16 +318,7 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
     for (int c = 0; c < MNSTAGE - 1; ++c)
         if (c < nchunks) issue(c);
     for (int c = 0; c < nchunks; ++c) {
-        // chunk c landed when at most the next chunk's NT loads per wave are
-        // outstanding (vector memory loads complete in order)
-        if (c + 1 < nchunks) {
-            if (NT == 3)
-                asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-            else
-                asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // every wave's part of chunk c is in LDS and every wave finished chunk
         // c-1, whose stage the next issue overwrites (a bare s_barrier:
         // __syncthreads() would also drain the later chunks' loads)
@@ -285,7 +337,7 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
             vec bv[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t)
-                bv[t] = *reinterpret_cast<const vec *>(sg + ((8 + wc * 2 + b) * NT + t) * OPERAND_BYTES);
+                bv[t] = *reinterpret_cast<const vec *>(sg + ((MBM / 32 + wc * 2 + b) * NT + t) * OPERAND_BYTES);
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
                 acc[a][b] = Split<SPLIT>::mfma(av[0][a], bv[0], acc[a][b]);
@@ -313,11 +365,12 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
     // SYM: off-diagonal tiles store (x, y) and (y, x); diagonal tiles store
     // x >= y and mirror x > y, so the two halves are the same values
     const bool diag = SYM && (I == J);
-    // whole off-diagonal tiles mirror through LDS: each wave writes its 64 x
-    // 32 block (one output, one a) transposed into its own region, then
-    // stores it back as rows of 32 consecutive x (128 B per row and store),
-    // instead of 16-byte pieces of 32 rows
-    const bool fastm = SYM && VEC && !diag && x0 + MBM <= na && y0 + MBM <= nb;
+    // off-diagonal tiles mirror through LDS: each wave writes its 64 x 32
+    // block (one output, one a) transposed into its own region, then stores it
+    // back as rows of 32 consecutive x (128 B per row), instead of 16-byte (or,
+    // unaligned, 4-byte) pieces of 32 rows
+    const bool fastm = SYM && !diag;
+    const bool whole = x0 + MBM <= na && y0 + MBN <= nb;
     float *const tr = reinterpret_cast<float *>(smem) + wave * 64 * MTRL;
     // lane's four x (8 rq + 4 (lane >> 5) ..) of row (lane & 31) + 32 b
     auto tr_put = [&](int rq, int b, const float (&v)[4]) {
@@ -326,6 +379,15 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
     };
     // the wave's transposed 64 x 32 block out as rows of 32 x
     auto tr_store = [&](float *out, int a) {
+        if (!VEC || !whole) {
+#pragma unroll 4
+            for (int it = 0; it < 32; ++it) {
+                const int ly = 2 * it + (lane >> 5), lx = lane & 31;
+                const int64_t y = y0 + wc * 64 + ly, x = x0 + wr * 64 + a * 32 + lx;
+                if (x < na && y < nb) out[y * ldo + x] = tr[ly * MTRL + lx];
+            }
+            return;
+        }
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
             const int ly = 8 * it + (lane >> 3), lx = (lane & 7) * 4;
@@ -367,28 +429,19 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
 #pragma unroll
                 for (int b = 0; b < 2; ++b) tr_put(rq, b, cv[b]);
             } else if (SYM) {
-                // (y, x) for the four x of this lane: one 16-byte store per
-                // output where the rows allow it
+                // the diagonal tile: (y, x) for the four x of this lane
 #pragma unroll
                 for (int b = 0; b < 2; ++b) {
                     const int64_t y = y0 + ly0 + b * 32;
                     const int64_t x = x0 + lx0;
                     if (y >= nb) continue;
                     const int64_t o = y * ldo + x;
-                    if (VEC && !diag && x + 3 < na) {
-                        *reinterpret_cast<float4 *>(args.corr + o) =
-                            make_float4(cv[b][0], cv[b][1], cv[b][2], cv[b][3]);
-                        *reinterpret_cast<float4 *>(args.ts + o) =
-                            make_float4(tv[b][0], tv[b][1], tv[b][2], tv[b][3]);
-                        *reinterpret_cast<float4 *>(args.pairs + o) = make_float4(fp, fp, fp, fp);
-                    } else {
 #pragma unroll
-                        for (int r4 = 0; r4 < 4; ++r4) {
-                            if (x + r4 >= na || (diag && x + r4 <= y)) continue;
-                            args.corr[o + r4] = cv[b][r4];
-                            args.ts[o + r4] = tv[b][r4];
-                            args.pairs[o + r4] = fp;
-                        }
+                    for (int r4 = 0; r4 < 4; ++r4) {
+                        if (x + r4 >= na || x + r4 <= y) continue;
+                        args.corr[o + r4] = cv[b][r4];
+                        args.ts[o + r4] = tv[b][r4];
+                        args.pairs[o + r4] = fp;
                     }
                 }
             }
@@ -407,6 +460,14 @@ __global__ __launch_bounds__(MTHREADS) void pmcc_tile_kernel(PmccTileArgs args)
     }
     if (fastm) {
         // pairs is one value: the wave's mirrored 64 x 64 block as rows
+        if (!VEC || !whole) {
+#pragma unroll 4
+            for (int ly = 0; ly < 64; ++ly) {
+                const int64_t y = y0 + wc * 64 + ly, x = x0 + wr * 64 + lane;
+                if (x < na && y < nb) args.pairs[y * ldo + x] = fp;
+            }
+            return;
+        }
 #pragma unroll
         for (int it = 0; it < 16; ++it) {
             const int ly = 4 * it + (lane >> 4), lx = (lane & 15) * 4;
@@ -1178,18 +1239,26 @@ PmccWs carve(int precision, int64_t na, int64_t nb, bool same, int64_t dim, void
 hipError_t launch_prep(int precision, const float *x, int64_t n, int64_t dim, int64_t ldx,
                        unsigned short *terms, float *iscale, float *z, hipStream_t stream)
 {
-    int64_t blocks = (operand_rows(n) + 3) / 4;
-    if (blocks > 65536) blocks = 65536;
-    const int64_t kp = padded_dim(dim);
-    if (precision == 0)
-        hipLaunchKernelGGL(pmcc_prep_kernel<PREP_FP32>, dim3((unsigned)blocks), dim3(256), 0,
-                           stream, x, n, dim, ldx, kp, terms, iscale, z);
-    else if (precision == 1)
-        hipLaunchKernelGGL(pmcc_prep_kernel<PREP_BF16>, dim3((unsigned)blocks), dim3(256), 0,
-                           stream, x, n, dim, ldx, kp, terms, iscale, z);
+    if (precision == 0) {
+        int64_t blocks = (n + 3) / 4;
+        if (blocks > 65536) blocks = 65536;
+        hipLaunchKernelGGL(pmcc_zscore_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, dim, ldx, z);
+        return hipGetLastError();
+    }
+    // workgroups per block of 32 variables: to fill the CUs, while each has a
+    // chunk per wave
+    const int64_t kp = padded_dim(dim), blocks = operand_rows(n) / 32;
+    int64_t split = 256 / (blocks > 0 ? blocks : 1), most = kp / OPERAND_K / (PTHREADS / 64);
+    if (split > most) split = most;
+    if (split < 1) split = 1;
+    const bool vec = ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    const dim3 grid((unsigned)((blocks < 65536 ? blocks : 65536) * split));
+    if (precision == 1)
+        hipLaunchKernelGGL(pmcc_prep_kernel<SPLIT_BF16>, grid, dim3(PTHREADS), 0, stream, x, n, dim, ldx, kp,
+                           (int)split, vec, terms, iscale);
     else
-        hipLaunchKernelGGL(pmcc_prep_kernel<PREP_FP16>, dim3((unsigned)blocks), dim3(256), 0,
-                           stream, x, n, dim, ldx, kp, terms, iscale, z);
+        hipLaunchKernelGGL(pmcc_prep_kernel<SPLIT_FP16>, grid, dim3(PTHREADS), 0, stream, x, n, dim, ldx, kp,
+                           (int)split, vec, terms, iscale);
     return hipGetLastError();
 }
 
@@ -1410,7 +1479,7 @@ hipError_t launch_pmcc(int use, int precision, const float *a, int64_t na, int64
     const int64_t sa = (args.tiles_a + MSUPER - 1) / MSUPER;
     const int64_t sbt = (args.tiles_b + MSUPER - 1) / MSUPER;
     args.super_b = sbt;
-    const int64_t ids = (same ? sa * (sa + 1) / 2 : sa * sbt) * MSUPER * MSUPER;
+    const int64_t ids = (same ? sa * (sa + 1) / 2 : sa * sbt) * MSUPER * MSUPER * 2;
     const bool vec = (ldo % 4 == 0) && ((reinterpret_cast<uintptr_t>(corr) |
                                          reinterpret_cast<uintptr_t>(ts) |
                                          reinterpret_cast<uintptr_t>(pairs)) & 15u) == 0;

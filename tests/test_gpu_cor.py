@@ -345,3 +345,30 @@ def test_pairwise_matrix_form_edges(dim, na, nb, scale):
         assert np.max(np.abs(c[ok] - corr[ok]), initial=0.0) <= 1e-5
         if xb is None:
             np.testing.assert_array_equal(c, c.T)
+
+
+@pytest.mark.parametrize("precision", ["bf16x3", "fp16x3"])
+@pytest.mark.parametrize("na,dim,pad", [(1, 40, 0), (127, 17, 1), (128, 512, 0), (129, 513, 3), (256, 33, 0),
+                                        (257, 100, 2), (384, 64, 0), (385, 1030, 1)])
+def test_everything_tile_edges(precision, na, dim, pad):
+    """The 256 x 128 tiles at their edges, rows of odd stride included.  A
+    pair of the self case is the pair of the two-matrix case (the same products
+    in the same order) on and below the diagonal, and mirrored above it; input
+    rows at an odd address are the same values as aligned ones."""
+    rng = np.random.default_rng(na * 7 + dim)
+    x = torch.from_numpy(rng.standard_normal((na, dim)).astype(np.float32) + 3).cuda()
+    bufs = [torch.full((na, na + pad), -7.0, device="cuda") for _ in range(3)]
+    got = gt.pmcc(x, precision=precision, out=tuple(b[:, :na] for b in bufs))
+    want = gt.pmcc(x, x.clone(), precision=precision)
+    flat = torch.zeros(na * dim + 1, device="cuda")
+    flat[1:] = x.reshape(-1)
+    shifted = gt.pmcc(flat[1:].view(na, dim), precision=precision)
+    for g, w, o in zip(got, want, shifted):
+        assert_bits_equal(g.tril().cpu().numpy(), w.tril().cpu().numpy())
+        assert_bits_equal(g.cpu().numpy(), g.t().contiguous().cpu().numpy())
+        assert_bits_equal(g.cpu().numpy(), o.cpu().numpy())
+    for b in bufs:
+        assert bool((b[:, na:] == -7.0).all())
+    z = x.double() - x.double().mean(1, keepdim=True)
+    z /= z.norm(dim=1, keepdim=True)
+    np.testing.assert_allclose(got[1].cpu().numpy(), (z @ z.t()).cpu().numpy(), rtol=0, atol=TOL)
