@@ -1,7 +1,7 @@
 // gt_gram.hip -- split-precision MFMA Gram form of the euclidean distance.
 //
 // d(x_i, x_j)^2 = ||x_i||^2 + ||x_j||^2 - 2 x_i.x_j.  The dot products of a
-// 256 x 256 tile of pairs run on the gfx950 matrix cores
+// 256 x 256 square of pairs (or half of one) run on the gfx950 matrix cores
 // (v_mfma_f32_32x32x16_{bf16,f16}) with FP32 accumulation.  A pre-pass splits
 // every FP32 input value once into 16-bit terms (stored in the workspace), and
 // the tile kernel accumulates the products whose error terms matter:
@@ -37,7 +37,7 @@
 namespace gt {
 namespace {
 
-constexpr int GBM = 256;        // tile side (points)
+constexpr int GBM = 256;        // side of a square of pairs (points)
 constexpr int GBK = 16;         // features per main-loop chunk (one MFMA k-step)
 constexpr int KPAD = 32;        // the split terms are zero-padded to a multiple of this
 constexpr int GSUPER = 4;       // super-tile side in tiles (L2 locality)
@@ -47,39 +47,42 @@ constexpr int FCAP = 1024;      // flagged pairs per fix-up pass
 // Gram-form values are finished with the hardware square root (v_sqrt_f32)
 // plus one residual correction (sqrt_rn), which rounds correctly for normal
 // inputs; d^2 below 2^-100 goes to the exact pass instead.
-constexpr int TERM_BYTES = GBM / 32 * OPERAND_BYTES;   // one split term of one side, one chunk (8 KB)
-constexpr int FIX_BYTES = 2 * GBM * FLD * 4;   // fix-up staging, both sides
 constexpr int LIST_BYTES = FCAP * 4;
-constexpr int SIDE_BYTES = 4 * GBM * 4 + 16 * 4;  // norms A, B, inverse scales A, B, scan
 
-// Wave layout of a 256 x 256 tile.  NW waves in a 4 (A rows) x NW/4 (B rows)
-// grid; each wave holds 64 x (256 / (NW/4)) pairs as 2 x NB blocks of 32 x 32
-// accumulators (NB = 8 / (NW/4)).  NW = 16: 64 x 64 per wave, 1024 threads,
-// 128 VGPRs per lane.  NW = 8: 64 x 128 per wave, 512 threads, up to 256
-// VGPRs per lane (the accumulators take 128).
+// A workgroup's tile: GAM rows j (side A) x 256 rows i (side B) on NW waves,
+// NW / 4 along A x 4 along B, 64 x 64 pairs each as 2 x 2 blocks of 32 x 32
+// accumulators (128 VGPRs per lane).  NW = 16: a whole square, one workgroup per
+// CU.  NW = 8: half a square, two workgroups per CU.
+constexpr int WC = 4;   // B-row groups
+constexpr int NB = 2;   // 32-row accumulator blocks along B per wave
 template <int NW>
-struct Waves {
+struct Tile {
     static constexpr int THREADS = NW * 64;
-    static constexpr int WC = NW / 4;             // B-row groups
-    static constexpr int NB = 8 / WC;             // 32-row accumulator blocks along B per wave
-    static constexpr int FUNITS = 2 * GBM * FBK / 4 / THREADS;  // fix-up float4 units per thread
-    static constexpr int FPER = FCAP / THREADS;   // fix-up list entries per thread
-    static constexpr int GPW = 16 / NW;           // 32-row load groups per wave per term
+    static constexpr int GAM = NW * 16;
+    static constexpr int PARTS = GBM / GAM;                                // workgroups per square
+    static constexpr int ABLOCKS = GAM / 32, BLOCKS = (GAM + GBM) / 32;    // operand blocks: A, both
+    static constexpr int FUNITS = (GAM + GBM) * FBK / 4 / THREADS;         // fix-up float4 units per thread
+    static constexpr int FPER = FCAP / THREADS;                            // fix-up list entries per thread
+    static constexpr int FIX_BYTES = (GAM + GBM) * FLD * 4;                // fix-up staging, both sides
+    static constexpr int SIDE_BYTES = 2 * (GAM + GBM) * 4 + 16 * 4;        // norms, inverse scales, scan
 };
 
-// LDS: [split terms, three stages | (aliased) fix-up staging + pair list]
-// [side data]
-template <int NT>
-struct TileLds {
-    // main-loop ring depth (two stages for BF16 measured no faster: 15.67 vs
-    // 15.55 ms on the 65536 x 512 mixture)
-    static constexpr int NSTAGE = 3;
-    static constexpr int STAGE = 2 * NT * TERM_BYTES;
+// LDS: [split terms | (aliased) fix-up staging + pair list] [side data]
+template <int NT, int NW>
+struct TileLds : Tile<NW> {
+    typedef Tile<NW> T;
+    static constexpr int PIECES = T::BLOCKS * NT;        // 1 KB each, per chunk
+    static constexpr int GPW = (PIECES + NW - 1) / NW;   // per wave
+    // main-loop ring depth: what two workgroups per CU leave room for (two
+    // stages with one: 15.67 vs 15.55 ms on the 65536 x 512 mixture, BF16)
+    static constexpr int NSTAGE = NW == 8 && NT == 3 ? 2 : 3;
+    static constexpr int STAGE = PIECES * OPERAND_BYTES;
     static constexpr int MAIN = NSTAGE * STAGE;
-    static constexpr int FIX = FIX_BYTES + LIST_BYTES;
+    static constexpr int FIX = T::FIX_BYTES + LIST_BYTES;
     static constexpr int REGION = MAIN > FIX ? MAIN : FIX;
     static constexpr int SIDE = REGION;
-    static constexpr int BYTES = REGION + SIDE_BYTES;
+    static constexpr int BYTES = REGION + T::SIDE_BYTES;
+    static_assert(NSTAGE == 2 || PIECES % NW == 0, "the same number of loads in flight in every wave");
 };
 
 struct GramArgs {
@@ -191,50 +194,48 @@ __device__ __forceinline__ void wait_vmcnt()
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef const __attribute__((address_space(1))) void gbl_void_t;
 
-// Main-loop LDS image of one chunk: side A (rows j), then side B (rows i), each
-// 8 blocks of 32 rows, each NT terms of 1 KB as they lie in memory.
+// Main-loop LDS image of one chunk: side A (rows j), then side B (rows i),
+// blocks of 32 rows, each NT terms of 1 KB as they lie in memory.
 // global_load_lds writes lane l's 16 B at the wave's LDS base + 16 l, so each
 // wave instruction moves one term of one block, eight whole lines; a lane's
-// operand read is its own 16 B, free of bank conflicts.  The 16 blocks (8 per
-// side) go to the waves round robin: wave w fills blocks w, w + NW, ... (block
-// g: side g / 8, rows 32 (g % 8) ..).  Blocks past the last one repeat it:
-// they only feed pairs that are never stored.
+// operand read is its own 16 B, free of bank conflicts.  These pieces go to the
+// waves round robin.  Blocks past the last one repeat it: they only feed pairs
+// that are never stored.
 // (Row-major terms moved 32 bytes of 32 rows per instruction, each line in four
 // parts: 65536 x 512 mixture, BF16, 15.77 -> 14.94 ms; 9001 x 130, FP16, 122 ->
-// 114 us.)
+// 114 us, both with one workgroup per CU.)
 template <int NT, int NW>
 __device__ __forceinline__ void chunk_sources(const GramArgs &args, int64_t i0, int64_t j0,
                                               int wave, int lane,
-                                              const unsigned short *(&gsrc)[Waves<NW>::GPW])
+                                              const unsigned short *(&gsrc)[TileLds<NT, NW>::GPW])
 {
     const int64_t last = operand_rows(args.n) / 32 - 1, nch = args.kp / OPERAND_K;
 #pragma unroll
-    for (int q = 0; q < Waves<NW>::GPW; ++q) {
-        const int g = wave + q * NW;
-        const int64_t rb = ((g >> 3) ? i0 : j0) / 32 + (g & 7);
-        gsrc[q] = args.terms + (rb < last ? rb : last) * nch * NT * OPERAND_VALUES + lane * 8;
+    for (int q = 0; q < TileLds<NT, NW>::GPW; ++q) {
+        const int p = min(wave + q * NW, TileLds<NT, NW>::PIECES - 1), g = p / NT;
+        constexpr int ABLOCKS = Tile<NW>::ABLOCKS;
+        const int64_t rb = g < ABLOCKS ? j0 / 32 + g : i0 / 32 + g - ABLOCKS;
+        gsrc[q] = args.terms + ((rb < last ? rb : last) * nch * NT + p % NT) * OPERAND_VALUES + lane * 8;
     }
 }
 
 template <int NT, int NW>
-__device__ __forceinline__ void issue_chunk(const unsigned short *const (&gsrc)[Waves<NW>::GPW],
+__device__ __forceinline__ void issue_chunk(const unsigned short *const (&gsrc)[TileLds<NT, NW>::GPW],
                                             unsigned char *stage, int wave, int chunk)
 {
     const int64_t off = (int64_t)chunk * NT * OPERAND_VALUES;
 #pragma unroll
-    for (int q = 0; q < Waves<NW>::GPW; ++q) {
-        const int g = wave + q * NW;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-            __builtin_amdgcn_global_load_lds((gbl_void_t *)(gsrc[q] + off + t * OPERAND_VALUES),
-                                             (lds_void_t *)(stage + (g * NT + t) * OPERAND_BYTES), 16, 0, 0);
-    }
+    for (int q = 0; q < TileLds<NT, NW>::GPW; ++q)
+        if (wave + q * NW < TileLds<NT, NW>::PIECES)
+            __builtin_amdgcn_global_load_lds((gbl_void_t *)(gsrc[q] + off),
+                                             (lds_void_t *)(stage + (wave + q * NW) * OPERAND_BYTES), 16, 0,
+                                             0);
 }
 
 // One chunk of MFMA products for this wave's pairs (acc[a][b]: A rows
 // wr*64 + a*32.., B rows wc*NB*32 + b*32..); sg = stage + the lane's operand
 // offset.
-template <int SPLIT, int NB>
+template <int SPLIT, int NW>
 __device__ __forceinline__ void mfma_chunk(f32x16_t (&acc)[2][NB], const unsigned char *sg, int wr,
                                            int wc)
 {
@@ -251,7 +252,7 @@ __device__ __forceinline__ void mfma_chunk(f32x16_t (&acc)[2][NB], const unsigne
         vec bv[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            bv[t] = *reinterpret_cast<const vec *>(sg + ((8 + wc * NB + b) * NT + t) * OPERAND_BYTES);
+            bv[t] = *reinterpret_cast<const vec *>(sg + ((Tile<NW>::ABLOCKS + wc * NB + b) * NT + t) * OPERAND_BYTES);
         // hh' first, then the cross terms in decreasing magnitude
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
@@ -268,19 +269,20 @@ __device__ __forceinline__ void mfma_chunk(f32x16_t (&acc)[2][NB], const unsigne
 }
 
 // Norms (and FP16 inverse row scales) of the tile's rows into LDS.
-template <int SPLIT>
+template <int SPLIT, int NW>
 __device__ __forceinline__ void load_side(const GramArgs &args, int64_t i0, int64_t j0, float *nA,
                                           float *nB, float *iA, float *iB)
 {
-    for (int t = threadIdx.x; t < 2 * GBM; t += blockDim.x) {
-        if (t < GBM) {
+    constexpr int GAM = Tile<NW>::GAM;
+    for (int t = threadIdx.x; t < GAM + GBM; t += Tile<NW>::THREADS) {
+        if (t < GAM) {
             const int64_t r = j0 + t;
             nA[t] = r < args.n ? args.norms[r] : 0.0f;
             if (SPLIT == SPLIT_FP16) iA[t] = r < args.n ? args.iscale[r] : 1.0f;
         } else {
-            const int64_t r = i0 + (t - GBM);
-            nB[t - GBM] = r < args.n ? args.norms[r] : 0.0f;
-            if (SPLIT == SPLIT_FP16) iB[t - GBM] = r < args.n ? args.iscale[r] : 1.0f;
+            const int64_t r = i0 + (t - GAM);
+            nB[t - GAM] = r < args.n ? args.norms[r] : 0.0f;
+            if (SPLIT == SPLIT_FP16) iB[t - GAM] = r < args.n ? args.iscale[r] : 1.0f;
         }
     }
 }
@@ -292,7 +294,7 @@ __device__ __forceinline__ void load_side(const GramArgs &args, int64_t i0, int6
 // of lane l is row 8(r/4) + 4(l/32) + r%4 (A side, j) and column l%32 (B
 // side, i); lanes 0..31 hold 32 consecutive i of one j, so packed stores are
 // contiguous runs.
-template <int SPLIT, int LAYOUT, int NB>
+template <int SPLIT, int LAYOUT>
 __device__ __forceinline__ void gram_epilogue(const f32x16_t (&acc)[2][NB], const GramArgs &args,
                                               int64_t i0, int64_t j0, bool interior, int wr,
                                               int wc, int lane, const float *nA, const float *nB,
@@ -383,7 +385,6 @@ __device__ __forceinline__ void gram_epilogue(const f32x16_t (&acc)[2][NB], cons
 }
 
 // Tile position of flag index `bit` of this lane: (A row << 16) | B row.
-template <int NB>
 __device__ __forceinline__ unsigned flag_entry(int bit, int wr, int li0, int lane)
 {
     const int a = bit / (NB * 16), b = (bit / 16) % NB, r = bit & 15;
@@ -414,26 +415,26 @@ __device__ __forceinline__ void store_exact(const GramArgs &args, int64_t i0, in
 template <int LAYOUT, bool VEC4, int NW>
 __device__ __forceinline__ void gram_fixup(const GramArgs &args, unsigned char *smem, int64_t i0,
                                            int64_t j0,
-                                           const unsigned long long (&fm)[Waves<NW>::NB / 2],
+                                           const unsigned long long (&fm)[NB / 2],
                                            int myoff, int total, int wr, int li0, int lane)
 {
-    typedef Waves<NW> W;
-    constexpr int THREADS = W::THREADS, FUNITS = W::FUNITS, FPER = W::FPER, NB = W::NB;
+    typedef Tile<NW> T;
+    constexpr int THREADS = T::THREADS, GAM = T::GAM, FUNITS = T::FUNITS, FPER = T::FPER;
     const int tid = threadIdx.x;
     float *fS = reinterpret_cast<float *>(smem);
-    unsigned int *list = reinterpret_cast<unsigned int *>(smem + FIX_BYTES);
+    unsigned int *list = reinterpret_cast<unsigned int *>(smem + T::FIX_BYTES);
     const int64_t n = args.n, k = args.k, ldx = args.ldx;
     // Staging unit e = tid + THREADS q (q < FUNITS): tile row e >> 3 (A side
     // rows first, then B side), features (e & 7) * 4..+3 of a chunk; the
     // unit's column is (tid & 7) * 4 for every q.  The accumulators are dead
     // here, so their registers hold a ring of FRING chunks in flight (the
     // pass is bound by load latency, not bandwidth).
-    constexpr int FRING = 2;
+    constexpr int FRING = NW == 16 ? 2 : 1;   // (two workgroups hide the latency too)
     int frow[FUNITS];
 #pragma unroll
     for (int q = 0; q < FUNITS; ++q) {
         const int row = (tid + THREADS * q) >> 3;
-        const int64_t g = row < GBM ? j0 + row : i0 + (row - GBM);
+        const int64_t g = row < GAM ? j0 + row : i0 + (row - GAM);
         frow[q] = (int)(g < n ? g : n - 1);
     }
     const float *const fx = args.x + (tid & 7) * 4;
@@ -471,7 +472,7 @@ __device__ __forceinline__ void gram_fixup(const GramArgs &args, unsigned char *
             if (tid + THREADS * c < cnt) {                                                 \
                 const float4 *ra = reinterpret_cast<const float4 *>(fS + (ent[c] >> 16) * FLD); \
                 const float4 *rb =                                                         \
-                    reinterpret_cast<const float4 *>(fS + (GBM + (ent[c] & 0xffffu)) * FLD); \
+                    reinterpret_cast<const float4 *>(fS + (GAM + (ent[c] & 0xffffu)) * FLD); \
                 float part = 0.0f;                                                         \
                 _Pragma("unroll") for (int q = 0; q < FBK / 4; ++q) {                      \
                     const float4 u = ra[q], v = rb[q];                                     \
@@ -498,7 +499,7 @@ __device__ __forceinline__ void gram_fixup(const GramArgs &args, unsigned char *
                     const int bit = __builtin_ctzll(m);
                     m &= m - 1;
                     if (rank >= base && rank < base + FCAP)
-                        list[rank - base] = flag_entry<NB>(qw * 64 + bit, wr, li0, lane);
+                        list[rank - base] = flag_entry(qw * 64 + bit, wr, li0, lane);
                     ++rank;
                 }
             }
@@ -509,7 +510,7 @@ __device__ __forceinline__ void gram_fixup(const GramArgs &args, unsigned char *
 #pragma unroll
         for (int c = 0; c < FPER; ++c) sum[c] = 0.0f;
         GT_FLOAD(fr0, 0);
-        if (nf > 1) GT_FLOAD(fr1, 1);
+        if (FRING == 2 && nf > 1) GT_FLOAD(fr1, 1);
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < FPER; ++c) {
@@ -518,7 +519,7 @@ __device__ __forceinline__ void gram_fixup(const GramArgs &args, unsigned char *
         }
         for (int ch = 0; ch < nf; ch += FRING) {
             GT_FSTEP(fr0, ch);
-            if (ch + 1 < nf) GT_FSTEP(fr1, ch + 1);
+            if (FRING == 2 && ch + 1 < nf) GT_FSTEP(fr1, ch + 1);
         }
 #pragma unroll
         for (int c = 0; c < FPER; ++c)
@@ -529,25 +530,28 @@ __device__ __forceinline__ void gram_fixup(const GramArgs &args, unsigned char *
 #undef GT_FLOAD
 }
 
-// One workgroup per 256 x 256 tile: main loop, epilogue, then the exact
-// pass of the flagged pairs.
+// One workgroup per tile: main loop, epilogue, then the exact pass of the
+// flagged pairs.  Bound: the matrix cores' power for long rows (65536 x 512
+// mixture, BF16: 13.2 TFLOP of products, 11.6 ms at the 1.14 PFLOP/s of a large
+// BF16 product, and 3.3 ms of exact pass: 14.9 ms), the stores for short ones.
 template <int SPLIT, int LAYOUT, bool VEC4, int NW>
-__global__ __launch_bounds__(NW * 64) void gram_tile_kernel(GramArgs args)
+__global__ __launch_bounds__(NW * 64, 4) void gram_tile_kernel(GramArgs args)
 {
-    typedef Waves<NW> W;
-    constexpr int NT = Split<SPLIT>::NT, NB = W::NB, GPW = W::GPW;
-    typedef TileLds<NT> L;
+    constexpr int NT = Split<SPLIT>::NT;
+    typedef TileLds<NT, NW> L;
+    constexpr int GPW = L::GPW, GAM = L::GAM;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[L::BYTES];
     float *nA = reinterpret_cast<float *>(smem + L::SIDE);
-    float *nB = nA + GBM, *iA = nB + GBM, *iB = iA + GBM;
+    float *nB = nA + GAM, *iA = nB + GBM, *iB = iA + GAM;
     int *scan_tmp = reinterpret_cast<int *>(iB + GBM);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave / W::WC, wc = wave % W::WC;
+    const int wr = wave / WC, wc = wave % WC;
 
     // Super-tiled lower-triangular schedule: super-tile s covers GSUPER x
     // GSUPER tiles; tiles above the diagonal or past the edge exit at once.
-    const int64_t id = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
+    const int64_t gid = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
+    const int64_t id = gid / L::PARTS;
     const int64_t st = id / (GSUPER * GSUPER);
     const int w = (int)(id % (GSUPER * GSUPER));
     int SI, SJ;
@@ -555,8 +559,9 @@ __global__ __launch_bounds__(NW * 64) void gram_tile_kernel(GramArgs args)
     const int64_t I = (int64_t)SI * GSUPER + w / GSUPER;
     const int64_t J = (int64_t)SJ * GSUPER + w % GSUPER;
     if (I >= args.T || J > I) return;
-    const int64_t i0 = I * GBM, j0 = J * GBM;
-    load_side<SPLIT>(args, i0, j0, nA, nB, iA, iB);
+    const int64_t i0 = I * GBM, j0 = J * GBM + gid % L::PARTS * GAM;
+    if (j0 >= args.n) return;
+    load_side<SPLIT, NW>(args, i0, j0, nA, nB, iA, iB);
 
     const unsigned short *gsrc[GPW];
     chunk_sources<NT, NW>(args, i0, j0, wave, lane, gsrc);
@@ -580,7 +585,7 @@ __global__ __launch_bounds__(NW * 64) void gram_tile_kernel(GramArgs args)
         // chunk c landed when at most the next chunk's loads of this wave
         // are outstanding (vector memory loads complete in order)
         if (NS == 3 && c + 1 < nchunks)
-            wait_vmcnt<NT * GPW>();
+            wait_vmcnt<GPW>();
         else
             wait_vmcnt<0>();
         // every wave's part of chunk c is in LDS, and every wave finished
@@ -590,14 +595,14 @@ __global__ __launch_bounds__(NW * 64) void gram_tile_kernel(GramArgs args)
         asm volatile("" ::: "memory");
         if (c + NS - 1 < nchunks)
             issue_chunk<NT, NW>(gsrc, smem + ((c + NS - 1) % NS) * L::STAGE, wave, c + NS - 1);
-        mfma_chunk<SPLIT, NB>(acc, smem + (c % NS) * L::STAGE + roff, wr, wc);
+        mfma_chunk<SPLIT, NW>(acc, smem + (c % NS) * L::STAGE + roff, wr, wc);
     }
     // the fix-up below reuses the stage memory
     __syncthreads();
 
     const bool interior = (I > J) && (i0 + GBM <= args.n);
     unsigned long long fm[NB / 2];
-    gram_epilogue<SPLIT, LAYOUT, NB>(acc, args, i0, j0, interior, wr, wc, lane, nA, nB, iA, iB, fm);
+    gram_epilogue<SPLIT, LAYOUT>(acc, args, i0, j0, interior, wr, wc, lane, nA, nB, iA, iB, fm);
     int cnt = 0;
 #pragma unroll
     for (int q = 0; q < NB / 2; ++q) cnt += __popcll(fm[q]);
@@ -748,35 +753,49 @@ __global__ __launch_bounds__(256) void row_prep_kernel(const float *__restrict__
     }
 }
 
-// 16 waves (64 x 64 pairs each).  8 waves of 64 x 128 pairs (512 threads,
-// about 200 VGPRs) give the same results bit for bit and measured slower:
-// 16.8 vs 15.9 ms on the 65536 x 512 mixture, 12.8 vs 12.5 ms on N(0, 1)
-// (BF16); the exact pass has half the loads in flight.
-constexpr int kGramWaves = 16;
-
-template <int SPLIT, int LAYOUT, bool VEC4>
-hipError_t launch_tiles(GramArgs &args, int64_t ids, hipStream_t stream)
+template <int SPLIT, int LAYOUT, bool VEC4, int NW>
+hipError_t launch_tiles(GramArgs &args, hipStream_t stream)
 {
+    const int64_t S = (args.T + GSUPER - 1) / GSUPER;
+    const int64_t ids = S * (S + 1) / 2 * GSUPER * GSUPER * Tile<NW>::PARTS;
     const int64_t max_ids = int64_t(1) << 23;
     for (int64_t off = 0; off < ids; off += max_ids) {
         args.id_offset = off;
         args.ids_this = (ids - off) < max_ids ? (ids - off) : max_ids;
-        hipLaunchKernelGGL((gram_tile_kernel<SPLIT, LAYOUT, VEC4, kGramWaves>),
-                           dim3((unsigned)args.ids_this), dim3(kGramWaves * 64), 0, stream, args);
+        hipLaunchKernelGGL((gram_tile_kernel<SPLIT, LAYOUT, VEC4, NW>), dim3((unsigned)args.ids_this),
+                           dim3(Tile<NW>::THREADS), 0, stream, args);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
+// Half squares while every half has a CU to itself (3000 points x 256 features
+// 74 -> 58 us in BF16, x 1024 162 -> 110), and for short rows, where a tile's
+// stores take as long as its products and the second workgroup fills them
+// (30000 x 64: 740 -> 716 us BF16, 649 -> 625 FP16; 9001 x 130 FP16 114 -> 109).
+// Else whole squares, which read fewer operands per pair (30000 x 1024 BF16
+// 4.73 ms whole, 5.16 halves).
+bool half_squares(const GramArgs &args, int terms)
+{
+    return args.T * (args.T + 1) <= 256 || args.kp * terms <= 512;
+}
+
+template <int SPLIT, int LAYOUT, bool VEC4>
+hipError_t launch_waves(GramArgs &args, hipStream_t stream)
+{
+    return half_squares(args, Split<SPLIT>::NT) ? launch_tiles<SPLIT, LAYOUT, VEC4, 8>(args, stream)
+                                                : launch_tiles<SPLIT, LAYOUT, VEC4, 16>(args, stream);
+}
+
 template <int SPLIT>
-hipError_t launch_layout(int layout, bool vec4, GramArgs &args, int64_t ids, hipStream_t stream)
+hipError_t launch_layout(int layout, bool vec4, GramArgs &args, hipStream_t stream)
 {
     if (layout == OUT_PACKED)
-        return vec4 ? launch_tiles<SPLIT, OUT_PACKED, true>(args, ids, stream)
-                    : launch_tiles<SPLIT, OUT_PACKED, false>(args, ids, stream);
-    return vec4 ? launch_tiles<SPLIT, OUT_FULL, true>(args, ids, stream)
-                : launch_tiles<SPLIT, OUT_FULL, false>(args, ids, stream);
+        return vec4 ? launch_waves<SPLIT, OUT_PACKED, true>(args, stream)
+                    : launch_waves<SPLIT, OUT_PACKED, false>(args, stream);
+    return vec4 ? launch_waves<SPLIT, OUT_FULL, true>(args, stream)
+                : launch_waves<SPLIT, OUT_FULL, false>(args, stream);
 }
 
 template <int SPLIT>
@@ -938,11 +957,9 @@ hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int
     args.ldd = ldd;
     args.T = (n + GBM - 1) / GBM;
     args.tau = tau;
-    const int64_t S = (args.T + GSUPER - 1) / GSUPER;
-    const int64_t ids = S * (S + 1) / 2 * GSUPER * GSUPER;
     const bool vec4 = rows_vec4(x, k, ldx);
-    return fp16 ? launch_layout<SPLIT_FP16>(layout, vec4, args, ids, stream)
-                : launch_layout<SPLIT_BF16>(layout, vec4, args, ids, stream);
+    return fp16 ? launch_layout<SPLIT_FP16>(layout, vec4, args, stream)
+                : launch_layout<SPLIT_BF16>(layout, vec4, args, stream);
 }
 
 }  // namespace gt

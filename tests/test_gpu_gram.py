@@ -195,3 +195,27 @@ def test_gram_rejects_other_methods():
     x = dev(wl.normal(10, 4))
     with pytest.raises(gt.GputoolsError, match="UNSUPPORTED"):
         gt.dist(x, "manhattan", precision="bf16x3")
+
+
+@pytest.mark.parametrize("precision", SPLITS)
+@pytest.mark.parametrize("layout", ["packed", "full"])
+@pytest.mark.parametrize("n,k", [(127, 40), (128, 300), (129, 171), (255, 256), (385, 257), (640, 20),
+                                 (3840, 300), (3841, 160), (3841, 161), (3841, 256), (3841, 257)])
+def test_gram_tile_halves(precision, layout, n, k):
+    """Half and whole squares of pairs at the edges of both and of the rule
+    between them (3840 points; 160 features in BF16, 256 in FP16), with groups
+    of near points that the exact pass recomputes."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((n, k)).astype(np.float32)
+    x[1::3] = x[0::3][: len(x[1::3])] + 1e-2 * x[1::3]
+    got = run(x, precision, layout)
+    if layout == "packed":
+        full = np.zeros((n, n), np.float32)
+        full[np.triu_indices(n, 1)] = got
+        got = full + full.T
+    rows = np.unique(np.concatenate([np.arange(0, n, max(1, n // 40)), [n - 1]]))
+    want = np.sqrt(((x[rows].astype(np.float64)[:, None, :] - x.astype(np.float64)[None]) ** 2).sum(-1)) \
+        if n < 1000 else torch.cdist(dev(x[rows]).double(), dev(x).double(),
+                                     compute_mode="donot_use_mm_for_euclid_dist").cpu().numpy()
+    print("case gram halves", precision, layout, n, k, flush=True)
+    assert max_rel(got[rows], want) <= RTOL
