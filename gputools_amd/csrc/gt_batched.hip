@@ -18,6 +18,8 @@
 #include "gt_common.h"
 #include "gt_internal.h"
 
+#include <type_traits>
+
 namespace gt {
 namespace {
 
@@ -56,13 +58,20 @@ __device__ __forceinline__ int side_index(int t, int m)
     return t * TM + m;
 }
 
+// Bound: the VALU (two operations per feature and pair).  1024 sets of 32 to
+// 2048 points (log-uniform), 16 to 128 features, euclidean, BM = 128: 1.60e10
+// terms, 0.81 ms at the rate of the vector unit; whole tiles make 2.03e10 of
+// them, the quarters that hold pairs 1.80e10.  1184 us with whole tiles and
+// 4-byte loads, 1136 by quarters, 1072 with 16-byte loads.  (Starting each
+// partial sum with its first term instead of zero took 1142, sqrt_rn before
+// the stores 1150: both undo the overlap of loads, roots and stores.)
 template <int OP, int BM>
-__global__ __launch_bounds__(BTHREADS) void batched_kernel(BatchedArgs args)
+__global__ __launch_bounds__(BTHREADS, 2) void batched_kernel(BatchedArgs args)
 {
     constexpr int TPS = 16;             // threads per tile side
     constexpr int TM = BM / TPS;        // pairs per thread per side
     constexpr int LD = BM + 4;
-    constexpr int LOADS = BM * BKC / BTHREADS;
+    constexpr int UNITS = (BM * BKC / 4 + BTHREADS - 1) / BTHREADS;   // 16 B units per thread and side
     __shared__ __attribute__((aligned(16))) float as_[BKC][LD];
     __shared__ __attribute__((aligned(16))) float bs_[BKC][LD];
 
@@ -80,17 +89,34 @@ __global__ __launch_bounds__(BTHREADS) void batched_kernel(BatchedArgs args)
         float *out = args.out + args.out_off[s];
         const int64_t i0 = (int64_t)I * BM, j0 = (int64_t)J * BM;
 
-        // global -> register staging, one chunk ahead of the LDS chunk
-        float sa[LOADS], sb[LOADS];
+        // global -> register staging, one chunk ahead of the LDS chunk: unit u
+        // is row u / 4, features (u % 4) * 4 .. + 3, one 16 B load where the
+        // set's rows are aligned (their writes to LDS meet no bank twice)
+        const bool vec = k % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+        float4 sa[UNITS], sb[UNITS];
+        auto row4 = [&](int64_t r, int64_t kk) {
+            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (r < n && kk < k) {
+                const float *p = x + r * k + kk;
+                if (vec) {
+                    v = *reinterpret_cast<const float4 *>(p);
+                } else {
+                    v.x = p[0];
+                    if (kk + 1 < k) v.y = p[1];
+                    if (kk + 2 < k) v.z = p[2];
+                    if (kk + 3 < k) v.w = p[3];
+                }
+            }
+            return v;
+        };
         auto gload = [&](int64_t kb) {
 #pragma unroll
-            for (int q = 0; q < LOADS; ++q) {
-                const int u = tid + BTHREADS * q;
-                const int row = u / BKC, kc = u % BKC;
-                const int64_t kk = kb + kc;
-                const int64_t ri = i0 + row, rj = j0 + row;
-                sa[q] = (rj < n && kk < k) ? x[rj * k + kk] : 0.0f;   // A side: j
-                sb[q] = (ri < n && kk < k) ? x[ri * k + kk] : 0.0f;   // B side: i
+            for (int q = 0; q < UNITS; ++q) {
+                const int u = tid + BTHREADS * q, row = u / 4;
+                if (BM * 4 < BTHREADS && u >= BM * 4) break;
+                const int64_t kk = kb + (u % 4) * 4;
+                sa[q] = row4(j0 + row, kk);   // A side: j
+                sb[q] = row4(i0 + row, kk);   // B side: i
             }
         };
 
@@ -100,42 +126,66 @@ __global__ __launch_bounds__(BTHREADS) void batched_kernel(BatchedArgs args)
 #pragma unroll
             for (int b = 0; b < TM; ++b) acc[a][b] = part[a][b] = 0.0f;
 
-        gload(0);
-        for (int64_t kb = 0; kb < k; kb += BKC) {
-            __syncthreads();
+        // QUADS: the quarters of the tile that hold a pair (bit 2 h + g: half h
+        // of the j, half g of the i; TM = 8, where a half is a run of four)
+        auto sweep = [&](auto quads) {
+            constexpr int QUADS = decltype(quads)::value;
+            auto on = [](int a, int b) { return TM < 8 || ((QUADS >> ((a >> 2) * 2 + (b >> 2))) & 1); };
+            constexpr bool ALL_A = TM < 8 || (QUADS & 12), ALL_B = TM < 8 || (QUADS & 10);
+            gload(0);
+            for (int64_t kb = 0; kb < k; kb += BKC) {
+                __syncthreads();
 #pragma unroll
-            for (int q = 0; q < LOADS; ++q) {
-                const int u = tid + BTHREADS * q;
-                const int row = u / BKC, kc = u % BKC;
-                as_[kc][row] = sa[q];
-                bs_[kc][row] = sb[q];
-            }
-            __syncthreads();
-            if (kb + BKC < k) gload(kb + BKC);
-            // the chunk's real features only (a set with d = 8 fills half)
-            const int nk = (k - kb) < BKC ? (int)(k - kb) : BKC;
-#pragma unroll 4
-            for (int kc = 0; kc < nk; ++kc) {
-                float av[TM], bv[TM];
-#pragma unroll
-                for (int m = 0; m < TM; ++m) {
-                    av[m] = as_[kc][side_index<BM, TM>(ty, m)];
-                    bv[m] = bs_[kc][side_index<BM, TM>(tx, m)];
+                for (int q = 0; q < UNITS; ++q) {
+                    const int u = tid + BTHREADS * q, row = u / 4, kc = (u % 4) * 4;
+                    if (BM * 4 < BTHREADS && u >= BM * 4) break;
+                    as_[kc][row] = sa[q].x;
+                    as_[kc + 1][row] = sa[q].y;
+                    as_[kc + 2][row] = sa[q].z;
+                    as_[kc + 3][row] = sa[q].w;
+                    bs_[kc][row] = sb[q].x;
+                    bs_[kc + 1][row] = sb[q].y;
+                    bs_[kc + 2][row] = sb[q].z;
+                    bs_[kc + 3][row] = sb[q].w;
                 }
+                __syncthreads();
+                if (kb + BKC < k) gload(kb + BKC);
+                // the chunk's real features only (a set with d = 8 fills half)
+                const int nk = (k - kb) < BKC ? (int)(k - kb) : BKC;
+#pragma unroll 4
+                for (int kc = 0; kc < nk; ++kc) {
+                    float av[TM], bv[TM];
 #pragma unroll
-                for (int a = 0; a < TM; ++a)
-#pragma unroll
-                    for (int b = 0; b < TM; ++b) bterm<OP>(part[a][b], av[a], bv[b]);
-            }
-            if (OP != OP_MAXIMUM) {
-#pragma unroll
-                for (int a = 0; a < TM; ++a)
-#pragma unroll
-                    for (int b = 0; b < TM; ++b) {
-                        acc[a][b] += part[a][b];
-                        part[a][b] = 0.0f;
+                    for (int m = 0; m < TM; ++m) {
+                        if (m < 4 || ALL_A) av[m] = as_[kc][side_index<BM, TM>(ty, m)];
+                        if (m < 4 || ALL_B) bv[m] = bs_[kc][side_index<BM, TM>(tx, m)];
                     }
+#pragma unroll
+                    for (int a = 0; a < TM; ++a)
+#pragma unroll
+                        for (int b = 0; b < TM; ++b)
+                            if (on(a, b)) bterm<OP>(part[a][b], av[a], bv[b]);
+                }
+                if (OP != OP_MAXIMUM) {
+#pragma unroll
+                    for (int a = 0; a < TM; ++a)
+#pragma unroll
+                        for (int b = 0; b < TM; ++b)
+                            if (on(a, b)) {
+                                acc[a][b] += part[a][b];
+                                part[a][b] = 0.0f;
+                            }
+                }
             }
+        };
+        if (TM < 8) {
+            sweep(std::integral_constant<int, 15>());
+        } else {
+            const bool wide = n - i0 > BM / 2;   // the second half of the i holds points
+            if (I > J)
+                wide ? sweep(std::integral_constant<int, 15>()) : sweep(std::integral_constant<int, 5>());
+            else
+                wide ? sweep(std::integral_constant<int, 11>()) : sweep(std::integral_constant<int, 1>());
         }
 #pragma unroll
         for (int a = 0; a < TM; ++a) {

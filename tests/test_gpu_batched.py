@@ -101,3 +101,26 @@ def test_batched_4096_sets():
             check_set(batched[int(b.out_off[s]):int(b.out_off[s]) +
                               int(sizes[s] * (sizes[s] - 1) // 2)].cpu().numpy(),
                       b.set_points(int(s)).cpu().numpy(), method)
+
+
+@pytest.mark.parametrize("method", ["euclidean", "manhattan", "maximum"])
+@pytest.mark.parametrize("tile", [1, 2, 3])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_batched_quarters_and_alignment(method, tile, shift):
+    """Sets whose last tile holds one point, half a tile or more, with feature
+    counts that allow 16-byte loads and not, at aligned and odd addresses.
+    The two-level sums of at most 40 terms err by less than 20 roundings."""
+    sizes = [2, 3, 64, 65, 127, 128, 129, 192, 193, 257]
+    dims = [1, 4, 8, 17, 16, 3, 20, 40, 33, 5]
+    rng = np.random.default_rng(17)
+    sets = [rng.standard_normal((n, k)).astype(np.float32) for n, k in zip(sizes, dims)]
+    flat = torch.zeros(sum(s.size for s in sets) + shift, device="cuda")
+    flat[shift:] = torch.from_numpy(np.concatenate([s.ravel() for s in sets])).cuda()
+    b = Batch(x=flat[shift:], sizes=np.array(sizes), dims=np.array(dims), method=method)
+    print("case batched quarters", method, tile, shift, flush=True)
+    b.run(tile)
+    for s, x in enumerate(sets):
+        d = np.abs(x[:, None, :].astype(np.float64) - x[None])
+        want = {"euclidean": np.sqrt((d * d).sum(-1)), "manhattan": d.sum(-1), "maximum": d.max(-1)}[method]
+        iu = np.triu_indices(len(x), 1)
+        np.testing.assert_allclose(b.result(s).cpu().numpy(), want[iu], rtol=20 * 2.0 ** -24, atol=0)
