@@ -99,66 +99,6 @@ struct GramArgs {
     float tau;
 };
 
-// Pre-pass: split every centred value x - c once into operand blocks
-// (gt_mfma.h); features k..kp-1 and rows past n are zero.  One thread per 8
-// consecutive features (one 16 B store per term), a wave per block of 32 rows
-// x 16 features.
-template <int SPLIT, bool VEC4>
-__global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x, int64_t n,
-                                                    int64_t k, int64_t ldx, int64_t kp,
-                                                    const float *__restrict__ center,
-                                                    const float *__restrict__ scales,
-                                                    unsigned short *__restrict__ terms)
-{
-    constexpr int NT = Split<SPLIT>::NT;
-    const int64_t nch = kp / OPERAND_K;
-    const int64_t blocks = operand_rows(n) / 32 * nch;
-    const int lane = threadIdx.x & 63;
-    for (int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); blk < blocks;
-         blk += (int64_t)gridDim.x * 4) {
-        int64_t rb, ch;
-        if (blocks <= 0xffffffffll) {
-            // 32-bit division (the 64-bit one is a long instruction sequence)
-            rb = (uint32_t)blk / (uint32_t)nch;
-            ch = (uint32_t)blk - (uint32_t)rb * (uint32_t)nch;
-        } else {
-            rb = blk / nch;
-            ch = blk % nch;
-        }
-        const int64_t row = rb * 32 + (lane & 31), c0 = ch * OPERAND_K + (lane >> 5) * 8;
-        const int64_t r = row < n ? row : n - 1;
-        const float sc = (SPLIT == SPLIT_FP16) ? scales[r] : 1.0f;
-        float v[8];
-        if (VEC4 && c0 + 8 <= k) {
-            const float4 a = *reinterpret_cast<const float4 *>(x + r * ldx + c0);
-            const float4 b = *reinterpret_cast<const float4 *>(x + r * ldx + c0 + 4);
-            const float4 ca = *reinterpret_cast<const float4 *>(center + c0);
-            const float4 cb = *reinterpret_cast<const float4 *>(center + c0 + 4);
-            v[0] = a.x - ca.x; v[1] = a.y - ca.y; v[2] = a.z - ca.z; v[3] = a.w - ca.w;
-            v[4] = b.x - cb.x; v[5] = b.y - cb.y; v[6] = b.z - cb.z; v[7] = b.w - cb.w;
-        } else {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) v[c] = (c0 + c < k) ? x[r * ldx + c0 + c] - center[c0 + c] : 0.0f;
-        }
-        unsigned short t[8][NT];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (SPLIT == SPLIT_FP16) v[c] *= sc;
-            Split<SPLIT>::split(v[c], t[c]);
-        }
-#pragma unroll
-        for (int q = 0; q < NT; ++q) {
-            uint4 w;
-            w.x = t[0][q] | ((unsigned)t[1][q] << 16);
-            w.y = t[2][q] | ((unsigned)t[3][q] << 16);
-            w.z = t[4][q] | ((unsigned)t[5][q] << 16);
-            w.w = t[6][q] | ((unsigned)t[7][q] << 16);
-            if (row >= n) w = make_uint4(0, 0, 0, 0);
-            *reinterpret_cast<uint4 *>(terms + (blk * NT + q) * OPERAND_VALUES + lane * 8) = w;
-        }
-    }
-}
-
 // Exclusive scan of one int per thread over a workgroup of NW waves.
 template <int NW>
 __device__ __forceinline__ int block_exclusive_scan(int v, int *tmp, int &total)
@@ -625,27 +565,51 @@ __global__ __launch_bounds__(NW * 64, 4) void gram_tile_kernel(GramArgs args)
 // integer centres); a constant column takes its value; a column holding a
 // NaN or an infinity is not moved.
 constexpr int CS_ROWS = 256;    // rows per partial-statistics block
+constexpr int PREP_THREADS = 1024, PREP_WAVES = PREP_THREADS / 64;
 
-__global__ __launch_bounds__(256) void colstats_partial_kernel(const float *__restrict__ x,
-                                                               int64_t n, int64_t k, int64_t ldx,
-                                                               float *__restrict__ psum,
-                                                               float *__restrict__ pmin,
-                                                               float *__restrict__ pmax)
+// 64 columns per workgroup, a wave per 16 rows, their sums combined in wave
+// order.  Bound: latency; 9001 x 130 12 us with a thread per column and all 256
+// rows, 5.0 us here.
+__global__ __launch_bounds__(PREP_THREADS) void colstats_partial_kernel(const float *__restrict__ x,
+                                                                        int64_t n, int64_t k, int64_t ldx,
+                                                                        float *__restrict__ psum,
+                                                                        float *__restrict__ pmin,
+                                                                        float *__restrict__ pmax)
 {
-    const int64_t r0 = (int64_t)blockIdx.x * CS_ROWS;
-    const int64_t r1 = (r0 + CS_ROWS < n) ? r0 + CS_ROWS : n;
-    for (int64_t c = (int64_t)blockIdx.y * 256 + threadIdx.x; c < k; c += (int64_t)gridDim.y * 256) {
+    constexpr int ROWS = CS_ROWS / PREP_WAVES;
+    __shared__ float red[3][PREP_WAVES][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r0 = (int64_t)blockIdx.x * CS_ROWS + wave * ROWS;
+    for (int64_t cb = (int64_t)blockIdx.y * 64; cb < k; cb += (int64_t)gridDim.y * 64) {
+        const int64_t c = cb + lane;
         float sum = 0.0f, mn = __builtin_inff(), mx = -__builtin_inff();
-#pragma unroll 8
-        for (int64_t r = r0; r < r1; ++r) {
-            const float v = x[r * ldx + c];
-            sum += v;              // a NaN or an infinity makes the sum non-finite
-            mn = fminf(mn, v);
-            mx = fmaxf(mx, v);
+        if (c < k) {
+            float v[ROWS];
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q) v[q] = r0 + q < n ? x[(r0 + q) * ldx + c] : 0.0f;
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q) {
+                if (r0 + q >= n) break;
+                sum += v[q];              // a NaN or an infinity makes the sum non-finite
+                mn = fminf(mn, v[q]);
+                mx = fmaxf(mx, v[q]);
+            }
         }
-        psum[blockIdx.x * k + c] = sum;
-        pmin[blockIdx.x * k + c] = mn;
-        pmax[blockIdx.x * k + c] = mx;
+        red[0][wave][lane] = sum;
+        red[1][wave][lane] = mn;
+        red[2][wave][lane] = mx;
+        __syncthreads();
+        if (wave == 0 && c < k) {
+            for (int w = 1; w < PREP_WAVES; ++w) {
+                sum += red[0][w][lane];
+                mn = fminf(mn, red[1][w][lane]);
+                mx = fmaxf(mx, red[2][w][lane]);
+            }
+            psum[blockIdx.x * k + c] = sum;
+            pmin[blockIdx.x * k + c] = mn;
+            pmax[blockIdx.x * k + c] = mx;
+        }
+        __syncthreads();
     }
 }
 
@@ -701,44 +665,71 @@ __global__ __launch_bounds__(256) void colstats_finish_kernel(const float *__res
     }
 }
 
-// ||x_i - c||^2 per row (and, for FP16, the power-of-two row scale and its
-// inverse): one wave per row.  The squares are summed with compensation
-// (each product split exactly by an fma, each addition's rounding error
-// recovered by TwoSum), so the norm is within about 2u of exact whatever k.
-__global__ __launch_bounds__(256) void row_prep_kernel(const float *__restrict__ x, int64_t n,
-                                                       int64_t k, int64_t ldx,
-                                                       const float *__restrict__ center,
-                                                       float *__restrict__ norms,
-                                                       float *__restrict__ scales,
-                                                       float *__restrict__ iscales)
+// ||v||^2 of one centred row by one wave, and max |v|.  The squares are summed
+// with compensation (each product split exactly by an fma, each addition's
+// rounding error recovered by TwoSum), so the norm is within about 2u of exact
+// whatever k.
+__device__ __forceinline__ void centred_norm(const float *xr, const float *center, int64_t k, float &norm,
+                                             float &m)
 {
 #pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < n; row += (int64_t)gridDim.x * 4) {
-        const float *xr = x + row * ldx;
-        float s = 0.0f, comp = 0.0f, m = 0.0f;
-        for (int64_t c = lane; c < k; c += 64) {
-            const float v = xr[c] - center[c];
-            const float p = v * v;
-            const float pe = fmaf(v, v, -p);          // v * v = p + pe exactly
-            const float t = s + p;
-            const float bp = t - s;
-            comp += ((s - (t - bp)) + (p - bp)) + pe;  // s + p = t + (TwoSum error)
-            s = t;
-            m = fmaxf(m, fabsf(v));
-        }
+    const int lane = threadIdx.x & 63;
+    float s = 0.0f, comp = 0.0f;
+    m = 0.0f;
+#pragma unroll 4
+    for (int64_t c = lane; c < k; c += 64) {
+        const float v = xr[c] - center[c];
+        const float p = v * v;
+        const float pe = fmaf(v, v, -p);          // v * v = p + pe exactly
+        const float t = s + p;
+        const float bp = t - s;
+        comp += ((s - (t - bp)) + (p - bp)) + pe;  // s + p = t + (TwoSum error)
+        s = t;
+        m = fmaxf(m, fabsf(v));
+    }
 #pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const float so = __shfl_xor(s, d, 64), co = __shfl_xor(comp, d, 64);
-            const float t = s + so;
-            const float bp = t - s;
-            comp = (comp + co) + ((s - (t - bp)) + (so - bp));
-            s = t;
-            m = fmaxf(m, __shfl_xor(m, d, 64));
-        }
-        if (lane == 0) {
-            norms[row] = s + comp;
-            if (scales) {
+    for (int d = 32; d >= 1; d >>= 1) {
+        const float so = __shfl_xor(s, d, 64), co = __shfl_xor(comp, d, 64);
+        const float t = s + so;
+        const float bp = t - s;
+        comp = (comp + co) + ((s - (t - bp)) + (so - bp));
+        s = t;
+        m = fmaxf(m, __shfl_xor(m, d, 64));
+    }
+    norm = s + comp;
+}
+
+// Row norms ||x_i - c||^2, for FP16 the power-of-two row scales and their
+// inverses, and every centred value x - c split once into operand blocks
+// (gt_mfma.h; features k..kp-1 and rows past n are zero).  `split` workgroups
+// per block of 32 rows: a wave per row for the norms, then a wave per chunk of
+// 16 features, one 1 KB block per term.  One launch and one read of the rows
+// from memory; a kernel for the norms and one for the terms took 5.1 + 8.5 us
+// at 9001 x 130, this one 13.5, and its
+// launch comes once.
+template <int SPLIT, bool VEC4>
+__global__ __launch_bounds__(PREP_THREADS) void row_prep_kernel(const float *__restrict__ x, int64_t n,
+                                                                int64_t k, int64_t ldx, int64_t kp, int split,
+                                                                const float *__restrict__ center,
+                                                                float *__restrict__ norms,
+                                                                float *__restrict__ scales,
+                                                                float *__restrict__ iscales,
+                                                                unsigned short *__restrict__ terms)
+{
+    constexpr int NT = Split<SPLIT>::NT;
+    __shared__ float row_scale[32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t part = blockIdx.x % split, blocks = operand_rows(n) / 32, nch = kp / OPERAND_K;
+    for (int64_t rb = blockIdx.x / split; rb < blocks; rb += gridDim.x / split) {
+        __syncthreads();   // the last block's scales are read
+        for (int q = wave; q < 32 && (SPLIT == SPLIT_FP16 || part == 0); q += PREP_WAVES) {
+            const int64_t row = rb * 32 + q;
+            if (row >= n) break;
+            float norm, m;
+            centred_norm(x + row * ldx, center, k, norm, m);
+            if (lane != 0) continue;
+            if (part == 0) norms[row] = norm;
+            if (SPLIT == SPLIT_FP16) {
                 // power of two that brings max|x - c| into [2^14, 2^15)
                 int e = 0;
                 if (m > 0.0f) {
@@ -746,8 +737,45 @@ __global__ __launch_bounds__(256) void row_prep_kernel(const float *__restrict__
                     if (e < -100) e = -100;
                     if (e > 100) e = 100;
                 }
-                scales[row] = ldexpf(1.0f, 14 - e);
-                iscales[row] = ldexpf(1.0f, e - 14);
+                row_scale[q] = ldexpf(1.0f, 14 - e);
+                if (part == 0) {
+                    scales[row] = row_scale[q];
+                    iscales[row] = ldexpf(1.0f, e - 14);
+                }
+            }
+        }
+        __syncthreads();
+        const int64_t row = rb * 32 + (lane & 31), r = row < n ? row : n - 1;
+        const float sc = SPLIT == SPLIT_FP16 && row < n ? row_scale[lane & 31] : 1.0f;
+        for (int64_t ch = part * PREP_WAVES + wave; ch < nch; ch += (int64_t)split * PREP_WAVES) {
+            const int64_t c0 = ch * OPERAND_K + (lane >> 5) * 8;
+            float v[8];
+            if (VEC4 && c0 + 8 <= k) {
+                const float4 a = *reinterpret_cast<const float4 *>(x + r * ldx + c0);
+                const float4 b = *reinterpret_cast<const float4 *>(x + r * ldx + c0 + 4);
+                const float4 ca = *reinterpret_cast<const float4 *>(center + c0);
+                const float4 cb = *reinterpret_cast<const float4 *>(center + c0 + 4);
+                v[0] = a.x - ca.x; v[1] = a.y - ca.y; v[2] = a.z - ca.z; v[3] = a.w - ca.w;
+                v[4] = b.x - cb.x; v[5] = b.y - cb.y; v[6] = b.z - cb.z; v[7] = b.w - cb.w;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) v[c] = (c0 + c < k) ? x[r * ldx + c0 + c] - center[c0 + c] : 0.0f;
+            }
+            unsigned short t[8][NT];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                if (SPLIT == SPLIT_FP16) v[c] *= sc;
+                Split<SPLIT>::split(v[c], t[c]);
+            }
+#pragma unroll
+            for (int q = 0; q < NT; ++q) {
+                uint4 w;
+                w.x = t[0][q] | ((unsigned)t[1][q] << 16);
+                w.y = t[2][q] | ((unsigned)t[3][q] << 16);
+                w.z = t[4][q] | ((unsigned)t[5][q] << 16);
+                w.w = t[6][q] | ((unsigned)t[7][q] << 16);
+                if (row >= n) w = make_uint4(0, 0, 0, 0);
+                *reinterpret_cast<uint4 *>(terms + ((rb * nch + ch) * NT + q) * OPERAND_VALUES + lane * 8) = w;
             }
         }
     }
@@ -799,17 +827,22 @@ hipError_t launch_layout(int layout, bool vec4, GramArgs &args, hipStream_t stre
 }
 
 template <int SPLIT>
-hipError_t launch_split(bool vec4, const float *x, int64_t n, int64_t k, int64_t ldx, const GramPrep &prep,
-                        hipStream_t stream)
+hipError_t launch_rows(bool vec4, const float *x, int64_t n, int64_t k, int64_t ldx, const GramPrep &prep,
+                       hipStream_t stream)
 {
-    int64_t blocks = (operand_rows(n) / 32 * (prep.kp / OPERAND_K) + 3) / 4;
-    if (blocks > 65536) blocks = 65536;
+    // workgroups per block of 32 rows: to fill the CUs, while each has a chunk
+    // per wave
+    const int64_t blocks = operand_rows(n) / 32;
+    int64_t split = 512 / (blocks > 0 ? blocks : 1), most = prep.kp / OPERAND_K / PREP_WAVES;
+    if (split > most) split = most;
+    if (split < 1) split = 1;
+    const dim3 grid((unsigned)((blocks < 65536 ? blocks : 65536) * split));
     if (vec4)
-        hipLaunchKernelGGL((split_kernel<SPLIT, true>), dim3((unsigned)blocks), dim3(256), 0, stream, x, n, k,
-                           ldx, prep.kp, prep.center, prep.scales, prep.terms);
+        hipLaunchKernelGGL((row_prep_kernel<SPLIT, true>), grid, dim3(PREP_THREADS), 0, stream, x, n, k, ldx,
+                           prep.kp, (int)split, prep.center, prep.norms, prep.scales, prep.iscales, prep.terms);
     else
-        hipLaunchKernelGGL((split_kernel<SPLIT, false>), dim3((unsigned)blocks), dim3(256), 0, stream, x, n,
-                           k, ldx, prep.kp, prep.center, prep.scales, prep.terms);
+        hipLaunchKernelGGL((row_prep_kernel<SPLIT, false>), grid, dim3(PREP_THREADS), 0, stream, x, n, k, ldx,
+                           prep.kp, (int)split, prep.center, prep.norms, prep.scales, prep.iscales, prep.terms);
     return hipGetLastError();
 }
 
@@ -904,9 +937,9 @@ hipError_t gram_prepare(int precision, const float *x, int64_t n, int64_t k, int
     float *pmax = reinterpret_cast<float *>(ws + 2 * pbytes);
     const bool fp16 = (precision == 2);
     {
-        const int64_t cb = (k + 255) / 256;
+        const int64_t cb = (k + 63) / 64;
         hipLaunchKernelGGL(colstats_partial_kernel, dim3((unsigned)csb, (unsigned)(cb < 1024 ? cb : 1024)),
-                           dim3(256), 0, stream, x, n, k, ldx, psum, pmin, pmax);
+                           dim3(PREP_THREADS), 0, stream, x, n, k, ldx, psum, pmin, pmax);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         const int64_t fb = (k + CS_COLS - 1) / CS_COLS;
@@ -915,18 +948,9 @@ hipError_t gram_prepare(int precision, const float *x, int64_t n, int64_t k, int
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    {
-        int64_t blocks = (n + 3) / 4;
-        if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL(row_prep_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, k,
-                           ldx, prep.center, prep.norms, fp16 ? prep.scales : nullptr,
-                           fp16 ? prep.iscales : nullptr);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
     const bool vec4 = rows_vec4(x, k, ldx);
-    return fp16 ? launch_split<SPLIT_FP16>(vec4, x, n, k, ldx, prep, stream)
-                : launch_split<SPLIT_BF16>(vec4, x, n, k, ldx, prep, stream);
+    return fp16 ? launch_rows<SPLIT_FP16>(vec4, x, n, k, ldx, prep, stream)
+                : launch_rows<SPLIT_BF16>(vec4, x, n, k, ldx, prep, stream);
 }
 
 // Above this tau nearly every pair would be recomputed: the request is
