@@ -8,8 +8,9 @@
 // v_bcnt_u32_b32, which adds to an accumulator).  From the row counts pa, pb:
 //   on in exactly one row = pa + pb - 2 (a & b),  on in either = pa + pb - (a & b).
 // Packed requests on one point set of up to SMALL_DIV_MAX features take the
-// matrix cores instead: one 0/1 byte per feature and v_mfma_i32_32x32x32_i8
-// give the same exact count of features on in both rows (binary_mfma_kernel).
+// matrix cores instead: four bits per feature (FP4, 0 or 1) and
+// v_mfma_f32_32x32x64_f8f6f4 give the same exact count of features on in both
+// rows, an FP32 sum of integers below 2^24 (binary_mfma_kernel).
 // The counts are exact integers; their ratio is rounded correctly to FP32,
 // which equals the FP32 rounding of the FP64 ratio R computes (double
 // rounding of a quotient from binary64 to binary32 is innocuous), so the
@@ -54,16 +55,23 @@ __device__ __forceinline__ float binary_value(uint32_t pa_plus_pb, uint32_t both
     return no == 0 ? 0.0f : q;
 }
 
+// The same from counts held as floats (exact: all are at most 2 SMALL_DIV_MAX).
+__device__ __forceinline__ float binary_value(float pa_plus_pb, float both)
+{
+    const float no = pa_plus_pb - both, nx = no - both;
+    const float q = small_quotient(nx, no);
+    return no == 0.0f ? 0.0f : q;
+}
+
 // The same value with y = RN(1/no) read from a table (lut[0] = 0: no = 0
 // implies nx = 0, and the sequence then gives +0).  RN(1/no) is one of the
 // reciprocals tests/exhaustive/small_div.c checks.
-__device__ __forceinline__ float binary_value_lut(uint32_t pa_plus_pb, uint32_t both, const float *lut)
+__device__ __forceinline__ float binary_value_lut(float pa_plus_pb, float both, const float *lut)
 {
-    const uint32_t no = pa_plus_pb - both, nx = no - both;
-    const float y = lut[no];
-    const float a = (float)nx, b = (float)no;
-    const float q0 = __fmul_rn(a, y);
-    const float r = fmaf(-q0, b, a);
+    const float no = pa_plus_pb - both, nx = no - both;
+    const float y = lut[(uint32_t)no];
+    const float q0 = __fmul_rn(nx, y);
+    const float r = fmaf(-q0, no, nx);
     return fmaf(r, y, q0);
 }
 
@@ -242,18 +250,20 @@ __global__ __launch_bounds__(BTHREADS) void binary_tile_kernel(BinaryArgs args)
 
 // ---------------------------------------------------------------------------
 // Packed whole-matrix requests: the counts on the matrix cores.  Each row is
-// one 0/1 byte per feature (zero-padded to a multiple of 32) and its count of
-// ones; v_mfma_i32_32x32x32_i8 sums the products of two rows' bytes exactly,
-// which is the number of features on in both.  The tiles are 256 x 256 (two
-// workgroups of 8 waves) or 128 x 128 (4 waves); chunks of 32 features (32 B
+// four bits per feature, FP4 (E2M1) 0 or 1, zero-padded to a multiple of 64, and
+// its count of ones; v_mfma_f32_32x32x64_f8f6f4 sums the products of two rows
+// exactly, which is the number of features on in both.  The tiles are 256 x 256
+// (two workgroups of 8 waves) or 128 x 128 (4 waves); chunks of 64 features (32 B
 // per row) reach LDS through global_load_lds into a ring of NSTAGE stages,
 // 16-byte halves swapped by ((R >> 2) ^ (R >> 3)) & 1 so that the operand
 // reads of consecutive rows hit distinct banks.
 // ---------------------------------------------------------------------------
 typedef int bin_i32x4_t __attribute__((ext_vector_type(4)));
-typedef int bin_i32x16_t __attribute__((ext_vector_type(16)));
+typedef int bin_i32x8_t __attribute__((ext_vector_type(8)));
+typedef float bin_f32x16_t __attribute__((ext_vector_type(16)));
 
-constexpr int QBK = 32;                  // features per chunk (bytes per row)
+constexpr int QBK = 32;                  // bytes per row and chunk
+constexpr int QFEATURES = 64;            // features per chunk
 constexpr int QSUPER = 4;                // super-tile side in tiles
 // Tile side: 256 x 256 pairs for large n; 128 x 128 (four workgroups per
 // CU) while the 256 schedule has fewer than QSMALL_ROUNDS rounds of 256 CUs
@@ -272,7 +282,7 @@ constexpr int64_t QSMALL_ROUNDS = 4;
 // with less LDS per workgroup.
 constexpr int QX = 32;
 constexpr int QXB = 5;                          // B blocks per wave
-// Reciprocal table entries (no = 0 .. 2 kb) when 2 kb < QLUT: an LDS read
+// Reciprocal table entries (no = 0 .. 2 x padded features) when fewer than QLUT: an LDS read
 // instead of v_rcp_f32 (a quarter-rate instruction) and the no = 0 select.
 constexpr int QLUT = 2048;
 template <int QA, int QB>
@@ -310,47 +320,45 @@ __device__ __forceinline__ void wait_vmcnt(int v)
     }
 }
 
-int64_t bytes_ld(int64_t k) { return (k + QBK - 1) / QBK * QBK; }
+int64_t bytes_ld(int64_t k) { return (k + QFEATURES - 1) / QFEATURES * QBK; }
 
-// One wave per row: bytes (x != 0) of 4 features per lane, and the row's
-// number of ones.
-__global__ __launch_bounds__(256) void binary_pack8_kernel(const float *__restrict__ x, int64_t n,
+// One wave per row: 64 features a step, a ballot of x != 0, whose bits lanes
+// 0..7 spread to FP4 values (1.0 is 2), eight to a word; and the row's number
+// of ones.
+__global__ __launch_bounds__(256) void binary_pack4_kernel(const float *__restrict__ x, int64_t n,
                                                            int64_t k, int64_t ldx, int64_t kb,
                                                            uint32_t *__restrict__ ind,
                                                            uint32_t *__restrict__ cnt)
 {
     const int lane = threadIdx.x & 63;
+    const int64_t steps = kb / QBK;
     for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < n;
          row += (int64_t)gridDim.x * 4) {
         const float *xr = x + row * ldx;
         uint32_t *ir = ind + row * (kb / 4);
         uint32_t ones = 0;
-        for (int64_t f0 = 0; f0 < kb; f0 += 256) {
-            const int64_t f = f0 + 4 * lane;
-            if (f >= kb) break;
-            uint32_t w = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const bool on = (f + e < k) && (xr[f + e] != 0.0f);
-                w |= (on ? 1u : 0u) << (8 * e);
-                ones += on ? 1u : 0u;
-            }
-            ir[f / 4] = w;
+#pragma unroll 4
+        for (int64_t st = 0; st < steps; ++st) {
+            const int64_t f = st * QFEATURES + lane;
+            const unsigned long long m = __ballot(f < k && xr[f < k ? f : 0] != 0.0f);
+            ones += (uint32_t)__popcll(m);
+            uint32_t w = (uint32_t)(m >> (8 * (lane & 7))) & 0xffu;
+            w = (w | w << 12) & 0x000f000fu;
+            w = (w | w << 6) & 0x03030303u;
+            w = (w | w << 3) & 0x11111111u;
+            if (lane < 8) ir[st * 8 + lane] = w << 1;
         }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) ones += __shfl_xor(ones, d, 64);
         if (lane == 0) cnt[row] = ones;
     }
 }
 
 struct BinMfmaArgs {
-    const unsigned char *ind;   // n x kb bytes
+    const unsigned char *ind;   // n x kb bytes, two features each
     const uint32_t *cnt;        // ones per row
     int64_t n, kb;
     float *out;                 // packed
     int64_t T;                  // tiles per side
     int64_t id_offset, ids_this;
-    int64_t stagger_below;      // odd workgroups below this id start late (first round)
 };
 
 // Line ownership.  Packed column j (the pairs (i, j), i > j) is one run of
@@ -382,6 +390,12 @@ __device__ __forceinline__ float lane_fetch(float v, int src_byte)
 
 // Only called with at most SMALL_DIV_MAX features: the quotient is
 // small_quotient's.
+// Bound: the stores and the quotients' VALU work, which follow each tile's
+// products; with many features the products.  30011 x 300: 513 us a call with
+// a byte per feature (v_mfma_i32_32x32x32_i8, twice the operand bytes and
+// products), 404 in FP4; 65536 x 300 2.59 -> 1.85 ms, 30011 x 4000 3.46 -> 1.86.
+// (Starting every second workgroup late, which helped the longer product
+// loop, gains nothing here.)
 template <int QA, int QB, bool LUT>
 __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::THREADS)) void binary_mfma_kernel(
     BinMfmaArgs args)
@@ -390,23 +404,14 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
     constexpr int QTERM = Q::TERM, QSTAGE = Q::STAGE, NW = Q::NW, NS = Q::NSTAGE, G = Q::G, GA = Q::GA;
     static_assert((NS - 2) * Q::GMAX <= 12, "wait_vmcnt covers the loads in flight");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[NS * QSTAGE + (QA + QB + QX) * 4];
-    uint32_t *cA = reinterpret_cast<uint32_t *>(smem + NS * QSTAGE);
-    uint32_t *cB = cA + QA;
+    float *cA = reinterpret_cast<float *>(smem + NS * QSTAGE);
+    float *cB = cA + QA;
     __shared__ float lut[LUT ? QLUT : 1];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wj = wave % Q::WJ, wi = wave / Q::WJ;   // A rows (j) 32 wj.., B rows (i) 128 wi..
 
     const int64_t gid = args.id_offset + xcd_remap(blockIdx.x, args.ids_this);
-    // Two 8-wave workgroups share a CU and have the same work, so if they
-    // start together they stay in step, and both store at once and then both
-    // run the matrix cores.  The odd workgroups of the first round start
-    // about 0.4 of a tile late, which keeps the pairs offset afterwards
-    // (65536 x 256, A/B on one box: 2.12 vs 2.30 ms).
-    if ((blockIdx.x & 1) && (int64_t)blockIdx.x < args.stagger_below) {
-        __builtin_amdgcn_s_sleep(127);
-        __builtin_amdgcn_s_sleep(127);
-    }
     const int part = (int)(gid % Q::PARTS);
     const int64_t id = gid / Q::PARTS;
     const int64_t st = id / (QSUPER * QSUPER);
@@ -420,14 +425,14 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
     if (j0 >= n) return;
     for (int t = tid; t < QA + QB + QX; t += Q::THREADS) {
         if (t < QA)
-            cA[t] = j0 + t < n ? args.cnt[j0 + t] : 0u;
+            cA[t] = j0 + t < n ? (float)args.cnt[j0 + t] : 0.0f;
         else
-            cB[t - QA] = i0 + t - QA < n ? args.cnt[i0 + t - QA] : 0u;
+            cB[t - QA] = i0 + t - QA < n ? (float)args.cnt[i0 + t - QA] : 0.0f;
     }
     if (LUT)
-        for (int t = tid; t <= 2 * args.kb; t += Q::THREADS) lut[t] = t ? 1.0f / (float)t : 0.0f;
-    auto value = [&](uint32_t pa_plus_pb, uint32_t both) {
-        return LUT ? binary_value_lut(pa_plus_pb, both, lut) : binary_value<true>(pa_plus_pb, both);
+        for (int t = tid; t <= 4 * args.kb; t += Q::THREADS) lut[t] = t ? 1.0f / (float)t : 0.0f;
+    auto value = [&](float pa_plus_pb, float both) {
+        return LUT ? binary_value_lut(pa_plus_pb, both, lut) : binary_value(pa_plus_pb, both);
     };
 
     // 32-row load groups: g < GA are A rows 32 g.., the rest B rows
@@ -458,11 +463,13 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
     const int lrow = lane & 31;
     const int roff = lrow * QBK + (((lane >> 5) ^ (((lrow >> 2) ^ (lrow >> 3)) & 1)) * 16);
 
-    bin_i32x16_t acc[QXB];
+    bin_f32x16_t acc[QXB];
 #pragma unroll
     for (int b = 0; b < QXB; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[b][r] = 0;
+        for (int r = 0; r < 16; ++r) acc[b][r] = 0.0f;
+    // FP4 operands take the first four of eight registers
+    auto wide = [](bin_i32x4_t v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1); };
 
     const int nchunks = (int)(args.kb / QBK);
     const int lpc = (G - wave + NW - 1) / NW;   // this wave's loads per chunk
@@ -483,7 +490,8 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
         for (int b = 0; b < QXB; ++b) {
             const bin_i32x4_t bv =
                 *reinterpret_cast<const bin_i32x4_t *>(sg + QTERM + (wi * 128 + b * 32) * QBK);
-            acc[b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, acc[b], 0, 0, 0);
+            acc[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wide(av), wide(bv), acc[b], 4, 4, 0, 127, 0,
+                                                                     127);
         }
     }
     __syncthreads();   // cA, cB and lut visible
@@ -494,7 +502,7 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
     const int lx = lane & 31;
     const bool hi = (lane >> 5) != 0;
     const int lib = wi * 128 + lx;
-    uint32_t pb[QXB];
+    float pb[QXB];
 #pragma unroll
     for (int b = 0; b < QXB; ++b) pb[b] = cB[lib + b * 32];
     const uint64_t fout = reinterpret_cast<uintptr_t>(args.out) >> 2;
@@ -515,10 +523,10 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
             const unsigned step_u = 4 * cw - 4 * dc - 10;
             const unsigned rc = base_u + (hi ? step_u : 0u);   // column j at row i0
             const unsigned e = (0u - (fw + rc)) & 31u;
-            const uint32_t pa = cA[wj * 32 + (int)dc + (hi ? 4 : 0)];
+            const float pa = cA[wj * 32 + (int)dc + (hi ? 4 : 0)];
             float v[QXB];
 #pragma unroll
-            for (int b = 0; b < QXB; ++b) v[b] = value(pa + pb[b], (uint32_t)acc[b][r]);
+            for (int b = 0; b < QXB; ++b) v[b] = value(pa + pb[b], acc[b][r]);
             // byte offsets from the wave-uniform outw stay in 32 bits
             char *const ob = reinterpret_cast<char *>(outw);
             if ((int)dc == lastc && (unsigned)lx < e)
@@ -545,14 +553,14 @@ __global__ __launch_bounds__((QTile<QA, QB>::THREADS), (1024 / QTile<QA, QB>::TH
         const int64_t e = line_gap(fout + (uint64_t)(pbj + i0));
         const int64_t lo = j + 1 >= i0 ? j + 1 : i0 + e;
         const int64_t hi_ = i0 + QB + e < n ? i0 + QB + e : n;
-        const uint32_t pa = cA[lj];
+        const float pa = cA[lj];
 #pragma unroll
         for (int b = 0; b < QXB; ++b) {
             // the last block is the next wave's first, except for the last wave
             if (b == QXB - 1 && wi != Q::WI - 1) continue;
             const int64_t i = i0 + lib + b * 32;
             if (i >= lo && i < hi_)
-                args.out[pbj + i] = value(pa + pb[b], (uint32_t)acc[b][r]);
+                args.out[pbj + i] = value(pa + pb[b], acc[b][r]);
         }
     }
 }
@@ -575,14 +583,6 @@ hipError_t launch_mfma_tiles(BinMfmaArgs &args, hipStream_t stream)
     args.T = (args.n + QB - 1) / QB;
     const int64_t S = (args.T + QSUPER - 1) / QSUPER;
     const int64_t ids = S * (S + 1) / 2 * QSUPER * QSUPER * Q::PARTS;
-    args.stagger_below = 0;
-    if (Q::PARTS == 2) {   // two workgroups per CU: stagger the first round
-        int dev = 0, cus = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e != hipSuccess) return e;
-        args.stagger_below = 2 * (int64_t)cus;
-    }
     const int64_t max_ids = int64_t(1) << 23;   // a multiple of PARTS
     for (int64_t off = 0; off < ids; off += max_ids) {
         args.id_offset = off;
@@ -600,8 +600,8 @@ hipError_t launch_mfma_tiles(BinMfmaArgs &args, hipStream_t stream)
 int64_t binary_words(int64_t k) { return (k + 31) / 32; }
 
 // Workspace of a binary call on one point set: the bit rows (with their
-// counts), then, up to SMALL_DIV_MAX features, the byte rows and counts of
-// the matrix-core form (a quarter of the input's size).
+// counts), then, up to SMALL_DIV_MAX features, the FP4 rows and counts of
+// the matrix-core form (an eighth of the input's size).
 size_t binary_workspace_bytes(int64_t n, int64_t k)
 {
     auto a256 = [](size_t v) { return (v + 255) / 256 * 256; };
@@ -630,7 +630,7 @@ hipError_t launch_binary_self(int layout, const float *x, int64_t n, int64_t k, 
     {
         int64_t blocks = (n + 3) / 4;
         if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL(binary_pack8_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, k,
+        hipLaunchKernelGGL(binary_pack4_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, k,
                            ldx, kb, reinterpret_cast<uint32_t *>(ind), cnt);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -641,7 +641,7 @@ hipError_t launch_binary_self(int layout, const float *x, int64_t n, int64_t k, 
     args.n = n;
     args.kb = kb;
     args.out = out;
-    const bool lut = 2 * kb < QLUT;
+    const bool lut = 4 * kb < QLUT;   // (two features a byte)
     const int64_t t256 = (n + 255) / 256;
     if (t256 * (t256 + 1) / 2 < QSMALL_ROUNDS * 256)
         return lut ? launch_mfma_tiles<128, 128, true>(args, stream)

@@ -499,3 +499,20 @@ def test_tile_sides_agree(method, k):
         else:
             off = ~np.eye(1037, n, dtype=bool)
             np.testing.assert_array_equal(cross[off], full[:1037][off])
+
+
+@pytest.mark.parametrize("n", [2, 129, 300])
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 63, 64, 65, 127, 129, 960, 961, 1025])
+def test_binary_packed_feature_edges(n, k):
+    """Packed binary distances at the edges of the words and chunks of features
+    and of the two quotient forms, bit for bit; a row of ones, an empty row,
+    and infinities and negative zero among the values."""
+    rng = np.random.default_rng(n * 2000 + k)
+    x = (rng.random((n, k)) < 0.4).astype(np.float32) * rng.standard_normal((n, k)).astype(np.float32)
+    x[0] = 1.0
+    x[1] = -0.0
+    if n > 2:
+        x[2, ::3] = np.inf
+        x[3, ::5] = -np.inf
+    got = gt.dist(torch.from_numpy(x).cuda(), "binary").cpu().numpy()
+    np.testing.assert_array_equal(got, orc.dist(x, "binary").astype(np.float32))
