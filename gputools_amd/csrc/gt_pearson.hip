@@ -191,13 +191,12 @@ __global__ __launch_bounds__(PTHREADS) void pmcc_prep_kernel(const float *__rest
 // ---------------------------------------------------------------------------
 // MFMA tile of use = "everything": corr(x, y) = z_x . z_y.
 // ---------------------------------------------------------------------------
-constexpr int MBM = 256;        // variables along x of a tile
-constexpr int MBN = 128;        // along y: two workgroups share a square of 256
+constexpr int MBM = 256;        // side of a square of pairs (variables), two workgroups'
 constexpr int MBK = 16;         // samples per main-loop chunk (one MFMA k-step)
 constexpr int MKPAD = 32;       // split terms are zero-padded to a multiple of this
-constexpr int MTHREADS = 512;   // 8 waves, 4 (x) x 2 (y), 64 x 64 pairs each
+constexpr int MTHREADS = 512;   // 8 waves of 64 x 64 pairs
 constexpr int MSUPER = 2;       // super-tile side in tiles (L2 locality)
-constexpr int MBLOCKS = (MBM + MBN) / 32;   // operand blocks of one term, one chunk
+constexpr int MBLOCKS = MBM / 2 * 3 / 32;   // operand blocks of one term, one chunk
 constexpr int MNSTAGE = 2;
 
 struct PmccTileArgs {
@@ -226,18 +225,22 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
 {
     typedef typename Split<SPLIT>::vec vec;
     constexpr int NT = Split<SPLIT>::NT;
+    // half a square: 256 x by 128 y where both (x, y) and (y, x) are stored; else
+    // 128 x by 256 y, whose rows of results are longer (5671 x 3400 variables x 27
+    // samples, FP16: 68 us with whole squares, 5% more with 128 y, 60 so)
+    constexpr int TX = SYM ? MBM : MBM / 2, TY = SYM ? MBM / 2 : MBM, WAVES_Y = TY / 64;
     constexpr int STAGE = MBLOCKS * NT * OPERAND_BYTES;
     // after the main loop the stages hold each wave's transpose region for
     // the mirrored stores: 64 rows of MTRL floats
     constexpr int MTRL = 36;
     constexpr int TRBYTES = (MTHREADS / 64) * 64 * MTRL * 4;
     constexpr int SBYTES = MNSTAGE * STAGE > TRBYTES ? MNSTAGE * STAGE : TRBYTES;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[SBYTES + (MBM + MBN) * 4];
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[SBYTES + (TX + TY) * 4];
     float *iA = reinterpret_cast<float *>(smem + SBYTES);
-    float *iB = iA + MBM;
+    float *iB = iA + TX;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave >> 1, wc = wave & 1;   // x rows wr*64.., y rows wc*64..
+    const int wr = wave / WAVES_Y, wc = wave % WAVES_Y;   // x rows wr*64.., y rows wc*64..
 
     // Super-tiled schedule: super-tile st covers MSUPER x MSUPER tiles; tiles
     // past the edge (or above the diagonal when SYM) exit at once.
@@ -258,17 +261,17 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
     const int64_t I = SI * MSUPER + w / MSUPER;
     const int64_t J = SJ * MSUPER + w % MSUPER;
     if (I >= args.tiles_a || J >= args.tiles_b || (SYM && J > I)) return;
-    const int64_t x0 = I * MBM, y0 = J * MBM + (gid & 1) * MBN;
+    const int64_t x0 = I * MBM + (SYM ? 0 : (gid & 1) * TX), y0 = J * MBM + (SYM ? (gid & 1) * TY : 0);
     const int64_t na = args.na, nb = args.nb, kp = args.kp;
-    if (y0 >= nb) return;
+    if (x0 >= na || y0 >= nb) return;
 
     if (SPLIT == SPLIT_FP16) {
-        if (tid < MBM) {
+        if (tid < TX) {
             const int64_t r = x0 + tid;
             iA[tid] = r < na ? args.isa[r] : 1.0f;
-        } else if (tid < MBM + MBN) {
-            const int64_t r = y0 + (tid - MBM);
-            iB[tid - MBM] = r < nb ? args.isb[r] : 1.0f;
+        } else if (tid < TX + TY) {
+            const int64_t r = y0 + (tid - TX);
+            iB[tid - TX] = r < nb ? args.isb[r] : 1.0f;
         }
     }
 
@@ -288,9 +291,9 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
 #pragma unroll
     for (int q = 0; q < PMAX; ++q) {
         const int p = min(wave + 8 * q, PIECES - 1), blk = p / NT;
-        const int lside = blk >= MBM / 32;
+        const int lside = blk >= TX / 32;
         const int64_t last = operand_rows(lside ? nb : na) / 32 - 1;
-        const int64_t rb = lside ? y0 / 32 + blk - MBM / 32 : x0 / 32 + blk;
+        const int64_t rb = lside ? y0 / 32 + blk - TX / 32 : x0 / 32 + blk;
         gsrc[q] = (lside ? args.tb : args.ta) +
                   ((rb < last ? rb : last) * (kp / OPERAND_K) * NT + p % NT) * OPERAND_VALUES + lane * 8;
     }
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
             vec bv[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t)
-                bv[t] = *reinterpret_cast<const vec *>(sg + ((MBM / 32 + wc * 2 + b) * NT + t) * OPERAND_BYTES);
+                bv[t] = *reinterpret_cast<const vec *>(sg + ((TX / 32 + wc * 2 + b) * NT + t) * OPERAND_BYTES);
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
                 acc[a][b] = Split<SPLIT>::mfma(av[0][a], bv[0], acc[a][b]);
@@ -370,7 +373,7 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
     // back as rows of 32 consecutive x (128 B per row), instead of 16-byte (or,
     // unaligned, 4-byte) pieces of 32 rows
     const bool fastm = SYM && !diag;
-    const bool whole = x0 + MBM <= na && y0 + MBN <= nb;
+    const bool whole = x0 + TX <= na && y0 + TY <= nb;
     float *const tr = reinterpret_cast<float *>(smem) + wave * 64 * MTRL;
     // lane's four x (8 rq + 4 (lane >> 5) ..) of row (lane & 31) + 32 b
     auto tr_put = [&](int rq, int b, const float (&v)[4]) {
@@ -496,10 +499,10 @@ struct PairwiseArgs {
     int64_t tiles_b;
     int64_t tile_offset, tiles_this;
     bool vec;   // ldo and the output pointers allow 16-byte stores
-    // tiles that pmcc_moments_kernel left (one byte per tile, 1 = left): only
-    // those run, with two passes; null: every tile runs
+    // LEFT: the tiles to run (one byte per tile, 1 = left), and each variable's
+    // power of two
     const uint8_t *left;
-    const float *scale_a, *scale_b;   // with left: each variable's power of two
+    const float *scale_a, *scale_b;
 };
 
 // A sample of a pair counts when both values are present (not NaN): counts
@@ -508,14 +511,15 @@ struct PairwiseArgs {
 // correlation.cu:53-150).  Masked samples are selected away, never multiplied
 // by zero, so an Inf beside a missing value does not leak into the sums.
 // Each chunk's sums are accumulated separately and then added to the totals.
-template <bool SYM>
+// LEFT: only the tiles that pmcc_moments_kernel left, with two passes.
+template <bool SYM, bool LEFT>
 __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs args)
 {
     __shared__ float lds[2][WBK][WLD];   // [0] x side, [1] y side; sample-major
     const int tid = threadIdx.x;
     const int tx = tid & 15, ty = tid >> 4;   // y = 4 tx + j, x = 4 ty + i
     const int64_t t = args.tile_offset + xcd_remap(blockIdx.x, args.tiles_this);
-    if (args.left && args.left[t] == 0) return;
+    if (LEFT && args.left[t] == 0) return;
     int64_t I, J;
     if (SYM) {
         int ti, tj;
@@ -536,15 +540,15 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     const float *pa = args.a + (va_ok ? (x0 + sv) * args.lda : 0);
     const float *pb = args.b + (vb_ok ? (y0 + sv) * args.ldb : 0);
     const float qnan = __builtin_nanf("");
-    const float fa = args.left && va_ok ? args.scale_a[x0 + sv] : 1.0f;
-    const float fb = args.left && vb_ok ? args.scale_b[y0 + sv] : 1.0f;
+    const float fa = LEFT && va_ok ? args.scale_a[x0 + sv] : 1.0f;
+    const float fb = LEFT && vb_ok ? args.scale_b[y0 + sv] : 1.0f;
     float ra[8], rb[8];
     auto gload = [&](int64_t kb) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const int64_t kk = kb + sk + q;
-            ra[q] = (va_ok && kk < dim) ? pa[kk] * fa : qnan;
-            rb[q] = (vb_ok && kk < dim) ? pb[kk] * fb : qnan;
+            ra[q] = (va_ok && kk < dim) ? (LEFT ? pa[kk] * fa : pa[kk]) : qnan;
+            rb[q] = (vb_ok && kk < dim) ? (LEFT ? pb[kk] * fb : pb[kk]) : qnan;
         }
     };
     auto stage = [&]() {
@@ -566,7 +570,7 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     // Where that subtraction cancels (Caa <= Saa / 16: a subset mean far from
     // c, a constant subset, fewer than two samples) or a sum is not finite
     // (Inf in the data), the tile runs the two passes below instead.
-    if (!args.left) {
+    if constexpr (!LEFT) {
         __shared__ float lds1[3][2][WBK][WLD];   // a', a'^2, presence; [side]
         gload(0);
         float csum[2] = {0.0f, 0.0f}, ccnt[2] = {0.0f, 0.0f};
@@ -970,8 +974,8 @@ struct MomentsArgs {
     int64_t id_offset, ids_this;
 };
 
-// A 128 x 64 tile of pairs; the operand blocks stream through a three-stage
-// LDS ring (direct loads; wave w < 7 moves term w of the six blocks).  A wave
+// A 64 x 64 tile of pairs; the operand blocks stream through a two-stage LDS
+// ring (direct loads).  A wave
 // holds 32 x 32 pairs: n = m m', Sa = a m', Sb = m b', Saa = q m', Sbb = m q'
 // and Sab = a b' take 1, 3, 3, 3, 3 and 6 products of 16 samples, all with
 // FP32 accumulation.  The second moments are two-level sums: `fold` chunks in
@@ -1426,12 +1430,18 @@ hipError_t launch_pmcc(int use, int precision, const float *a, int64_t na, int64
         for (int64_t off = 0; off < total; off += max_tiles) {
             args.tile_offset = off;
             args.tiles_this = (total - off) < max_tiles ? (total - off) : max_tiles;
-            if (same)
-                hipLaunchKernelGGL(pmcc_pairwise_kernel<true>, dim3((unsigned)args.tiles_this),
-                                   dim3(WTHREADS), 0, stream, args);
-            else
-                hipLaunchKernelGGL(pmcc_pairwise_kernel<false>, dim3((unsigned)args.tiles_this),
-                                   dim3(WTHREADS), 0, stream, args);
+            const dim3 grid((unsigned)args.tiles_this), block(WTHREADS);
+            if (args.left) {
+                if (same)
+                    hipLaunchKernelGGL((pmcc_pairwise_kernel<true, true>), grid, block, 0, stream, args);
+                else
+                    hipLaunchKernelGGL((pmcc_pairwise_kernel<false, true>), grid, block, 0, stream, args);
+            } else {
+                if (same)
+                    hipLaunchKernelGGL((pmcc_pairwise_kernel<true, false>), grid, block, 0, stream, args);
+                else
+                    hipLaunchKernelGGL((pmcc_pairwise_kernel<false, false>), grid, block, 0, stream, args);
+            }
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
