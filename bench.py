@@ -193,6 +193,12 @@ def _valu_roof(flops, ms):
             "frac": round(tf / 157.3, 4)}
 
 
+def _mfma_roof(flops, ms, peak):
+    tf = flops / (ms * 1e-3) / 1e12
+    return {"bound": "mfma", "achieved": round(tf, 2), "peak": peak, "unit": "TFLOP/s",
+            "frac": round(tf / peak, 4)}
+
+
 def _roof(flops, hbm_bytes, ms):
     # the binding resource: FP32 VALU at 157.3 TFLOP/s or HBM at 8 TB/s,
     # whichever takes longer for this work
@@ -300,7 +306,8 @@ def path_backward(torch, gt, wl, steps, warmup, out):
     ms_bw = _timed(lambda: gt.dist_backward(x, grad, "euclidean"), steps, warmup, torch)
     # algorithmic work per pair: about 6k flop (the difference, its square and
     # sum to recompute d, and the weighted difference added to both rows' dX);
-    # D is recomputed, not read.  The kernel's two-owner sweep does more.
+    # D is recomputed, not read.  The kernel does more (split products on the
+    # matrix cores, each pair for both owners).
     out["backward_euclidean_16384x128"] = {
         "ms": round(ms_bw, 4), "algorithmic_flops": 6.0 * k * pairs,
         "roofline": _valu_roof(6.0 * pairs * k, ms_bw)}
@@ -330,13 +337,13 @@ def path_small(torch, gt, wl, steps, warmup, out):
 
 def path_hclust(torch, gt, wl, steps, warmup, out):
     # clustering stage (gpuDistClust's second half) on the 8192 x 256 N(0,1)
-    # euclidean matrix: n - 1 sequential merge rounds on one workgroup, so the
-    # figure of merit is time per round.  The reference's loop rescans the
+    # euclidean matrix: n - 1 sequential merge rounds, shared by the workgroups
+    # of one XCD, so the figure of merit is time per round.  The reference's loop rescans the
     # lower triangle every round: n^3/6 FP32 reads, whose HBM time alone is
     # given as the reference's floor.
     # Our kernel reads O(n^2) in all, so it is bound by the latency of its
-    # n - 1 dependent rounds (argmin, update, repair, rescan, each ending in a
-    # barrier), not by bandwidth.  The floor per round is measured with the
+    # n - 1 dependent rounds (exchange of candidates, update, repair, rescan),
+    # not by bandwidth.  The floor per round is measured with the
     # same kernel at n = 64, where every phase has almost nothing to do.
     def run_rounds(d, m):
         torch.cuda.synchronize()
@@ -372,9 +379,9 @@ def path_pmcc(torch, gt, wl, steps, warmup, out):
     # self case (half the tiles computed, every value stored twice).  Each
     # pair gets pairs, corr and t-score: 12 B of output, which bounds the
     # "everything" path; its algorithmic work is one 1024-long dot product
-    # per unique pair.  pairwise.complete.obs (10% NaN) is per-pair VALU
-    # work: one pass of 6 fused products per sample (count, two shifted sums,
-    # three second moments), 12 flops.
+    # per unique pair.  pairwise.complete.obs (10% NaN) forms six sums of
+    # products per pair and sample (count, two shifted sums, three second
+    # moments), 12 flops, on the matrix cores from split operands (19 products).
     nv, size = 8192, 1024
     a = torch.from_numpy(wl.normal(nv, size, seed=6)).cuda()
     outs = tuple(torch.empty((nv, nv), dtype=torch.float32, device="cuda") for _ in range(3))
@@ -394,29 +401,24 @@ def path_pmcc(torch, gt, wl, steps, warmup, out):
                 steps, warmup, torch)
     cor["pairwise_complete_fp32"] = {
         "ms": round(ms, 4), "pairs_per_s": round(nv * nv / (ms * 1e-3), 1),
-        "roofline": _valu_roof(12.0 * size * nv * (nv + 1) / 2, ms)}
+        "roofline": _mfma_roof(12.0 * size * nv * (nv + 1) / 2, ms, 2500.0)}
     out["pmcc_self_8192x1024"] = cor
 
 
 def path_kendall(torch, gt, wl, steps, warmup, out):
     # gpuCor(x, method = "kendall"): 1024 variables x 2048 samples N(0,1),
     # self case.  Algorithmic work of the count for variables without ties or
-    # NaN (this workload): per unique pair of variables and 32 sample pairs,
-    # one XOR and one popcount-accumulate (32-bit integer VALU lane
-    # operations; 256 CUs x 64 lanes x 2.4 GHz = 39.3 T/s).
+    # NaN (this workload): per unique pair of variables one product of signs
+    # per sample pair, on the FP4 matrix cores (10 PFLOP/s dense).
     nv, size = 1024, 2048
     a = torch.from_numpy(wl.normal(nv, size, seed=8)).cuda()
     tau = torch.empty((nv, nv), dtype=torch.float64, device="cuda")
     ms = _timed(lambda: gt.kendall(a, out=tau), steps, warmup, torch)
-    q, r = divmod(size - 1, 32)
-    words = 16 * q * (q + 1) + r * (q + 1)
-    ops = 2.0 * words * nv * (nv + 1) / 2
-    tops = ops / (ms * 1e-3) / 1e12
+    products = nv * (nv + 1) / 2 * size * (size - 1) / 2
     out["kendall_self_1024x2048"] = {
         "ms": round(ms, 4), "pairs_per_s": round(nv * nv / (ms * 1e-3), 1),
-        "sample_pairs_per_s": round(nv * (nv + 1) / 2 * size * (size - 1) / 2 / (ms * 1e-3), 1),
-        "roofline": {"bound": "valu", "achieved": round(tops, 2), "peak": 39.3,
-                     "unit": "T int32 lane-ops/s", "frac": round(tops / 39.3, 4)}}
+        "sample_pairs_per_s": round(products / (ms * 1e-3), 1),
+        "roofline": _mfma_roof(2.0 * products, ms, 10000.0)}
 
 
 PATHS = {"methods": path_methods, "binary_large": path_binary_large, "uniform": path_uniform,

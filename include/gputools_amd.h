@@ -351,7 +351,9 @@ int gt_dist_batched(const float *x, const int64_t *x_offsets, const int64_t *siz
  * use GT_USE_EVERYTHING: precision FP32 (VALU), BF16X3 or FP16X3 (MFMA on
  * standardised variables); GT_USE_PAIRWISE: FP32 only.  The workspace
  * (gt_pmcc_workspace_size, same != 0 for the self case) holds the
- * standardised variables; none is needed for GT_USE_PAIRWISE. */
+ * standardised variables.  For GT_USE_PAIRWISE it is optional: the matrix
+ * cores' operands where that form is faster (0 bytes elsewhere); without it
+ * the VALU does the work. */
 int gt_pmcc_workspace_size(int use, int precision, int64_t na, int64_t nb, int64_t dim, int same,
                            size_t *bytes);
 int gt_pmcc(int use, int precision, const float *a, int64_t na, int64_t lda, const float *b,
@@ -370,8 +372,8 @@ int gt_ttest(const float *pairs, const float *corr, int64_t n, float *ts, void *
  * are counted exactly in integers; the quotient follows the reference's FP32
  * / FP64 steps (inst/cuda/kendall.cu:40-45).  b == NULL (or b == a with the
  * same shape) is the self case.  The workspace (gt_kendall_workspace_size)
- * holds three bit planes of n(n-1)/2 bits per variable, per-variable flags,
- * a small per-chunk table of the bits past row ends, and the counts. */
+ * holds bit planes of the sample pairs (a segment of them at a time, within
+ * three bits per pair and variable or 64 MiB), flags, and the counts. */
 int gt_kendall_workspace_size(int64_t na, int64_t nb, int64_t n, int same, size_t *bytes);
 int gt_kendall(const float *a, int64_t na, int64_t lda, const float *b, int64_t nb, int64_t ldb,
                int64_t n, double *tau, int64_t ldt, void *workspace, size_t workspace_bytes,
