@@ -13,8 +13,8 @@
 //   - hclust_init_kernel (many workgroups, one wave per row) puts +inf on the
 //     diagonal, sets every count to 1 and computes each row's minimum over
 //     columns 0..r-1 (value and column);
-//   - hclust_group_kernel (32 workgroups on one XCD, see there) runs the n - 1
-//     rounds from 8 to 32768 points;
+//   - hclust_group_kernel (32 workgroups on one XCD, or one up to 256 points, see
+//     there) runs the n - 1 rounds up to 32768 points;
 //   - hclust_merge_kernel (one persistent workgroup of 1024 threads) runs them
 //     elsewhere, and where the 32 found no room together.  Per round: the argmin over the cached row minima, the
 //     update of row and column sup (row and column sub become +inf), then the
@@ -43,6 +43,8 @@
 #include "gt_common.h"
 #include "gt_internal.h"
 
+#include <type_traits>
+
 namespace gt {
 namespace {
 
@@ -68,18 +70,19 @@ struct HclustArgs {
     float *height;
     bool vec4;         // rows start 16 B aligned
     struct HcGroup *group;   // hclust_group_kernel's meeting point; null without it
+    int lgp;                 // log2 of its workgroups
 };
 
 // Meeting point of the workgroups of hclust_group_kernel (cleared by the init
 // kernel).
-constexpr int GP = 32;               // workgroups, all on one XCD
+constexpr int GP_MAX = 32;           // workgroups, all on one XCD
 constexpr int GMAX_N = 32768;        // a tie key fits 15 bits
 constexpr unsigned G_ABORT = 0xffffu;
 struct HcGroup {
     unsigned arrive[16];             // workgroups seen, per XCD
     unsigned chosen;                 // 0 none yet, 1 + XCD, or G_ABORT
     unsigned pad[47];
-    unsigned long long rec[2][GP][2];   // [round parity][workgroup]: what it found
+    unsigned long long rec[2][GP_MAX][2];   // [round parity][workgroup]: what it found
 };
 static_assert(sizeof(HcGroup) + 255 <= HC_GROUP_BYTES, "workspace share, any alignment");
 
@@ -619,12 +622,12 @@ __global__ __launch_bounds__(HTHREADS) void hclust_merge_kernel(HclustArgs a)
 // The merge rounds on the 32 CUs of one XCD
 // ---------------------------------------------------------------------------
 // One workgroup's round is a chain of memory round trips with LDS work on all
-// rows' state between them, and one CU issues every scattered store.  Here GP
+// rows' state between them, and one CU issues every scattered store.  Here 32
 // workgroups share the rounds.  Rows are owned in blocks of 32, round robin; a
 // workgroup keeps the cached minima of its rows in LDS, and every workgroup
 // keeps all sizes (each sees every merge).  Per round:
 //   - wave 0 sends out the workgroup's best row and its part of the minimum of
-//     the row rewritten last round as two tagged 64-bit words, reads all GP
+//     the row rewritten last round as two tagged 64-bit words, reads all
 //     records and comes to the same pair as the others (the order on (value,
 //     tie key) is total, so the grouping does not matter), and lists its rows
 //     whose cached minimum is at column sub or sup;
@@ -635,19 +638,19 @@ __global__ __launch_bounds__(HTHREADS) void hclust_merge_kernel(HclustArgs a)
 //     sup joins afterwards.
 // The workgroups must run on one XCD: they exchange data through its L2, where
 // stores complete and which loads that pass the L1 by read.  GLAUNCH are
-// launched, the first XCD that has GP of them is chosen and the others leave.
-// If none has GP within 50 ms (a busy device), nobody starts and
+// launched, the first XCD that has 32 of them is chosen and the others leave.
+// If none has 32 within 50 ms (a busy device), nobody starts and
 // hclust_merge_kernel, launched behind, does the work; otherwise that leaves
 // at once.
 // Bound: the round's latency, most of it dependent instructions of single
-// waves.  Average linkage, n = 8192 (independent normal points): 4.2 us a
+// waves.  Average linkage, n = 8192 (independent normal points): 3.9 us a
 // round, of which 0.2 gather, 0.5 exchange, 0.4 choice of the pair, 0.35 list,
-// 1.0 rewrite and 1.3 beside it where some workgroup scans a row (0.8 of the
-// rounds have one).  One workgroup took 21.6 us; whole runs 177 -> 34 ms, at
-// 1024 points 8.9 -> 3.2 ms, at 32768 4680 -> 299 ms.
-// From 8 points (51 us against 66; at 3 points 38 against 36, the larger launch)
-// to what 15-bit tie keys and the LDS hold (9.1 against 143 us a round there).
-constexpr int GROUP_MIN_N = 8;
+// 1.0 rewrite and 1.1 beside it where some workgroup scans a row (0.84 of the
+// rounds have one).  hclust_merge_kernel took 21.6 us; whole runs 177 -> 32 ms,
+// at 1000 points 8.7 -> 3.0 ms, at 32768 4680 -> 299 ms.
+// Up to here one workgroup does this kernel's rounds and meets nobody (64 points:
+// 3.3 us a round against 3.6 with the meetings, 256: 3.1 and 3.2, 512: 3.9 and 3.1).
+constexpr int GALONE_N = 256;
 constexpr int GTHREADS = 1024, GWAVES = GTHREADS / 64;
 constexpr int GLAUNCH = 320;
 constexpr unsigned long long GJOIN_TICKS = 5000000ull;      // 50 ms of the 100 MHz clock
@@ -761,7 +764,7 @@ __device__ __forceinline__ void wave_min2(float v, float w, float &mv, float &mw
 }
 
 // rows per workgroup, a multiple of 32
-__host__ __device__ __forceinline__ int group_rows(int n) { return ((n + 31) / 32 + GP - 1) / GP * 32; }
+__host__ __device__ __forceinline__ int group_rows(int n, int lgp) { return (((n + 31) / 32 - 1 >> lgp) + 1) * 32; }
 
 template <int METHOD>
 __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
@@ -777,10 +780,12 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     HcGroup *const grp = a.group;
-    if (tid == 0) {
+    const int lgp = a.lgp, gp = 1 << lgp;
+    if (tid == 0) s_g = 0;   // a workgroup alone meets nobody
+    if (tid == 0 && lgp > 0) {
         const unsigned xcc = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & 15u;   // HW_REG_XCC_ID
         const unsigned t = atomicAdd(&grp->arrive[xcc], 1u);
-        if (t == GP - 1) atomicCAS(&grp->chosen, 0u, xcc + 1u);
+        if (t == (unsigned)gp - 1) atomicCAS(&grp->chosen, 0u, xcc + 1u);
         const unsigned long long began = wall_clock64();
         unsigned c = 0u;
         while (c == 0u) {
@@ -789,13 +794,13 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
             if (late) break;
             __builtin_amdgcn_s_sleep(4);
         }
-        s_g = (c == xcc + 1u && t < GP) ? (int)t : -1;
+        s_g = (c == xcc + 1u && t < (unsigned)gp) ? (int)t : -1;
     }
     __syncthreads();
     const int g = s_g;
     if (g < 0) return;
 
-    const int n = a.n, rows = group_rows(n), words = (n + 31) / 32;
+    const int n = a.n, rows = group_rows(n, lgp), words = (n + 31) / 32;
     const int64_t ldd = a.ldd;
     float *const minv = hs_dyn;                                   // own rows: cached minimum,
     unsigned *const mink = reinterpret_cast<unsigned *>(minv + rows);   // its column's key,
@@ -805,9 +810,9 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
     unsigned *const scank = reinterpret_cast<unsigned *>(minv + 5 * rows);
     unsigned *const live = reinterpret_cast<unsigned *>(minv + 6 * rows);   // bit per cluster, sup's off
     float *const cnt = reinterpret_cast<float *>(live + words);   // sizes of all clusters
-    auto row_of = [&](int l) { return ((l >> 5) * GP + g) * 32 + (l & 31); };
-    auto mine = [&](int r) { return ((r >> 5) & (GP - 1)) == g; };
-    auto local = [&](int r) { return (r >> 5) / GP * 32 + (r & 31); };
+    auto row_of = [&](int l) { return (((l >> 5) << lgp) + g) * 32 + (l & 31); };
+    auto mine = [&](int r) { return ((r >> 5) & (gp - 1)) == g; };
+    auto local = [&](int r) { return (r >> (5 + lgp)) * 32 + (r & 31); };
     for (int c = tid; c < n; c += GTHREADS) cnt[c] = 1.0f;
     for (int w = tid; w < words; w += GTHREADS)
         live[w] = n - w * 32 >= 32 ? ~0u : (1u << (n - w * 32)) - 1;
@@ -866,7 +871,7 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
             }
             if (last >= 0 && lane == 0) atomicOr(&live[last >> 5], 1u << (last & 31));
             // (the last round's stores are complete, so the record may go out)
-            unsigned long long *const rec = grp->rec[iter & 1][0];
+            unsigned long long w0, w1;   // best row; part of row `last`
             {
                 float mb, mp;
                 wave_min2(bv, pv, mb, mp);
@@ -876,22 +881,22 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
                 const unsigned q = (unsigned)__builtin_amdgcn_readlane((int)pk, wp & 63) & 0x7fffu;
                 const float v = wb < 0 ? INFINITY : lane_of(bv, wb & 63);
                 const float qv = wp < 0 ? INFINITY : lane_of(pv, wp & 63);
-                if (lane < 2) {
-                    const unsigned hi = __float_as_uint(lane == 0 ? v : qv);
-                    const unsigned lo = lane == 0 ? (k << 17 | c << 2 | tag) : (q << 2 | tag);
-                    store_shared(rec + g * 2 + lane, ((unsigned long long)hi << 32) | lo);
-                }
+                w0 = ((unsigned long long)__float_as_uint(v) << 32) | (k << 17 | c << 2 | tag);
+                w1 = ((unsigned long long)__float_as_uint(qv) << 32) | (q << 2 | tag);
             }
             // ---- all records ---------------------------------------------------
-            unsigned long long w0 = 0, w1 = 0;
             bool failed = false;
-            for (unsigned spin = 0;; ++spin) {
-                w0 = load_shared(rec + (lane & (GP - 1)) * 2);
-                w1 = load_shared(rec + (lane & (GP - 1)) * 2 + 1);
-                if (__builtin_amdgcn_ballot_w64((w0 & 3u) != tag || (w1 & 3u) != tag) == 0) break;
-                if (spin == 5000000u) {
-                    failed = true;   // a partner is gone: about a second
-                    break;
+            if (lgp > 0) {
+                unsigned long long *const rec = grp->rec[iter & 1][0];
+                if (lane < 2) store_shared(rec + g * 2 + lane, lane == 0 ? w0 : w1);
+                for (unsigned spin = 0;; ++spin) {
+                    w0 = load_shared(rec + (lane & (gp - 1)) * 2);
+                    w1 = load_shared(rec + (lane & (gp - 1)) * 2 + 1);
+                    if (__builtin_amdgcn_ballot_w64((w0 & 3u) != tag || (w1 & 3u) != tag) == 0) break;
+                    if (spin == 5000000u) {
+                        failed = true;   // a partner is gone: about a second
+                        break;
+                    }
                 }
             }
             asm volatile("" ::: "memory");
@@ -903,8 +908,8 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
                 }
                 if (lane == 0) s_nres = -1;
             } else {
-                const float v = lane < GP ? __uint_as_float((unsigned)(w0 >> 32)) : INFINITY;
-                const float lv = lane < GP ? __uint_as_float((unsigned)(w1 >> 32)) : INFINITY;
+                const float v = lane < gp ? __uint_as_float((unsigned)(w0 >> 32)) : INFINITY;
+                const float lv = lane < gp ? __uint_as_float((unsigned)(w1 >> 32)) : INFINITY;
                 const unsigned k = (unsigned)w0 >> 17, kc = ((unsigned)w0 >> 2) & 0x7fffu;
                 const unsigned lk = ((unsigned)w1 >> 2) & 0x7fffu;
                 float mv, ml;
@@ -1067,32 +1072,55 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
             for (int cb = c0; cb < c1; cb += 1024) {
                 const int cc = cb + lane * 4;
                 f32x4 x[4];
-                load_four(row, min(cc, c1 - 4) * 4, min(cc + 256, c1 - 4) * 4, min(cc + 512, c1 - 4) * 4,
-                          min(cc + 768, c1 - 4) * 4, x);
-                float best = INFINITY;
+                float best;
+                int first_at;
+                // the lane's first minimum over `units` of its four 16 B units, in
+                // key order: columns 0, 2, 1, 3 of four, each over the units (four
+                // short chains, then two)
+                auto scan = [&](auto units) {
+                    constexpr int NU = decltype(units)::value;
+                    unsigned open[NU];   // bits of the live columns
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (cb + u * 256 >= c1) {
-                        x[u] = f32x4{INFINITY, INFINITY, INFINITY, INFINITY};
-                        continue;
+                    for (int u = 0; u < NU; ++u) {
+                        const int cu = cc + u * 256;
+                        const unsigned w = live[min(cu >> 5, words - 1)];
+                        open[u] = cu < c1 ? w >> (cu & 31) : 0u;
                     }
-                    const int cu = cc + u * 256;
-                    const unsigned w = cu < c1 ? live[cu >> 5] >> (cu & 31) : 0u;
+                    load_four(row, min(cc, c1 - 4) * 4, min(cc + 256, c1 - 4) * 4, min(cc + 512, c1 - 4) * 4,
+                              min(cc + 768, c1 - 4) * 4, x);
+                    float bv[4];
+                    int bo[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        x[u][e] = (w >> e) & 1u ? x[u][e] : INFINITY;
-                        best = x[u][e] < best ? x[u][e] : best;   // (passes NaN over)
+                    for (int c = 0; c < 4; ++c) {
+                        const int e = (c >> 1) | ((c << 1) & 2);
+                        bv[c] = INFINITY;
+                        bo[c] = -1;
+#pragma unroll
+                        for (int u = 0; u < NU; ++u) {
+                            const unsigned on = (unsigned)((int)(open[u] << (31 - e)) >> 31);   // all bits or none
+                            const float y = __uint_as_float((__float_as_uint(x[u][e]) & on) | (0x7f800000u & ~on));
+                            const bool t = y < bv[c];   // (passes NaN over)
+                            bv[c] = t ? y : bv[c];
+                            bo[c] = t ? c * 4 + u : bo[c];
+                        }
                     }
-                }
+#pragma unroll
+                    for (int c = 0; c < 4; c += 2) {
+                        const bool t = bv[c + 1] < bv[c];
+                        bv[c] = t ? bv[c + 1] : bv[c];
+                        bo[c] = t ? bo[c + 1] : bo[c];
+                    }
+                    const bool hi = bv[2] < bv[0];
+                    best = hi ? bv[2] : bv[0];
+                    first_at = hi ? bo[2] : bo[0];
+                };
+                if (c1 - cb <= 256)
+                    scan(std::integral_constant<int, 1>());
+                else
+                    scan(std::integral_constant<int, 4>());
                 const float m = wave_min(best);
                 if (m < INFINITY && m <= v) {
-                    // this lane's first in key order: columns 0, 2, 1, 3 of four
-                    int at = -1;
-#pragma unroll
-                    for (int o = 15; o >= 0; --o) {
-                        const int e = (o >> 3) | ((o >> 1) & 2), u = o & 3;
-                        at = x[u][e] == m ? o : at;
-                    }
+                    const int at = best == m ? first_at : -1;
                     const unsigned bk =
                         at < 0 ? NO_KEY : key_of(cc) + ((unsigned)(at >> 2) << 13) + ((unsigned)(at & 3) << 3);
                     const int w = winner(at < 0 ? INFINITY : m, bk, m);
@@ -1167,7 +1195,7 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
     }
 }
 
-unsigned group_lds(int n) { return (unsigned)((n + 31) / 32 * 4 + 4 * n + 24 * group_rows(n)); }
+unsigned group_lds(int n, int lgp) { return (unsigned)((n + 31) / 32 * 4 + 4 * n + 24 * group_rows(n, lgp)); }
 
 }  // namespace
 
@@ -1191,7 +1219,10 @@ hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lam
     a.height = height;
     a.vec4 = (ldd % 4 == 0) && ((reinterpret_cast<uintptr_t>(d) & 15) == 0);
     a.group = nullptr;
-    if (state == HC_STATE_AUTO && group && n >= GROUP_MIN_N && n <= GMAX_N)
+    a.lgp = n <= GALONE_N ? 0 : 5;
+    // up to what 15-bit tie keys and the LDS hold (32768 points: 9.1 us a round,
+    // one workgroup of hclust_merge_kernel 143)
+    if (state == HC_STATE_AUTO && group && n <= GMAX_N)
         a.group = reinterpret_cast<HcGroup *>((reinterpret_cast<uintptr_t>(group) + 255) & ~(uintptr_t)255);
     int64_t blocks = (n + 3) / 4;
     if (blocks > 65536) blocks = 65536;
@@ -1208,13 +1239,13 @@ hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lam
 #define GT_HC_CASE(m)                                                                          \
     case m:                                                                                    \
         if (a.group) {                                                                         \
-            const unsigned gl = group_lds((int)n);                                             \
+            const unsigned gl = group_lds((int)n, a.lgp);                                      \
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(hclust_group_kernel<m>),    \
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)gl);      \
             if (e != hipSuccess) return e;                                                     \
-            hipLaunchKernelGGL(hclust_group_kernel<m>, dim3(GLAUNCH), dim3(GTHREADS), gl,      \
-                               stream, a);                                                     \
-            if ((e = hipGetLastError()) != hipSuccess) return e;                               \
+            hipLaunchKernelGGL(hclust_group_kernel<m>, dim3(a.lgp ? GLAUNCH : 1),              \
+                               dim3(GTHREADS), gl, stream, a);                                 \
+            if ((e = hipGetLastError()) != hipSuccess || a.lgp == 0) return e;                 \
         }                                                                                      \
         if (lds) {                                                                             \
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(hclust_merge_kernel<m, true>), \

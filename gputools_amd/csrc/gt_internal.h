@@ -113,8 +113,8 @@ enum HcMethod {
 // Clustering on a full n x n device matrix d (row stride ldd, destroyed).
 // count, minv, minc: n entries of workspace each; group: HC_GROUP_BYTES or null;
 // sub, sup, height: n - 1.
-// state: HC_STATE_AUTO shares the rounds among the workgroups of one XCD from
-// 8 to 32768 points if group is given; elsewhere one workgroup keeps the
+// state: HC_STATE_AUTO shares the rounds among the workgroups of one XCD up to
+// 32768 points if group is given; elsewhere one workgroup keeps the
 // per-row state in LDS up to HC_LDS_MAX_N points and in global memory above.
 // HC_STATE_LDS / HC_STATE_GLOBAL force one workgroup and a placement (LDS only
 // up to HC_LDS_MAX_N).

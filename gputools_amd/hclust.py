@@ -155,7 +155,7 @@ def hclust(d, method="complete", lam: float = 0.5, beta: float = 0.5, stream=Non
     tensors ``sub``, ``sup`` and float32 ``height`` of length n - 1: at step s
     the clusters represented by sub[s] < sup[s] merge at height[s].
     ``state`` places the kernel's per-row state: "auto" (shared among
-    workgroups from 8 to 32768 points; else one workgroup, in LDS up to 9216
+    workgroups up to 32768 points; else one workgroup, in LDS up to 9216
     points, in global memory above), "lds" or "global" (one workgroup); every
     placement gives the same result."""
     import torch

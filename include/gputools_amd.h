@@ -275,7 +275,7 @@ int gt_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float 
 
 /* Where the clustering kernel keeps its per-row state (counts, cached row
  * minima, the rewritten row): GT_HC_STATE_AUTO as gt_hclust does (shared among
- * workgroups from 8 to 32768 points; else one workgroup, in LDS up to
+ * workgroups up to 32768 points; else one workgroup, in LDS up to
  * GT_HC_LDS_MAX_N points, in global memory above), or one workgroup and its
  * placement forced (LDS only up to GT_HC_LDS_MAX_N).  All run the same merge
  * rounds and give the same merges and heights bit for bit. */

@@ -244,3 +244,14 @@ def test_hclust_workgroup_edges(n, data):
             res.append([t.cpu().numpy() for t in gt.hclust(buf[:, :n], method, state=state)])
         for a, b in zip(*res):
             np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [2, 255, 256, 257, 288, 290])
+def test_hclust_one_workgroup_limit(n):
+    """One workgroup of the several-workgroup form, up to 256 points, and the
+    first sizes above, against the oracle, on distances with many ties."""
+    rng = np.random.default_rng(5000 + n)
+    d = full_matrix(rng.integers(0, 3, size=(n, 4)))
+    for method in ("single", "average", "ward"):
+        print("case hclust one workgroup n=%d %s" % (n, method), flush=True)
+        assert_same(d, method)
