@@ -75,6 +75,7 @@ struct PlanesArgs {
     int64_t nvb, fstride, ngroups;
     int64_t tile_begin, ntiles;   // this segment's tiles of sample pairs
     int64_t runs;
+    int64_t run;         // tiles per workgroup
 };
 
 constexpr int KRUN = 4;      // tiles per workgroup
@@ -91,7 +92,8 @@ typedef const __attribute__((address_space(4))) float uniform_float_t;
 // samples from 0.52 ms (a ballot per 64 pairs, moved between lanes) to
 // 0.23 ms.  Bound: VALU issue (1.2e8 wave instructions, 108 per word of 64
 // lanes: 80 in the column loop, the rest masks, tests and the LDS transpose).
-// A word with a zero difference or a non-finite value is redone with the
+// A word with a zero difference or a non-finite value is redone (from the columns
+// in the lanes: few variables with ties took 76 us of scalar loads, 15 so) with the
 // three comparisons; if it holds a tie (or a NaN may be about), its group is
 // flagged and the N and E words of the whole group are stored.
 __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
@@ -105,8 +107,8 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t n = args.n, jwn = column_words(n);
     const int64_t vb = blockIdx.x / args.runs, run = blockIdx.x % args.runs;
-    const int64_t tb = run * KRUN;
-    const int nt = (int)(args.ntiles - tb < KRUN ? args.ntiles - tb : KRUN);
+    const int64_t tb = run * args.run;
+    const int nt = (int)(args.ntiles - tb < args.run ? args.ntiles - tb : args.run);
     const int64_t t0 = args.tile_begin + tb;
     // row block of tile t0: the last rb with tiles_before(rb) <= t0
     int64_t rb;
@@ -133,13 +135,13 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
             xi[vv] = x[v * args.ldx + i] + 0.0f;
         }
     };
-    // the three comparisons of 32 columns, column u in bit u; the columns from
-    // cols on repeat the last one
-    auto exact = [&](float a, uniform_float_t *xj, int cols, uint32_t &gt, uint32_t &lt, uint32_t &eq) {
+    // the three comparisons of 32 columns, column u in bit u, which lane u holds
+    // (scalar loads here would be waited for one after the other)
+    auto exact = [&](float a, float xl, uint32_t &gt, uint32_t &lt, uint32_t &eq) {
         gt = lt = eq = 0u;
 #pragma unroll 8
         for (int u = 31; u >= 0; --u) {
-            const float b = xj[u < cols ? u : cols - 1];
+            const float b = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(xl), u));
             gt = (gt << 1) | (b > a ? 1u : 0u);
             lt = (lt << 1) | (b < a ? 1u : 0u);
             eq = (eq << 1) | (b == a ? 1u : 0u);
@@ -156,7 +158,8 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
         const int lo = (int)(rb * 64 - j0) + lane + 1;   // -n .. 64
         uint32_t valid = cols >= 32 ? 0xffffffffu : (1u << cols) - 1u;
         if (lo > 0) valid &= lo >= 32 ? 0u : 0xffffffffu << lo;
-        unsigned sp = 0;
+        unsigned sp = 0, compared = 0;   // compared: the variables with ltw and eqw
+        uint32_t ltw[8], eqw[8];         // x_j < x_i and x_j == x_i
         uint32_t *const pb = buf[k & 1] + slot + wave * 8 * 4;
 #pragma unroll
         for (int vv = 0; vv < 8; ++vv) {
@@ -173,13 +176,23 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
                     m = d < m ? d : m;
                 }
             } else {
-                m = 0u;
+                // the columns from cols on repeat the last one
+#pragma unroll
+                for (int u = 31; u >= 0; --u) {
+                    const uint32_t d = __float_as_uint(
+                        xi[vv] - __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(xl), u)));
+                    w = __builtin_amdgcn_alignbit(w, d, 31);
+                    m = d < m ? d : m;
+                }
             }
             const bool odd = !(fabsf(xi[vv]) < INFINITY) || !(fabsf(xl) < INFINITY);
             const unsigned long long oddw = __builtin_amdgcn_ballot_w64(odd);
             if (__builtin_amdgcn_ballot_w64(m == 0u) | oddw) {
                 uint32_t lt, eq;
-                exact(xi[vv], xj, cols, w, lt, eq);
+                exact(xi[vv], xl, w, lt, eq);
+                ltw[vv] = lt;
+                eqw[vv] = eq;
+                compared |= 1u << vv;
                 const unsigned long long tied = __builtin_amdgcn_ballot_w64((eq & valid) != 0u);
                 if (oddw) {
                     sp = 0xffu;
@@ -206,13 +219,15 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
         if (mask != 0u) {
             const int q = lane >> 3;
             uint32_t *const po = pt + q * KGWORDS + ((lane >> 2) & 1) * 128 + (lane & 3);
+#pragma unroll
             for (int vv = 0; vv < 8; ++vv) {
-                const int64_t v = v0 + vv < args.nvar ? v0 + vv : args.nvar - 1;
-                uint32_t gt, lt, eq;
-                exact(xi[vv], (uniform_float_t *)(x + v * args.ldx + j0), cols, gt, lt, eq);
+                // not compared: no tie and nothing odd, so N = ~P and E = 0
+                const bool c = (compared >> vv) & 1u;
+                const uint32_t lt = c ? (ltw[vv] & valid) | ~valid : ~pb[vv * 4];
+                const uint32_t eq = c ? eqw[vv] & valid : 0u;
                 if ((mask >> q) & 1u) {
-                    po[pstride + (wave * 8 + vv) * 4] = (lt & valid) | ~valid;
-                    po[2 * pstride + (wave * 8 + vv) * 4] = eq & valid;
+                    po[pstride + (wave * 8 + vv) * 4] = lt;
+                    po[2 * pstride + (wave * 8 + vv) * 4] = eq;
                 }
             }
         }
@@ -587,7 +602,10 @@ hipError_t launch_planes(const float *x, int64_t nvar, int64_t n, int64_t ldx, u
     args.ngroups = seg * KTG;
     args.tile_begin = begin;
     args.ntiles = tiles;
-    args.runs = (tiles + KRUN - 1) / KRUN;
+    // tiles per workgroup: as many as leave about four workgroups per CU
+    args.run = nvb * tiles / 1024;
+    args.run = args.run < 1 ? 1 : args.run > KRUN ? KRUN : args.run;
+    args.runs = (tiles + args.run - 1) / args.run;
     hipLaunchKernelGGL(kendall_planes_kernel, dim3((unsigned)(nvb * args.runs)), dim3(256), 0,
                        stream, args);
     return hipGetLastError();
@@ -652,7 +670,10 @@ hipError_t launch_kendall(const float *a, int64_t na, int64_t lda, const float *
             // step, so that one's barrier and LDS waits lie under the other's
             // products), so the number of workgroups is kept just under a
             // multiple of 512 (the multiple, up to 4, that leaves the fewest
-            // idle), with at least 16 groups each to fill and drain the ring.
+            // idle), with at least 16 groups each, as long as a whole tile's
+            // 32768 additions to the counts take; fewer, down to 2, where tiles
+            // hold fewer pairs (43 variables x 87 samples with ties: 54 us with 16
+            // groups, 14 with 2; 300 x 300 variables x 200: 53 and 77 us in all).
             int64_t splits = 1;
             double best = 0.0;
             for (int r = 1; r <= 4; ++r) {
@@ -664,7 +685,9 @@ hipError_t launch_kendall(const float *a, int64_t na, int64_t lda, const float *
                     splits = s;
                 }
             }
-            if (splits > args.ngroups / 16) splits = args.ngroups / 16;
+            int64_t least = na * nb / args.ntiles / 2048;
+            least = least < 2 ? 2 : least > 16 ? 16 : least;
+            if (splits > args.ngroups / least) splits = args.ngroups / least;
             if (splits < 1) splits = 1;
             args.split_g = (args.ngroups + splits - 1) / splits;
             if (args.split_g > KMAXGROUPS) args.split_g = KMAXGROUPS;
