@@ -239,3 +239,23 @@ def test_kendall_segments():
         torch.cuda.synchronize()
         want, _ = orc.kendall(a, a if bb is None else bb, nthreads=8)
         assert_same(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("na,nb,n", [(1, 1, 2), (5, 3, 33), (20, 20, 65), (43, 40, 87), (33, 31, 161), (217, 48, 129)])
+@pytest.mark.parametrize("kind", ["ordinal", "one_tie", "holes"])
+def test_kendall_few_variables_with_ties(na, nb, n, kind):
+    """Few variables (tiles with few pairs are split over more workgroups), with
+    last column tiles of 1 to 32 columns, words compared for some variables of a
+    block and not for others, and NaN and infinities: exact."""
+    rng = np.random.default_rng(na * 1000 + n)
+    a, b = (rng.standard_normal((m, n)).astype(np.float32) for m in (na, nb))
+    if kind == "ordinal":
+        a, b = (np.round(v * 2).astype(np.float32) for v in (a, b))
+    elif kind == "one_tie":
+        a[:: 3, 0] = a[:: 3, n - 1]
+    else:
+        a[rng.random(a.shape) < 0.05] = np.nan
+        b[rng.random(b.shape) < 0.05] = np.inf
+    want, _ = orc.kendall(a, b, nthreads=8)
+    got = gt.kendall(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda())
+    np.testing.assert_array_equal(got.cpu().numpy(), want)
