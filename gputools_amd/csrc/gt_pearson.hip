@@ -487,6 +487,9 @@ constexpr int WBM = 64;        // variables per tile side
 constexpr int WBK = 32;        // samples per LDS chunk
 constexpr int WTHREADS = 256;  // 16 x 16 lanes, 4 x 4 pairs each
 constexpr int WLD = WBM + 4;   // LDS row length (16-byte aligned rows)
+// second moments whose squares neither overflowed nor lost bits that count (a
+// sum of up to 2^24 of them)
+constexpr float MOMENT_MIN = 0x1p-100f, MOMENT_MAX = 0x1p120f;
 
 struct PairwiseArgs {
     const float *a;
@@ -500,7 +503,7 @@ struct PairwiseArgs {
     int64_t tile_offset, tiles_this;
     bool vec;   // ldo and the output pointers allow 16-byte stores
     // LEFT: the tiles to run (one byte per tile, 1 = left), and each variable's
-    // power of two
+    // power of two (pmcc_moments_prep_kernel)
     const uint8_t *left;
     const float *scale_a, *scale_b;
 };
@@ -511,7 +514,13 @@ struct PairwiseArgs {
 // correlation.cu:53-150).  Masked samples are selected away, never multiplied
 // by zero, so an Inf beside a missing value does not leak into the sums.
 // Each chunk's sums are accumulated separately and then added to the totals.
-// LEFT: only the tiles that pmcc_moments_kernel left, with two passes.
+// LEFT: only the tiles that pmcc_moments_kernel left, with two passes over the
+// values as they are.  A variable's power of two fits its largest value, which a
+// pair need not contain (one 1e30 beside ordinary values, missing in the
+// partner, would scale the pair's squares to nothing).  The passes run again
+// with it only where a variable of the tile is far from 1 in scale and a pair's
+// squares over- or underflowed; such pairs take the scaled moments if those are
+// in range.
 template <bool SYM, bool LEFT>
 __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs args)
 {
@@ -540,8 +549,8 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     const float *pa = args.a + (va_ok ? (x0 + sv) * args.lda : 0);
     const float *pb = args.b + (vb_ok ? (y0 + sv) * args.ldb : 0);
     const float qnan = __builtin_nanf("");
-    const float fa = LEFT && va_ok ? args.scale_a[x0 + sv] : 1.0f;
-    const float fb = LEFT && vb_ok ? args.scale_b[y0 + sv] : 1.0f;
+    float fa = 1.0f, fb = 1.0f;   // LEFT: factors of this lane's variables
+    unsigned settled = 0;         // LEFT: the pairs whose moments were in range without factors
     float ra[8], rb[8];
     auto gload = [&](int64_t kb) {
 #pragma unroll
@@ -675,7 +684,8 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
     }
 
     // ---- two passes (tiles the one pass does not settle) -------------------
-    {
+#pragma unroll 1
+    for (int attempt = 0; attempt < (LEFT ? 2 : 1); ++attempt) {
         float s1[4][4], s2[4][4];
     #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -803,6 +813,45 @@ __global__ __launch_bounds__(WTHREADS) void pmcc_pairwise_kernel(PairwiseArgs ar
                     qab[i][j] += pab[i][j];
                 }
         }
+        if constexpr (LEFT) {
+            // the first attempt's correlations, if there is a second
+            __shared__ float kept[16][WTHREADS];
+            unsigned in_range = 0;
+            bool again = false;
+    #pragma unroll
+            for (int i = 0; i < 4; ++i)
+    #pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool ok = qa[i][j] >= MOMENT_MIN && qa[i][j] <= MOMENT_MAX &&
+                                    qb[i][j] >= MOMENT_MIN && qb[i][j] <= MOMENT_MAX;   // (not for NaN)
+                    in_range |= ok ? 1u << (i * 4 + j) : 0u;
+                    const bool inside = x0 + ty * 4 + i < args.na && y0 + tx * 4 + j < args.nb;
+                    again = again || (inside && !ok);
+                }
+            if (attempt > 0) {
+    #pragma unroll
+                for (int i = 0; i < 4; ++i)
+    #pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (((in_range & ~settled) >> (i * 4 + j) & 1u) == 0) {
+                            qab[i][j] = kept[i * 4 + j][tid];
+                            qa[i][j] = qb[i][j] = 1.0f;
+                        }
+                break;
+            }
+            settled = in_range;
+            fa = va_ok ? args.scale_a[x0 + sv] : 1.0f;
+            fb = vb_ok ? args.scale_b[y0 + sv] : 1.0f;
+            // (with every largest value within 2^+-40, no sum overflows, and
+            // factors would not bring back what underflows)
+            const bool far = !(fa >= 0x1p-40f && fa <= 0x1p40f && fb >= 0x1p-40f && fb <= 0x1p40f);
+            if (__syncthreads_or(far) == 0 || __syncthreads_or(again) == 0) break;
+    #pragma unroll
+            for (int i = 0; i < 4; ++i)
+    #pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    kept[i * 4 + j][tid] = qab[i][j] / (sqrtf(qa[i][j]) * sqrtf(qb[i][j]));
+        }
     }
 
 finish:
@@ -872,9 +921,11 @@ finish:
 // past dim and rows past the last variable are zero in all seven.  The shift c
 // is the mean of the present values among the first 32 samples; the scale is
 // the power of two that brings max |v - c| to [1, 2), so that the terms stay
-// clear of the denormal range (the correlation does not depend on it; the
-// two passes over the tiles that are left use it as well).
+// clear of the denormal range.  A pair need not contain that largest value:
+// where its own squares are below MOMENTS_FLOOR on average, their terms run into
+// the denormal range, and the pair is left to the two passes.
 constexpr int QT = 7;
+constexpr float MOMENTS_FLOOR = 0x1p-90f;
 enum { Q_VALUE = 0, Q_SQUARE = 3, Q_MASK = 6 };
 constexpr int QTHREADS = 1024;
 
@@ -1106,7 +1157,8 @@ __global__ __launch_bounds__(QWAVES * 64, 2) void pmcc_moments_kernel(MomentsArg
         const float qb = sbb[r] - sb[r] * sb[r] / n;
         const float qab = sab[r] - sa[r] * sb[r] / n;
         const bool inside = x < na && y < nb && (!diag || x >= y);
-        ill = ill || (inside && !(qa > saa[r] * 0.0625f && qb > sbb[r] * 0.0625f));
+        ill = ill || (inside && !(qa > saa[r] * 0.0625f && qb > sbb[r] * 0.0625f &&
+                                  fminf(saa[r], sbb[r]) >= n * MOMENTS_FLOOR));
         rv[r] = qab / (sqrtf(qa) * sqrtf(qb));
         tv[r] = t_score<true>(n, rv[r]);
         if (inside) {

@@ -372,3 +372,40 @@ def test_everything_tile_edges(precision, na, dim, pad):
     z = x.double() - x.double().mean(1, keepdim=True)
     z /= z.norm(dim=1, keepdim=True)
     np.testing.assert_allclose(got[1].cpu().numpy(), (z @ z.t()).cpu().numpy(), rtol=0, atol=TOL)
+
+
+@pytest.mark.parametrize("at", [5, 150])
+@pytest.mark.parametrize("fill", [1e4, 1e10, 1e15, 3e18, 1e19, 1e20, 3e20, 1e22, 1e24, -1e30, 9.97e36])
+def test_pairwise_large_value_missing_in_partner(fill, at):
+    """One large value (a fill value, say) in a variable, at a sample that its
+    partners lack: it belongs to none of the pairs, whose correlations are those
+    of the other samples, with and without a workspace.  In the first 32 samples
+    it moves the shift, elsewhere only the scale.  The two-level FP32 sums of
+    200 terms are within 40 roundings (2.4e-6) of the oracle."""
+    rng = np.random.default_rng(at)
+    dim, na, nb = 200, 70, 40
+    a = np.ascontiguousarray(_data(rng, dim, na, shift=1.0).T, dtype=np.float32)
+    b = np.ascontiguousarray(_data(rng, dim, nb).T + a[:nb], dtype=np.float32)
+    a[rng.random(a.shape) < 0.05] = np.nan
+    b[:, at] = np.nan
+    a[3, at] = a[66, at] = fill
+    b[7, at + 9] = fill
+    a[:, at + 9] = np.nan
+    # self case: one variable holds the value, the others lack the sample
+    c = a.copy()
+    c[:, at] = np.nan
+    c[3, at] = fill
+    print("case pairwise large value %g at %d" % (fill, at), flush=True)
+    for x, y in ((a, b), (c, None)):
+        pairs, corr = orc.pmcc(x, x if y is None else y, "pairwise.complete.obs")
+        if y is None:
+            corr[3, 3] = 1.0
+        ad = torch.from_numpy(x).cuda()
+        bd = None if y is None else torch.from_numpy(y).cuda()
+        for workspace in (True, False):
+            need, (p, r, t) = _pmcc_capi(ad, bd, workspace)
+            assert need > 0
+            np.testing.assert_array_equal(p, pairs)
+            if y is None:
+                r[3, 3] = 1.0   # its squares may overflow
+            np.testing.assert_allclose(r, corr, rtol=0, atol=1e-5)
