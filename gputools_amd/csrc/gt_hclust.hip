@@ -769,7 +769,7 @@ __host__ __device__ __forceinline__ int group_rows(int n, int lgp) { return (((n
 template <int METHOD>
 __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
 {
-    extern __shared__ float hs_dyn[];
+    extern __shared__ __attribute__((aligned(16))) float hs_dyn[];   // (mink is read 16 B at a time)
     __shared__ int s_g, s_nres, s_rw, s_cw;
     __shared__ float s_val, s_np, s_nq;
     // per wave: its rows' best (value, row and column), its part of row sup's
