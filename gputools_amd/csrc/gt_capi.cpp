@@ -199,6 +199,16 @@ bool injected_alloc_failure()
     return n >= 1 && ++g_fi_seen == n;
 }
 
+// The same for the clustering workgroups' meeting: GT_FAIL_MEETING=join (they
+// never come together) or partner (one is given up at once).
+int injected_meeting_failure()
+{
+    const char *v = getenv("GT_FAIL_MEETING");
+    if (v == nullptr) return gt::HC_FAULT_NONE;
+    return strcmp(v, "join") == 0 ? gt::HC_FAULT_JOIN
+           : strcmp(v, "partner") == 0 ? gt::HC_FAULT_PARTNER : gt::HC_FAULT_NONE;
+}
+
 hipError_t device_malloc(void **p, size_t bytes)
 {
     if (injected_alloc_failure()) {
@@ -382,7 +392,8 @@ int run_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float
     const size_t part = round_up((size_t)n * 4, 256);
     GT_HIP(gt::launch_hclust(d, n, ldd, method, lambda, beta, reinterpret_cast<float *>(w),
                              reinterpret_cast<float *>(w + part), reinterpret_cast<int *>(w + 2 * part),
-                             ws_bytes >= hclust_ws_bytes(n) ? w + 3 * part : nullptr, sub, sup, height, state, stream));
+                             ws_bytes >= hclust_ws_bytes(n) ? w + 3 * part : nullptr, sub, sup, height, state,
+                             injected_meeting_failure(), stream));
     return GT_OK;
 }
 
@@ -407,6 +418,8 @@ int hclust_device_to_host(float *d, int64_t n, int64_t ldd, int method, float la
     GT_HIP(hipMemcpy(sub_h, dsub, len * 4, hipMemcpyDeviceToHost));
     GT_HIP(hipMemcpy(sup_h, dsup, len * 4, hipMemcpyDeviceToHost));
     GT_HIP(hipMemcpy(height_h, dh, len * 4, hipMemcpyDeviceToHost));
+    if (sub_h[len - 1] >= sup_h[len - 1])
+        return fail(GT_ERR_HIP, "clustering stopped early: a workgroup of its kernel was not seen for about a second");
     return GT_OK;
 }
 

@@ -71,6 +71,7 @@ struct HclustArgs {
     bool vec4;         // rows start 16 B aligned
     struct HcGroup *group;   // hclust_group_kernel's meeting point; null without it
     int lgp;                 // log2 of its workgroups
+    int fault;               // HcFault: a failure forced by a test
 };
 
 // Meeting point of the workgroups of hclust_group_kernel (cleared by the init
@@ -653,6 +654,9 @@ __global__ __launch_bounds__(HTHREADS) void hclust_merge_kernel(HclustArgs a)
 constexpr int GALONE_N = 256;
 constexpr int GTHREADS = 1024, GWAVES = GTHREADS / 64;
 constexpr int GLAUNCH = 320;
+// Polls of a partner's record before it is given up: about a second of running
+// (not of the clock, which goes on while a queue is swapped out).
+constexpr unsigned GPOLLS = 5000000u;
 constexpr unsigned long long GJOIN_TICKS = 5000000ull;      // 50 ms of the 100 MHz clock
 
 // End of a round: also this wave's stores are complete.
@@ -785,7 +789,7 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
     if (tid == 0 && lgp > 0) {
         const unsigned xcc = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & 15u;   // HW_REG_XCC_ID
         const unsigned t = atomicAdd(&grp->arrive[xcc], 1u);
-        if (t == (unsigned)gp - 1) atomicCAS(&grp->chosen, 0u, xcc + 1u);
+        if (t == (unsigned)gp - 1 && a.fault != HC_FAULT_JOIN) atomicCAS(&grp->chosen, 0u, xcc + 1u);
         const unsigned long long began = wall_clock64();
         unsigned c = 0u;
         while (c == 0u) {
@@ -893,15 +897,16 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
                     w0 = load_shared(rec + (lane & (gp - 1)) * 2);
                     w1 = load_shared(rec + (lane & (gp - 1)) * 2 + 1);
                     if (__builtin_amdgcn_ballot_w64((w0 & 3u) != tag || (w1 & 3u) != tag) == 0) break;
-                    if (spin == 5000000u) {
-                        failed = true;   // a partner is gone: about a second
+                    if (spin == (a.fault == HC_FAULT_PARTNER ? 0u : GPOLLS)) {
+                        failed = true;
                         break;
                     }
                 }
             }
             asm volatile("" ::: "memory");
             if (failed) {
-                // never seen: what is left is marked as no merge
+                // a partner is gone; d is half rewritten, so what is left is marked
+                // as no merge (sub == sup, NaN), which host callers get as an error
                 for (int i = iter + lane; g == 0 && i + 1 < n; i += 64) {
                     a.height[i] = __builtin_nanf("");
                     a.sub[i] = a.sup[i] = 0;
@@ -1201,7 +1206,7 @@ unsigned group_lds(int n, int lgp) { return (unsigned)((n + 31) / 32 * 4 + 4 * n
 
 hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float beta,
                          float *count, float *minv, int *minc, void *group, int *sub, int *sup,
-                         float *height, int state, hipStream_t stream)
+                         float *height, int state, int fault, hipStream_t stream)
 {
     if (n < 2) return hipSuccess;
     HclustArgs a;
@@ -1219,6 +1224,7 @@ hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lam
     a.height = height;
     a.vec4 = (ldd % 4 == 0) && ((reinterpret_cast<uintptr_t>(d) & 15) == 0);
     a.group = nullptr;
+    a.fault = fault;
     a.lgp = n <= GALONE_N ? 0 : 5;
     // up to what 15-bit tie keys and the LDS hold (32768 points: 9.1 us a round,
     // one workgroup of hclust_merge_kernel 143)

@@ -118,12 +118,17 @@ enum HcMethod {
 // per-row state in LDS up to HC_LDS_MAX_N points and in global memory above.
 // HC_STATE_LDS / HC_STATE_GLOBAL force one workgroup and a placement (LDS only
 // up to HC_LDS_MAX_N).
+// fault: tests force a failure of the several workgroups: they never come
+// together (one workgroup then does the rounds), or a partner's record is given
+// up on the first poll that does not find it.  That marks the rounds that are
+// left with sub == sup == 0 and a NaN height.
 enum HcState { HC_STATE_AUTO = 0, HC_STATE_LDS = 1, HC_STATE_GLOBAL = 2 };
+enum HcFault { HC_FAULT_NONE = 0, HC_FAULT_JOIN = 1, HC_FAULT_PARTNER = 2 };
 constexpr int64_t HC_LDS_MAX_N = 9216;
 constexpr size_t HC_GROUP_BYTES = 4096;
 hipError_t launch_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float beta,
                          float *count, float *minv, int *minc, void *group, int *sub, int *sup,
-                         float *height, int state, hipStream_t stream);
+                         float *height, int state, int fault, hipStream_t stream);
 
 // Pearson correlation (gpuCor).  use: 0 everything, 1 pairwise.complete.obs.
 // precision (use 0 only): 0 FP32 VALU, 1 BF16 three-term, 2 FP16 two-term

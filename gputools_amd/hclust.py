@@ -157,7 +157,8 @@ def hclust(d, method="complete", lam: float = 0.5, beta: float = 0.5, stream=Non
     ``state`` places the kernel's per-row state: "auto" (shared among
     workgroups up to 32768 points; else one workgroup, in LDS up to 9216
     points, in global memory above), "lds" or "global" (one workgroup); every
-    placement gives the same result."""
+    placement gives the same result.  (Should the shared form's workgroups lose
+    each other, the merges not made read sub == sup == 0, height NaN.)"""
     import torch
     if not isinstance(d, torch.Tensor) or not d.is_cuda or d.dtype != torch.float32:
         raise TypeError("d must be a float32 torch tensor on the GPU")

@@ -269,7 +269,11 @@ int gt_hclust_workspace_size(int64_t n, size_t *bytes);
  * (inst/cuda/hcluster.cu:4-400).  Writes the n - 1 merges to device arrays:
  * at step s the clusters represented by sub[s] < sup[s] (0-based point
  * indices) merge at height[s]; the merged cluster keeps index sup[s].  Ties
- * and arithmetic follow the reference bit for bit.  n below 2^24. */
+ * and arithmetic follow the reference bit for bit.  n below 2^24.
+ * The launch is asynchronous.  Should a workgroup not hear from another one for
+ * about a second (a kernel that the device stopped serving), the merges not yet
+ * made read sub == sup == 0 with a NaN height, the last one among them; the
+ * host-to-host entry points return GT_ERR_HIP then. */
 int gt_hclust(float *d, int64_t n, int64_t ldd, int method, float lambda, float beta, int *sub,
               int *sup, float *height, void *workspace, size_t workspace_bytes, void *stream);
 

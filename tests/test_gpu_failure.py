@@ -169,3 +169,72 @@ def test_gt_dist_device_full_and_kendall_release():
         return s == _lib.GT_OK, _lib.last_error() if s else ""
 
     assert fail_each_allocation(kendall) == 3
+
+
+def _cluster_matrix(n, seed):
+    x = torch.from_numpy(wl.normal(n, 5, seed=seed)).cuda()
+    return gt.dist(x, layout="full")
+
+
+def _hclust_chosen(d, method):
+    """hclust on the device through the C ABI: its results and the XCD choice in
+    the workspace's meeting point (0: none, 1 + XCD, or 0xffff: given up)."""
+    n = d.shape[0]
+    size = ctypes.c_size_t()
+    L = _lib.lib()
+    assert L.gt_hclust_workspace_size(n, ctypes.byref(size)) == 0
+    ws = torch.full((size.value,), 0xA5, dtype=torch.uint8, device="cuda")
+    out = [torch.empty(n - 1, dtype=t, device="cuda") for t in (torch.int32, torch.int32, torch.float32)]
+    assert L.gt_hclust(d.data_ptr(), n, d.stride(0), L.gt_hclust_method_from_name(method.encode()), 0.5, 0.5,
+                       *(t.data_ptr() for t in out), ws.data_ptr(), size.value, None) == 0
+    torch.cuda.synchronize()
+    at = ws.data_ptr() + size.value - 4096
+    at = (at + 255) // 256 * 256 + 64 - ws.data_ptr()
+    return [t.cpu().numpy() for t in out], int(ws[at:at + 4].cpu().numpy().view(np.uint32)[0])
+
+
+@pytest.mark.parametrize("n", [257, 1000, 9300])
+def test_hclust_without_room_for_the_workgroups(n):
+    """The clustering workgroups do not come together: one workgroup does the
+    rounds, with the same merges; without the failure an XCD is chosen."""
+    d = _cluster_matrix(n, 47)
+    print("case hclust without room n=%d" % n, flush=True)
+    want, chosen = _hclust_chosen(d.clone(), "average")
+    assert 1 <= chosen <= 16
+    os.environ["GT_FAIL_MEETING"] = "join"
+    try:
+        got, chosen = _hclust_chosen(d.clone(), "average")
+    finally:
+        del os.environ["GT_FAIL_MEETING"]
+    assert chosen == 0xFFFF
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g.view(np.uint32), w.view(np.uint32))
+
+
+def test_hclust_lost_workgroup_is_an_error():
+    """A workgroup that gives another one up ends the kernel; host callers get
+    an error, device callers merges with sub == sup."""
+    n = 700
+    d = _cluster_matrix(n, 48)
+    host = np.ascontiguousarray(d.cpu().numpy())
+    sub, sup = np.zeros(n - 1, np.int32), np.zeros(n - 1, np.int32)
+    height = np.zeros(n - 1, np.float32)
+    L = _lib.lib()
+
+    def call():
+        return L.gt_hclust_host(host.ctypes.data, n, n, L.gt_hclust_method_from_name(b"average"), 0.5, 0.5,
+                                sub.ctypes.data, sup.ctypes.data, height.ctypes.data)
+
+    print("case hclust lost workgroup", flush=True)
+    os.environ["GT_FAIL_MEETING"] = "partner"
+    try:
+        assert call() == _lib.GT_ERR_HIP
+        assert "stopped early" in _lib.last_error()
+        got, chosen = _hclust_chosen(d.clone(), "average")
+    finally:
+        del os.environ["GT_FAIL_MEETING"]
+    assert got[0][-1] == got[1][-1] == 0 and np.isnan(got[2][-1])
+    assert call() == 0
+    want = orc.hclust(host, "average")
+    for g, w in zip((sub, sup, height), want):
+        np.testing.assert_array_equal(g, w)
