@@ -640,7 +640,7 @@ __global__ __launch_bounds__(HTHREADS) void hclust_merge_kernel(HclustArgs a)
 // The workgroups must run on one XCD: they exchange data through its L2, where
 // stores complete and which loads that pass the L1 by read.  GLAUNCH are
 // launched, the first XCD that has 32 of them is chosen and the others leave.
-// If none has 32 within 50 ms (a busy device), nobody starts and
+// If none has 32 in time (a busy device, masked CUs), nobody starts and
 // hclust_merge_kernel, launched behind, does the work; otherwise that leaves
 // at once.
 // Bound: the round's latency, most of it dependent instructions of single
@@ -657,7 +657,10 @@ constexpr int GLAUNCH = 320;
 // Polls of a partner's record before it is given up: about a second of running
 // (not of the clock, which goes on while a queue is swapped out).
 constexpr unsigned GPOLLS = 5000000u;
-constexpr unsigned long long GJOIN_TICKS = 5000000ull;      // 50 ms of the 100 MHz clock
+// The wait for room: 1 us per point (100 MHz clock), a tenth to a fifth of what the
+// rounds take in hclust_merge_kernel (5.9 us a round at 257 points, 8.5 at 1000,
+// 19 at 8192).  They come together in some us where there is room.
+constexpr unsigned long long GJOIN_TICKS = 100ull;
 
 // End of a round: also this wave's stores are complete.
 __device__ __forceinline__ void round_barrier()
@@ -793,7 +796,7 @@ __global__ __launch_bounds__(GTHREADS) void hclust_group_kernel(HclustArgs a)
         const unsigned long long began = wall_clock64();
         unsigned c = 0u;
         while (c == 0u) {
-            const bool late = wall_clock64() - began > GJOIN_TICKS;
+            const bool late = wall_clock64() - began > GJOIN_TICKS * (unsigned long long)a.n;
             c = atomicCAS(&grp->chosen, 0u, late ? G_ABORT : 0u);
             if (late) break;
             __builtin_amdgcn_s_sleep(4);

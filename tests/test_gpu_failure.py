@@ -238,3 +238,33 @@ def test_hclust_lost_workgroup_is_an_error():
     want = orc.hclust(host, "average")
     for g, w in zip((sub, sup, height), want):
         np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("n", [257, 600])
+def test_hclust_short_wait_for_room(n):
+    """Where the workgroups find no room together (masked CUs, other work) the
+    wait before one workgroup takes over follows the work it could save: small
+    calls don't wait for tens of milliseconds."""
+    import time
+    d = _cluster_matrix(n, 49)
+
+    def best(state):
+        times = []
+        for _ in range(5):
+            c = d.clone()
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            gt.hclust(c, "average", state=state)
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - t0)
+        return min(times)
+
+    alone = best("lds")
+    os.environ["GT_FAIL_MEETING"] = "join"
+    try:
+        handed_over = best("auto")
+    finally:
+        del os.environ["GT_FAIL_MEETING"]
+    print("case hclust wait n=%d: %.2f ms alone, %.2f ms handed over" % (n, alone * 1e3, handed_over * 1e3), flush=True)
+    # one microsecond per point, and as much again for the launches
+    assert handed_over - alone <= 2e-6 * n + 1e-3
