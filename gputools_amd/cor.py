@@ -170,13 +170,19 @@ def pmcc(a, b=None, use="everything", precision: str = "bf16x3", stream=None, ou
     nbytes = ctypes.c_size_t()
     check(lib().gt_pmcc_workspace_size(u, prec, na, nb, dim, 1 if b is None else 0,
                                        ctypes.byref(nbytes)))
-    ws = torch.empty(max(nbytes.value, 1), dtype=torch.uint8, device=a.device)
+    try:
+        ws = torch.empty(max(nbytes.value, 1), dtype=torch.uint8, device=a.device)
+    except torch.cuda.OutOfMemoryError:
+        if u != USES.index("pairwise.complete.obs"):
+            raise
+        # runs without its workspace too
+        ws, nbytes.value = None, 0
     s = stream if stream is not None else torch.cuda.current_stream()
     check(lib().gt_pmcc(u, prec, a.data_ptr(), na, a.stride(0),
                         None if b is None else b.data_ptr(), nb,
                         a.stride(0) if b is None else b.stride(0), dim, pairs.data_ptr(),
-                        corr.data_ptr(), ts.data_ptr(), pairs.stride(0), ws.data_ptr(),
-                        nbytes.value, s.cuda_stream or None))
+                        corr.data_ptr(), ts.data_ptr(), pairs.stride(0),
+                        None if ws is None else ws.data_ptr(), nbytes.value, s.cuda_stream or None))
     return pairs, corr, ts
 
 

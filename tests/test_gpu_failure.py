@@ -268,3 +268,45 @@ def test_hclust_short_wait_for_room(n):
     print("case hclust wait n=%d: %.2f ms alone, %.2f ms handed over" % (n, alone * 1e3, handed_over * 1e3), flush=True)
     # one microsecond per point, and as much again for the launches
     assert handed_over - alone <= 2e-6 * n + 1e-3
+
+
+def _table(n, dim, seed):
+    x = np.ascontiguousarray(wl.normal(n, dim, seed=seed))
+    x[np.random.default_rng(seed).random(x.shape) < 0.05] = np.nan
+    return x
+
+
+def test_pairwise_without_room_for_its_workspace():
+    """pairwise.complete.obs needs no workspace: where it finds none, the call
+    runs without (host entry point and package function)."""
+    n, dim = 400, 3000
+    a, b = _table(n, dim, 50), _table(n, dim, 51)
+    outs = [np.zeros(n * n, np.float32) for _ in range(3)]
+    cu, cn, cs = ctypes.c_int(1), ctypes.c_int(n), ctypes.c_int(dim)
+    # variables 4.8 MB, results 1.9 MB, workspace 35 MB
+    os.environ["GT_FAIL_ALLOC_ABOVE"] = str(8 << 20)
+    try:
+        ok, msg = c_call(_lib.lib().rpmcc, ctypes.byref(cu), a.ctypes.data_as(FP), ctypes.byref(cn),
+                         b.ctypes.data_as(FP), ctypes.byref(cn), ctypes.byref(cs),
+                         *(o.ctypes.data_as(FP) for o in outs))
+    finally:
+        del os.environ["GT_FAIL_ALLOC_ABOVE"]
+    assert ok, msg
+    pairs, corr = orc.pmcc(a, b, "pairwise.complete.obs")
+    np.testing.assert_array_equal(outs[0].reshape(n, n), pairs)
+    assert np.max(np.abs(outs[1].reshape(n, n) - corr)) <= 1e-5
+
+    ad, bd = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    res = tuple(torch.empty((n, n), device="cuda") for _ in range(3))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    limit = torch.cuda.memory_reserved() + (10 << 20)
+    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        gt.pmcc(ad, bd, use="pairwise.complete.obs", precision="fp32", out=res)
+        got = res[1].cpu().numpy()
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            gt.pmcc(ad.nan_to_num_(), bd.nan_to_num_(), precision="bf16x3", out=res)   # needs its workspace
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert np.max(np.abs(got - corr)) <= 1e-5
