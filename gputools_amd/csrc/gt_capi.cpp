@@ -755,7 +755,7 @@ int gt_dist_device_full(const float *x_host, int64_t n, int64_t k, int method, f
     if ((s = dx.alloc((size_t)n * (size_t)k * sizeof(float), "hipMalloc(points)")) != GT_OK) return s;
     if ((s = dws.alloc(ws_bytes, "hipMalloc(workspace)")) != GT_OK) return s;
     // Pitched n x n result, as distanceLeaveOnGpu allocates it (cudaMallocPitch).
-    hipError_t e = injected_alloc_failure()
+    hipError_t e = injected_alloc_failure((size_t)n * sizeof(float) * (size_t)n)
                        ? hipErrorOutOfMemory
                        : hipMallocPitch(&d, &pitch, (size_t)n * sizeof(float), (size_t)n);
     if (e != hipSuccess) return hip_fail(e, "hipMallocPitch(distances)");
