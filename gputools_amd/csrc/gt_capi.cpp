@@ -891,6 +891,9 @@ int gt_pmcc(int use, int precision, const float *a, int64_t na, int64_t lda, con
                         workspace_bytes);
         workspace = nullptr;
     }
+    // (its operands are moved 16 bytes at a time; a pairwise call takes any
+    // pointer, as it once did without reading it)
+    if (use == GT_USE_PAIRWISE && (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) workspace = nullptr;
     GT_HIP(gt::launch_pmcc(use, precision, a, na, lda, b, nb, ldb, same, dim, pairs, corr, ts, ldo,
                            workspace, static_cast<hipStream_t>(stream)));
     return GT_OK;

@@ -409,3 +409,28 @@ def test_pairwise_large_value_missing_in_partner(fill, at):
             if y is None:
                 r[3, 3] = 1.0   # its squares may overflow
             np.testing.assert_allclose(r, corr, rtol=0, atol=1e-5)
+
+
+@pytest.mark.parametrize("shift", [0, 1, 8])
+def test_pairwise_workspace_at_any_address(shift):
+    """A pairwise call may be given any pointer and any number of bytes as its
+    workspace; what is not aligned for the matrix-core form is not used."""
+    import ctypes
+    rng = np.random.default_rng(11)
+    x = np.ascontiguousarray(_data(rng, 90, 70).T, dtype=np.float32)
+    x[rng.random(x.shape) < 0.1] = np.nan
+    a = torch.from_numpy(x).cuda()
+    need = ctypes.c_size_t()
+    L = gt.lib()
+    assert L.gt_pmcc_workspace_size(1, 0, 70, 70, 90, 1, ctypes.byref(need)) == 0 and need.value > 0
+    ws = torch.full((need.value + 16,), 0xFF, dtype=torch.uint8, device="cuda")
+    outs = [torch.full((70, 70), 7.0, device="cuda") for _ in range(3)]
+    print("case pairwise workspace shift", shift, flush=True)
+    assert L.gt_pmcc(1, 0, a.data_ptr(), 70, 90, None, 70, 90, 90, outs[0].data_ptr(), outs[1].data_ptr(),
+                     outs[2].data_ptr(), 70, ws.data_ptr() + shift, need.value, None) == 0
+    torch.cuda.synchronize()
+    if shift:
+        assert bool((ws == 0xFF).all())
+    pairs, corr = orc.pmcc(x, x, "pairwise.complete.obs")
+    np.testing.assert_array_equal(outs[0].cpu().numpy(), pairs)
+    np.testing.assert_allclose(outs[1].cpu().numpy(), corr, rtol=0, atol=1e-5)
