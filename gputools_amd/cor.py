@@ -25,7 +25,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import check, lib
-from .dist import pmatch
+from .dist import _workspace, pmatch
 
 COR_METHODS = ("pearson", "kendall")
 USES = ("everything", "pairwise.complete.obs")
@@ -171,7 +171,7 @@ def pmcc(a, b=None, use="everything", precision: str = "bf16x3", stream=None, ou
     check(lib().gt_pmcc_workspace_size(u, prec, na, nb, dim, 1 if b is None else 0,
                                        ctypes.byref(nbytes)))
     try:
-        ws = torch.empty(max(nbytes.value, 1), dtype=torch.uint8, device=a.device)
+        ws = _workspace(nbytes.value, a.device, stream)
     except torch.cuda.OutOfMemoryError:
         if u != USES.index("pairwise.complete.obs"):
             raise
@@ -212,7 +212,7 @@ def kendall(a, b=None, stream=None, out=None, workspace=None):
     nbytes = ctypes.c_size_t()
     check(lib().gt_kendall_workspace_size(na, nb, n, 1 if b is None else 0, ctypes.byref(nbytes)))
     if workspace is None:
-        ws = torch.empty(max(nbytes.value, 1), dtype=torch.uint8, device=a.device)
+        ws = _workspace(max(nbytes.value, 1), a.device, stream)
     else:
         if workspace.dtype != torch.uint8 or not workspace.is_cuda or workspace.numel() < nbytes.value:
             raise ValueError("workspace must be a uint8 CUDA tensor of at least %d bytes"

@@ -214,6 +214,21 @@ def _torch():
     return torch
 
 
+def _workspace(nbytes, device, stream=None):
+    """nbytes of workspace (None for 0) for work on ``stream``: memory comes from
+    the current stream's pool, which must not give it out again before another
+    stream is done with it."""
+    torch = _torch()
+    if not nbytes:
+        return None
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if stream is not None:
+        if not isinstance(stream, torch.cuda.Stream):   # anything with a cuda_stream
+            stream = torch.cuda.ExternalStream(stream.cuda_stream, device=ws.device)
+        ws.record_stream(stream)
+    return ws
+
+
 def _stream_ptr(stream=None) -> Optional[int]:
     torch = _torch()
     s = stream if stream is not None else torch.cuda.current_stream()
@@ -264,7 +279,7 @@ def dist(x, method="euclidean", p: float = 2.0, precision: str = "fp32",
             out = torch.empty((n, n), dtype=torch.float32, device=x.device)
     ldd = out.stride(0) if lay == _lib.LAYOUT_FULL else n
     ws_bytes = workspace_size(n, k, m, precision)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    ws = _workspace(ws_bytes, x.device, stream)
     check(lib().gt_dist_ws(x.data_ptr() if x.numel() else None, n, k, x.stride(0) if n else k,
                            m, float(p), prec, lay, out.data_ptr() if out.numel() else None, ldd,
                            ws.data_ptr() if ws is not None else None, ws_bytes,

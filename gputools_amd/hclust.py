@@ -27,7 +27,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import check, lib
-from .dist import Dist, METHODS, _as_points, pmatch
+from .dist import Dist, METHODS, _as_points, _workspace, pmatch
 
 # the clustering methods gpuHclust / gpuDistClust accept (R/gpuHclust.R:43-44)
 R_CLUST_METHODS = ("ward", "single", "complete", "average", "mcquitty", "median", "centroid",
@@ -171,7 +171,7 @@ def hclust(d, method="complete", lam: float = 0.5, beta: float = 0.5, stream=Non
     height = torch.empty(m, dtype=torch.float32, device=d.device)
     b = ctypes.c_size_t()
     check(lib().gt_hclust_workspace_size(n, ctypes.byref(b)))
-    ws = torch.empty(max(b.value, 1), dtype=torch.uint8, device=d.device)
+    ws = _workspace(max(b.value, 1), d.device, stream)
     s = stream if stream is not None else torch.cuda.current_stream()
     check(lib().gt_hclust_state(d.data_ptr(), n, d.stride(0), hclust_method_id(method),
                                 float(lam), float(beta), sub.data_ptr() if m else None,

@@ -434,3 +434,36 @@ def test_pairwise_workspace_at_any_address(shift):
     pairs, corr = orc.pmcc(x, x, "pairwise.complete.obs")
     np.testing.assert_array_equal(outs[0].cpu().numpy(), pairs)
     np.testing.assert_allclose(outs[1].cpu().numpy(), corr, rtol=0, atol=1e-5)
+
+
+@pytest.mark.parametrize("call", ["pairwise", "everything", "kendall", "dist", "hclust"])
+def test_workspace_on_another_stream(call):
+    """A call on a stream that is busy keeps its workspace while the current
+    stream allocates and writes memory of the same size."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn((500, 300), generator=g, device="cuda")
+    fn = {"pairwise": lambda **kw: gt.pmcc(x, use="pairwise.complete.obs", precision="fp32", **kw)[1],
+          "everything": lambda **kw: gt.pmcc(x, precision="bf16x3", **kw)[1],
+          "kendall": lambda **kw: gt.kendall(x, **kw),
+          "dist": lambda **kw: gt.dist(x, precision="bf16x3", **kw),
+          "hclust": lambda **kw: gt.hclust(d.clone(), "average", **kw)[2]}[call]
+    d = gt.dist(x, layout="full")
+    want = fn()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    d = d.clone()
+    print("case workspace on another stream:", call, flush=True)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(50_000_000)
+    if call == "hclust":      # its matrix must live as long
+        c = d.clone()
+        side.wait_stream(torch.cuda.current_stream())
+        got = gt.hclust(c, "average", stream=side)[2]
+    else:
+        got = fn(stream=side)
+    trash = [torch.full((size,), 0xFF, dtype=torch.uint8, device="cuda")
+             for size in [1 << s for s in range(9, 27)]]
+    torch.cuda.synchronize()
+    del trash
+    assert torch.equal(got, want)
