@@ -276,7 +276,7 @@ def _table(n, dim, seed):
     return x
 
 
-def test_pairwise_without_room_for_its_workspace():
+def test_pairwise_without_room_for_its_workspace(monkeypatch):
     """pairwise.complete.obs needs no workspace: where it finds none, the call
     runs without (host entry point and package function)."""
     n, dim = 400, 3000
@@ -298,15 +298,16 @@ def test_pairwise_without_room_for_its_workspace():
 
     ad, bd = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
     res = tuple(torch.empty((n, n), device="cuda") for _ in range(3))
-    torch.cuda.synchronize()
-    torch.cuda.empty_cache()
-    limit = torch.cuda.memory_reserved() + (10 << 20)
-    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
-    try:
-        gt.pmcc(ad, bd, use="pairwise.complete.obs", precision="fp32", out=res)
-        got = res[1].cpu().numpy()
-        with pytest.raises(torch.cuda.OutOfMemoryError):
-            gt.pmcc(ad.nan_to_num_(), bd.nan_to_num_(), precision="bf16x3", out=res)   # needs its workspace
-    finally:
-        torch.cuda.set_per_process_memory_fraction(1.0)
+    real = torch.empty
+
+    def no_room(*args, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.cuda.OutOfMemoryError("no room for a workspace")
+        return real(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_room)
+    gt.pmcc(ad, bd, use="pairwise.complete.obs", precision="fp32", out=res)
+    got = res[1].cpu().numpy()
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        gt.pmcc(ad.nan_to_num_(), bd.nan_to_num_(), precision="bf16x3", out=res)   # needs its workspace
     assert np.max(np.abs(got - corr)) <= 1e-5
