@@ -730,7 +730,9 @@ __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
 // those of row j are added over the lane's four rows, then over the wave by
 // data-parallel adds.  Each term is w (y_i - y_j): sums of w and of w y_j apart
 // cancel where points are close.  Both sides go to partial slices, which
-// mds_finish_kernel adds in a fixed order: deterministic, no atomics.
+// mds_finish_kernel adds in a fixed order: deterministic, no atomics.  The
+// slices are about n / 128 for each row: beyond MDS_SLICE_BYTES the row blocks are
+// taken some at a time, each pass adding to dY.
 // Bound: VALU issue (about 45 instructions per pair with 2 features, two of them
 // FP64; delta alone would take 0.11 ms).  16384 x 2: 0.67 ms for the sweep, which
 // visits each pair from both rows and pads 2 features to 4, 0.18 ms here; the
@@ -744,8 +746,13 @@ struct MdsArgs {
     int64_t n, q, ldy;
     const float *delta;
     int jw;                    // columns per wave: 16, 32 or 64
-    float *ipart, *jpart;      // [slice][feature][row]: rows i by column block, rows j by row block
-    double *partials;          // stress, one per workgroup
+    int64_t c0, c1;            // this pass's row blocks
+    int t0;                    // tiles before them
+    // [slice][feature][row]: rows i of the pass (irows of them) by column block,
+    // rows j by row block of the pass; the pointers are those of row 0 and block 0
+    float *ipart, *jpart;
+    int irows;
+    double *partials;          // stress, one per workgroup (of this pass)
 };
 
 // Sum over the wave, in lane 63.
@@ -820,7 +827,7 @@ __global__ __launch_bounds__(256) void mds_small_kernel(MdsArgs args)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t n = args.n;
     // row block ci has f (ci + 1) column blocks, f = 256 / (4 jw)
-    const int64_t t = blockIdx.x;
+    const int64_t t = args.t0 + blockIdx.x;
     const int f = 64 / args.jw;
     int ci, cm;
     tri_tile(t / f, ci, cm);
@@ -901,7 +908,7 @@ __global__ __launch_bounds__(256) void mds_small_kernel(MdsArgs args)
                 for (int c = 0; c < Q; ++c) {
                     float v = wi[r][c];
                     for (int w = 0; w < 3; ++w) v += red[w][r * 64 + lane][c];
-                    if (i < n && c < args.q) args.ipart[(cj * args.q + c) * n + i] = v;
+                    if (i < n && c < args.q) args.ipart[(cj * args.q + c) * args.irows + i] = v;
                 }
             }
     }
@@ -909,19 +916,22 @@ __global__ __launch_bounds__(256) void mds_small_kernel(MdsArgs args)
     for (int d = 32; d >= 1; d >>= 1) stress += __shfl_xor(stress, d, 64);
     if (lane == 0) red_s[wave] = stress;
     __syncthreads();
-    if (tid == 0) args.partials[t] = ((red_s[0] + red_s[1]) + red_s[2]) + red_s[3];
+    if (tid == 0) args.partials[blockIdx.x] = ((red_s[0] + red_s[1]) + red_s[2]) + red_s[3];
 }
 
-// dY_r from the slices of row r: its column blocks as a
-// row i, then the row blocks from its own on as a row j.  MSUM threads a row;
-// the last workgroup adds the stress partials.
+// dY_r from the slices of row r in this pass: its column blocks as a row i, then
+// the row blocks from its own on as a row j; rows of earlier passes only as a
+// row j, added to what they have.  MSUM threads a row; the last workgroup adds
+// the stress partials (stress null: not the last pass).
 __global__ __launch_bounds__(256) void mds_finish_kernel(MdsArgs args, float *__restrict__ dy, int64_t lddy,
                                                          int64_t count, double *__restrict__ stress)
 {
     if (blockIdx.x == gridDim.x - 1) {
+        if (stress == nullptr) return;
         __shared__ double s_[256];
         double s = 0.0;
-        for (int64_t e = threadIdx.x; e < count; e += 256) s += args.partials[e];
+        const double *const all = args.partials - args.t0;
+        for (int64_t e = threadIdx.x; e < count; e += 256) s += all[e];
         s_[threadIdx.x] = s;
         __syncthreads();
         for (int d = 128; d >= 1; d >>= 1) {
@@ -935,21 +945,24 @@ __global__ __launch_bounds__(256) void mds_finish_kernel(MdsArgs args, float *__
     __shared__ float red[MSUM][ROWS];
     const int lr = threadIdx.x % ROWS, part = threadIdx.x / ROWS;
     const int64_t n = args.n, row = (int64_t)blockIdx.x * ROWS + lr, ci = row / MI;
-    const int64_t islices = 64 / args.jw * (ci + 1), slices = islices + (n + MI - 1) / MI - ci;
+    const bool earlier = ci < args.c0;
+    const int64_t first = earlier ? args.c0 : ci;
+    const int64_t islices = earlier ? 0 : 64 / args.jw * (ci + 1), slices = islices + args.c1 - first;
+    const bool in = row < n && ci < args.c1;
     for (int64_t c = 0; c < args.q; ++c) {
         float v = 0.0f;
-        if (row < n)
+        if (in)
 #pragma unroll 4
             for (int64_t e = part; e < slices; e += MSUM)
-                v += e < islices ? args.ipart[(e * args.q + c) * n + row]
-                                 : args.jpart[((ci + e - islices) * args.q + c) * n + row];
+                v += e < islices ? args.ipart[(e * args.q + c) * args.irows + row]
+                                 : args.jpart[((first + e - islices) * args.q + c) * n + row];
         __syncthreads();
         red[part][lr] = v;
         __syncthreads();
         float total = red[0][lr];
 #pragma unroll
         for (int e = 1; e < MSUM; ++e) total += red[e][lr];
-        if (part == 0 && row < n) dy[row * lddy + c] = total;
+        if (part == 0 && in) dy[row * lddy + c] = earlier ? dy[row * lddy + c] + total : total;
     }
 }
 
@@ -1160,12 +1173,28 @@ bool mds_small_applies(int64_t n, int64_t q) { return n >= 2 && (q <= 6 || (q <=
 
 // Slices of the rows as i (column blocks) and as j (row blocks).
 int64_t mds_islices(int64_t n) { return 64 / mds_jw(n) * ((n + MI - 1) / MI); }
-size_t mds_slices(int64_t n) { return (size_t)mds_islices(n) + (size_t)((n + MI - 1) / MI); }
+
+// Row blocks of a pass: all of them while the slices fit MDS_SLICE_BYTES (up to
+// 32768 x 8), else what fits, at least one (65536 x 8: 6.59 ms with 1.07 GB in one
+// pass, 7.30 with 128 MB, 6.84 with 256).
+constexpr size_t MDS_SLICE_BYTES = (size_t)256 << 20;
+size_t mds_slice_bytes(int64_t n, int64_t q, int64_t blocks)
+{
+    const int64_t ni = (n + MI - 1) / MI, irows = blocks == ni ? n : blocks * MI;
+    return (size_t)(mds_islices(n) * irows + blocks * n) * (size_t)q * sizeof(float);
+}
+int64_t mds_pass_blocks(int64_t n, int64_t q)
+{
+    const int64_t ni = (n + MI - 1) / MI;
+    if (mds_slice_bytes(n, q, ni) <= MDS_SLICE_BYTES) return ni;
+    const int64_t blocks = (int64_t)(MDS_SLICE_BYTES / mds_slice_bytes(n, q, 1));
+    return blocks < 1 ? 1 : blocks;
+}
 
 template <int Q>
 void launch_mds_small(const MdsArgs &args, bool grad, hipStream_t stream)
 {
-    const dim3 grid((unsigned)mds_tiles(args.n));
+    const dim3 grid((unsigned)(64 / args.jw * (args.c1 * (args.c1 + 1) / 2) - args.t0));
     if (grad)
         hipLaunchKernelGGL((mds_small_kernel<Q, true>), grid, dim3(256), 0, stream, args);
     else
@@ -1182,7 +1211,7 @@ int64_t mds_partials_count(int64_t n, int64_t q)
 
 size_t mds_workspace_bytes(int64_t n, int64_t q)
 {
-    if (mds_small_applies(n, q)) return mds_slices(n) * (size_t)n * (size_t)q * sizeof(float);
+    if (mds_small_applies(n, q)) return mds_slice_bytes(n, q, mds_pass_blocks(n, q));
     return sweep_workspace_bytes(n, q);
 }
 
@@ -1234,24 +1263,33 @@ hipError_t launch_mds(const float *y, int64_t n, int64_t q, int64_t ldy, const f
         ma.q = q;
         ma.ldy = ldy;
         ma.delta = delta;
-        ma.ipart = workspace;
         ma.jw = mds_jw(n);
-        ma.jpart = dy ? workspace + (size_t)mds_islices(n) * (size_t)n * (size_t)q : nullptr;
-        ma.partials = partials;
-        switch (q) {
-        case 1: launch_mds_small<1>(ma, dy != nullptr, stream); break;
-        case 2: launch_mds_small<2>(ma, dy != nullptr, stream); break;
-        case 3: launch_mds_small<3>(ma, dy != nullptr, stream); break;
-        case 4: launch_mds_small<4>(ma, dy != nullptr, stream); break;
-        case 5: case 6: launch_mds_small<6>(ma, dy != nullptr, stream); break;
-        default: launch_mds_small<8>(ma, dy != nullptr, stream); break;
+        const int64_t ni = (n + MI - 1) / MI, blocks = dy ? mds_pass_blocks(n, q) : ni;
+        for (int64_t c0 = 0; c0 < ni; c0 += blocks) {
+            ma.c0 = c0;
+            ma.c1 = c0 + blocks < ni ? c0 + blocks : ni;
+            const int64_t end = ma.c1 * MI < n ? ma.c1 * MI : n;
+            ma.irows = (int)(end - c0 * MI);
+            ma.t0 = (int)(64 / ma.jw * (c0 * (c0 + 1) / 2));
+            ma.partials = partials + ma.t0;
+            ma.ipart = dy ? workspace - c0 * MI : nullptr;
+            ma.jpart = dy ? workspace + mds_islices(n) * ma.irows * q - c0 * q * n : nullptr;
+            switch (q) {
+            case 1: launch_mds_small<1>(ma, dy != nullptr, stream); break;
+            case 2: launch_mds_small<2>(ma, dy != nullptr, stream); break;
+            case 3: launch_mds_small<3>(ma, dy != nullptr, stream); break;
+            case 4: launch_mds_small<4>(ma, dy != nullptr, stream); break;
+            case 5: case 6: launch_mds_small<6>(ma, dy != nullptr, stream); break;
+            default: launch_mds_small<8>(ma, dy != nullptr, stream); break;
+            }
+            hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+            const unsigned rows = dy ? (unsigned)((end + 256 / MSUM - 1) / (256 / MSUM)) : 0u;
+            hipLaunchKernelGGL(mds_finish_kernel, dim3(rows + 1), dim3(256), 0, stream, ma, dy, lddy,
+                               mds_tiles(n), ma.c1 == ni ? stress : nullptr);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
         }
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        const unsigned rows = dy ? (unsigned)((n + 256 / MSUM - 1) / (256 / MSUM)) : 0u;
-        hipLaunchKernelGGL(mds_finish_kernel, dim3(rows + 1), dim3(256), 0, stream, ma, dy, lddy, mds_tiles(n),
-                           stress);
-        return hipGetLastError();
+        return hipSuccess;
     }
     BwArgs args;
     args.x = y;

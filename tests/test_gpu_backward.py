@@ -223,3 +223,49 @@ def test_mds_few_features(n, q):
             s2, dy2 = _mds(yd, dd, True)
             assert s2.item() == s.item()                              # deterministic
             np.testing.assert_array_equal(dy.cpu().numpy(), dy2.cpu().numpy())
+
+
+def _mds_reference(y, delta):
+    """Stress and gradient in FP64 on the GPU, some rows at a time."""
+    n = y.shape[0]
+    yd = y.double()
+    stress, dy = 0.0, torch.zeros_like(yd)
+    cols = torch.arange(n, device="cuda")
+    for i in range(0, n, 1024):
+        rows = cols[i:i + 1024]
+        diff2 = sum((yd[i:i + 1024, c, None] - yd[None, :, c]).square_() for c in range(y.shape[1]))
+        d = diff2.sqrt_()
+        hi, lo = torch.maximum(rows[:, None], cols), torch.minimum(rows[:, None], cols)
+        at = lo * n - lo * (lo + 1) // 2 + hi - lo - 1
+        off = hi != lo
+        dl = torch.where(off, delta[at.clamp_(0, delta.numel() - 1)].double(), torch.zeros((), dtype=torch.float64, device="cuda"))
+        r = torch.where(off, d - dl, torch.zeros_like(d))
+        stress += 0.5 * r.square().sum().item()
+        w = torch.where(d > 0, 2.0 * r / d, torch.zeros_like(d))
+        dy[i:i + 1024] = yd[i:i + 1024] * w.sum(1, keepdim=True) - w @ yd
+    return stress, dy
+
+
+@pytest.mark.parametrize("n,q", [(33025, 8), (50001, 8), (65793, 2)])
+def test_mds_scratch_is_bounded(n, q):
+    """The partial slices of the few-feature form grow with n^2; beyond 256 MiB
+    the rows are taken in several passes (two or three here, with a ragged
+    last block)."""
+    import os
+    g = torch.Generator(device="cuda").manual_seed(n)
+    y = torch.randn((n, q), generator=g, device="cuda")
+    y[n - 1] = y[3]
+    delta = torch.rand(n * (n - 1) // 2, generator=g, device="cuda") * 3.0
+    from gputools_amd.autograd import _mds
+    print("case mds bounded scratch n=%d q=%d" % (n, q), flush=True)
+    os.environ["GT_FAIL_ALLOC_ABOVE"] = str((256 << 20) + (4 << 20))   # and the stress partials
+    try:
+        s, dy = _mds(y, delta, True)
+        s2, dy2 = _mds(y, delta, True)
+        s3, _ = _mds(y, delta, False)
+    finally:
+        del os.environ["GT_FAIL_ALLOC_ABOVE"]
+    assert s2.item() == s.item() == s3.item() and torch.equal(dy, dy2)
+    want_s, want = _mds_reference(y, delta)
+    assert abs(s.item() - want_s) <= 1e-6 * want_s
+    assert_grad_close(dy.cpu().numpy(), want.cpu().numpy())
