@@ -871,17 +871,26 @@ static size_t terms_bytes(int64_t rows, int64_t k, int precision)
                     sizeof(unsigned short));
 }
 
+// Above this tau nearly every pair would be recomputed: the request is
+// computed by the FP32 difference kernel instead (from 8305 features on in BF16,
+// 15457 in FP16), which needs no workspace.
+constexpr float GRAM_TAU_MAX = 0.9f;
+
+static int64_t terms_rows(int64_t n, int64_t k, int precision)
+{
+    return gram_tau(precision, k) > GRAM_TAU_MAX ? n : operand_rows(n);
+}
+
 // Bytes of gram_workspace_bytes that come from rounding the rows up to 32: at
-// most GRAM_ROW_SLACK at the feature counts that use them (GRAM_TAU_MAX below:
-// up to 8304 in BF16, 15456 in FP16).
+// most GRAM_ROW_SLACK.
 size_t gram_rounding_bytes(int64_t n, int64_t k, int precision)
 {
-    return terms_bytes(operand_rows(n), k, precision) - terms_bytes(n, k, precision);
+    return terms_bytes(terms_rows(n, k, precision), k, precision) - terms_bytes(n, k, precision);
 }
 
 size_t gram_workspace_bytes(int64_t n, int64_t k, int precision)
 {
-    return terms_bytes(operand_rows(n), k, precision) + 3 * align256((size_t)n * sizeof(float)) + align256((size_t)k * sizeof(float)) +
+    return terms_bytes(terms_rows(n, k, precision), k, precision) + 3 * align256((size_t)n * sizeof(float)) + align256((size_t)k * sizeof(float)) +
            3 * align256((size_t)colstats_blocks(n) * (size_t)k * sizeof(float));
 }
 
@@ -952,10 +961,6 @@ hipError_t gram_prepare(int precision, const float *x, int64_t n, int64_t k, int
     return fp16 ? launch_rows<SPLIT_FP16>(vec4, x, n, k, ldx, prep, stream)
                 : launch_rows<SPLIT_BF16>(vec4, x, n, k, ldx, prep, stream);
 }
-
-// Above this tau nearly every pair would be recomputed: the request is
-// computed by the FP32 difference kernel instead.
-constexpr float GRAM_TAU_MAX = 0.9f;
 
 hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int64_t k,
                        int64_t ldx, float *out, int64_t ldd, void *workspace, hipStream_t stream)

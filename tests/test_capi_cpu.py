@@ -184,3 +184,22 @@ def test_noalloc_rejects_oversized_requests_before_the_device():
     # ordinary argument errors come first, as for gt_dist
     s, msg = _status(L.gt_dist_noalloc, dummy, 10, 4, 4, 9, 2.0, 0, 0, dummy, 10, None)
     assert s == _lib.GT_ERR_INVALID and "method" in msg
+
+
+@pytest.mark.parametrize("prec,terms,limit", [(1, 3, 8304), (2, 2, 15456)])
+def test_split_workspace_of_few_points(prec, terms, limit):
+    """The split terms are laid out for rows in multiples of 32; beyond the
+    feature counts that use them (where the FP32 kernel takes the call) a few
+    points don't ask for 32 rows."""
+    L = _lib.lib()
+    b = ctypes.c_size_t()
+
+    def need(n, k):
+        assert L.gt_dist_workspace_size(n, k, 0, prec, ctypes.byref(b)) == 0
+        return b.value
+
+    for n, k in ((2, limit + 1), (2, 10 ** 7), (33, 10 ** 6)):
+        kp = (k + 31) // 32 * 32
+        blocks = (n + 255) // 256
+        assert need(n, k) <= 2 * terms * n * kp + 12 * n + 4 * k + 12 * blocks * k + 8 * 256
+    assert need(2, limit) > 32 * 2 * terms * limit
