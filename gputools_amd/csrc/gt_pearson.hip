@@ -1266,6 +1266,22 @@ size_t side_bytes(int precision, int64_t rows, int64_t dim)
            align256((size_t)rows * sizeof(float));
 }
 
+// The form that computes a call of use = "everything": the split terms are laid
+// out for variables in multiples of 32, so a few long variables would take up to
+// 32 times their bytes (2 x 10^8 samples 19 GB, BF16).  Where the rounding adds
+// half of them again and more than 256 MB (one tile of few variables then), the
+// FP32 form does the work, in 4 bytes a value: its products and sums are no less
+// exact (see the sums of gt_plain.hip), and such a call takes about as long (20
+// variables x 100000: 3.7 ms, BF16 5.9, FP16 3.4).
+int everything_form(int precision, int64_t na, int64_t nb, bool same, int64_t dim)
+{
+    if (precision == 0) return 0;
+    const double value = 2.0 * prep_terms(precision) * (double)padded_dim(dim);
+    const double rows = (double)na + (same ? 0.0 : (double)nb);
+    const double rounded = (double)operand_rows(na) + (same ? 0.0 : (double)operand_rows(nb));
+    return rounded >= 1.5 * rows && (rounded - rows) * value > 268435456.0 ? 0 : precision;
+}
+
 PmccWs carve(int precision, int64_t na, int64_t nb, bool same, int64_t dim, void *ws)
 {
     PmccWs w;
@@ -1411,6 +1427,7 @@ size_t pmcc_workspace_bytes(int use, int precision, int64_t na, int64_t nb, bool
 {
     if (dim <= 0 || na <= 0 || nb <= 0) return 0;
     if (use == 1) return moments_plan(na, nb, same, dim).bytes;
+    precision = everything_form(precision, na, nb, same, dim);
     return side_bytes(precision, na, dim) + (same ? 0 : side_bytes(precision, nb, dim));
 }
 
@@ -1500,6 +1517,7 @@ hipError_t launch_pmcc(int use, int precision, const float *a, int64_t na, int64
         return hipSuccess;
     }
 
+    precision = everything_form(precision, na, nb, same, dim);
     PmccWs w = carve(precision, na, nb, same, dim, workspace);
     hipError_t e = launch_prep(precision, a, na, dim, lda, w.ta, w.isa, w.za, stream);
     if (e != hipSuccess) return e;

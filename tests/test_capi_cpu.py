@@ -203,3 +203,21 @@ def test_split_workspace_of_few_points(prec, terms, limit):
         blocks = (n + 255) // 256
         assert need(n, k) <= 2 * terms * n * kp + 12 * n + 4 * k + 12 * blocks * k + 8 * 256
     assert need(2, limit) > 32 * 2 * terms * limit
+
+
+@pytest.mark.parametrize("prec,terms", [(1, 3), (2, 2)])
+def test_pearson_workspace_of_few_long_variables(prec, terms):
+    """The split terms are laid out for variables in multiples of 32; a few long
+    variables take the FP32 form rather than 32 times their bytes."""
+    L = _lib.lib()
+    b = ctypes.c_size_t()
+    for na, nb, dim, same in ((1, 1, 10 ** 8, 0), (2, 2, 10 ** 8, 1), (1, 20, 10 ** 8, 0), (21, 21, 10 ** 7, 1)):
+        rows = na if same else na + nb
+        assert L.gt_pmcc_workspace_size(0, prec, na, nb, dim, same, ctypes.byref(b)) == 0
+        assert b.value <= 2 * terms * rows * (dim + 31) + 4 * rows + 4 * 256
+    # otherwise the rounded rows, at most half again or 256 MB more
+    for na, nb, dim, same in ((2, 2, 1000, 1), (2, 4000, 10 ** 6, 0), (64, 64, 10 ** 7, 1)):
+        rows = na if same else na + nb
+        assert L.gt_pmcc_workspace_size(0, prec, na, nb, dim, same, ctypes.byref(b)) == 0
+        plain = 2 * terms * rows * dim
+        assert plain <= b.value <= max(1.5 * plain, plain + (1 << 28)) + 2 * terms * rows * 32 + 4 * rows + 4096

@@ -467,3 +467,22 @@ def test_workspace_on_another_stream(call):
     torch.cuda.synchronize()
     del trash
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("precision", ["bf16x3", "fp16x3"])
+@pytest.mark.parametrize("na,nb,dim", [(3, 0, 3000003), (1, 2, 1500001)])
+def test_everything_few_long_variables(precision, na, nb, dim):
+    """Few and long variables run in the FP32 form (their split terms would take
+    many times their bytes): the same bits as that, and sums of millions of terms
+    no further from FP64 than one level of FP32 sums in steps of 16 would be."""
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    a = torch.randn((na, dim), generator=g, device="cuda") + 2.0
+    b = torch.randn((nb, dim), generator=g, device="cuda") + a[0] if nb else None
+    print("case few long variables", precision, na, nb, dim, flush=True)
+    got = gt.pmcc(a, b, precision=precision)
+    want = gt.pmcc(a, b, precision="fp32")
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+    za, zb = (v.double() - v.double().mean(1, keepdim=True) for v in (a, a if b is None else b))
+    za, zb = (z / z.norm(dim=1, keepdim=True) for z in (za, zb))
+    np.testing.assert_allclose(got[1].cpu().numpy(), (za @ zb.t()).cpu().numpy(), rtol=0, atol=TOL)
