@@ -66,16 +66,25 @@ __host__ __device__ __forceinline__ int64_t pair_tiles(int64_t n)
 // ---------------------------------------------------------------------------
 // Planes pass
 // ---------------------------------------------------------------------------
-struct PlanesArgs {
+struct PlanesSide {
     const float *x;
-    int64_t nvar, n, ldx;
+    int64_t nvar, ldx;
     uint32_t *planes;    // plane p (0 = P, 1 = N, 2 = E), block vb, group g at
                          // ((p * nvb + vb) * ngroups + g) * KGWORDS
     uint8_t *flags;      // flags[g * fstride + vb]: the group's N and E words are stored
-    int64_t nvb, fstride, ngroups;
+    int64_t nvb, fstride;
+};
+
+struct PlanesArgs {
+    PlanesSide a, b;     // b.nvb = 0: the self case
+    int64_t n, ngroups;
     int64_t tile_begin, ntiles;   // this segment's tiles of sample pairs
     int64_t runs;
     int64_t run;         // tiles per workgroup
+    // the counts, cleared here before the first count pass adds to them (by
+    // stores, not a memset node, so that a captured graph replays correctly)
+    unsigned long long *count;
+    int64_t ncount;
 };
 
 constexpr int KRUN = 4;      // tiles per workgroup
@@ -105,8 +114,16 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
     __shared__ unsigned special[3];   // per tile: groups whose N and E words are needed
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int64_t e = (int64_t)blockIdx.x * 256 + tid; e < args.ncount; e += (int64_t)gridDim.x * 256)
+        args.count[e] = 0ull;
     const int64_t n = args.n, jwn = column_words(n);
-    const int64_t vb = blockIdx.x / args.runs, run = blockIdx.x % args.runs;
+    int64_t vb = blockIdx.x / args.runs;
+    const int64_t run = blockIdx.x % args.runs;
+    const bool second = vb >= args.a.nvb;
+    if (second) vb -= args.a.nvb;
+    const int64_t nvb = second ? args.b.nvb : args.a.nvb, nvar = second ? args.b.nvar : args.a.nvar;
+    const int64_t ldx = second ? args.b.ldx : args.a.ldx, fstride = second ? args.b.fstride : args.a.fstride;
+    uint8_t *const flags = second ? args.b.flags : args.a.flags;
     const int64_t tb = run * args.run;
     const int nt = (int)(args.ntiles - tb < args.run ? args.ntiles - tb : args.run);
     const int64_t t0 = args.tile_begin + tb;
@@ -120,9 +137,9 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
     }
     int64_t jw = 2 * rb + (t0 - tiles_before(rb, jwn));
     const int64_t v0 = vb * KVB + wave * 8;
-    const float *const x = args.x;
-    const int64_t pstride = args.nvb * args.ngroups * KGWORDS;
-    uint32_t *const pv = args.planes + vb * args.ngroups * KGWORDS;
+    const float *const x = second ? args.b.x : args.a.x;
+    const int64_t pstride = nvb * args.ngroups * KGWORDS;
+    uint32_t *const pv = (second ? args.b.planes : args.a.planes) + vb * args.ngroups * KGWORDS;
     const int slot = (lane >> 3) * QS + ((lane >> 2) & 1) * HS + (lane & 3);
 
     float xi[8];
@@ -131,8 +148,8 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
         if (i > n - 1) i = n - 1;
 #pragma unroll
         for (int vv = 0; vv < 8; ++vv) {
-            const int64_t v = v0 + vv < args.nvar ? v0 + vv : args.nvar - 1;
-            xi[vv] = x[v * args.ldx + i] + 0.0f;
+            const int64_t v = v0 + vv < nvar ? v0 + vv : nvar - 1;
+            xi[vv] = x[v * ldx + i] + 0.0f;
         }
     };
     // the three comparisons of 32 columns, column u in bit u, which lane u holds
@@ -163,8 +180,8 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
         uint32_t *const pb = buf[k & 1] + slot + wave * 8 * 4;
 #pragma unroll
         for (int vv = 0; vv < 8; ++vv) {
-            const int64_t v = v0 + vv < args.nvar ? v0 + vv : args.nvar - 1;
-            const float *xv = x + v * args.ldx + j0;
+            const int64_t v = v0 + vv < nvar ? v0 + vv : nvar - 1;
+            const float *xv = x + v * ldx + j0;
             uniform_float_t *xj = (uniform_float_t *)xv;
             const float xl = xv[(lane & 31) < cols ? lane & 31 : cols - 1];
             uint32_t w = 0u, m = 0xffffffffu;
@@ -215,7 +232,7 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
                 *reinterpret_cast<const uint4 *>(buf[k & 1] + q * QS + (l >> 5) * HS + (l & 31) * 4);
         }
         const unsigned mask = special[k % 3];
-        if (tid < KTG) args.flags[(g + tid) * args.fstride + vb] = (uint8_t)((mask >> tid) & 1u);
+        if (tid < KTG) flags[(g + tid) * fstride + vb] = (uint8_t)((mask >> tid) & 1u);
         if (mask != 0u) {
             const int q = lane >> 3;
             uint32_t *const po = pt + q * KGWORDS + ((lane >> 2) & 1) * 128 + (lane & 3);
@@ -344,8 +361,9 @@ __global__ __launch_bounds__(KTHREADS, 2) void kendall_count_kernel(KendallArgs 
     if (g1 > args.ngroups) g1 = args.ngroups;
     if (g0 >= g1) return;
     const int ng = (int)(g1 - g0);
-    // a wave with no pair x >= y only helps to load
-    const bool idle = SYM && y0 + wy * 64 > x0 + wx * 128 + 127;
+    // a wave with no pair, or none x >= y, only helps to load
+    const bool idle = x0 + wx * 128 >= args.na || y0 + wy * 64 >= args.nb ||
+                      (SYM && y0 + wy * 64 > x0 + wx * 128 + 127);
 
     // wave w loads blocks 3 w .. 3 w + 2 of the 8 + 4; blocks past a side's last
     // one repeat it (they only feed pairs that are not stored)
@@ -586,20 +604,12 @@ KendallPlan kendall_plan(int64_t na, int64_t nb, bool same, int64_t n)
     return k;
 }
 
-hipError_t launch_planes(const float *x, int64_t nvar, int64_t n, int64_t ldx, uint32_t *planes,
-                         uint8_t *flags, int64_t nvb, int64_t fstride, int64_t seg, int64_t begin,
-                         int64_t tiles, hipStream_t stream)
+// One launch for both sides, which clears the counts too: small calls take as
+// long as their launches.
+hipError_t launch_planes(PlanesArgs &args, int64_t begin, int64_t tiles, hipStream_t stream)
 {
-    PlanesArgs args;
-    args.x = x;
-    args.nvar = nvar;
-    args.n = n;
-    args.ldx = ldx;
-    args.planes = planes;
-    args.flags = flags;
-    args.nvb = nvb;
-    args.fstride = fstride;
-    args.ngroups = seg * KTG;
+    const int64_t nvb = args.a.nvb + args.b.nvb;
+    args.ngroups = tiles * KTG;
     args.tile_begin = begin;
     args.ntiles = tiles;
     // tiles per workgroup: as many as leave about four workgroups per CU
@@ -636,10 +646,12 @@ hipError_t launch_kendall(const float *a, int64_t na, int64_t lda, const float *
         uint8_t *fb = same ? fa : reinterpret_cast<uint8_t *>(ws + k.off_fb);
         count = reinterpret_cast<unsigned long long *>(ws + k.off_count);
         nopair = (unsigned long long)k.tiles * KTG * KGW * 32 - (unsigned long long)n * (n - 1) / 2;
-        // the counts are added to: cleared by a fill kernel, not a memset
-        // node, so that a captured graph replays correctly
-        e = launch_fill(reinterpret_cast<float *>(count), na * nb * 2, 0.0f, stream);
-        if (e != hipSuccess) return e;
+        PlanesArgs planes = {};
+        planes.a = {a, na, lda, pa, fa, k.nvb_a, k.fs_a};
+        if (!same) planes.b = {b, nb, ldb, pb, fb, k.nvb_b, k.fs_b};
+        planes.n = n;
+        planes.count = count;
+        planes.ncount = na * nb;
         KendallArgs args;
         args.pa = pa;
         args.pb = pb;
@@ -655,16 +667,12 @@ hipError_t launch_kendall(const float *a, int64_t na, int64_t lda, const float *
         args.ldc = nb;
         const int64_t ta = (na + KBX - 1) / KBX;
         args.tiles_b = (nb + KBY - 1) / KBY;
-        args.ntiles = same ? ta * (ta + 1) : ta * args.tiles_b;
+        // (self case: the last tile may lie past the last variable)
+        args.ntiles = same ? ta * (ta + 1) - (args.tiles_b < 2 * ta ? 1 : 0) : ta * args.tiles_b;
         for (int64_t begin = 0; begin < k.tiles; begin += k.seg) {
             const int64_t tiles = k.tiles - begin < k.seg ? k.tiles - begin : k.seg;
-            e = launch_planes(a, na, n, lda, pa, fa, k.nvb_a, k.fs_a, tiles, begin, tiles, stream);
-            if (e != hipSuccess) return e;
-            if (!same) {
-                e = launch_planes(b, nb, n, ldb, pb, fb, k.nvb_b, k.fs_b, tiles, begin, tiles,
-                                  stream);
-                if (e != hipSuccess) return e;
-            }
+            if ((e = launch_planes(planes, begin, tiles, stream)) != hipSuccess) return e;
+            planes.ncount = 0;   // cleared by the first segment
             args.ngroups = tiles * KTG;
             // Ranges of groups: two workgroups run on a CU at a time (out of
             // step, so that one's barrier and LDS waits lie under the other's

@@ -259,3 +259,22 @@ def test_kendall_few_variables_with_ties(na, nb, n, kind):
     want, _ = orc.kendall(a, b, nthreads=8)
     got = gt.kendall(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda())
     np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("na", [1, 64, 65, 128, 129, 192, 256, 320, 384, 385])
+def test_kendall_self_last_tile(na):
+    """Self case where the last tile (256 x 128), or some of its 128 x 64 parts,
+    lie past the last variable; the counts are cleared by the planes pass, so a
+    workspace of ones, used twice, gives the same."""
+    import ctypes
+    rng = np.random.default_rng(na)
+    x = rng.standard_normal((na, 70)).astype(np.float32)
+    x[na // 2:, 3] = x[na // 2:, 69]
+    need = ctypes.c_size_t()
+    assert gt.lib().gt_kendall_workspace_size(na, na, 70, 1, ctypes.byref(need)) == 0
+    ws = torch.full((need.value,), 0xFF, dtype=torch.uint8, device="cuda")
+    print("case kendall self last tile na=%d" % na, flush=True)
+    want, _ = orc.kendall(x, x, nthreads=8)
+    xd = torch.from_numpy(x).cuda()
+    for _ in range(2):
+        assert_same(gt.kendall(xd, workspace=ws).cpu().numpy(), want)
