@@ -1203,35 +1203,35 @@ void launch_mds_small(const MdsArgs &args, bool grad, hipStream_t stream)
 
 }  // namespace
 
-int64_t mds_partials_count(int64_t n, int64_t q)
+int64_t mds_partials_count(int64_t n, int64_t q, bool lean)
 {
-    if (mds_small_applies(n, q)) return mds_tiles(n);
+    if (!lean && mds_small_applies(n, q)) return mds_tiles(n);
     return (n + BI - 1) / BI * j_splits(n, q);
 }
 
-size_t mds_workspace_bytes(int64_t n, int64_t q)
-{
-    if (mds_small_applies(n, q)) return mds_slice_bytes(n, q, mds_pass_blocks(n, q));
-    return sweep_workspace_bytes(n, q);
-}
-
-size_t backward_workspace_bytes(int op, int64_t n, int64_t k)
-{
-    if (n < 2 || k < 1) return 0;
-    if (gradient_applies(op, n, k)) return gradient_plan(n, k).bytes;
-    return sweep_workspace_bytes(n, k);
-}
-
-size_t sweep_workspace_bytes(int64_t n, int64_t k)
+static size_t sweep_workspace_bytes(int64_t n, int64_t k)
 {
     if (n < 2 || k < 1) return 0;
     const int js = j_splits(n, k);
     return js > 1 ? (size_t)js * (size_t)n * (size_t)k * sizeof(float) : 0;
 }
 
+size_t mds_workspace_bytes(int64_t n, int64_t q, bool lean)
+{
+    if (!lean && mds_small_applies(n, q)) return mds_slice_bytes(n, q, mds_pass_blocks(n, q));
+    return sweep_workspace_bytes(n, q);
+}
+
+size_t backward_workspace_bytes(int op, int64_t n, int64_t k, bool lean)
+{
+    if (n < 2 || k < 1) return 0;
+    if (!lean && gradient_applies(op, n, k)) return gradient_plan(n, k).bytes;
+    return sweep_workspace_bytes(n, k);
+}
+
 hipError_t launch_backward(int op, const float *x, int64_t n, int64_t k, int64_t ldx, float p,
                            const float *g_packed, float *dx, int64_t lddx, float *workspace,
-                           hipStream_t stream)
+                           bool lean, hipStream_t stream)
 {
     if (n <= 0 || k <= 0) return hipSuccess;
     BwArgs args;
@@ -1247,16 +1247,16 @@ hipError_t launch_backward(int op, const float *x, int64_t n, int64_t k, int64_t
     args.p = p;
     args.pm1 = p - 1.0f;
     args.left = nullptr;
-    if (gradient_applies(op, n, k)) return launch_gradient(args, workspace, stream);
+    if (!lean && gradient_applies(op, n, k)) return launch_gradient(args, workspace, stream);
     const int bop = (op == OP_EUCLID) ? BW_EUCLID : (op == OP_MINK3) ? BW_MINK3 : BW_MINKP;
     return launch_mode<MODE_GRAD>(bop, args, stream);
 }
 
 hipError_t launch_mds(const float *y, int64_t n, int64_t q, int64_t ldy, const float *delta,
                       float *dy, int64_t lddy, double *stress, double *partials, float *workspace,
-                      hipStream_t stream)
+                      bool lean, hipStream_t stream)
 {
-    if (mds_small_applies(n, q)) {
+    if (!lean && mds_small_applies(n, q)) {
         MdsArgs ma;
         ma.y = y;
         ma.n = n;
@@ -1307,7 +1307,7 @@ hipError_t launch_mds(const float *y, int64_t n, int64_t q, int64_t ldy, const f
     hipError_t e = launch_mode<MODE_MDS>(BW_EUCLID, args, stream);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, stream, partials,
-                       mds_partials_count(n, q), stress);
+                       mds_partials_count(n, q, lean), stress);
     return hipGetLastError();
 }
 

@@ -259,6 +259,15 @@ struct Scratch {
         return GT_OK;
     }
 
+    // `bytes`, or where there is no room for them `less`.
+    int acquire_either(size_t bytes, size_t less, bool &took_less, hipStream_t s)
+    {
+        int r = acquire(bytes, s);
+        took_less = r == GT_ERR_ALLOC && less < bytes;
+        if (took_less && (r = acquire(less, s)) == GT_OK) g_err[0] = '\0';
+        return r;
+    }
+
     int release()
     {
         if (!ptr) return GT_OK;
@@ -1161,10 +1170,12 @@ int gt_dist_backward(const float *x, int64_t n, int64_t k, int64_t ldx, int meth
     else if (p == 3.0f) op = gt::OP_MINK3;
     // partial dX slices when the row blocks are few (stream-ordered scratch)
     Scratch ws;
-    int s = ws.acquire(gt::backward_workspace_bytes(op, n, k), hs);
+    bool lean = false;
+    int s = ws.acquire_either(gt::backward_workspace_bytes(op, n, k, false),
+                              gt::backward_workspace_bytes(op, n, k, true), lean, hs);
     if (s != GT_OK) return s;
     const hipError_t e = gt::launch_backward(op, x, n, k, ldx, p, g_packed, dx, lddx,
-                                             static_cast<float *>(ws.ptr), hs);
+                                             static_cast<float *>(ws.ptr), lean, hs);
     const int r = ws.release();
     if (e != hipSuccess) return hip_fail(e, "gt_dist_backward");
     return r;
@@ -1178,11 +1189,15 @@ int gt_mds_stress(const float *y, int64_t n, int64_t q, int64_t ldy, const float
     if (stress_dev == nullptr) return fail(GT_ERR_INVALID, "null stress pointer");
     if (n > 1 && (y == nullptr || delta_packed == nullptr)) return fail(GT_ERR_INVALID, "null pointer");
     hipStream_t hs = static_cast<hipStream_t>(stream);
-    const int64_t parts = n > 1 ? gt::mds_partials_count(n, q) : 1;
-    const size_t pbytes = round_up((size_t)parts * sizeof(double), 256);
-    const size_t dbytes = (n > 1 && dy != nullptr) ? gt::mds_workspace_bytes(n, q) : 0;
+    size_t pbytes[2], dbytes[2];   // of both forms
+    for (int form = 0; form < 2; ++form) {
+        const int64_t parts = n > 1 ? gt::mds_partials_count(n, q, form == 1) : 1;
+        pbytes[form] = round_up((size_t)parts * sizeof(double), 256);
+        dbytes[form] = (n > 1 && dy != nullptr) ? gt::mds_workspace_bytes(n, q, form == 1) : 0;
+    }
     Scratch ws;
-    int s = ws.acquire(pbytes + dbytes, hs);
+    bool lean = false;
+    int s = ws.acquire_either(pbytes[0] + dbytes[0], pbytes[1] + dbytes[1], lean, hs);
     if (s != GT_OK) return s;
     hipError_t e;
     if (n < 2) {
@@ -1192,9 +1207,9 @@ int gt_mds_stress(const float *y, int64_t n, int64_t q, int64_t ldy, const float
     } else {
         e = gt::launch_mds(y, n, q, ldy, delta_packed, dy, lddy, stress_dev,
                            static_cast<double *>(ws.ptr),
-                           dbytes ? reinterpret_cast<float *>(static_cast<char *>(ws.ptr) + pbytes)
-                                  : nullptr,
-                           hs);
+                           dbytes[lean] ? reinterpret_cast<float *>(static_cast<char *>(ws.ptr) + pbytes[lean])
+                                        : nullptr,
+                           lean, hs);
     }
     const int r = ws.release();
     if (e != hipSuccess) return hip_fail(e, "gt_mds_stress");

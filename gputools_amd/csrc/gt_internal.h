@@ -74,19 +74,19 @@ hipError_t launch_gram(int precision, int layout, const float *x, int64_t n, int
 // Backward (dL/dX) and fused MDS stress.  op: OP_EUCLID, OP_MINK3 or OP_MINKP.
 // workspace: backward_workspace_bytes(op, n, k) (partial dX slices when the j
 // blocks are split over workgroups, and the matrix-core form's operands; 0
-// otherwise); the sweep alone takes sweep_workspace_bytes.
-size_t backward_workspace_bytes(int op, int64_t n, int64_t k);
-size_t sweep_workspace_bytes(int64_t n, int64_t k);
-size_t mds_workspace_bytes(int64_t n, int64_t q);
+// otherwise).
+// lean: the sweep over both owners of a pair whatever the size, in at most 16
+// slices of dX, for where there is no room for the faster form's workspace.
+size_t backward_workspace_bytes(int op, int64_t n, int64_t k, bool lean);
+size_t mds_workspace_bytes(int64_t n, int64_t q, bool lean);
 hipError_t launch_backward(int op, const float *x, int64_t n, int64_t k, int64_t ldx,
                            float p, const float *g_packed, float *dx, int64_t lddx,
-                           float *workspace, hipStream_t stream);
-// partials: mds_partials_count(n, q) doubles; workspace (with dy):
-// mds_workspace_bytes.
-int64_t mds_partials_count(int64_t n, int64_t q);
+                           float *workspace, bool lean, hipStream_t stream);
+// partials: mds_partials_count doubles; workspace (with dy): mds_workspace_bytes.
+int64_t mds_partials_count(int64_t n, int64_t q, bool lean);
 hipError_t launch_mds(const float *y, int64_t n, int64_t q, int64_t ldy,
                       const float *delta, float *dy, int64_t lddy, double *stress,
-                      double *partials, float *workspace, hipStream_t stream);
+                      double *partials, float *workspace, bool lean, hipStream_t stream);
 
 // Batched persistent kernel.  tile: 1..3 (32, 64, 128 pairs per side).
 int batched_tile_side(int tile);

@@ -311,3 +311,38 @@ def test_pairwise_without_room_for_its_workspace(monkeypatch):
     with pytest.raises(torch.cuda.OutOfMemoryError):
         gt.pmcc(ad.nan_to_num_(), bd.nan_to_num_(), precision="bf16x3", out=res)   # needs its workspace
     assert np.max(np.abs(got - corr)) <= 1e-5
+
+
+def test_gradient_and_mds_without_room_for_the_faster_form():
+    """The matrix-core gradient and the MDS form that visits each pair once take
+    more scratch than the sweep over both owners of a pair: where there is no
+    room for it, the sweep runs."""
+    from gputools_amd.autograd import _mds
+    rng = np.random.default_rng(60)
+    n, k = 2000, 64
+    x = rng.standard_normal((n, k)).astype(np.float32)
+    g = rng.standard_normal(n * (n - 1) // 2).astype(np.float32)
+    xd, gd = torch.from_numpy(x).cuda(), torch.from_numpy(g).cuda()
+    m = 4000
+    y = rng.standard_normal((m, 2)).astype(np.float32)
+    delta = (rng.random(m * (m - 1) // 2) * 3.0).astype(np.float32)
+    yd, dd = torch.from_numpy(y).cuda(), torch.from_numpy(delta).cuda()
+    usual, (s_usual, dy_usual) = gt.dist_backward(xd, gd), _mds(yd, dd, True)
+
+    def limited(limit, call):
+        os.environ["GT_FAIL_ALLOC_ABOVE"] = str(limit)
+        try:
+            return call()
+        finally:
+            del os.environ["GT_FAIL_ALLOC_ABOVE"]
+
+    dx = limited(9000000, lambda: gt.dist_backward(xd, gd))        # 9.8 MB, sweep 8.2
+    s, dy = limited(1000000, lambda: _mds(yd, dd, True))           # 1.5 MB, sweep 0.5
+    assert not torch.equal(dx, usual) and not torch.equal(dy, dy_usual)
+    for got, want in ((dx, orc.dist_backward(x, g.astype(np.float64), "euclidean")),
+                      (dy, orc.mds_stress(y, delta.astype(np.float64))[1])):
+        got = got.cpu().numpy().astype(np.float64)
+        assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    assert abs(s.item() - s_usual.item()) <= 1e-6 * s_usual.item()
+    with pytest.raises(gt.GputoolsError, match="ALLOC"):           # nor for the sweep
+        limited(1000, lambda: gt.dist_backward(xd, gd))
