@@ -348,7 +348,14 @@ constexpr int GTL = 36;                // row of a wave's transposed block of G
 constexpr int GOWN = 512 + 1024;       // floats of a wave's region: G, or near pairs and distances
 static_assert(32 * GTL <= GOWN, "transpose region");
 constexpr float GRAD_W_MIN = 0x1p-100f;
-constexpr int GRAD_NEAR_MAX = 160;     // near pairs of a 32 x 32 block, on average
+constexpr int GRAD_NEAR_MAX = 256;     // near pairs of a 32 x 32 block, on average
+constexpr int GRAD_SAMPLES = 512;      // blocks of 32 x 32 pairs; a thread of gradient_kernel each
+static_assert(GRAD_SAMPLES == GW * 64, "samples");
+
+__device__ __forceinline__ uint16_t *gradient_samples(uint8_t *left)
+{
+    return reinterpret_cast<uint16_t *>(left) - GRAD_SAMPLES;
+}
 
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));   // rows start anywhere
 
@@ -372,28 +379,72 @@ struct GradArgs {
     float *dx;
     int64_t lddx;
     float *dxp;                        // gridDim.y > 1: partial dX slices
-    uint8_t *left;                     // per BI rows: 1 = left to backward_kernel
+    // per BI rows: 1 = left to backward_kernel; before them the near pairs of the
+    // blocks that gradient_sample visits
+    uint8_t *left;
     int64_t jblocks;                   // blocks of 32 rows j, per workgroup
     float tau;
 };
 
+// Near pairs of sample s, a block of 32 x 32 pairs, from the first terms alone: the
+// rows i of the samples are spread over all rows, and so are the rows j of the
+// even ones; those of the odd ones follow the rows i, which shows clusters that
+// lie in order.
+__device__ __forceinline__ void gradient_sample(const GradArgs &args, int s, int nch)
+{
+    typedef Split<SPLIT_BF16> S;
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int64_t n = args.n, nblk = operand_rows(n) / 32;
+    const int64_t ib = s * nblk / GRAD_SAMPLES;
+    const int64_t jb = (ib + (s & 1 ? 1 : 1 + s * (int64_t)617 % nblk)) % nblk;
+    const unsigned short *const a = args.terms + jb * nch * 3 * OPERAND_VALUES + lane * 8;
+    const unsigned short *const b = args.terms + ib * nch * 3 * OPERAND_VALUES + lane * 8;
+    const int64_t i = ib * 32 + (lane & 31);
+    const float ni = args.norms[i < n ? i : n - 1];
+    float nj[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int64_t j = jb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        nj[r] = args.norms[j < n ? j : n - 1];
+    }
+    f32x16_t w;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) w[r] = 0.0f;
+#pragma unroll 8
+    for (int c = 0; c < nch; ++c)
+        w = S::mfma(*reinterpret_cast<const bf16x8_t *>(a + c * 3 * OPERAND_VALUES),
+                    *reinterpret_cast<const bf16x8_t *>(b + c * 3 * OPERAND_VALUES), w);
+    int near = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int64_t j = jb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        const float ss = ni + nj[r], d2 = fmaf(-2.0f, w[r], ss);
+        const bool ok = d2 >= fmaf(args.tau, ss, GRAM_SQRT_MIN) && d2 < 0x1p127f;
+        near += __popcll(__builtin_amdgcn_ballot_w64(i < n && j < n && i != j && !ok));
+    }
+    if (lane == 0) gradient_samples(args.left)[s] = (uint16_t)near;
+}
+
 // B operands of the second product: block jb (32 rows j), feature block cb (32
 // features), step s (sixteen j: 16 s + 8 p + 4 h + e, p < 2, e < 4), term t at
 // (((jb * ncb + cb) * 2 + s) * 3 + t) * OPERAND_VALUES, lane 32 h + c.  Also
-// clears `left`.
-__global__ __launch_bounds__(256) void gradient_terms_kernel(const float *__restrict__ x, int64_t n,
-                                                             int64_t k, int64_t ldx, int64_t ncb,
-                                                             const float *__restrict__ center,
-                                                             unsigned short *__restrict__ tterms,
-                                                             uint8_t *__restrict__ left)
+// clears `left`, and the first workgroups count the samples.
+__global__ __launch_bounds__(256) void gradient_terms_kernel(GradArgs args, int64_t ncb,
+                                                             unsigned short *__restrict__ tterms)
 {
+    constexpr int SAMPLERS = GRAD_SAMPLES / 4;   // workgroups
+    if (blockIdx.x < SAMPLERS) {
+        gradient_sample(args, (int)blockIdx.x * 4 + (threadIdx.x >> 6), (int)ncb * 2);
+        return;
+    }
     const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int64_t n = args.n, k = args.k, ldx = args.ldx;
+    const int64_t wg = (int64_t)blockIdx.x - SAMPLERS, wgs = (int64_t)gridDim.x - SAMPLERS;
+    const float *const __restrict__ x = args.x, *const __restrict__ center = args.center;
     const int64_t nleft = (n + BI - 1) / BI;
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < nleft; t += (int64_t)gridDim.x * 256)
-        left[t] = 0;
+    for (int64_t t = wg * 256 + threadIdx.x; t < nleft; t += wgs * 256) args.left[t] = 0;
     const int64_t blocks = operand_rows(n) / 32 * ncb * 2;
-    for (int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); blk < blocks;
-         blk += (int64_t)gridDim.x * 4) {
+    for (int64_t blk = wg * 4 + (threadIdx.x >> 6); blk < blocks; blk += wgs * 4) {
         const int64_t s = blk & 1, cb = (blk >> 1) % ncb, jb = (blk >> 1) / ncb;
         const int64_t c = cb * 32 + (lane & 31);
         unsigned short t[8][3];
@@ -426,9 +477,16 @@ __global__ __launch_bounds__(256) void gradient_terms_kernel(const float *__rest
 // VALU), 1.1 ms here; the relative error of dX against FP64 8.2e-7 -> 4.0e-7.
 // A pair with d^2 < tau (||x_i||^2 + ||x_j||^2), or a d^2 that is not a normal
 // number, is recomputed from FP32 differences.  Rows with a weight that is not
-// finite or too small for three BF16 terms, or with many near pairs, are left to
-// backward_kernel (8000 x 128 in 32, 8 and 4 clusters: 0.52, 0.90 and 1.35 ms
-// with every near pair taken here, 1.28 ms for the sweep).
+// finite or too small for three BF16 terms, or (in the blocks that one wave has
+// seen) more near pairs than GRAD_NEAR_MAX, are left to backward_kernel, and so are
+// all rows where the samples show many near pairs: more than 144 of 1024 (80 up
+// to 32 features, where the sweep is faster).  In ms, here and in the sweep, with
+// 64 and 128 of 1024 near: 16384 x 128 2.51, 3.42 and 5.19; 3000 x 48 0.122,
+// 0.141 and 0.175; 16384 x 32 1.29, 1.63 and 1.73; 6000 x 32 0.28, 0.42 and 0.26.
+// Left without samples, by each wave once it had seen too many, a row was found
+// after other waves had done their work on it: 12000 x 128 with one dominant
+// direction 5.15 ms, in 8 clusters that lie in order 4.20, with the samples 3.24
+// and 3.22, the sweep 3.20.
 template <int NC>
 __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
 {
@@ -447,6 +505,25 @@ __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
     const int64_t nblk = operand_rows(n) / 32;
     const int64_t jb0 = (int64_t)blockIdx.y * args.jblocks;
     const int64_t jb1 = jb0 + args.jblocks < nblk ? jb0 + args.jblocks : nblk;
+    {
+        // many near pairs, or clusters in order: all rows are left
+        const int v = gradient_samples(args.left)[tid];
+        const int ordered = __syncthreads_count((tid & 1) && v > 256);
+        int sum = tid & 1 ? 0 : v;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+        int *const part = reinterpret_cast<int *>(smem);
+        if (lane == 0) part[wave] = sum;
+        __syncthreads();
+        sum = 0;
+        for (int w = 0; w < GW; ++w) sum += part[w];
+        __syncthreads();   // the region is free again
+        if (sum > (NC == 2 ? 80 : 144) * (GRAD_SAMPLES / 2) || ordered > GRAD_SAMPLES / 8) {
+            if (blockIdx.y == 0 && tid < GROWS / BI && (int64_t)blockIdx.x * GROWS + tid * BI < n)
+                args.left[(int64_t)blockIdx.x * (GROWS / BI) + tid] = 1;
+            return;
+        }
+    }
     bool idle = i0 >= n;                              // only helps to load
     const int64_t i = i0 + col;
     const int64_t ic = i < n ? i : n - 1;
@@ -1016,10 +1093,11 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 // its rule (5 features, 4000 points: 206 us, and 115 for the sweep); with few
 // points the pre-passes cost more than they save (times in us, sweep and here:
 // 1000 x 96 50 and 55, 2000 x 96 88 and 70; 2000 x 32 41 and 58, 4000 x 32 122
-// and 77).  A sweep that needs no workspace can be captured; it stays.
+// and 77; at 3000 x 32 95 and 74, but 130 where all rows are left).  A sweep that
+// needs no workspace can be captured; it stays.
 bool gradient_applies(int op, int64_t n, int64_t k)
 {
-    return op == OP_EUCLID && k <= 128 && ((k > 32 && n >= 1500) || (k >= 16 && n >= 3000)) &&
+    return op == OP_EUCLID && k <= 128 && ((k > 32 && n >= 1500) || (k >= 16 && n >= 4000)) &&
            j_splits(n, k) > 1;
 }
 
@@ -1039,6 +1117,7 @@ GradPlan gradient_plan(int64_t n, int64_t k)
     size_t p = align256(gram_workspace_bytes(n, k, 1));
     g.off_tterms = p;
     p += (size_t)operand_rows(n) * (size_t)g.kp * 3 * sizeof(unsigned short);
+    p += GRAD_SAMPLES * sizeof(uint16_t);
     g.off_left = p;
     p += align256((size_t)nblk);
     g.off_slices = p;
@@ -1128,8 +1207,8 @@ hipError_t launch_gradient(BwArgs &args, void *workspace, hipStream_t stream)
     ga.tau = fmaxf(gram_tau(1, args.k), 0.25f);
     int64_t blocks = (operand_rows(args.n) / 32 * g.ncb * 2 + 3) / 4;
     if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(gradient_terms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, args.x, args.n,
-                       args.k, args.ldx, g.ncb, prep.center, const_cast<unsigned short *>(ga.tterms), ga.left);
+    hipLaunchKernelGGL(gradient_terms_kernel, dim3((unsigned)(GRAD_SAMPLES / 4 + blocks)), dim3(256), 0, stream, ga,
+                       g.ncb, const_cast<unsigned short *>(ga.tterms));
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const dim3 grid((unsigned)((args.n + GROWS - 1) / GROWS), (unsigned)g.slices);
     switch (g.ncb) {

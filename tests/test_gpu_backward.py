@@ -269,3 +269,50 @@ def test_mds_scratch_is_bounded(n, q):
     want_s, want = _mds_reference(y, delta)
     assert abs(s.item() - want_s) <= 1e-6 * want_s
     assert_grad_close(dy.cpu().numpy(), want.cpu().numpy())
+
+
+@pytest.mark.parametrize("data", ["dominant", "ordered", "tiny"])
+def test_gradient_of_many_near_pairs_costs_the_sweep(data):
+    """Data whose pairs are mostly near by the rule of the matrix-core form (one
+    dominant direction; clusters that lie in order; values whose squares are
+    denormal) is left to the sweep as a whole, before work is done on it: the
+    same values as the sweep's, in about its time."""
+    import os
+    n, k = 6000, 64
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.randn((n, k), generator=gen, device="cuda")
+    if data == "dominant":
+        x[:, 0] *= 40.0
+    elif data == "ordered":
+        x = x * 1e-2 + torch.randn((8, k), generator=gen, device="cuda")[torch.arange(n, device="cuda") * 8 // n]
+    else:
+        x *= 1e-17
+    g = torch.randn(n * (n - 1) // 2, generator=gen, device="cuda")
+    print("case gradient of near pairs %s" % data, flush=True)
+
+    def timed():
+        times = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(4):
+                dx = gt.dist_backward(x, g)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        return dx, min(times)
+
+    dx, usual = timed()
+    os.environ["GT_FAIL_ALLOC_ABOVE"] = "26000000"   # the sweep's 25 MB, not the operands beside it
+    try:
+        want, sweep = timed()
+    finally:
+        del os.environ["GT_FAIL_ALLOC_ABOVE"]
+    assert torch.equal(dx, want)
+    assert usual <= 1.4 * sweep, (usual, sweep)      # 1.05; 1.6 to 1.8 without the samples
+
+
+@pytest.mark.parametrize("n,k,data", [(4000, 16, "uniform"), (4009, 31, "clusters"), (4001, 32, "duplicates")])
+def test_matrix_core_gradient_of_few_features(n, k, data):
+    """The same up to 32 features, where the form begins at 4000 points."""
+    test_matrix_core_gradient(n, k, data)
