@@ -2,7 +2,11 @@
 
 ``pdist(x, method, p)`` returns the packed distance vector (R 'dist' order)
 and differentiates through ``gt_dist_backward`` (euclidean, minkowski p >= 1),
-which recomputes distances tile by tile instead of storing them.
+which recomputes distances tile by tile instead of storing them.  ``precision``
+is the forward's.  The euclidean backward of many points with 16 to 128 features
+sums products of values split into three BF16 terms: its error is 0.4 to 0.8 of
+FP32 sums' for dense upstream gradients, up to 1.7 times it where few near pairs
+make up a row.
 
 ``mds_stress(y, delta)`` is the metric-MDS objective
 S(Y) = sum_{i<j} (||y_i - y_j|| - delta_ij)^2 with delta packed; forward and

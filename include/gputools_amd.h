@@ -309,9 +309,16 @@ int gt_hclust_host(const float *d_host, int64_t n, int64_t ldd, int method, floa
 int gt_hclust_format(int64_t len, const int *sub, const int *sup, int *merge, int *order);
 
 /* Backward of the packed distance vector: dX (n x k, row stride lddx) =
- * sum_j G_ij * d(d_ij)/d(x_i) for euclidean (any precision flag is ignored:
- * FP32) and minkowski (p >= 1).  G is packed dL/dD.  D is recomputed
- * tile-by-tile and never stored.  Pairs with d_ij == 0 contribute 0. */
+ * sum_j G_ij * d(d_ij)/d(x_i) for euclidean and minkowski (p >= 1).  G is
+ * packed dL/dD.  D is recomputed tile-by-tile and never stored.  Pairs with
+ * d_ij == 0 contribute 0.
+ * FP32 throughout, except for euclidean with 16 to 128 features and many points
+ * (from 1500 on, 4000 up to 32 features): there D and dX come from products of
+ * values split into three BF16 terms (24 bits), summed in FP32, and pairs closer
+ * than half the root of their squared norms' sum from FP32 differences.  The
+ * error against FP64 is 0.4 to 0.8 of the FP32 sweep's where most of G is not
+ * zero, and up to 1.7 times it where a few near pairs make up a row (both lose
+ * to the cancellation of near points there). */
 int gt_dist_backward(const float *x, int64_t n, int64_t k, int64_t ldx, int method,
                      float p, const float *g_packed, float *dx, int64_t lddx,
                      void *stream);

@@ -316,3 +316,44 @@ def test_gradient_of_many_near_pairs_costs_the_sweep(data):
 def test_matrix_core_gradient_of_few_features(n, k, data):
     """The same up to 32 features, where the form begins at 4000 points."""
     test_matrix_core_gradient(n, k, data)
+
+
+def test_gradient_error_with_dominant_directions():
+    """Three features of five times the others' spread, and upstream gradients at
+    the nearest pairs alone: a distance is then up to half the size of the norms
+    it comes from in the matrix-core form, and few terms make up a row.  Rows of
+    dX are not much further from FP64 than the sweep's, which takes differences."""
+    import os
+    n, k = 4000, 128
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn((n, k), generator=gen, device="cuda")
+    x[:, :3] *= 5.0
+    g = torch.randn(n * (n - 1) // 2, generator=gen, device="cuda")
+    d = gt.dist(x)
+    g *= d <= torch.quantile(d[torch.randint(d.numel(), (1000000,), generator=gen, device="cuda")], 0.01)
+    print("case gradient of near pairs alone", flush=True)
+    dx = gt.dist_backward(x, g)
+    os.environ["GT_FAIL_ALLOC_ABOVE"] = "33000000"   # the sweep's 32.8 MB, not the operands beside it
+    try:
+        sweep = gt.dist_backward(x, g)
+    finally:
+        del os.environ["GT_FAIL_ALLOC_ABOVE"]
+    assert not torch.equal(dx, sweep)
+    xd = x.double()
+    w = torch.zeros((n, n), dtype=torch.float64, device="cuda")
+    w[torch.ones((n, n), dtype=torch.bool, device="cuda").triu_(1)] = g.double()
+    w += w.T.clone()
+    d2 = torch.zeros_like(w)
+    for f in range(k):
+        d2 += (xd[:, f, None] - xd[None, :, f]).square_()
+    w /= d2.sqrt_().fill_diagonal_(1.0)
+    want = torch.empty_like(xd)
+    for f in range(k):
+        want[:, f] = (w * (xd[:, f, None] - xd[None, :, f])).sum(1)
+
+    def worst_row(got):
+        some = want.norm(dim=1) > 0          # (rows without a near pair are zero)
+        return ((got.double() - want).norm(dim=1) / want.norm(dim=1))[some].max().item()
+
+    ours, theirs = worst_row(dx), worst_row(sweep)
+    assert ours <= 1.8 * theirs, (ours, theirs)
