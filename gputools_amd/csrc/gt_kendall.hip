@@ -152,17 +152,20 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
             xi[vv] = x[v * ldx + i] + 0.0f;
         }
     };
-    // the three comparisons of 32 columns, column u in bit u, which lane u holds
-    // (scalar loads here would be waited for one after the other)
-    auto exact = [&](float a, float xl, uint32_t &gt, uint32_t &lt, uint32_t &eq) {
+    // the three comparisons of up to 32 columns, column u in bit u, which lane u
+    // holds (scalar loads here would be waited for one after the other), eight at
+    // a time: few samples have one tile of few columns
+    auto exact = [&](float a, float xl, int cols, uint32_t &gt, uint32_t &lt, uint32_t &eq) {
         gt = lt = eq = 0u;
-#pragma unroll 8
-        for (int u = 31; u >= 0; --u) {
-            const float b = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(xl), u));
-            gt = (gt << 1) | (b > a ? 1u : 0u);
-            lt = (lt << 1) | (b < a ? 1u : 0u);
-            eq = (eq << 1) | (b == a ? 1u : 0u);
-        }
+#pragma unroll 1
+        for (int u0 = (cols - 1) & ~7; u0 >= 0; u0 -= 8)
+#pragma unroll
+            for (int u = u0 + 7; u >= u0; --u) {
+                const float b = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(xl), u));
+                gt = (gt << 1) | (b > a ? 1u : 0u);
+                lt = (lt << 1) | (b < a ? 1u : 0u);
+                eq = (eq << 1) | (b == a ? 1u : 0u);
+            }
     };
     load_rows();
     if (tid == 0) special[0] = 0u;
@@ -192,21 +195,15 @@ __global__ __launch_bounds__(256) void kendall_planes_kernel(PlanesArgs args)
                     w = __builtin_amdgcn_alignbit(w, d, 31);
                     m = d < m ? d : m;
                 }
-            } else {
-                // the columns from cols on repeat the last one
-#pragma unroll
-                for (int u = 31; u >= 0; --u) {
-                    const uint32_t d = __float_as_uint(
-                        xi[vv] - __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(xl), u)));
-                    w = __builtin_amdgcn_alignbit(w, d, 31);
-                    m = d < m ? d : m;
-                }
             }
             const bool odd = !(fabsf(xi[vv]) < INFINITY) || !(fabsf(xl) < INFINITY);
             const unsigned long long oddw = __builtin_amdgcn_ballot_w64(odd);
-            if (__builtin_amdgcn_ballot_w64(m == 0u) | oddw) {
+            // (a tile of fewer columns, the only one of few samples, is compared at
+            // once: 300 variables x 7 samples 15.8 us with the differences first,
+            // which took each x_i - x_i for a tie, 8.1 so)
+            if (cols < 32 || (__builtin_amdgcn_ballot_w64(m == 0u) | oddw)) {
                 uint32_t lt, eq;
-                exact(xi[vv], xl, w, lt, eq);
+                exact(xi[vv], xl, cols, w, lt, eq);
                 ltw[vv] = lt;
                 eqw[vv] = eq;
                 compared |= 1u << vv;

@@ -278,3 +278,10 @@ def test_kendall_self_last_tile(na):
     xd = torch.from_numpy(x).cuda()
     for _ in range(2):
         assert_same(gt.kendall(xd, workspace=ws).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n", [3, 8, 9, 24, 31])
+@pytest.mark.parametrize("kind", ["ordinal", "one_tie", "holes"])
+def test_kendall_few_samples(n, kind):
+    """One tile of fewer than 32 columns, compared eight at a time."""
+    test_kendall_few_variables_with_ties(70, 33, n, kind)
