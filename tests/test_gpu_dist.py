@@ -516,3 +516,30 @@ def test_binary_packed_feature_edges(n, k):
         x[3, ::5] = -np.inf
     got = gt.dist(torch.from_numpy(x).cuda(), "binary").cpu().numpy()
     np.testing.assert_array_equal(got, orc.dist(x, "binary").astype(np.float32))
+
+
+@pytest.mark.parametrize("n", [11264, 11265, 11700])
+@pytest.mark.parametrize("k", [960, 961])
+def test_binary_large_tiles_at_the_table_limit(n, k):
+    """960 features are the most that the packed matrix-core tiles divide with
+    the reciprocal table (four entries per byte of two features, below 2048);
+    961 take v_rcp_f32.  Up to 11264 points run the 128 x 128 tiles, more the
+    128 x 256 ones.  Every element written (the output starts as NaN); tile-edge
+    columns and random pairs bit-exact."""
+    x = wl.bernoulli(n, k, seed=n + k)
+    x[7] = 0.0
+    print("case binary large tiles", n, k, flush=True)
+    got = torch.full((n * (n - 1) // 2,), float("nan"), device="cuda")
+    gt.dist(dev(x), "binary", out=got)
+    torch.cuda.synchronize()
+    assert not torch.isnan(got).any()
+    rng = np.random.default_rng(n + k)
+    edge = [0, 7, 127, 128, 255, 256, 11135, 11136, n - 2]
+    jj = np.concatenate([np.repeat(edge, n), rng.integers(0, n, 100000)])
+    ii = np.concatenate([np.tile(np.arange(n), len(edge)), rng.integers(0, n, 100000)])
+    keep = ii != jj
+    ii, jj = ii[keep], jj[keep]
+    hi, lo = np.maximum(ii, jj), np.minimum(ii, jj)
+    idx = lo * n - lo * (lo + 1) // 2 + (hi - lo - 1)
+    vals = got[torch.from_numpy(idx).cuda()].cpu().numpy()
+    np.testing.assert_array_equal(vals, orc.dist_pairs(x, hi, lo, "binary").astype(np.float32))
