@@ -255,3 +255,41 @@ def test_hclust_one_workgroup_limit(n):
     for method in ("single", "average", "ward"):
         print("case hclust one workgroup n=%d %s" % (n, method), flush=True)
         assert_same(d, method)
+
+
+@pytest.mark.parametrize("n", [16385, 20000, 32767, 32768, 32769])
+def test_hclust_many_points_single_linkage(n):
+    """Up to 32768 points the workgroups of one XCD share the rounds (their keys
+    of 15 bits hold the last index, and the LDS is nearly full), from 32769 on
+    one workgroup works alone.  Heights are the minimum spanning tree's weights,
+    and the meeting point shows that the workgroups did meet."""
+    from test_gpu_failure import _cluster_matrix, _hclust_chosen
+    print("case hclust many points n=%d" % n, flush=True)
+    d = _cluster_matrix(n, 69)
+    best, inf = d[0].clone(), torch.full((n,), float("inf"), device="cuda")
+    in_tree = torch.zeros(n, dtype=torch.bool, device="cuda")
+    in_tree[0] = True
+    want = torch.empty(n - 1, device="cuda")
+    for t in range(n - 1):
+        cand = torch.where(in_tree, inf, best)
+        j = cand.argmin().reshape(1)
+        want[t:t + 1] = cand[j]
+        in_tree[j] = True
+        best = torch.minimum(best, d[j][0])
+    (sub, sup, h), chosen = _hclust_chosen(d, "single")
+    assert (1 <= chosen <= 16) == (n <= 32768)
+    assert (sub < sup).all() and np.array_equal(np.sort(sub), np.setdiff1d(np.arange(n), sup[-1:]))
+    np.testing.assert_array_equal(h, np.sort(want.cpu().numpy()))
+
+
+@pytest.mark.parametrize("n,method", [(16385, "ward"), (20000, "flexible group"), (32768, "average")])
+def test_hclust_many_points_equal_one_workgroup(n, method):
+    """The shared rounds against one workgroup's, bit for bit."""
+    from test_gpu_failure import _cluster_matrix, _hclust_chosen
+    print("case hclust many points %s n=%d" % (method, n), flush=True)
+    d = _cluster_matrix(n, 70)
+    got, chosen = _hclust_chosen(d.clone(), method)
+    assert 1 <= chosen <= 16
+    want = gt.hclust(d, method, state="global")
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g.view(np.uint32), w.cpu().numpy().view(np.uint32))
