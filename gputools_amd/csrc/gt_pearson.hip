@@ -276,12 +276,13 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
     }
 
     // ---- main loop: direct global -> LDS loads, MNSTAGE-deep, MFMA products
-    // LDS chunk image: side x, then side y, each 8 blocks of 32 rows, each NT
-    // terms of 1 KB as they lie in memory (gt_mfma.h).  global_load_lds writes
-    // lane l's 16 B at the wave's LDS base + 16 l: wave w moves block w (0-7
-    // side x, 8-15 side y), one term per instruction, and a lane's operand read
-    // is its own 16 B, free of bank conflicts.  Blocks past the last one repeat
-    // it: they only feed pairs that are never stored.
+    // LDS chunk image: side x, then side y, 12 blocks of 32 rows together (8 + 4
+    // where SYM, else 4 + 8), each NT terms of 1 KB as they lie in memory
+    // (gt_mfma.h).  These pieces go to the 8 waves round robin, one per
+    // instruction: global_load_lds writes lane l's 16 B at the wave's LDS base +
+    // 16 l, and a lane's operand read is its own 16 B, free of bank conflicts.
+    // Blocks past the last one repeat it: they only feed pairs that are never
+    // stored.
     // (Row-major terms moved 32 bytes of 32 rows per instruction: 8192 x 1024
     // self, BF16, 643 -> 613 us.)
     typedef __attribute__((address_space(3))) void lds_void_t;
@@ -323,8 +324,7 @@ __global__ __launch_bounds__(MTHREADS, 4) void pmcc_tile_kernel(PmccTileArgs arg
     for (int c = 0; c < nchunks; ++c) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // every wave's part of chunk c is in LDS and every wave finished chunk
-        // c-1, whose stage the next issue overwrites (a bare s_barrier:
-        // __syncthreads() would also drain the later chunks' loads)
+        // c-1, whose stage the next issue overwrites
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (c + MNSTAGE - 1 < nchunks) issue(c + MNSTAGE - 1);

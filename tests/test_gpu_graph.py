@@ -1,7 +1,7 @@
 """gt_dist_ws captured in a HIP graph (torch.cuda.CUDAGraph).
 
 A caller that owns the workspace can capture the whole distance call: the
-packed binary path (byte rows, matrix-core tiles with their staggered start)
+packed binary path (FP4 rows, matrix-core tiles)
 and the split-precision euclidean path (column statistics and centres, the
 split, the norms, the Gram tiles and their exact pass).  The library records
 no memset nodes.  Each graph is replayed several times with eager work
