@@ -360,11 +360,13 @@ int gt_dist_batched(const float *x, const int64_t *x_offsets, const int64_t *siz
  * t-score.  b == NULL (or b == a with the same shape) correlates A with
  * itself: the result is exactly symmetric and half the tiles are computed.
  * use GT_USE_EVERYTHING: precision FP32 (VALU), BF16X3 or FP16X3 (MFMA on
- * standardised variables); GT_USE_PAIRWISE: FP32 only.  The workspace
- * (gt_pmcc_workspace_size, same != 0 for the self case) holds the
- * standardised variables.  For GT_USE_PAIRWISE it is optional: the matrix
- * cores' operands where that form is faster (0 bytes elsewhere); without it
- * the VALU does the work. */
+ * standardised variables; a few long variables run as FP32); GT_USE_PAIRWISE:
+ * FP32 only.  The workspace (gt_pmcc_workspace_size, same != 0 for the self
+ * case) holds the standardised variables.  For GT_USE_PAIRWISE it is optional:
+ * the matrix cores' operands where that form is faster (0 bytes elsewhere),
+ * values and squares in three BF16 terms (24 bits) whose products are summed in
+ * FP32, with an rms error of 0.5 to 1.0 of the VALU form's; without it the VALU
+ * does the work. */
 int gt_pmcc_workspace_size(int use, int precision, int64_t na, int64_t nb, int64_t dim, int same,
                            size_t *bytes);
 int gt_pmcc(int use, int precision, const float *a, int64_t na, int64_t lda, const float *b,
