@@ -388,15 +388,16 @@ struct GradArgs {
 
 // Near pairs of sample s, a block of 32 x 32 pairs, from the first terms alone: the
 // rows i of the samples are spread over all rows, and so are the rows j of the
-// even ones; those of the odd ones follow the rows i, which shows clusters that
-// lie in order.
+// even ones; those of the odd ones are the rows i, which shows near points that
+// lie in order (the eight waves of a workgroup meet such a block one after the
+// other, each while the others wait).
 __device__ __forceinline__ void gradient_sample(const GradArgs &args, int s, int nch)
 {
     typedef Split<SPLIT_BF16> S;
     const int lane = threadIdx.x & 63, h = lane >> 5;
     const int64_t n = args.n, nblk = operand_rows(n) / 32;
     const int64_t ib = s * nblk / GRAD_SAMPLES;
-    const int64_t jb = (ib + (s & 1 ? 1 : 1 + s * (int64_t)617 % nblk)) % nblk;
+    const int64_t jb = s & 1 ? ib : (ib + 1 + s * (int64_t)617 % nblk) % nblk;
     const unsigned short *const a = args.terms + jb * nch * 3 * OPERAND_VALUES + lane * 8;
     const unsigned short *const b = args.terms + ib * nch * 3 * OPERAND_VALUES + lane * 8;
     const int64_t i = ib * 32 + (lane & 31);
@@ -486,7 +487,9 @@ __global__ __launch_bounds__(256) void gradient_terms_kernel(GradArgs args, int6
 // Left without samples, by each wave once it had seen too many, a row was found
 // after other waves had done their work on it: 12000 x 128 with one dominant
 // direction 5.15 ms, in 8 clusters that lie in order 4.20, with the samples 3.24
-// and 3.22, the sweep 3.20.
+// and 3.22, the sweep 3.20.  Of the samples on the diagonal more than a quarter may
+// not hold more than 400 near pairs: in groups of 12 and 32 rows that lie in order
+// 3000 x 64 took 0.178 and 0.41 ms here, 0.175 in the sweep.
 template <int NC>
 __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
 {
@@ -506,9 +509,9 @@ __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
     const int64_t jb0 = (int64_t)blockIdx.y * args.jblocks;
     const int64_t jb1 = jb0 + args.jblocks < nblk ? jb0 + args.jblocks : nblk;
     {
-        // many near pairs, or clusters in order: all rows are left
+        // many near pairs, or groups of near points in order: all rows are left
         const int v = gradient_samples(args.left)[tid];
-        const int ordered = __syncthreads_count((tid & 1) && v > 256);
+        const int ordered = __syncthreads_count((tid & 1) && v > 400);
         int sum = tid & 1 ? 0 : v;
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
@@ -701,7 +704,7 @@ __global__ __launch_bounds__(GW * 64, 2) void gradient_kernel(GradArgs args)
             }
             __builtin_amdgcn_wave_barrier();
             seen_near += near;
-            if (seen >= 1 && seen_near > (seen + 1) * GRAD_NEAR_MAX) {
+            if (seen_near > (seen < 1 ? 2 : seen + 1) * GRAD_NEAR_MAX) {
                 // points in a few clusters: differences throughout are cheaper
                 bad = idle = true;
                 continue;

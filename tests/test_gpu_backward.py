@@ -357,3 +357,37 @@ def test_gradient_error_with_dominant_directions():
 
     ours, theirs = worst_row(dx), worst_row(sweep)
     assert ours <= 1.8 * theirs, (ours, theirs)
+
+
+@pytest.mark.parametrize("rows", [16, 32, 64])
+def test_gradient_of_near_points_in_order_costs_the_sweep(rows):
+    """Groups of near points next to each other (only the blocks on the diagonal
+    hold near pairs, up to all of theirs): left to the sweep as a whole."""
+    import os
+    n, k = 3000, 64
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    at = torch.arange(n, device="cuda") // rows
+    x = 1e-2 * torch.randn((n, k), generator=gen, device="cuda") + torch.randn((n // rows + 1, k), generator=gen, device="cuda")[at]
+    g = torch.randn(n * (n - 1) // 2, generator=gen, device="cuda")
+    print("case gradient of groups of %d in order" % rows, flush=True)
+
+    def timed():
+        times = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(8):
+                dx = gt.dist_backward(x, g)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        return dx, min(times)
+
+    dx, usual = timed()
+    os.environ["GT_FAIL_ALLOC_ABOVE"] = "13000000"   # the sweep's 12.3 MB, not the operands beside it
+    try:
+        want, sweep = timed()
+    finally:
+        del os.environ["GT_FAIL_ALLOC_ABOVE"]
+    assert torch.equal(dx, want)
+    assert usual <= 1.5 * sweep, (usual, sweep)      # 1.15; 1.3 (16 rows) and 2.3 (32) with samples beside the diagonal
