@@ -923,11 +923,16 @@ int gt_ttest(const float *pairs, const float *corr, int64_t n, float *ts, void *
     return GT_OK;
 }
 
+// The planes are moved 16 bytes at a time, straight into LDS too: a workspace
+// that begins elsewhere is used from its next such address on.
+static constexpr size_t KENDALL_WS_ALIGN = 16;
+
 int gt_kendall_workspace_size(int64_t na, int64_t nb, int64_t n, int same, size_t *bytes)
 {
     if (bytes == nullptr) return fail(GT_ERR_INVALID, "null bytes pointer");
     if (na < 0 || nb < 0 || n < 0) return fail(GT_ERR_INVALID, "negative size");
     *bytes = gt::kendall_workspace_bytes(na, same ? na : nb, same != 0, n);
+    if (*bytes > 0) *bytes += KENDALL_WS_ALIGN;
     return GT_OK;
 }
 
@@ -943,11 +948,13 @@ int gt_kendall(const float *a, int64_t na, int64_t lda, const float *b, int64_t 
     }
     int s = check_kendall_args(a, na, lda, b, nb, ldb, n, tau, ldt);
     if (s != GT_OK) return s;
+    const uintptr_t at = reinterpret_cast<uintptr_t>(workspace);
     const size_t need = gt::kendall_workspace_bytes(na, nb, same, n);
-    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
-        return fail(GT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need,
+    const size_t skip = round_up(at, KENDALL_WS_ALIGN) - at;
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need + skip))
+        return fail(GT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need + skip,
                     workspace_bytes);
-    GT_HIP(gt::launch_kendall(a, na, lda, b, nb, ldb, same, n, tau, ldt, workspace,
+    GT_HIP(gt::launch_kendall(a, na, lda, b, nb, ldb, same, n, tau, ldt, static_cast<char *>(workspace) + skip,
                               static_cast<hipStream_t>(stream)));
     return GT_OK;
 }

@@ -386,7 +386,8 @@ int gt_ttest(const float *pairs, const float *corr, int64_t n, float *ts, void *
  * / FP64 steps (inst/cuda/kendall.cu:40-45).  b == NULL (or b == a with the
  * same shape) is the self case.  The workspace (gt_kendall_workspace_size)
  * holds bit planes of the sample pairs (a segment of them at a time, within
- * three bits per pair and variable or 64 MiB), flags, and the counts. */
+ * three bits per pair and variable or 64 MiB), flags, and the counts; it may
+ * begin at any address (16 bytes of it are for the planes' alignment). */
 int gt_kendall_workspace_size(int64_t na, int64_t nb, int64_t n, int same, size_t *bytes);
 int gt_kendall(const float *a, int64_t na, int64_t lda, const float *b, int64_t nb, int64_t ldb,
                int64_t n, double *tau, int64_t ldt, void *workspace, size_t workspace_bytes,

@@ -285,3 +285,22 @@ def test_kendall_self_last_tile(na):
 def test_kendall_few_samples(n, kind):
     """One tile of fewer than 32 columns, compared eight at a time."""
     test_kendall_few_variables_with_ties(70, 33, n, kind)
+
+
+@pytest.mark.parametrize("offset", [0, 8, 16, 24])
+def test_kendall_workspace_at_any_eight_bytes(offset):
+    """The planes move 16 bytes at a time; a workspace that begins elsewhere is
+    used from its next 16 bytes on, within the size that was asked for."""
+    import ctypes
+    rng = np.random.default_rng(offset)
+    x = np.round(rng.standard_normal((70, 90)) * 3).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    need = ctypes.c_size_t()
+    assert gt.lib().gt_kendall_workspace_size(70, 70, 90, 1, ctypes.byref(need)) == 0
+    buf = torch.full((need.value + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    assert buf.data_ptr() % 16 == 0
+    print("case kendall workspace at +%d" % offset, flush=True)
+    got = gt.kendall(xd, workspace=buf[offset:offset + need.value])
+    assert torch.equal(got, gt.kendall(xd))
+    torch.cuda.synchronize()
+    assert (buf[:offset] == 0x5A).all() and (buf[offset + need.value:] == 0x5A).all()
